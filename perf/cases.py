@@ -19,7 +19,7 @@ import sys
 
 import torch
 
-sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cogni-ml_amd"))
+sys.path.insert(0, os.path.join(os.getcwd(), "cogni-ml_amd"))   # the working folder is the root of the tree that is timed
 
 from cogni_ml_amd import hip, quant  # noqa: E402
 from cogni_ml_amd.ffn_sequence import FFNSequenceRunner  # noqa: E402
