@@ -4,6 +4,7 @@
 #include "kernels/dequant.hpp"
 #include "kernels/gemv.hpp"
 #include "kernels/gemv_plain.hpp"
+#include "kernels/gemm_terms.hpp"
 #include "kernels/gemv_mfma.hpp"
 #include "kernels/gemv_mfma_q6k.hpp"
 #include "kernels/gemv_mt.hpp"

@@ -312,6 +312,45 @@ static inline GEMV_HD bool gemm_tile_of(unsigned id, unsigned mtiles, unsigned n
   return b < nb && *nt < ntiles && *mt < mtiles;
 }
 
+// ---- several tokens of F32, F16, IQ4_NL or Q8_0 weights (gemm_terms.hpp): eight wavefronts = eight k-slices per tile.
+// Workgroups go to the XCDs round-robin: the token tiles of one row of weight tiles follow each other on one XCD, so that
+// its L2 fetches the weights once.
+#define GEMM_TERMS_WAVES 8
+static inline GEMV_HD void gemm_terms_tile(unsigned id, unsigned mtiles, unsigned* mt, unsigned* nt) {
+  const unsigned x = id % GEMM_XCD_COUNT, l = id / GEMM_XCD_COUNT;
+  *mt = l % mtiles;
+  *nt = (l / mtiles) * GEMM_XCD_COUNT + x;
+}
+// Which calls take these kernels. F16 and F32: the row kernels re-read a row per four tokens and are level for the first few
+// of a short row (F16, us, row kernel | tile: 512 -> 512 at 4 tokens 3.3 | 3.5, at 8 4.6 | 3.5; 2048 -> 2048 at 2 tokens
+// 6.2 | 6.3, at 3 7.5 | 6.4; 4096 -> 4096 at 2 13.5 | 10.0). IQ4_NL: always (one token of 1024 -> 3584 11.6 | 4.4). Q8_0: what
+// the one-pass kernels leave - more than eight tokens (9 of 1024 -> 3584: 9.6 | 4.6), and rows that are no multiple of 256 from
+// three (4000 -> 4096 at 2 tokens 10.0 | 9.1, at 3 12.3 | 9.1; 1000 -> 2041 at 2 4.5 | 4.7, at 3 5.3 | 4.7).
+#define GEMM_TERMS_Q80_FROM 3u
+static inline int gemm_terms_take(unsigned type, unsigned tokens, unsigned in_dim) {
+  if (type == 20) return 1;
+  if (type == 0 || type == 1) return tokens >= 5u || (tokens >= 3u && tokens * (unsigned long long)in_dim >= 4096u) || (tokens == 2u && in_dim >= 4096u);
+  if (type != 8) return 0;
+  return tokens > 8u || (tokens >= GEMM_TERMS_Q80_FROM && ((in_dim & 255u) != 0 || in_dim > GEMV_MT_MAX_IN_DIM));
+}
+// The tile (16 tm tokens x 16 tn rows) that takes the least time when the launch runs in rounds of 256 workgroups: a round
+// of 1 x 1 tiles is the unit, the others measured against it (4096 columns of Q8_0, one round each: 6.4 / 8.8 / 13.9 / 21.2 /
+// 34.6 us above an empty launch).
+static inline unsigned gemm_terms_plan(unsigned tokens, unsigned out_dim, unsigned* tm, unsigned* tn) {
+  static const unsigned shape[5][3] = {{1, 1, 100}, {1, 2, 140}, {2, 2, 220}, {2, 4, 335}, {4, 4, 545}};
+  unsigned best = 0;
+  unsigned long long cost = ~0ull;
+  for (unsigned i = 0; i < 5; i++) {
+    const unsigned long long mt = (tokens + 16ull * shape[i][0] - 1) / (16ull * shape[i][0]), nt = (out_dim + 16ull * shape[i][1] - 1) / (16ull * shape[i][1]);
+    const unsigned long long c = ((mt * nt + 255ull) / 256ull) * shape[i][2];
+    if (c < cost) cost = c, best = i;
+  }
+  *tm = shape[best][0];
+  *tn = shape[best][1];
+  const unsigned mt = (tokens + 16 * *tm - 1) / (16 * *tm), nt = (out_dim + 16 * *tn - 1) / (16 * *tn);
+  return mt * ((nt + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT) * GEMM_XCD_COUNT;
+}
+
 // ---- one-pass kernel, rows above 4096 values: what a streamed unit waits for (gemv_mt.hpp)
 // vmcnt value that says "operand set i and unit i of a streamed row group have landed" (T = 1, S super-blocks per
 // k-slice, NSLOT units in LDS). Issue order: set 0, unit 0, set 1, unit 1, units 2 .. min(S, NSLOT) - 1 up front; behind unit

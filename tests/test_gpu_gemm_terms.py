@@ -1,0 +1,48 @@
+"""Several tokens of F32, F16, IQ4_NL and Q8_0 weights on the matrix cores (activations as three bfloat16 terms): fp32 precision
+at every tile shape and remainder, against the oracle."""
+import numpy as np
+import pytest
+
+from cogni_ml_amd import quant, synth
+from gpu_common import DevArray, gpu  # noqa: F401
+from helpers import F16, F32, IQ4_NL, Q8_0
+
+pytestmark = pytest.mark.gpu
+
+# (in_dim, out_dim, tokens): every tile (1x1, 1x2, 2x2, 2x4, 4x4 sixteens), one more and one less than a tile, a row that ends
+# inside a step of 32 (only F32 and F16 have such rows of any length; the block formats clip their last block), fewer steps than
+# wavefronts, one row, one token (IQ4_NL)
+CASES = [(96, 40, 9), (1024, 3584, 17), (1056, 4111, 33), (544, 2064, 64), (288, 4097, 129), (512, 4096, 200), (32, 1, 16),
+         (4128, 17, 15), (1000, 33, 31), (70, 5, 65), (5, 3, 6), (2048, 300, 1), (2048, 300, 3)]
+
+
+@pytest.mark.parametrize("t", [F32, F16, IQ4_NL, Q8_0])
+@pytest.mark.parametrize("in_dim,out_dim,tokens", CASES)
+def test_terms_kernels_match_the_oracle(gpu, oracle, t, in_dim, out_dim, tokens):
+    rng = np.random.default_rng(t * 7919 + in_dim * 13 + out_dim * 7 + tokens)
+    raw = synth.make_weights(rng, t, out_dim, in_dim)
+    x = synth.make_activations(rng, tokens, in_dim)
+    x[:: 7] *= np.float32(1e-6)
+    x[3:: 11] *= np.float32(1e5)                       # terms of very different size in one sum
+    res = rng.standard_normal(tokens * out_dim).astype(np.float32)
+    print("case type=%d in_dim=%d out_dim=%d tokens=%d" % (t, in_dim, out_dim, tokens), flush=True)
+    want = oracle.matmul_add(x, tokens, in_dim, raw, t, out_dim, np.zeros(out_dim, dtype=np.float32), threads=16)
+    row = raw.size // out_dim
+    dense = np.stack([oracle.dequantize(raw[r * row:(r + 1) * row], t, in_dim) for r in range(out_dim)]).astype(np.float64)
+    mags = np.abs(x.reshape(tokens, in_dim).astype(np.float64)) @ np.abs(dense).T
+    # the term products left out are below 3 * 2^-24 of a product; a sum goes through at most 32 + 2 roundings inside a step of
+    # 32, one per step of a k-slice (an eighth of them), eight for the slices and one for the block scale; the oracle's own
+    # result is rounded once
+    bound = (3 + 34 + (in_dim / 32) / 8 + 1 + 8 + 1 + 1) * 2.0 ** -24 * mags.reshape(-1) + 1e-37
+    w, xd, od, rd = DevArray(raw), DevArray(x), DevArray(np.full(tokens * out_dim, np.nan, dtype=np.float32)), DevArray(res)
+    try:
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim)
+        err = np.abs(got.astype(np.float64) - want)
+        assert np.all(err <= bound), (err - bound).max()
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens, rd.ptr)
+        assert np.array_equal(od.read(np.float32, tokens * out_dim), got + res)
+        assert quant.gemv_passes(t, tokens, in_dim, out_dim) == 1 or (t == Q8_0 and tokens <= 8)
+    finally:
+        for a in (w, xd, od, rd):
+            a.close()
