@@ -2,7 +2,7 @@
 
 The HIP counterpart of the reference's QwenOutputHeadRunner (src/ml/cuda/qwen_output_head_runner.cr:6-7, 659-760; launches
 :937-940): the default decode-facing path reads back only the top-1 id and value per token; the full logits are read
-only on request (read_logits), through the plain GEMV. Groups of up to eight tokens share one pass over the weights.
+only on request (read_logits), from the same pass over the weights. Groups of up to eight tokens share one pass.
 """
 import numpy as np
 
@@ -75,19 +75,21 @@ class QwenOutputHeadRunner:
         st = hip.current_stream_handle()
         h, t = self.hidden, self.weights.output_type
         normed = self._normed.ptr + 4 * tok0 * h
-        if self._from and count >= self._from:
-            quant.rmsnorm_pack_dev(self._x.ptr + 4 * tok0 * h, self._norm.ptr, normed if self._logits is not None else 0, t,
-                                   self._image.ptr, h, count, self.eps, st)
-            quant.gemv_packed_top1_dev(self._w.ptr, t, self._image.ptr, self._partial_ids.ptr + 4 * tok0 * self._stride,
-                                       self._partial_values.ptr + 4 * tok0 * self._stride, self._top1_ids.ptr + 4 * tok0,
-                                       self._top1_values.ptr + 4 * tok0, h, self.vocab, count, st)
+        lg = self._logits.ptr + 4 * tok0 * self.vocab if self._logits is not None else 0   # stored by the pass that finds the top-1
+        packed = self._from and count >= self._from
+        if packed:
+            quant.rmsnorm_pack_dev(self._x.ptr + 4 * tok0 * h, self._norm.ptr, 0, t, self._image.ptr, h, count, self.eps, st)
         else:
             quant.rmsnorm_dev(self._x.ptr + 4 * tok0 * h, self._norm.ptr, normed, h, count, self.eps, st)
-            quant.gemv_top1_dev(self._w.ptr, t, normed, self._partial_ids.ptr + 4 * tok0 * self._stride,
-                                self._partial_values.ptr + 4 * tok0 * self._stride, self._top1_ids.ptr + 4 * tok0,
-                                self._top1_values.ptr + 4 * tok0, h, self.vocab, count, st)
-        if self._logits is not None:
-            quant.gemv_dev(self._w.ptr, t, normed, self._logits.ptr + 4 * tok0 * self.vocab, h, self.vocab, count, 0, st)
+        src = self._image.ptr if packed else normed
+        out = (self._partial_ids.ptr + 4 * tok0 * self._stride, self._partial_values.ptr + 4 * tok0 * self._stride,
+               self._top1_ids.ptr + 4 * tok0, self._top1_values.ptr + 4 * tok0)
+        if lg:
+            top1 = quant.gemv_packed_top1_logits_dev if packed else quant.gemv_top1_logits_dev
+            top1(self._w.ptr, t, src, *out, lg, h, self.vocab, count, st)
+        else:
+            top1 = quant.gemv_packed_top1_dev if packed else quant.gemv_top1_dev
+            top1(self._w.ptr, t, src, *out, h, self.vocab, count, st)
 
     def _run_token(self, tok):
         self._launch(tok, 1)

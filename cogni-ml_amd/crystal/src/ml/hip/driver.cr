@@ -106,6 +106,12 @@ lib LibCogniHIP
   fun cogni_gemv_top1_dev(w_raw : UInt64, w_type : UInt32, x : UInt64, partial_ids : UInt64, partial_values : UInt64,
                           top1_ids : UInt64, top1_values : UInt64, in_dim : UInt32, out_dim : UInt32, tokens : UInt32,
                           stream : Void*) : Int32
+  fun cogni_gemv_top1_logits_dev(w_raw : UInt64, w_type : UInt32, x : UInt64, partial_ids : UInt64, partial_values : UInt64,
+                                 top1_ids : UInt64, top1_values : UInt64, logits : UInt64, in_dim : UInt32, out_dim : UInt32,
+                                 tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemv_packed_top1_logits_dev(w_raw : UInt64, w_type : UInt32, image : UInt64, partial_ids : UInt64,
+                                        partial_values : UInt64, top1_ids : UInt64, top1_values : UInt64, logits : UInt64,
+                                        in_dim : UInt32, out_dim : UInt32, tokens : UInt32, stream : Void*) : Int32
   fun cogni_gemm_workspace_bytes(w_type : UInt32, in_dim : UInt32, tokens : UInt32) : LibC::SizeT
   fun cogni_gemm_workspace_bytes_split(w_type : UInt32, in_dim : UInt32, out_dim : UInt32, tokens : UInt32) : LibC::SizeT
   fun cogni_gemm_dev(w_raw : UInt64, w_type : UInt32, x : UInt64, bias : UInt64, out : UInt64,

@@ -877,14 +877,28 @@ uint32_t cogni_gemv_top1_partials(uint32_t w_type, uint32_t out_dim) {
   return most;
 }
 
-int cogni_gemv_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t partial_ids, uint64_t partial_values,
-                        uint64_t top1_ids, uint64_t top1_values, uint32_t in_dim, uint32_t out_dim, uint32_t tokens,
-                        void* stream) {
+static int top1_packed_launch(uint64_t w_raw, uint32_t w_type, uint64_t image, uint64_t partial_ids, uint64_t partial_values, uint64_t logits,
+                              uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream) {
+  const bool q6 = w_type == COGNI_TYPE_Q6_K;
+  const uint32_t grid = gemv_mt_grid(w_type, in_dim, out_dim), lds = gemv_mt_lds_bytes(w_type);
+  if (logits) {
+    void* params[] = {&w_raw, &image, &partial_ids, &partial_values, &logits, &in_dim, &out_dim, &tokens};
+    return launch(q6 ? "q6_k_gemv_mt_top1_logits_partial_f32" : "q4_k_gemv_mt_top1_logits_partial_f32", grid, GEMV_MT_WAVES * 64, lds, params, stream);
+  }
+  void* params[] = {&w_raw, &image, &partial_ids, &partial_values, &in_dim, &out_dim, &tokens};
+  return launch(q6 ? "q6_k_gemv_mt_top1_partial_f32" : "q4_k_gemv_mt_top1_partial_f32", grid, GEMV_MT_WAVES * 64, lds, params, stream);
+}
+
+// cogni_gemv_top1_dev, with the row values stored as well when `logits` is given: from the same launch where the kernel has
+// that form, else (three or four tokens of a row the one-pass kernel does not take that early) by cogni_gemv_dev in front of it.
+static int top1_launch(const char* who, uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t partial_ids, uint64_t partial_values,
+                       uint64_t top1_ids, uint64_t top1_values, uint64_t logits, uint32_t in_dim, uint32_t out_dim, uint32_t tokens,
+                       void* stream) {
   if (!gemv_type(w_type))
     return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for fused matmul: ") + type_name(w_type));
   if (!w_raw || !x || !partial_ids || !partial_values || !top1_ids || !top1_values)
-    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_top1_dev: null device pointer");
-  if (in_dim == 0 || out_dim == 0 || tokens == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_top1_dev: zero dimension");
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  if (in_dim == 0 || out_dim == 0 || tokens == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": zero dimension");
   if (k_quant(w_type) && (in_dim % 256) != 0)
     return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(type_name(w_type)) + " GEMV requires in_dim multiple of 256, got " + std::to_string(in_dim));
   const uint32_t cap = top1_token_cap(w_type), stride = cogni_gemv_top1_partials(w_type, out_dim);
@@ -897,7 +911,7 @@ int cogni_gemv_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t pa
     int rc = 0;
     // the group's partial results: [token in group][workgroup], inside the group's share of the caller's buffers
     uint64_t xm = x + (uint64_t)t0 * in_dim * 4, pi = partial_ids + (uint64_t)t0 * stride * 4, pv = partial_values + (uint64_t)t0 * stride * 4;
-    uint64_t oi = top1_ids + (uint64_t)t0 * 4, ov = top1_values + (uint64_t)t0 * 4;
+    uint64_t oi = top1_ids + (uint64_t)t0 * 4, ov = top1_values + (uint64_t)t0 * 4, lg = logits ? logits + (uint64_t)t0 * out_dim * 4 : 0;
     // up to eight tokens of a Q4_K or Q6_K matrix the one-pass kernel takes, from the token count at which pack + one
     // pass is the faster way to the logits: the weights once for the whole group, the arg-max inside
     const uint32_t from = (w_type == COGNI_TYPE_Q4_K || w_type == COGNI_TYPE_Q6_K) ? gemv_mt_from(w_type, in_dim, out_dim) : 0;
@@ -908,9 +922,7 @@ int cogni_gemv_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t pa
         grid = gemv_mt_grid(w_type, in_dim, out_dim);
         rc = cogni_gemv_pack_dev(xm, w_type, in_dim, m, image, stream);
         if (rc != 0) return rc;
-        void* params[] = {&w_raw, &image, &pi, &pv, &in_dim, &out_dim, &m};
-        rc = launch(w_type == COGNI_TYPE_Q6_K ? "q6_k_gemv_mt_top1_partial_f32" : "q4_k_gemv_mt_top1_partial_f32", grid,
-                    GEMV_MT_WAVES * 64, gemv_mt_lds_bytes(w_type), params, stream);
+        rc = top1_packed_launch(w_raw, w_type, image, pi, pv, lg, in_dim, out_dim, m, stream);
         if (rc != 0) return rc;
         void* rparams[] = {&pi, &pv, &oi, &ov, &grid};
         rc = launch("top1_reduce_f32", m, 1024, 0, rparams, stream);
@@ -928,14 +940,20 @@ int cogni_gemv_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t pa
       block = GEMV_MFMA_WAVES * 64;
       shmem = gemv_mfma_lds_bytes(w_type, (int)m, in_dim);
       name = std::string(type_prefix(w_type)) + "_gemv_mfma_top1_partial_f32_tbatch" + std::to_string(m);
+      if (lg) {
+        rc = cogni_gemv_dev(w_raw, w_type, xm, 0, lg, in_dim, out_dim, m, stream);
+        if (rc != 0) return rc;
+        lg = 0;
+      }
     } else {
       rc = cogni_gemv_launch_dims(w_type, m, in_dim, out_dim, &grid, &block, &shmem);
       if (rc != 0) return rc;
-      name = std::string(type_prefix(w_type)) + "_gemv_top1_partial_f32";
+      name = std::string(type_prefix(w_type)) + (lg ? "_gemv_top1_logits_partial_f32" : "_gemv_top1_partial_f32");
       if (m > 1) name += "_tbatch" + std::to_string(m);
     }
     void* params[] = {&w_raw, &xm, &pi, &pv, &in_dim, &out_dim};
-    rc = launch(name.c_str(), grid, block, shmem, params, stream);
+    void* lparams[] = {&w_raw, &xm, &pi, &pv, &lg, &in_dim, &out_dim};
+    rc = launch(name.c_str(), grid, block, shmem, lg ? lparams : params, stream);
     if (rc != 0) return rc;
     void* rparams[] = {&pi, &pv, &oi, &ov, &grid};
     rc = launch("top1_reduce_f32", m, 1024, 0, rparams, stream);
@@ -944,24 +962,52 @@ int cogni_gemv_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t pa
   return 0;
 }
 
+int cogni_gemv_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t partial_ids, uint64_t partial_values,
+                        uint64_t top1_ids, uint64_t top1_values, uint32_t in_dim, uint32_t out_dim, uint32_t tokens,
+                        void* stream) {
+  return top1_launch("cogni_gemv_top1_dev", w_raw, w_type, x, partial_ids, partial_values, top1_ids, top1_values, 0, in_dim, out_dim, tokens,
+                     stream);
+}
+
+int cogni_gemv_top1_logits_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t partial_ids, uint64_t partial_values,
+                               uint64_t top1_ids, uint64_t top1_values, uint64_t logits, uint32_t in_dim, uint32_t out_dim,
+                               uint32_t tokens, void* stream) {
+  if (!logits) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_top1_logits_dev: null device pointer");
+  return top1_launch("cogni_gemv_top1_logits_dev", w_raw, w_type, x, partial_ids, partial_values, top1_ids, top1_values, logits, in_dim,
+                     out_dim, tokens, stream);
+}
+
+// Top-1 against a packed image; `logits` may be 0.
+static int top1_packed(const char* who, uint64_t w_raw, uint32_t w_type, uint64_t image, uint64_t partial_ids, uint64_t partial_values,
+                       uint64_t top1_ids, uint64_t top1_values, uint64_t logits, uint32_t in_dim, uint32_t out_dim, uint32_t tokens,
+                       void* stream) {
+  if (!w_raw || !image || !partial_ids || !partial_values || !top1_ids || !top1_values)
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  if (out_dim == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": zero dimension");
+  if ((w_type != COGNI_TYPE_Q4_K && w_type != COGNI_TYPE_Q6_K) || tokens == 0 || tokens > (uint32_t)GEMV_MT_MAX_TOKENS ||
+      !gemv_mt_supported(w_type, 2, in_dim))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": no one-pass top-1 kernel for this type, token count and in_dim");
+  uint32_t grid = gemv_mt_grid(w_type, in_dim, out_dim);
+  if (grid > cogni_gemv_top1_partials(w_type, out_dim))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": the partial buffers are sized by cogni_gemv_top1_partials");
+  if (int rc = top1_packed_launch(w_raw, w_type, image, partial_ids, partial_values, logits, in_dim, out_dim, tokens, stream)) return rc;
+  void* rparams[] = {&partial_ids, &partial_values, &top1_ids, &top1_values, &grid};
+  return launch("top1_reduce_f32", tokens, 1024, 0, rparams, stream);
+}
+
 int cogni_gemv_packed_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t image, uint64_t partial_ids, uint64_t partial_values,
                                uint64_t top1_ids, uint64_t top1_values, uint32_t in_dim, uint32_t out_dim, uint32_t tokens,
                                void* stream) {
-  if (!w_raw || !image || !partial_ids || !partial_values || !top1_ids || !top1_values)
-    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_top1_dev: null device pointer");
-  if (out_dim == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_top1_dev: zero dimension");
-  if ((w_type != COGNI_TYPE_Q4_K && w_type != COGNI_TYPE_Q6_K) || tokens == 0 || tokens > (uint32_t)GEMV_MT_MAX_TOKENS ||
-      !gemv_mt_supported(w_type, 2, in_dim))
-    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_top1_dev: no one-pass top-1 kernel for this type, token count and in_dim");
-  uint32_t grid = gemv_mt_grid(w_type, in_dim, out_dim);
-  if (grid > cogni_gemv_top1_partials(w_type, out_dim))
-    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_top1_dev: the partial buffers are sized by cogni_gemv_top1_partials");
-  void* params[] = {&w_raw, &image, &partial_ids, &partial_values, &in_dim, &out_dim, &tokens};
-  int rc = launch(w_type == COGNI_TYPE_Q6_K ? "q6_k_gemv_mt_top1_partial_f32" : "q4_k_gemv_mt_top1_partial_f32", grid,
-                  GEMV_MT_WAVES * 64, gemv_mt_lds_bytes(w_type), params, stream);
-  if (rc != 0) return rc;
-  void* rparams[] = {&partial_ids, &partial_values, &top1_ids, &top1_values, &grid};
-  return launch("top1_reduce_f32", tokens, 1024, 0, rparams, stream);
+  return top1_packed("cogni_gemv_packed_top1_dev", w_raw, w_type, image, partial_ids, partial_values, top1_ids, top1_values, 0, in_dim,
+                     out_dim, tokens, stream);
+}
+
+int cogni_gemv_packed_top1_logits_dev(uint64_t w_raw, uint32_t w_type, uint64_t image, uint64_t partial_ids, uint64_t partial_values,
+                                      uint64_t top1_ids, uint64_t top1_values, uint64_t logits, uint32_t in_dim, uint32_t out_dim,
+                                      uint32_t tokens, void* stream) {
+  if (!logits) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_top1_logits_dev: null device pointer");
+  return top1_packed("cogni_gemv_packed_top1_logits_dev", w_raw, w_type, image, partial_ids, partial_values, top1_ids, top1_values, logits,
+                     in_dim, out_dim, tokens, stream);
 }
 
 int cogni_rmsnorm_dev(uint64_t x, uint64_t norm, uint64_t out, uint32_t dim, uint32_t tokens, float eps, void* stream) {

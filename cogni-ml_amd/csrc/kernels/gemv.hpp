@@ -42,7 +42,9 @@
 // (bin/cuda_ffn_sequence_probe.cr:46-84) in one launch.
 // TOP1: instead of the row values the workgroup stores, per token, the largest of its rows and that row's index
 // (out[m * gridDim.x + blockIdx.x], top_ids[same]); of equal values the lowest row wins. The reference's
-// q6_k_gemv_top1_partial_f32 (src/ml/cuda/kernels/q6k_gemv_probe.ptx:1331-1580) for the output head.
+// q6_k_gemv_top1_partial_f32 (src/ml/cuda/kernels/q6k_gemv_probe.ptx:1331-1580) for the output head. With `logits` the row
+// values are stored there as well (logits[m * out_dim + row], the bits of the plain kernel), so that a head that wants both
+// reads its weights once: the Q6_K 151936 x 4096 head with norm and reduce, one token, 190 us as two passes, 103 as one.
 // LIST (with DUAL, M = 1): up to three matrices of one row length and any row counts as one matrix of all their rows
 // (q | k | v of a decoder layer: the reference's qmatvec_many seam, src/ml/gguf/qwen35_cpu.cr:1419-1445); `list` names
 // them, w / w_b / out / out_b / out_dim are not used.
@@ -58,7 +60,7 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
                                           const float* __restrict__ residual, float* __restrict__ out,
                                           u32 in_dim, u32 out_dim, const uint8_t* __restrict__ w_b = nullptr,
                                           float* __restrict__ out_b = nullptr, u32* __restrict__ top_ids = nullptr,
-                                          const GemvList* list = nullptr) {
+                                          const GemvList* list = nullptr, float* __restrict__ logits = nullptr) {
   constexpr int R = RO ? RO : F::rows(M);
   constexpr int MG = M < F::MG_MAX ? M : F::MG_MAX;   // tokens held in registers at a time
   constexpr int NG = (M + MG - 1) / MG;
@@ -286,6 +288,7 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
         for (int r = 0; r < R; r++) {
           const float v = wave_sum(acc[r][m]);
           if (row0 + r < out_dim && v > top_best[m]) top_best[m] = v, top_best_id[m] = row0 + r;   // rows ascend
+          if (logits && lane == 0 && row0 + r < out_dim) logits[(size_t)m * out_dim + row0 + r] = v;
         }
       }
     } else {
@@ -564,6 +567,13 @@ __device__ __forceinline__ void gemv_entry(const uint8_t* w, const float* x, con
     gemv_core<FMT, M, false, false, false, true>(w, x, nullptr, partial_values, in_dim, out_dim, nullptr, nullptr, \
                                                  partial_ids);                                                   \
   }
+// the same with the row values stored as well: (w_raw, x, partial_ids, partial_values, logits, in_dim, out_dim)
+#define GEMV_TOP1_LOGITS_ENTRY(NAME, FMT, M)                                                                     \
+  extern "C" __global__ __launch_bounds__(GEMV_BLOCK) GEMV_OCC(M) void NAME(const uint8_t* w, const float* x, u32* partial_ids, \
+                                                                 float* partial_values, float* logits, u32 in_dim, u32 out_dim) { \
+    gemv_core<FMT, M, false, false, false, true>(w, x, nullptr, partial_values, in_dim, out_dim, nullptr, nullptr, \
+                                                 partial_ids, nullptr, logits);                                  \
+  }
 
 typedef FmtK45<false> FmtQ4K;
 typedef FmtK45<true> FmtQ5K;
@@ -596,6 +606,12 @@ GEMV_TOP1_ENTRY(q6_k_gemv_top1_partial_f32, FmtQ6K, 1)
 GEMV_TOP1_ENTRY(q6_k_gemv_top1_partial_f32_tbatch2, FmtQ6K, 2)
 GEMV_TOP1_ENTRY(q6_k_gemv_top1_partial_f32_tbatch3, FmtQ6K, 3)
 GEMV_TOP1_ENTRY(q8_0_gemv_top1_partial_f32, FmtQ80, 1)
+GEMV_TOP1_LOGITS_ENTRY(q4_k_gemv_top1_logits_partial_f32, FmtQ4K, 1)
+GEMV_TOP1_LOGITS_ENTRY(q4_k_gemv_top1_logits_partial_f32_tbatch2, FmtQ4K, 2)
+GEMV_TOP1_LOGITS_ENTRY(q5_k_gemv_top1_logits_partial_f32, FmtQ5K, 1)
+GEMV_TOP1_LOGITS_ENTRY(q6_k_gemv_top1_logits_partial_f32, FmtQ6K, 1)
+GEMV_TOP1_LOGITS_ENTRY(q6_k_gemv_top1_logits_partial_f32_tbatch2, FmtQ6K, 2)
+GEMV_TOP1_LOGITS_ENTRY(q8_0_gemv_top1_logits_partial_f32, FmtQ80, 1)
 
 // (partial_ids, partial_values, out_ids, out_values, count): the largest of `count` partial values and its id, per
 // token (grid.x = tokens; partial_* + token * count, out_* + token). Of equal values the lowest id wins, which is

@@ -620,11 +620,12 @@ struct MtArgs {
 // swiglu_f32): the values of the pair launch followed by swiglu_f32, bit for bit, without the gate and up vectors in memory.
 // TOP1 (one matrix): instead of the row values the workgroup stores, per token, the largest of the rows it walked and
 // that row's index (out[0][m * gridDim.x + blockIdx.x], top_ids[same]; of equal values the lowest row wins): the partial
-// results top1_reduce_f32 finishes, as q6_k_gemv_top1_partial_f32 writes them for one token.
+// results top1_reduce_f32 finishes, as q6_k_gemv_top1_partial_f32 writes them for one token. With `logits` the row values are
+// stored as well (logits[m * rows + row]).
 template <class F, int SBW, int T, bool SWIGLU = false, bool TOP1 = false>
 __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __restrict__ image,
                                              const float* __restrict__ residual, u32 in_dim, u32 tokens,
-                                             u32* __restrict__ top_ids = nullptr) {
+                                             u32* __restrict__ top_ids = nullptr, float* __restrict__ logits = nullptr) {
   constexpr bool STREAM = SBW > 2;
   constexpr int NTOK = F::NTOK;   // token rows of the partial sums: 8, or 16 single-term tokens
   static_assert(NTOK == 8 || (NTOK == 16 && !TOP1), "sixteen tokens: rows or SwiGLU, no top-1");
@@ -760,6 +761,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
           // competes as minus infinity under the highest index)
           const bool real = row < a.rows[0];
           top1_take(top_v, top_i, real ? v : -__builtin_inff(), real ? row : 0xFFFFFFFFu);
+          if (logits && real) logits[(size_t)m * a.rows[0] + row] = v;
         } else if (row < a.rows[0]) {
           const size_t oi = (size_t)m * a.rows[0] + row;
           if (residual) v += residual[oi];
@@ -909,24 +911,24 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
 // constants. Shapes outside gemv_mt_supported() must not be launched.
 template <class F, bool TOP1 = false>
 __device__ __forceinline__ void gemv_mt_dispatch(const MtArgs& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens,
-                                                 u32* top_ids = nullptr) {
+                                                 u32* top_ids = nullptr, float* logits = nullptr) {
   const u32 ntiles = (a.rows[0] + a.rows[1] + a.rows[2] + 15) >> 4;
   const u32 t = gemv_mt_tiles(F::TYPE, in_dim, ntiles);
   switch (gemv_mt_padded_sb(in_dim) >> 3) {
     case 1:
-      if (t <= 1) gemv_mt_core<F, 1, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids);
-      else if (t == 2) gemv_mt_core<F, 1, 2, false, TOP1>(a, image, residual, in_dim, tokens, top_ids);
-      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 1, 3, false, TOP1>(a, image, residual, in_dim, tokens, top_ids);
+      if (t <= 1) gemv_mt_core<F, 1, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if (t == 2) gemv_mt_core<F, 1, 2, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 1, 3, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
       break;
     case 2:
-      if (t <= 1) gemv_mt_core<F, 2, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids);
-      else if (t == 2) gemv_mt_core<F, 2, 2, false, TOP1>(a, image, residual, in_dim, tokens, top_ids);
-      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 2, 3, false, TOP1>(a, image, residual, in_dim, tokens, top_ids);
+      if (t <= 1) gemv_mt_core<F, 2, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if (t == 2) gemv_mt_core<F, 2, 2, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 2, 3, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
       break;
-    case 3: gemv_mt_core<F, 3, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids); break;
-    case 4: gemv_mt_core<F, 4, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids); break;
-    case 5: gemv_mt_core<F, 5, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids); break;
-    default: gemv_mt_core<F, 6, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids); break;
+    case 3: gemv_mt_core<F, 3, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 4: gemv_mt_core<F, 4, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 5: gemv_mt_core<F, 5, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    default: gemv_mt_core<F, 6, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
   }
 }
 
@@ -953,19 +955,30 @@ GEMV_MT_ENTRY(q8_0_gemv_mt16_f32, MtQ80x16)
 // partial_*[token * gridDim.x + workgroup], finished by top1_reduce_f32 with count = gridDim.x. The one-token kernel's
 // parameter order (src/ml/cuda/kernels/q6k_gemv_probe.ptx:1331-1338) with the image in the place of x and the token count
 // behind.
+// The logits form (parameter `logits` behind partial_values) stores the row values as well.
+#define GEMV_MT_TOP1_BODY(FMT, LOGITS)                                                                                    \
+  /* the absent matrices' row counts: a zero the optimizer cannot see through (with literal zeros it folds the lookup */  \
+  /* of a row's matrix away, and this release of the compiler crashes in its control-flow simplification doing so)    */  \
+  u32 none;                                                                                                               \
+  asm volatile("s_mov_b32 %0, 0" : "=s"(none));                                                                           \
+  const MtArgs a = {{w, w, w}, {partial_values, partial_values, partial_values}, {out_dim, none, none}};                  \
+  gemv_mt_dispatch<FMT, true>(a, image, nullptr, in_dim, tokens, partial_ids, LOGITS);
 #define GEMV_MT_TOP1_ENTRY(NAME, FMT)                                                                                    \
   extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void NAME(const uint8_t* w, const uint8_t* image,          \
                                                                         u32* partial_ids, float* partial_values,         \
                                                                         u32 in_dim, u32 out_dim, u32 tokens) {           \
-    /* the absent matrices' row counts: a zero the optimizer cannot see through (with literal zeros it folds the lookup */ \
-    /* of a row's matrix away, and this release of the compiler crashes in its control-flow simplification doing so)    */ \
-    u32 none;                                                                                                            \
-    asm volatile("s_mov_b32 %0, 0" : "=s"(none));                                                                        \
-    const MtArgs a = {{w, w, w}, {partial_values, partial_values, partial_values}, {out_dim, none, none}};               \
-    gemv_mt_dispatch<FMT, true>(a, image, nullptr, in_dim, tokens, partial_ids);                                         \
+    GEMV_MT_TOP1_BODY(FMT, nullptr)                                                                                      \
+  }
+#define GEMV_MT_TOP1_LOGITS_ENTRY(NAME, FMT)                                                                             \
+  extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void NAME(const uint8_t* w, const uint8_t* image,          \
+                                                                        u32* partial_ids, float* partial_values,         \
+                                                                        float* logits, u32 in_dim, u32 out_dim, u32 tokens) { \
+    GEMV_MT_TOP1_BODY(FMT, logits)                                                                                       \
   }
 GEMV_MT_TOP1_ENTRY(q4_k_gemv_mt_top1_partial_f32, MtQ4K)
 GEMV_MT_TOP1_ENTRY(q6_k_gemv_mt_top1_partial_f32, MtQ6K)
+GEMV_MT_TOP1_LOGITS_ENTRY(q4_k_gemv_mt_top1_logits_partial_f32, MtQ4K)
+GEMV_MT_TOP1_LOGITS_ENTRY(q6_k_gemv_mt_top1_logits_partial_f32, MtQ6K)
 
 // (w_gate, w_up, image, out, in_dim, out_dim, tokens): out[m][o] = silu(gate . x) * (up . x); block 512, grid = min(256,
 // ceil(out_dim / 16)), dynamic shared memory as q4_k_gemv_mt_f32. The parameter list of q4_k_dual_gemv_swiglu_f32 with the

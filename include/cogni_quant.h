@@ -353,6 +353,17 @@ int cogni_gemv_packed_top1_dev(uint64_t w_raw, uint32_t w_type, uint64_t image, 
                                uint64_t top1_ids, uint64_t top1_values, uint32_t in_dim, uint32_t out_dim, uint32_t tokens,
                                void* stream);
 
+/* The two with the row values as well: logits[m*out_dim + o], the same sums the arg-max compares, from the same pass over the
+ * weights ("<prefix>_gemv_top1_logits_partial_f32[_tbatchM]" | "<prefix>_gemv_mt_top1_logits_partial_f32": parameter `logits`
+ * behind partial_values). Three or four tokens of a row that only the matrix-core kernel takes go through cogni_gemv_dev and
+ * then the top-1. */
+int cogni_gemv_top1_logits_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t partial_ids, uint64_t partial_values,
+                               uint64_t top1_ids, uint64_t top1_values, uint64_t logits, uint32_t in_dim, uint32_t out_dim,
+                               uint32_t tokens, void* stream);
+int cogni_gemv_packed_top1_logits_dev(uint64_t w_raw, uint32_t w_type, uint64_t image, uint64_t partial_ids, uint64_t partial_values,
+                                      uint64_t top1_ids, uint64_t top1_values, uint64_t logits, uint32_t in_dim, uint32_t out_dim,
+                                      uint32_t tokens, void* stream);
+
 /* cogni_gemv_top1_dev for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): the same launches and the same results, with the per-workgroup partial
  * results in a static device array inside the library instead of caller-owned buffers. No counterpart in the
