@@ -190,7 +190,11 @@ class QwenProjectionStackRunner:
             # every projection still to come of the same input, type and row length joins this launch (q | k | v | gate | up:
             # their input is this one's, so it exists already) - the prefill counterpart of the qmatvec_many seam
             grp = [e for e in ents[idx:] if e[0] not in done and (e[1], int(e[2]), e[4]) == (src, int(t), in_dim)][:6]
-            if len(grp) >= 2 and int(t) in list_types:
+            if quant.gemm_stream_takes(t, in_dim, sum(e[3] for e in grp), count):
+                quant.gemm_stream_dev([self._w[e[0]].ptr for e in grp], t, ws.ptr, nbytes, [self._act[e[0]].ptr for e in grp],
+                                      [e[3] for e in grp], in_dim, count, 0, stream)
+                done.update(e[0] for e in grp)
+            elif len(grp) >= 2 and int(t) in list_types:
                 quant.gemm_packed_many_dev([self._w[e[0]].ptr for e in grp], t, ws.ptr, nbytes, [self._act[e[0]].ptr for e in grp],
                                            [e[3] for e in grp], in_dim, count, stream)
                 done.update(e[0] for e in grp)

@@ -398,6 +398,32 @@ def gemm_packed_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, wor
         ctypes.c_size_t(next_workspace_bytes), ctypes.c_uint32(in_dim), ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
 
 
+def gemm_stream_takes(w_type, in_dim, rows, tokens):
+    """Whether the router and the runners take the short-prefill kernels for a launch of `rows` rows in all."""
+    return bool(hip.lib().cogni_gemm_stream_takes(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(in_dim), ctypes.c_uint32(rows),
+                                                  ctypes.c_uint32(tokens)))
+
+
+def gemm_stream_dev(w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, in_dim, tokens, residual_ptr=0, stream=None):
+    """One to six matrices of one type and row length against the same packed activations, weights streamed (short prefills)."""
+    n = len(w_ptrs)
+    if not (n == len(out_ptrs) == len(out_dims)):
+        raise ValueError("w_ptrs, out_ptrs and out_dims must have one entry per matrix")
+    _check(hip.lib().cogni_gemm_stream_dev((ctypes.c_uint64 * n)(*w_ptrs), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(workspace_ptr),
+                                           ctypes.c_size_t(workspace_bytes), ctypes.c_uint64(residual_ptr), (ctypes.c_uint64 * n)(*out_ptrs),
+                                           (ctypes.c_uint32 * n)(*out_dims), ctypes.c_uint32(n), ctypes.c_uint32(in_dim),
+                                           ctypes.c_uint32(tokens), stream))
+
+
+def gemm_stream_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, workspace_bytes, out_ptr, next_type, next_workspace_ptr,
+                                next_workspace_bytes, in_dim, out_dim, tokens, stream=None):
+    """gemm_packed_swiglu_pack_dev for short prefills (weights streamed)."""
+    _check(hip.lib().cogni_gemm_stream_swiglu_pack_dev(
+        ctypes.c_uint64(w_gate_ptr), ctypes.c_uint64(w_up_ptr), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(workspace_ptr),
+        ctypes.c_size_t(workspace_bytes), ctypes.c_uint64(out_ptr), ctypes.c_uint32(int(next_type)), ctypes.c_uint64(next_workspace_ptr),
+        ctypes.c_size_t(next_workspace_bytes), ctypes.c_uint32(in_dim), ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
+
+
 def matmul_dev(w_ptr, w_type, x_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr=0, workspace_bytes=0, bias_ptr=0,
                stream=None):
     """The GEMV/GEMM router (tokens > threshold and Q4_K -> GEMM)."""

@@ -1363,10 +1363,9 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
   return launch(names[w_type == COGNI_TYPE_Q5_K][m64][n128], gemm_grid_x(mtiles, end), 256, 0, params, stream);
 }
 
-int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
-                                      uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
-                                      uint32_t out_dim, uint32_t tokens, void* stream) {
-  const char* who = "cogni_gemm_packed_swiglu_pack_dev";
+static int swiglu_pack_check(const char* who, uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes,
+                             uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
+                             uint32_t tokens) {
   if (w_type != COGNI_TYPE_Q4_K)
     return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the fused gate/up SwiGLU GEMM: ") + type_name(w_type));
   if (!gemm_type(next_type))
@@ -1377,11 +1376,96 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
   if ((out_dim % 256) != 0) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": out_dim must be a multiple of 256");
   if (next_workspace_bytes < cogni_gemm_workspace_bytes(next_type, out_dim, tokens))
     return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": next_workspace too small (cogni_gemm_workspace_bytes)");
+  return 0;
+}
+
+int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
+                                      uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
+                                      uint32_t out_dim, uint32_t tokens, void* stream) {
+  if (int rc = swiglu_pack_check("cogni_gemm_packed_swiglu_pack_dev", w_gate, w_up, w_type, workspace, workspace_bytes, next_type, next_workspace,
+                                 next_workspace_bytes, in_dim, out_dim, tokens))
+    return rc;
   const uint32_t mtiles = (tokens + 127) / 128, ntiles = (out_dim + 95) / 96;
   void* params[] = {&w_gate, &w_up, &workspace, &out, &next_workspace, &in_dim, &out_dim, &tokens};
   static const char* const names[2][2] = {{"q4_k_gemm_swiglu_pack_q4k_f16", "q4_k_gemm_swiglu_pack_q4k_m64_f16"},
                                           {"q4_k_gemm_swiglu_pack_q6k_f16", "q4_k_gemm_swiglu_pack_q6k_m64_f16"}};
   return launch(names[next_type == COGNI_TYPE_Q6_K][tokens <= 64], gemm_grid_x(mtiles, ntiles), 256, 0, params, stream);
+}
+
+// Short prefills: the weights streamed through workgroups of four wavefronts (kernels/gemm_stream.hpp). The same packed
+// activations, planes and precision as the tile kernels above.
+static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t add,
+                              uint32_t add_stride, const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim,
+                              uint32_t tokens, void* stream) {
+  const size_t packed_bytes = cogni_gemm_workspace_bytes(w_type, in_dim, tokens);
+  if (packed_bytes > GEMM_STREAM_MAX_PACKED) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": packed activations of 2 GiB or more");
+  uint64_t rows = 0;
+  for (uint32_t i = 0; i < count; i++) rows += out_dims[i];
+  // planes that fit behind the packed activations (one matrix only)
+  uint32_t planes_max = 1;
+  if (count == 1) {
+    const size_t fit = (workspace_bytes - packed_bytes) / ((size_t)tokens * out_dims[0] * sizeof(float));
+    planes_max = fit < 2 ? 1u : (fit < GEMM_STREAM_MAX_SPLITS ? (uint32_t)fit : GEMM_STREAM_MAX_SPLITS);
+  }
+  const GemmStreamPlan p = gemm_stream_plan(w_type, tokens, in_dim, rows, planes_max);
+  GemmManyArgs list{};
+  uint32_t end = 0;
+  for (uint32_t i = 0; i < count; i++) {
+    list.w[i] = w_raw[i];
+    list.out[i] = p.splits > 1 ? workspace + packed_bytes : outs[i];
+    list.out_dim[i] = out_dims[i];
+    list.tile_end[i] = end += (out_dims[i] + 32 * p.rt - 1) / (32 * p.rt);
+  }
+  list.count = count;
+  char name[64];
+  std::snprintf(name, sizeof name, "%s_gemm_stream_f16_%ux%u", type_prefix(w_type), p.t, p.rt);
+  uint64_t kadd = p.splits > 1 ? 0 : add;
+  void* params[] = {&list, &workspace, &kadd, &add_stride, &in_dim, &tokens};
+  if (int rc = launch(name, gemm_stream_grid(tokens, p.t, end), 256, 0, params, stream, p.splits)) return rc;
+  if (p.splits == 1) return 0;
+  uint64_t planes = workspace + packed_bytes, out = outs[0];
+  uint32_t out_dim = out_dims[0], total = tokens * out_dim, splits = p.splits;
+  void* sum[] = {&planes, &add, &out, &total, &out_dim, &splits, &add_stride};
+  return launch("gemm_sum_splits_f32", (total + 1023) / 1024, 256, 0, sum, stream);
+}
+
+int cogni_gemm_stream_takes(uint32_t w_type, uint32_t in_dim, uint32_t rows, uint32_t tokens) {
+  return gemm_type(w_type) && in_dim != 0 && in_dim % 256 == 0 && rows != 0 && gemm_stream_take(w_type, tokens, in_dim, rows);
+}
+
+int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t residual,
+                          const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_stream_dev";
+  if (!w_raw || !outs || !out_dims || count == 0 || count > 6) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": one to six matrices");
+  if (residual && count != 1) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": a residual goes with one matrix");
+  for (uint32_t i = 0; i < count; i++) {
+    if (!w_raw[i] || !outs[i]) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+    if (int rc = gemm_check(who, w_type, in_dim, out_dims[i], tokens, workspace, workspace_bytes)) return rc;
+  }
+  return gemm_stream_launch(who, w_raw, w_type, workspace, workspace_bytes, residual, residual ? out_dims[0] : 0, outs, out_dims, count, in_dim,
+                            tokens, stream);
+}
+
+int cogni_gemm_stream_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
+                                      uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
+                                      uint32_t out_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_stream_swiglu_pack_dev";
+  if (int rc = swiglu_pack_check(who, w_gate, w_up, w_type, workspace, workspace_bytes, next_type, next_workspace, next_workspace_bytes, in_dim,
+                                 out_dim, tokens))
+    return rc;
+  if (cogni_gemm_workspace_bytes(w_type, in_dim, tokens) > GEMM_STREAM_MAX_PACKED)
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": packed activations of 2 GiB or more");
+  const uint32_t t = gemm_stream_tokens(tokens);
+  GemmManyArgs list{};
+  list.w[0] = w_gate;
+  list.out[0] = out;
+  list.out_dim[0] = out_dim;
+  list.tile_end[0] = (out_dim + 31) / 32;
+  list.count = 1;
+  char name[64];
+  std::snprintf(name, sizeof name, "q4_k_gemm_stream_swiglu_pack_%s_f16_%ux2", next_type == COGNI_TYPE_Q6_K ? "q6k" : "q4k", t);
+  void* params[] = {&list, &w_up, &workspace, &next_workspace, &in_dim, &tokens};
+  return launch(name, gemm_stream_grid(tokens, t, list.tile_end[0]), 256, 0, params, stream);
 }
 
 int cogni_set_gemm_threshold(int32_t tokens) {
@@ -1415,6 +1499,12 @@ int cogni_matmul_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias,
       if (!w_raw || !x || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_matmul_dev: null device pointer");
       if (int rc = cogni_gemv_pack16_dev(x, w_type, in_dim, tokens, workspace, stream)) return rc;
       return cogni_gemv_packed16_dev(&w_raw, w_type, workspace, 0, &out, &out_dim, 1, in_dim, tokens, stream);
+    }
+    if (in_dim % 256 == 0 && gemm_stream_take(w_type, tokens, in_dim, out_dim)) {
+      if (!w_raw || !x || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_matmul_dev: null device pointer");
+      if (int rc = gemm_check("cogni_matmul_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;
+      if (int rc = cogni_gemm_pack_dev(x, w_type, in_dim, tokens, workspace, workspace_bytes, stream)) return rc;
+      return gemm_stream_launch("cogni_matmul_dev", &w_raw, w_type, workspace, workspace_bytes, bias, 0, &out, &out_dim, 1, in_dim, tokens, stream);
     }
     return cogni_gemm_dev(w_raw, w_type, x, bias, out, in_dim, out_dim, tokens, workspace, workspace_bytes, stream);
   }

@@ -351,6 +351,56 @@ static inline unsigned gemm_terms_plan(unsigned tokens, unsigned out_dim, unsign
   return mt * ((nt + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT) * GEMM_XCD_COUNT;
 }
 
+// ---- short prefills of Q4_K, Q5_K and Q6_K (gemm_stream.hpp): a workgroup takes 32 t tokens x 32 rt rows
+#define GEMM_STREAM_MAX_SPLITS 8u
+#define GEMM_STREAM_MAX_PACKED 0x7FFFFFFFu   // bytes of packed activations the kernels can address
+typedef struct {
+  unsigned t, rt, splits;
+} GemmStreamPlan;
+static inline unsigned gemm_stream_tokens(unsigned tokens) { return tokens <= 32u ? 1u : 2u; }
+// Rows of a workgroup and k splits: the cheapest of (super-blocks a wavefront walks) x (time of one, by type and tile) x
+// (load), plus the plane sum. The load is what workgroups that share a compute unit cost each other: 1 up to one workgroup per
+// unit, 1.7 more for every further one (Q4_K, 64 tokens x 32 rows, 4096 columns: 128 workgroups 9.2 us, 256 10.0, 384 19.5, 960
+// 39.1; 64 rows: 192 workgroups 16.9, 480 31.9). Q6_K at 64 tokens x 64 rows does not fit the registers.
+static inline GemmStreamPlan gemm_stream_plan(unsigned type, unsigned tokens, unsigned in_dim, unsigned long long rows, unsigned planes_max) {
+  static const unsigned us100[3][2][2] = {{{100, 160}, {150, 260}}, {{170, 260}, {200, 320}}, {{200, 420}, {260, 0}}};   // [type][t][rt]
+  const unsigned ty = type == 14u ? 2u : (type == 13u ? 1u : 0u), t = gemm_stream_tokens(tokens), nkb = in_dim >> 8;
+  const unsigned long long mt = (tokens + 32u * t - 1u) / (32u * t);
+  GemmStreamPlan best;
+  unsigned long long least = ~0ull;
+  unsigned rt, s;
+  best.t = t;
+  best.rt = best.splits = 1;
+  for (rt = 1; rt <= 2u; rt++)
+    for (s = 1; s <= planes_max && (s == 1u || 4u * s <= nkb); s *= 2u) {
+      const unsigned step = us100[ty][t - 1u][rt - 1u];
+      const unsigned long long wgs = mt * ((rows + 32u * rt - 1u) / (32u * rt)) * s;
+      const unsigned long long load = wgs <= 180u ? 256u : (wgs * 17u) / 10u - 50u;   // in 256ths
+      const unsigned long long cost = ((nkb + 4u * s - 1u) / (4u * s)) * step * (load < 256u ? 256u : load) / 256u + (s > 1u ? 300u : 0u);
+      if (step && cost < least) least = cost, best.rt = rt, best.splits = s;
+    }
+  return best;
+}
+static inline unsigned gemm_stream_grid(unsigned tokens, unsigned t, unsigned ntiles) {
+  const unsigned mt = (tokens + 32u * t - 1u) / (32u * t);
+  return mt * ((ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT) * GEMM_XCD_COUNT;
+}
+// Which launches take these kernels: more tokens than the sixteen-token one-pass kernels have, and no more weights x groups of
+// 64 tokens (in values) than the line up to which they measured ahead of the tile kernels (us, tile | stream). One group, Q4_K
+// 4096 -> 12288 at 32 tokens 19.0 | 14.0, 64 21.6 | 16.9; 12288 -> 12288 at 24 37.1 | 31.7, at 48 40.3 | 39.8; Q6_K 12288 ->
+// 4096 at 32 22.8 | 18.9, at 64 23.9 | 23.0. More: Q4_K 1024 -> 3072 at 512 18.2 | 10.1, 2048 -> 2048 at 1024 25.5 | 16.9, 2048 ->
+// 4096 at 512 24.6 | 15.8, at 1024 24.2 | 29.4; rows of 4096 and more hold on longer (4096 -> 4096 at 512 29.9 | 26.4, at 1024
+// 40.5 | 53.2; 4096 -> 12288 at 128 31.7 | 25.8). Q6_K 4096 -> 4096 at 256 23.9 | 21.8, at 512 33.5 | 39.8.
+static inline int gemm_stream_take(unsigned type, unsigned tokens, unsigned in_dim, unsigned long long rows) {
+  const unsigned long long groups = (tokens + 63ull) / 64ull, values = groups * in_dim * rows;
+  unsigned long long most = 1ull << 26;
+  if (tokens <= 16u || 256ull * ((tokens + 127ull) / 128ull) * in_dim > GEMM_STREAM_MAX_PACKED) return 0;
+  if (type == 14u) most = tokens <= 32u ? 100000000ull : 1ull << 26;
+  else if (tokens <= 64u) most = 160000000ull;
+  else if (in_dim >= 4096u) most = 140000000ull;
+  return values <= most;
+}
+
 // ---- one-pass kernel, rows above 4096 values: what a streamed unit waits for (gemv_mt.hpp)
 // vmcnt value that says "operand set i and unit i of a streamed row group have landed" (T = 1, S super-blocks per
 // k-slice, NSLOT units in LDS). Issue order: set 0, unit 0, set 1, unit 1, units 2 .. min(S, NSLOT) - 1 up front; behind unit

@@ -464,6 +464,21 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
 int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                       uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
                                       uint32_t out_dim, uint32_t tokens, void* stream);
+/* The short-prefill forms of the packed GEMMs: the weights streamed through many small workgroups instead of tiles of 128
+ * tokens that have a compute unit to themselves. They read the same packed activations, their operands are rounded as the
+ * tile kernels round them (fp16, fp32 sums; the order of the sums differs), and cogni_matmul_dev and the resident runners take
+ * them where cogni_gemm_stream_takes says so: `rows` is the sum of the row counts of what is launched together.
+ * cogni_gemm_stream_dev: one to six matrices of one type (Q4_K, Q5_K, Q6_K) and row length; a [tokens][out_dim] residual (0: none;
+ * it may be the output) goes with one matrix. The k range is split as far as planes fit behind the packed activations
+ * (cogni_gemm_workspace_bytes_split). cogni_gemm_stream_swiglu_pack_dev: as cogni_gemm_packed_swiglu_pack_dev (Q4_K; `out` may be
+ * null); of the absent tokens of the packed block only those of the last tile of 32 are written (zeros). Any token count is taken
+ * as long as the packed activations are below 2 GiB. */
+int cogni_gemm_stream_takes(uint32_t w_type, uint32_t in_dim, uint32_t rows, uint32_t tokens);
+int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t residual,
+                          const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
+int cogni_gemm_stream_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
+                                      uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
+                                      uint32_t out_dim, uint32_t tokens, void* stream);
 /* The launch cogni_gemm_packed_dev makes for a shape and a workspace of `workspace_bytes`: kernel name, grid (x: tiles,
  * y: k splits; with y > 1 gemm_sum_splits_f32 follows) and block, for hosts that launch by name (level 1) and for
  * callers who want to know which of the two Q4_K tilings a shape gets. Any out pointer may be null. The counterpart of

@@ -1,0 +1,104 @@
+"""The short-prefill GEMM kernels (weights streamed, four k-slices per workgroup) against the oracle and the tile kernels."""
+import numpy as np
+import pytest
+
+from cogni_ml_amd import quant, synth
+from gpu_common import DevArray, gpu  # noqa: F401
+from helpers import Q4_K, Q5_K, Q6_K
+
+pytestmark = pytest.mark.gpu
+
+# (in_dim, out_dim, tokens): one super-block (three of the four k-slices idle), five (uneven slices), a k split; one row, rows that
+# end inside a tile and inside a group of four, tall enough for 64-row tiles; one more and one less than a token tile, the
+# last token tile empty but for one
+CASES = [(256, 32, 17), (256, 1, 32), (1280, 33, 33), (1024, 100, 64), (512, 8200, 31), (768, 6147, 65), (12288, 70, 48),
+         (4096, 64, 129), (2048, 130, 97)]
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("in_dim,out_dim,tokens", CASES)
+def test_router_and_residual(gpu, oracle, t, in_dim, out_dim, tokens):
+    """The router takes these shapes to the new kernels: within the GEMM's bound of the oracle, a bias and a residual on top of
+    the very same sums, and the sums those of the tile kernel up to the order of fp32 additions."""
+    assert quant.gemm_stream_takes(t, in_dim, out_dim, tokens)
+    rng = np.random.default_rng(t * 7919 + in_dim * 13 + out_dim * 7 + tokens)
+    raw = synth.make_weights(rng, t, out_dim, in_dim)
+    x = synth.make_activations(rng, tokens, in_dim)
+    bias, res = rng.standard_normal(out_dim).astype(np.float32), rng.standard_normal(tokens * out_dim).astype(np.float32)
+    print("case type=%d in_dim=%d out_dim=%d tokens=%d" % (t, in_dim, out_dim, tokens), flush=True)
+    wsb = quant.gemm_workspace_bytes(t, in_dim, tokens, out_dim)
+    w, xd, ws = DevArray(raw), DevArray(x), DevArray(nbytes=wsb)
+    od, rd, bd = DevArray(np.full(tokens * out_dim + 64, np.nan, dtype=np.float32)), DevArray(res), DevArray(bias)
+    try:
+        quant.matmul_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens, ws.ptr, wsb)
+        got = od.read(np.float32, tokens * out_dim + 64)
+        assert np.isnan(got[tokens * out_dim:]).all()          # nothing behind the output
+        got = got[:tokens * out_dim]
+        rows = rng.choice(tokens, min(tokens, 8), replace=False)
+        want = oracle.matmul_add(np.ascontiguousarray(x.reshape(tokens, in_dim)[rows]).reshape(-1), len(rows), in_dim, raw, t, out_dim,
+                                 np.zeros(out_dim, dtype=np.float32), threads=16).reshape(len(rows), out_dim)
+        # binary16 activations and weights: the bound of every GEMM here
+        assert np.abs(got.reshape(tokens, out_dim)[rows].astype(np.float64) - want).max() <= 2e-3 * np.abs(want).max()
+        quant.gemm_packed_dev(w.ptr, t, ws.ptr, wsb, od.ptr, in_dim, out_dim, tokens)
+        tile = od.read(np.float32, tokens * out_dim)
+        # the same products (11 + 11 bits, exact in fp32) added in another order: at most one rounding per addition on either
+        # side, of a partial sum that is at most the sum of the magnitudes, which is sqrt(in_dim) times a typical result
+        assert np.abs(got - tile).max() <= 2 * 2.0 ** -24 * np.sqrt(in_dim) * in_dim * np.abs(tile).max()
+        assert np.linalg.norm(got - tile) <= 1e-5 * np.linalg.norm(tile)
+        quant.matmul_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens, ws.ptr, wsb, bd.ptr)
+        assert np.array_equal(od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim), got.reshape(tokens, out_dim) + bias)
+        quant.gemm_stream_dev([w.ptr], t, ws.ptr, wsb, [rd.ptr], [out_dim], in_dim, tokens, rd.ptr)   # in place
+        assert np.array_equal(rd.read(np.float32, tokens * out_dim), got + res)
+    finally:
+        for a in (w, xd, ws, od, rd, bd):
+            a.close()
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("tokens", [24, 70])
+def test_list_of_matrices(gpu, t, tokens):
+    """Every output of a list is that of the matrix by itself, unsplit, up to the tile height (which does not enter the sums)."""
+    in_dim, outs = 1536, [512, 33, 1, 260, 64]
+    rng = np.random.default_rng(tokens + t)
+    raws = [DevArray(synth.make_weights(rng, t, o, in_dim)) for o in outs]
+    xd = DevArray(synth.make_activations(rng, tokens, in_dim))
+    wsb = quant.gemm_workspace_bytes(t, in_dim, tokens)
+    ws = DevArray(nbytes=wsb)
+    ods = [DevArray(np.full(tokens * o, np.nan, dtype=np.float32)) for o in outs]
+    try:
+        quant.gemm_pack_dev(xd.ptr, t, in_dim, tokens, ws.ptr, wsb)
+        quant.gemm_stream_dev([w.ptr for w in raws], t, ws.ptr, wsb, [o.ptr for o in ods], outs, in_dim, tokens)
+        got = [o.read(np.float32, tokens * n) for o, n in zip(ods, outs)]
+        for w, o, n, g in zip(raws, ods, outs, got):
+            quant.gemm_stream_dev([w.ptr], t, ws.ptr, wsb, [o.ptr], [n], in_dim, tokens)
+            assert np.array_equal(o.read(np.float32, tokens * n), g)
+    finally:
+        for a in raws + ods + [xd, ws]:
+            a.close()
+
+
+@pytest.mark.parametrize("next_type", [Q4_K, Q6_K])
+@pytest.mark.parametrize("in_dim,out_dim,tokens", [(256, 256, 17), (1280, 768, 33), (4096, 512, 64), (512, 256, 130)])
+def test_gate_up_swiglu_pack(gpu, in_dim, out_dim, tokens, next_type):
+    """silu(gate) * up within a few roundings of the tile kernel's, and the packed block what the pack kernel makes of it."""
+    rng = np.random.default_rng(in_dim + out_dim + tokens)
+    g, u = (DevArray(synth.make_weights(rng, Q4_K, out_dim, in_dim)) for _ in range(2))
+    xd = DevArray(synth.make_activations(rng, tokens, in_dim))
+    wsb, nxb = quant.gemm_workspace_bytes(Q4_K, in_dim, tokens), quant.gemm_workspace_bytes(next_type, out_dim, tokens)
+    ws, nx, ref, out = DevArray(nbytes=wsb), DevArray(np.zeros(nxb, dtype=np.uint8)), DevArray(nbytes=nxb), DevArray(nbytes=4 * tokens * out_dim)
+    try:
+        quant.gemm_pack_dev(xd.ptr, Q4_K, in_dim, tokens, ws.ptr, wsb)
+        quant.gemm_packed_swiglu_dev(g.ptr, u.ptr, Q4_K, ws.ptr, wsb, out.ptr, in_dim, out_dim, tokens)
+        tile = out.read(np.float32, tokens * out_dim)
+        quant.gemm_stream_swiglu_pack_dev(g.ptr, u.ptr, Q4_K, ws.ptr, wsb, out.ptr, next_type, nx.ptr, nxb, in_dim, out_dim, tokens)
+        got, packed = out.read(np.float32, tokens * out_dim), nx.read(np.uint8, nxb)
+        assert np.linalg.norm(got - tile) <= 2e-5 * np.linalg.norm(tile)
+        quant.gemm_pack_dev(out.ptr, next_type, out_dim, tokens, ref.ptr, nxb)
+        assert np.array_equal(packed, ref.read(np.uint8, nxb))    # (the tiles of absent tokens are zeros in both here)
+        nx2 = DevArray(np.zeros(nxb, dtype=np.uint8))
+        quant.gemm_stream_swiglu_pack_dev(g.ptr, u.ptr, Q4_K, ws.ptr, wsb, 0, next_type, nx2.ptr, nxb, in_dim, out_dim, tokens)
+        assert np.array_equal(nx2.read(np.uint8, nxb), packed)
+        nx2.close()
+    finally:
+        for a in (g, u, xd, ws, nx, ref, out):
+            a.close()
