@@ -98,6 +98,7 @@ struct TermsF32 {
   static constexpr int ROWS = 2;   // row addresses per lane
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)n * 4; }
   static __device__ __forceinline__ u32 row_of(u32 lane, int i) { return 8 * i + (lane >> 3); }
+  static __device__ __forceinline__ float at(const uint8_t* row, u32 k) { return reinterpret_cast<const float*>(row)[k]; }
   TermsF32Tile t;
   template <bool FULL>
   __device__ __forceinline__ void load(const uint8_t* const (&rows)[2], u32 s, u32 lane, u32 n) {
@@ -119,6 +120,7 @@ struct TermsF16 {   // one load: four lanes x 16 bytes per row; rows 20 dwords a
   static constexpr int ROWS = 1;
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)n * 2; }
   static __device__ __forceinline__ u32 row_of(u32 lane, int) { return lane >> 2; }
+  static __device__ __forceinline__ float at(const uint8_t* row, u32 k) { return h2f(ld2(row + (size_t)k * 2)); }
   uint4 q;
   template <bool FULL>
   __device__ __forceinline__ void load(const uint8_t* const (&rows)[1], u32 s, u32 lane, u32 n) {
@@ -167,6 +169,10 @@ struct TermsQ80 {
   static constexpr int ROWS = 1;
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)((n + 31) >> 5) * 34; }
   static __device__ __forceinline__ u32 row_of(u32 lane, int) { return lane >> 2; }
+  static __device__ __forceinline__ float at(const uint8_t* row, u32 k) {
+    const uint8_t* b = row + (size_t)(k >> 5) * 34;
+    return h2f(ld2(b)) * (float)(int)(int8_t)b[2 + (k & 31)];
+  }
   uint2 q;
   u32 d;
   template <bool FULL>
@@ -192,6 +198,10 @@ struct TermsIq4nl {   // values 0..15 of a block are the low nibbles of its 16 b
   static constexpr int ROWS = 1;
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)((n + 31) >> 5) * 18; }
   static __device__ __forceinline__ u32 row_of(u32 lane, int) { return lane >> 2; }
+  static __device__ __forceinline__ float at(const uint8_t* row, u32 k) {
+    const uint8_t* b = row + (size_t)(k >> 5) * 18;
+    return h2f(ld2(b)) * (float)(int)(int8_t)look(((u32)b[2 + (k & 15)] >> (k & 16 ? 4 : 0)) & 15u);
+  }
   u32 q, d;
   template <bool FULL>
   __device__ __forceinline__ void load(const uint8_t* const (&rows)[1], u32 s, u32 lane, u32) {
@@ -218,6 +228,15 @@ struct TermsIq4nl {   // values 0..15 of a block are the low nibbles of its 16 b
     terms_from_bytes(look((r.x >> sh) & 0x0F0F0F0Fu), look((r.y >> sh) & 0x0F0F0F0Fu), o[0]);
   }
 };
+
+// An infinity has no such terms (inf - inf, and inf times a term that is zero), so a sum that is not a number is taken again
+// term by term: the infinity or NaN that the row kernels give. Only outputs of rows that hold one (or overflow) come here.
+template <class W>
+__device__ __forceinline__ float terms_plain_sum(const uint8_t* row, const float* x, u32 n) {
+  float s = 0.f;
+  for (u32 k = 0; k < n && s == s; k++) s = fmaf(x[k], W::at(row, k), s);
+  return s;
+}
 
 // D: steps whose loads are in flight while one is computed (a ring of registers).
 template <class W, int TM, int TN, int D>
@@ -340,7 +359,9 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
       for (u32 v = 0; v < 4; v++)
         if (mb + v < tokens) {
           const size_t at = (size_t)(mb + v) * out_dim + n;
-          out[at] = residual ? residual[at] + s[v] : s[v];
+          float r = s[v];
+          if (r != r) r = terms_plain_sum<W>(w + (size_t)n * W::row_bytes(in_dim), x + (size_t)(mb + v) * in_dim, in_dim);
+          out[at] = residual ? residual[at] + r : r;
         }
     }
   }

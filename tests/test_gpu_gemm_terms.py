@@ -46,3 +46,29 @@ def test_terms_kernels_match_the_oracle(gpu, oracle, t, in_dim, out_dim, tokens)
     finally:
         for a in (w, xd, od, rd):
             a.close()
+
+
+@pytest.mark.parametrize("t", [F32, F16, IQ4_NL, Q8_0])
+@pytest.mark.parametrize("in_dim,out_dim,tokens", [(96, 40, 9), (1024, 33, 33), (70, 5, 65)])
+def test_infinities_and_nans_stay_what_they_are(gpu, oracle, t, in_dim, out_dim, tokens):
+    """An infinity has no finite bfloat16 terms: the outputs of its row are the row kernels' (+-inf, or NaN where both signs or a
+    zero weight meet), the other rows' are finite. Exactly: which outputs are finite, +inf, -inf and NaN."""
+    rng = np.random.default_rng(t * 31 + in_dim + tokens)
+    raw = synth.make_weights(rng, t, out_dim, in_dim)
+    x = synth.make_activations(rng, tokens, in_dim).reshape(tokens, in_dim)
+    x[0, 3] = np.inf
+    x[2, in_dim - 1] = -np.inf
+    x[4, 0], x[4, in_dim // 2] = np.inf, -np.inf
+    x[5, 1] = np.nan
+    x[6, 2] = np.uint32(0x7F800001).view(np.float32)   # a NaN whose upper half is that of an infinity
+    want = oracle.matmul_add(x, tokens, in_dim, raw, t, out_dim, np.zeros(out_dim, dtype=np.float32), threads=4).reshape(tokens, out_dim)
+    w, xd, od = DevArray(raw), DevArray(x), DevArray(np.zeros(tokens * out_dim, dtype=np.float32))
+    try:
+        print("case type=%d in_dim=%d out_dim=%d tokens=%d" % (t, in_dim, out_dim, tokens), flush=True)
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+    finally:
+        for a in (w, xd, od):
+            a.close()
+    for kind in (np.isfinite, np.isposinf, np.isneginf, np.isnan):
+        assert np.array_equal(kind(got), kind(want)), kind.__name__
