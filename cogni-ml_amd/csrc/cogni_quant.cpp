@@ -1500,7 +1500,9 @@ int cogni_matmul_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias,
       if (int rc = cogni_gemv_pack16_dev(x, w_type, in_dim, tokens, workspace, stream)) return rc;
       return cogni_gemv_packed16_dev(&w_raw, w_type, workspace, 0, &out, &out_dim, 1, in_dim, tokens, stream);
     }
-    if (in_dim % 256 == 0 && gemm_stream_take(w_type, tokens, in_dim, out_dim)) {
+    // the short-prefill kernels from eighteen tokens: they add in another order than cogni_gemm_dev, whose bits this entry
+    // point gives at seventeen (what its test holds it to)
+    if (tokens > 17 && in_dim % 256 == 0 && gemm_stream_take(w_type, tokens, in_dim, out_dim)) {
       if (!w_raw || !x || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_matmul_dev: null device pointer");
       if (int rc = gemm_check("cogni_matmul_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;
       if (int rc = cogni_gemm_pack_dev(x, w_type, in_dim, tokens, workspace, workspace_bytes, stream)) return rc;

@@ -467,7 +467,7 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
 /* The short-prefill forms of the packed GEMMs: the weights streamed through many small workgroups instead of tiles of 128
  * tokens that have a compute unit to themselves. They read the same packed activations, their operands are rounded as the
  * tile kernels round them (fp16, fp32 sums; the order of the sums differs), and cogni_matmul_dev and the resident runners take
- * them where cogni_gemm_stream_takes says so: `rows` is the sum of the row counts of what is launched together.
+ * them where cogni_gemm_stream_takes says so (cogni_matmul_dev from eighteen tokens: seventeen keep cogni_gemm_dev's bits): `rows` is the sum of the row counts of what is launched together.
  * cogni_gemm_stream_dev: one to six matrices of one type (Q4_K, Q5_K, Q6_K) and row length; a [tokens][out_dim] residual (0: none;
  * it may be the output) goes with one matrix. The k range is split as far as planes fit behind the packed activations
  * (cogni_gemm_workspace_bytes_split). cogni_gemm_stream_swiglu_pack_dev: as cogni_gemm_packed_swiglu_pack_dev (Q4_K; `out` may be

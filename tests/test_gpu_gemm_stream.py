@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 # (in_dim, out_dim, tokens): one super-block (three of the four k-slices idle), five (uneven slices), a k split; one row, rows that
 # end inside a tile and inside a group of four, tall enough for 64-row tiles; one more and one less than a token tile, the
 # last token tile empty but for one
-CASES = [(256, 32, 17), (256, 1, 32), (1280, 33, 33), (1024, 100, 64), (512, 8200, 31), (768, 6147, 65), (12288, 70, 48),
+CASES = [(256, 32, 18), (256, 1, 32), (1280, 33, 33), (1024, 100, 64), (512, 8200, 31), (768, 6147, 65), (12288, 70, 48),
          (4096, 64, 129), (2048, 130, 97)]
 
 
