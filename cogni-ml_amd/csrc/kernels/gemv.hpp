@@ -606,12 +606,6 @@ GEMV_TOP1_ENTRY(q6_k_gemv_top1_partial_f32, FmtQ6K, 1)
 GEMV_TOP1_ENTRY(q6_k_gemv_top1_partial_f32_tbatch2, FmtQ6K, 2)
 GEMV_TOP1_ENTRY(q6_k_gemv_top1_partial_f32_tbatch3, FmtQ6K, 3)
 GEMV_TOP1_ENTRY(q8_0_gemv_top1_partial_f32, FmtQ80, 1)
-GEMV_TOP1_LOGITS_ENTRY(q4_k_gemv_top1_logits_partial_f32, FmtQ4K, 1)
-GEMV_TOP1_LOGITS_ENTRY(q4_k_gemv_top1_logits_partial_f32_tbatch2, FmtQ4K, 2)
-GEMV_TOP1_LOGITS_ENTRY(q5_k_gemv_top1_logits_partial_f32, FmtQ5K, 1)
-GEMV_TOP1_LOGITS_ENTRY(q6_k_gemv_top1_logits_partial_f32, FmtQ6K, 1)
-GEMV_TOP1_LOGITS_ENTRY(q6_k_gemv_top1_logits_partial_f32_tbatch2, FmtQ6K, 2)
-GEMV_TOP1_LOGITS_ENTRY(q8_0_gemv_top1_logits_partial_f32, FmtQ80, 1)
 
 // (partial_ids, partial_values, out_ids, out_values, count): the largest of `count` partial values and its id, per
 // token (grid.x = tokens; partial_* + token * count, out_* + token). Of equal values the lowest id wins, which is

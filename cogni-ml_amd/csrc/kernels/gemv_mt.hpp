@@ -977,8 +977,6 @@ GEMV_MT_ENTRY(q8_0_gemv_mt16_f32, MtQ80x16)
   }
 GEMV_MT_TOP1_ENTRY(q4_k_gemv_mt_top1_partial_f32, MtQ4K)
 GEMV_MT_TOP1_ENTRY(q6_k_gemv_mt_top1_partial_f32, MtQ6K)
-GEMV_MT_TOP1_LOGITS_ENTRY(q4_k_gemv_mt_top1_logits_partial_f32, MtQ4K)
-GEMV_MT_TOP1_LOGITS_ENTRY(q6_k_gemv_mt_top1_logits_partial_f32, MtQ6K)
 
 // (w_gate, w_up, image, out, in_dim, out_dim, tokens): out[m][o] = silu(gate . x) * (up . x); block 512, grid = min(256,
 // ceil(out_dim / 16)), dynamic shared memory as q4_k_gemv_mt_f32. The parameter list of q4_k_dual_gemv_swiglu_f32 with the
