@@ -3,9 +3,10 @@
 // These types have no fp16-precision prefill form (the reference computes them in full precision at every token count,
 // src/ml/gguf/quant_matmul.cr:216-368), so every operand is split into bfloat16 terms that lose nothing: an fp32 value is
 // exactly three of them (8 + 8 + 8 significand bits, by truncation; bfloat16 has the exponent range of fp32, so no scaling),
-// a binary16 weight two, a Q8_0 or IQ4_NL code one (the block scale is applied to the 32-value sum in fp32). A product is the
-// sum of the term products that reach 2^-24 of it: 3 instructions of v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32 for the codes,
-// 5 for binary16, 6 for fp32 weights.
+// a binary16 weight two, a Q8_0 or IQ4_NL code one (the block scale is applied to the 32-value sum in fp32). Truncated terms are
+// below 2^-7 and 2^-15 of the value and have its sign, so what is left out of a product is a bias: all term products are taken
+// but the last one of fp32 weights, x2 w2, below 2^-30. 3 instructions of v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32 for the
+// codes, 6 for binary16, 8 for fp32 weights. (Without x1 w2 and x2 w1: up to 7.8 x 2^-24 of a product, 0.7 on average.)
 //
 // Kernel ABI: (w_raw, x, residual | null, out, in_dim:u32, out_dim:u32, tokens:u32), names <type>_gemm_terms_f32_<TM>x<TN>:
 // a workgroup of eight wavefronts takes 16 TM tokens x 16 TN rows, grid gemm_terms_plan (gemv_config.h). The
@@ -304,14 +305,14 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
       const float d = W::scale(wl, lane);
 #pragma unroll
       for (int t = 0; t < TM; t++) {
-        // term i of x against term j of w, the products below 2^-24 left out (i + j > 2), smallest first; the sum over the
-        // step's 32 values joins the running sum in one rounding
+        // term i of x against term j of w, i + j <= 3, smallest first; the sum over the step's 32 values joins the running sum
+        // in one rounding
         terms_f4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ij = 2; ij >= 0; ij--)
+        for (int ij = 3; ij >= 0; ij--)
 #pragma unroll
           for (int j = 0; j < W::TERMS; j++)
-            if (ij - j >= 0) p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t][ij - j], B[j], p, 0, 0, 0);
+            if (ij - j >= 0 && ij - j < 3) p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t][ij - j], B[j], p, 0, 0, 0);
 #pragma unroll
         for (int v = 0; v < 4; v++) acc[t][c][v] = W::SCALED ? fmaf(d, p[v], acc[t][c][v]) : acc[t][c][v] + p[v];
       }
@@ -349,9 +350,14 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
   __syncthreads();
   // a lane's four sums are tokens 4 (lane / 16) .. + 3 of its tile for weight row lane % 16
   for (u32 i = wave; i < TM * TN; i += GEMM_TERMS_WAVES) {
-    terms_f4 s = part[i * 64 + lane];
+    terms_f4 p[GEMM_TERMS_WAVES];
 #pragma unroll
-    for (u32 k = 1; k < GEMM_TERMS_WAVES; k++) s += part[(k * (TM * TN) + i) * 64 + lane];
+    for (u32 k = 0; k < GEMM_TERMS_WAVES; k++) p[k] = part[(k * (TM * TN) + i) * 64 + lane];
+#pragma unroll
+    for (u32 h = GEMM_TERMS_WAVES / 2; h; h >>= 1)   // in pairs: three roundings on the way, not seven
+#pragma unroll
+      for (u32 k = 0; k < h; k++) p[k] += p[k + h];
+    const terms_f4 s = p[0];
     const u32 n = n0 + 16 * (i % TN) + row;
     const u32 mb = m0 + 16 * (i / TN) + 4 * kg;
     if (n < out_dim) {

@@ -1,9 +1,11 @@
 """Several tokens of F32, F16, IQ4_NL and Q8_0 weights on the matrix cores (activations as three bfloat16 terms): fp32 precision
 at every tile shape and remainder, against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from cogni_ml_amd import quant, synth
+from cogni_ml_amd import hip, quant, synth
 from gpu_common import DevArray, gpu  # noqa: F401
 from helpers import F16, F32, IQ4_NL, Q8_0
 
@@ -30,10 +32,10 @@ def test_terms_kernels_match_the_oracle(gpu, oracle, t, in_dim, out_dim, tokens)
     row = raw.size // out_dim
     dense = np.stack([oracle.dequantize(raw[r * row:(r + 1) * row], t, in_dim) for r in range(out_dim)]).astype(np.float64)
     mags = np.abs(x.reshape(tokens, in_dim).astype(np.float64)) @ np.abs(dense).T
-    # the term products left out are below 3 * 2^-24 of a product; a sum goes through at most 32 + 2 roundings inside a step of
-    # 32, one per step of a k-slice (an eighth of them), eight for the slices and one for the block scale; the oracle's own
-    # result is rounded once
-    bound = (3 + 34 + (in_dim / 32) / 8 + 1 + 8 + 1 + 1) * 2.0 ** -24 * mags.reshape(-1) + 1e-37
+    # the term product left out (fp32 weights) is below 2^-30 of a product; a sum goes through at most 32 + 2 roundings inside a
+    # step of 32, one per step of a k-slice (an eighth of them), three for the slices and one for the block scale; the oracle's
+    # own result is rounded once
+    bound = (2.0 ** -6 + 34 + (in_dim / 32) / 8 + 1 + 3 + 1 + 1) * 2.0 ** -24 * mags.reshape(-1) + 1e-37
     w, xd, od, rd = DevArray(raw), DevArray(x), DevArray(np.full(tokens * out_dim, np.nan, dtype=np.float32)), DevArray(res)
     try:
         quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
@@ -72,3 +74,66 @@ def test_infinities_and_nans_stay_what_they_are(gpu, oracle, t, in_dim, out_dim,
             a.close()
     for kind in (np.isfinite, np.isposinf, np.isneginf, np.isnan):
         assert np.array_equal(kind(got), kind(want)), kind.__name__
+
+
+@pytest.mark.parametrize("t", [F32, F16])
+@pytest.mark.parametrize("in_dim", [1, 2, 3])
+def test_no_term_product_is_missing(gpu, t, in_dim):
+    """Values whose bfloat16 terms behind the first are as large as they get, all of one sign: a term product left out shows (the
+    smallest of them is 3.3 * 2^-24 of the sum with binary16 weights, as much each with fp32). Bound: a matrix instruction may drop
+    what lies below the last place of its result (2 * 2^-24, here that of the sum of the smaller term products as the leading one
+    joins it; 2^-6 of that before), and one rounding of the result."""
+    out_dim, tokens = 20, 6
+    rng = np.random.default_rng(in_dim + t)
+    x = (np.full((tokens, in_dim), 0x3F80FFFF, dtype=np.uint32).view(np.float32) * np.float32(2.0) ** rng.integers(-3, 4, (tokens, 1))).astype(np.float32)
+    if t == F32:
+        dense = (np.full((out_dim, in_dim), 0x3F80FFFF, dtype=np.uint32).view(np.float32) * np.float32(2.0) ** rng.integers(-3, 4, (out_dim, 1))).astype(np.float32)
+    else:
+        dense = (np.full((out_dim, in_dim), 0x3C07, dtype=np.uint16).view(np.float16) * np.float16(2.0) ** rng.integers(-3, 4, (out_dim, 1))).astype(np.float16)
+    want = x.astype(np.float64) @ dense.astype(np.float64).T
+    w, xd, od = DevArray(dense), DevArray(x), DevArray(np.full(tokens * out_dim, np.nan, dtype=np.float32))
+    try:
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+    finally:
+        for a in (w, xd, od):
+            a.close()
+    err = np.abs(got.astype(np.float64) - want) / want * 2.0 ** 24
+    assert err.max() <= 3 + 2.0 ** -4, err.max()
+
+
+@pytest.mark.parametrize("t,kernel", [(F32, "f32_gemv_plain_f32"), (F16, "f16_gemv_plain_f32"), (IQ4_NL, "iq4_nl_gemv_plain_f32")])
+@pytest.mark.parametrize("in_dim", [256, 1024, 4096])
+@pytest.mark.parametrize("positive", [False, True])
+def test_no_further_from_64_bits_than_the_row_kernel(gpu, oracle, t, kernel, in_dim, positive):
+    """The error in the 2-norm against 64-bit sums of the row kernel (a chain of fused multiply-adds per lane) on the same inputs, of
+    mixed signs and all of one: not exceeded but by what another order of the same number of roundings changes (a tenth)."""
+    out_dim, tokens = 512, 33
+    rng = np.random.default_rng(t + in_dim + positive)
+    raw = synth.make_weights(rng, t, out_dim, in_dim)
+    x = synth.make_activations(rng, tokens, in_dim).reshape(tokens, in_dim)
+    if positive:
+        x = np.abs(x)
+        if t == F32:
+            raw = np.abs(raw.view(np.float32)).view(np.uint8)
+        elif t == F16:
+            raw = np.abs(raw.view(np.float16)).view(np.uint8)
+        else:
+            raw.reshape(-1, 18)[:, 2:] |= 0x88   # the upper half of the table is positive
+    row = raw.size // out_dim
+    dense = np.stack([oracle.dequantize(raw[r * row:(r + 1) * row], t, in_dim) for r in range(out_dim)]).astype(np.float64)
+    want = x.astype(np.float64) @ dense.T
+    w, xd, od = DevArray(raw), DevArray(x), DevArray(nbytes=4 * tokens * out_dim)
+    try:
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+        params = hip.KernelParams(*[ctypes.c_uint64(v) for v in (w.ptr, xd.ptr, 0, od.ptr)], *[ctypes.c_uint32(v) for v in (in_dim, out_dim, tokens)])
+        module = hip.HIPModule.load_builtin()
+        hip.launch(module.function(kernel), (out_dim + 3) // 4, 1, 1, 256, 1, 1, params, kernel)
+        rows = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+        module.close()
+    finally:
+        for a in (w, xd, od):
+            a.close()
+    assert np.linalg.norm(rows - want) <= 1e-6 * np.linalg.norm(want)
+    assert np.linalg.norm(got - want) <= 1.1 * np.linalg.norm(rows - want)
