@@ -230,13 +230,24 @@ struct TermsIq4nl {   // values 0..15 of a block are the low nibbles of its 16 b
   }
 };
 
-// An infinity has no such terms (inf - inf, and inf times a term that is zero), so a sum that is not a number is taken again
-// term by term: the infinity or NaN that the row kernels give. Only outputs of rows that hold one (or overflow) come here.
+// What has no such terms: an infinity (inf - inf, and inf times a term that is zero), and a block whose codes times x leave the range of
+// fp32 before the block scale brings them back. A sum that is no finite number is therefore taken again from plain fp32 products, as
+// the row kernels do: a wavefront takes four tokens against one row at a time, lanes over k, all wavefronts of the workgroup share
+// the tile's. F16 2048 x 2048, 33 tokens, us (a lane per sum, walking the row alone | this | the row kernel): one infinity 178 | 24 | 42, one
+// in every token 818 | 63 | 42, every value a NaN 10 | 16 | 41; F32 4096 x 4096, 33 tokens, one infinity 383 | 59 | 177; Q8_0 1024 -> 3584,
+// 200 tokens, one infinity 140 | 43, one in every token 3650 | 310.
 template <class W>
-__device__ __forceinline__ float terms_plain_sum(const uint8_t* row, const float* x, u32 n) {
-  float s = 0.f;
-  for (u32 k = 0; k < n && s == s; k++) s = fmaf(x[k], W::at(row, k), s);
-  return s;
+__device__ __forceinline__ void terms_plain_sums(const uint8_t* row, const float* const (&x)[4], u32 n, u32 lane, float (&s)[4]) {
+#pragma unroll
+  for (int v = 0; v < 4; v++) s[v] = 0.f;
+#pragma unroll 4
+  for (u32 k = lane; k < n; k += 64) {
+    const float w = W::at(row, k);
+#pragma unroll
+    for (int v = 0; v < 4; v++) s[v] = fmaf(x[v][k], w, s[v]);
+  }
+#pragma unroll
+  for (int v = 0; v < 4; v++) s[v] = wave_sum(s[v]);
 }
 
 // D: steps whose loads are in flight while one is computed (a ring of registers).
@@ -246,7 +257,8 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
   constexpr u32 XD = 16 * TERMS_F32_STRIDE;                      // dwords of 16 rows of x
   constexpr u32 WAVE_DWORDS = TM * XD + TN * W::LDS_DWORDS;      // a wavefront's region
   constexpr u32 PART_DWORDS = GEMM_TERMS_WAVES * TM * TN * 256;  // the k-slices' sums, behind the loop
-  constexpr u32 LDS_DWORDS = GEMM_TERMS_WAVES * WAVE_DWORDS > PART_DWORDS ? GEMM_TERMS_WAVES * WAVE_DWORDS : PART_DWORDS;
+  constexpr u32 END_DWORDS = PART_DWORDS + GEMM_TERMS_WAVES;     // and a flag of each wavefront
+  constexpr u32 LDS_DWORDS = GEMM_TERMS_WAVES * WAVE_DWORDS > END_DWORDS ? GEMM_TERMS_WAVES * WAVE_DWORDS : END_DWORDS;
   __shared__ uint4 lds4[(LDS_DWORDS + 3) / 4];
   const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const u32 row = lane & 15, kg = lane >> 4;
@@ -349,7 +361,9 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
     for (int c = 0; c < TN; c++) part[(wave * (TM * TN) + t * TN + c) * 64 + lane] = acc[t][c];
   __syncthreads();
   // a lane's four sums are tokens 4 (lane / 16) .. + 3 of its tile for weight row lane % 16
-  for (u32 i = wave; i < TM * TN; i += GEMM_TERMS_WAVES) {
+  u32 again = 0;   // four bits a tile: the lane's sums that are no finite numbers
+#pragma unroll
+  for (u32 i = wave, j = 0; i < TM * TN; i += GEMM_TERMS_WAVES, j++) {
     terms_f4 p[GEMM_TERMS_WAVES];
 #pragma unroll
     for (u32 k = 0; k < GEMM_TERMS_WAVES; k++) p[k] = part[(k * (TM * TN) + i) * 64 + lane];
@@ -357,7 +371,6 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
     for (u32 h = GEMM_TERMS_WAVES / 2; h; h >>= 1)   // in pairs: three roundings on the way, not seven
 #pragma unroll
       for (u32 k = 0; k < h; k++) p[k] += p[k + h];
-    const terms_f4 s = p[0];
     const u32 n = n0 + 16 * (i % TN) + row;
     const u32 mb = m0 + 16 * (i / TN) + 4 * kg;
     if (n < out_dim) {
@@ -365,8 +378,51 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
       for (u32 v = 0; v < 4; v++)
         if (mb + v < tokens) {
           const size_t at = (size_t)(mb + v) * out_dim + n;
-          float r = s[v];
-          if (r != r) r = terms_plain_sum<W>(w + (size_t)n * W::row_bytes(in_dim), x + (size_t)(mb + v) * in_dim, in_dim);
+          const float r = p[0][v];
+          if (__builtin_isfinite(r)) out[at] = residual ? residual[at] + r : r;
+          else again |= 1u << (4 * j + v);
+        }
+    }
+  }
+  u32* const flag = reinterpret_cast<u32*>(lds4) + PART_DWORDS;
+  const bool any = __builtin_amdgcn_ballot_w64(again != 0) != 0;
+  if (lane == 0) flag[wave] = any;
+  __syncthreads();
+  u32 sum = 0;
+#pragma unroll
+  for (u32 k = 0; k < GEMM_TERMS_WAVES; k++) sum |= flag[k];
+  if (__builtin_amdgcn_readfirstlane(sum) == 0) return;
+  // All wavefronts share the tile's sums that have to be taken again (the k-slices' sums in LDS have been read). A NaN among the first
+  // values of a token, as in a row of NaNs, is the answer for all its sums.
+  u32* const todo = reinterpret_cast<u32*>(lds4);
+  u32* const nan = todo + TM * TN * 64;
+  for (u32 i = wave, j = 0; i < TM * TN; i += GEMM_TERMS_WAVES, j++) todo[i * 64 + lane] = (again >> (4 * j)) & 15u;
+  for (u32 t = wave; t < 16 * TM; t += GEMM_TERMS_WAVES) {
+    const float v = lane < in_dim ? x[(size_t)min(m0 + t, tokens - 1) * in_dim + lane] : 0.f;
+    const bool is = __builtin_amdgcn_ballot_w64(v != v) != 0;
+    if (lane == 0) nan[t] = is;
+  }
+  __syncthreads();
+  for (u32 q = wave; q < TM * TN * 64; q += GEMM_TERMS_WAVES) {
+    const u32 which = __builtin_amdgcn_readfirstlane(todo[q]);
+    if (which == 0) continue;
+    const u32 i = q >> 6, n = n0 + 16 * (i % TN) + (q & 15), t0 = 16 * (i / TN) + 4 * ((q >> 4) & 3), mb = m0 + t0;
+    u32 known = 0;
+    const float* xs[4];
+#pragma unroll
+    for (u32 v = 0; v < 4; v++) {
+      known |= nan[t0 + v] << v;
+      xs[v] = x + (size_t)min(mb + v, tokens - 1) * in_dim;
+    }
+    known = __builtin_amdgcn_readfirstlane(known);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    if (which & ~known) terms_plain_sums<W>(w + (size_t)n * W::row_bytes(in_dim), xs, in_dim, lane, s);
+    if (lane == 0) {
+#pragma unroll
+      for (u32 v = 0; v < 4; v++)
+        if (which & (1u << v)) {
+          const size_t at = (size_t)(mb + v) * out_dim + n;
+          const float r = known & (1u << v) ? __builtin_nanf("") : s[v];
           out[at] = residual ? residual[at] + r : r;
         }
     }

@@ -137,3 +137,66 @@ def test_no_further_from_64_bits_than_the_row_kernel(gpu, oracle, t, kernel, in_
             a.close()
     assert np.linalg.norm(rows - want) <= 1e-6 * np.linalg.norm(want)
     assert np.linalg.norm(got - want) <= 1.1 * np.linalg.norm(rows - want)
+
+
+@pytest.mark.parametrize("t", [Q8_0, IQ4_NL])
+@pytest.mark.parametrize("in_dim,out_dim,tokens", [(1024, 33, 9), (288, 100, 70)])
+def test_activations_near_the_top_of_the_fp32_range(gpu, oracle, t, in_dim, out_dim, tokens):
+    """|x| of 1e35 and more, outputs up to 1e38: a block's codes times x leave the fp32 range before the scale brings them back, the
+    result does not. It is finite in the oracle's 64-bit sums and has to be here, to the bar of the one-pass kernels."""
+    rng = np.random.default_rng(t + in_dim)
+    raw = synth.make_weights(rng, t, out_dim, in_dim)
+    x = synth.make_activations(rng, tokens, in_dim).reshape(tokens, in_dim)
+    x[0] *= np.float32(1e35)
+    x[1] *= np.float32(1e36)
+    x[tokens - 1, in_dim - 32:] *= np.float32(2e36)
+    want = oracle.matmul_add(x, tokens, in_dim, raw, t, out_dim, np.zeros(out_dim, dtype=np.float32), threads=4).reshape(tokens, out_dim)
+    assert np.isfinite(want).all()
+    w, xd, od = DevArray(raw), DevArray(x), DevArray(nbytes=4 * tokens * out_dim)
+    try:
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+    finally:
+        for a in (w, xd, od):
+            a.close()
+    assert np.isfinite(got).all()
+    for m in range(tokens):
+        assert np.max(np.abs(got[m].astype(np.float64) - want[m])) <= 2e-5 * np.max(np.abs(want[m]).astype(np.float64)), m
+
+
+@pytest.mark.parametrize("t", [F32, F16])
+@pytest.mark.parametrize("in_dim,out_dim,tokens", [(96, 40, 9), (1024, 70, 33), (512, 4097, 129), (70, 5, 65)])
+def test_infinite_weights_leave_the_other_rows_alone(gpu, oracle, t, in_dim, out_dim, tokens):
+    """Rows with an infinity, two of both signs and a NaN, in the first and in the last (partial) tile: which outputs are finite,
+    +inf, -inf and NaN is what the oracle says, with and without a residual, and every other output keeps its bits."""
+    rng = np.random.default_rng(t + in_dim + out_dim)
+    dense = synth.make_weights(rng, t, out_dim, in_dim).view(np.float32 if t == F32 else np.float16).reshape(out_dim, in_dim)
+    x = synth.make_activations(rng, tokens, in_dim).reshape(tokens, in_dim)
+    x[1, 0] = 0.0
+    res = rng.standard_normal(tokens * out_dim).astype(np.float32)
+    bad = dense.copy()
+    bad[0, 0] = np.inf                      # NaN against the zero of token 1
+    bad[2, 3], bad[2, in_dim - 1] = np.inf, -np.inf
+    bad[out_dim - 1, in_dim // 2] = -np.inf
+    bad[out_dim - 2, in_dim - 1] = np.nan
+    touched = [0, 2, out_dim - 1, out_dim - 2]
+    want = oracle.matmul_add(x, tokens, in_dim, np.ascontiguousarray(bad[touched]).view(np.uint8).reshape(-1), t, 4, np.zeros(4, dtype=np.float32),
+                             threads=4).reshape(tokens, 4)
+    good, w, xd, rd, od = DevArray(dense), DevArray(bad), DevArray(x), DevArray(res), DevArray(nbytes=4 * tokens * out_dim)
+    try:
+        print("case type=%d in_dim=%d out_dim=%d tokens=%d" % (t, in_dim, out_dim, tokens), flush=True)
+        quant.gemv_dev(good.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        plain = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+        quant.gemv_dev(w.ptr, t, xd.ptr, rd.ptr, in_dim, out_dim, tokens, rd.ptr)   # in place
+        added = rd.read(np.float32, tokens * out_dim).reshape(tokens, out_dim)
+    finally:
+        for a in (good, w, xd, rd, od):
+            a.close()
+    rest = np.setdiff1d(np.arange(out_dim), touched)
+    assert np.array_equal(got[:, rest], plain[:, rest])
+    assert np.array_equal(added[:, rest], plain[:, rest] + res.reshape(tokens, out_dim)[:, rest])
+    for kind in (np.isfinite, np.isposinf, np.isneginf, np.isnan):
+        assert np.array_equal(kind(got[:, touched]), kind(want)), kind.__name__
+        assert np.array_equal(kind(added[:, touched]), kind(want)), kind.__name__
