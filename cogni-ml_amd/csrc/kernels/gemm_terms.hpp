@@ -7,6 +7,9 @@
 // below 2^-7 and 2^-15 of the value and have its sign, so what is left out of a product is a bias: all term products are taken
 // but the last one of fp32 weights, x2 w2, below 2^-30. 3 instructions of v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32 for the
 // codes, 6 for binary16, 8 for fp32 weights. (Without x1 w2 and x2 w1: up to 7.8 x 2^-24 of a product, 0.7 on average.)
+// The instruction reads a term below 2^-126 as zero, and the third term of a value is as small as its last place: fp32 operands are
+// split times 2^24, which brings the last place of the smallest subnormal above that, and the sums are brought back at the end
+// (unscaled, activations around 2^-112 / 2^-120 / 2^-128 were off by 2.6e-7 / 7e-5 / 0.018 of the result, the row kernels by 9e-8).
 //
 // Kernel ABI: (w_raw, x, residual | null, out, in_dim:u32, out_dim:u32, tokens:u32), names <type>_gemm_terms_f32_<TM>x<TN>:
 // a workgroup of eight wavefronts takes 16 TM tokens x 16 TN rows, grid gemm_terms_plan (gemv_config.h). The
@@ -17,8 +20,9 @@
 // IQ4_NL, 64 tokens: 34 us against 18.7; with four steps in flight instead of one 40), so a wavefront loads its steps with
 // neighbouring lanes on neighbouring bytes of a row, up to two ahead, and turns them through a region of LDS that no other
 // wavefront uses: no barrier in the loop.
-// What bounds it: small calls the chain load - LDS - sums (4 us), large ones the vector instructions that split x (5.5 per
-// value and 64 rows: 4096 x 4096 Q8_0, 256 tokens, 40 us = 215 TFLOP/s of results, 650 of matrix instructions).
+// What bounds it: small calls the chain load - LDS - sums (4 us), large ones the vector instructions that split x (6.5 per
+// value and 64 rows, one of them the scale: Q8_0 1024 -> 3584, 200 tokens 14.2 us without it, 14.7 with) beside the waits of two wavefronts
+// per SIMD (4096 x 4096 Q8_0, 256 tokens, 41 us = 207 TFLOP/s of results, 620 of matrix instructions).
 // Measured, row kernels (Q8_0: one-pass launches of eight tokens) -> these: Q8_0 1024 -> 3584, 9 / 48 / 200 tokens 9.6 / 35 /
 // 143 -> 4.6 / 7.1 / 14.3 us; F16 2048 -> 2048, 33 tokens 39.9 -> 8.3; F32 4096 -> 4096, 33 tokens 173 -> 23; IQ4_NL 4096 ->
 // 4096, 1 / 64 tokens 39 / 1923 -> 9.5 / 19.
@@ -69,8 +73,10 @@ __device__ __forceinline__ float4 terms_load4(const float* row, u32 k, u32 n) {
   }
 }
 
-// Rows of 32 fp32 values in LDS, 36 dwords apart (the 16-byte reads of sixteen rows then fall on all 64 banks).
+// Rows of 32 fp32 values in LDS, 36 dwords apart (the 16-byte reads of sixteen rows then fall on all 64 banks). get(): the
+// lane's operand times TERMS_F32_SCALE (from 2^104 on an infinity, whose sums are taken again).
 #define TERMS_F32_STRIDE 36u
+#define TERMS_F32_SCALE 0x1p24f
 struct TermsF32Tile {   // 16 rows: two loads of eight rows x 8 lanes x 16 bytes
   float4 v[2];
   template <bool FULL>
@@ -87,14 +93,18 @@ struct TermsF32Tile {   // 16 rows: two loads of eight rows x 8 lanes x 16 bytes
     const float4 a = q[0], b = q[1];
     o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
     o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
+#pragma unroll
+    for (int e = 0; e < 8; e++) o[e] *= TERMS_F32_SCALE;
   }
 };
 
 // ---- weight formats: sixteen rows x 32 values. rows(): the addresses a lane loads from; load<FULL>() / put(): registers, LDS;
-// terms(): the operand's terms; scale(): what the step's sum is multiplied by.
+// terms(): the operand's terms; scale(): what the step's sum is multiplied by; UNSCALE: what brings the sums back from the scale
+// of the terms (those of x are always scaled).
 struct TermsF32 {
   static constexpr int TERMS = 3;
   static constexpr bool SCALED = false;
+  static constexpr float UNSCALE = 1.0f / (TERMS_F32_SCALE * TERMS_F32_SCALE);
   static constexpr u32 LDS_DWORDS = 16 * TERMS_F32_STRIDE;
   static constexpr int ROWS = 2;   // row addresses per lane
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)n * 4; }
@@ -117,6 +127,7 @@ struct TermsF32 {
 struct TermsF16 {   // one load: four lanes x 16 bytes per row; rows 20 dwords apart
   static constexpr int TERMS = 2;
   static constexpr bool SCALED = false;
+  static constexpr float UNSCALE = 1.0f / TERMS_F32_SCALE;
   static constexpr u32 STRIDE = 20, LDS_DWORDS = 16 * STRIDE;
   static constexpr int ROWS = 1;
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)n * 2; }
@@ -166,6 +177,7 @@ __device__ __forceinline__ void terms_from_bytes(u32 a, u32 b, bf16x8_t& t) {
 struct TermsQ80 {
   static constexpr int TERMS = 1;
   static constexpr bool SCALED = true;
+  static constexpr float UNSCALE = 1.0f / TERMS_F32_SCALE;
   static constexpr u32 STRIDE = 10, LDS_DWORDS = 16 * STRIDE + 16;   // rows of 8 dwords 10 apart, then the scales
   static constexpr int ROWS = 1;
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)((n + 31) >> 5) * 34; }
@@ -195,6 +207,7 @@ struct TermsQ80 {
 struct TermsIq4nl {   // values 0..15 of a block are the low nibbles of its 16 bytes, 16..31 the high ones
   static constexpr int TERMS = 1;
   static constexpr bool SCALED = true;
+  static constexpr float UNSCALE = 1.0f / TERMS_F32_SCALE;
   static constexpr u32 STRIDE = 6, LDS_DWORDS = 16 * STRIDE + 16;
   static constexpr int ROWS = 1;
   static __device__ __forceinline__ size_t row_bytes(u32 n) { return (size_t)((n + 31) >> 5) * 18; }
@@ -230,8 +243,8 @@ struct TermsIq4nl {   // values 0..15 of a block are the low nibbles of its 16 b
   }
 };
 
-// What has no such terms: an infinity (inf - inf, and inf times a term that is zero), and a block whose codes times x leave the range of
-// fp32 before the block scale brings them back. A sum that is no finite number is therefore taken again from plain fp32 products, as
+// What has no such terms: an infinity (inf - inf, and inf times a term that is zero), and sums that leave the range of fp32 times the
+// scale of the terms, or before the block scale brings them back. A sum that is no finite number is therefore taken again from plain fp32 products, as
 // the row kernels do: a wavefront takes four tokens against one row at a time, lanes over k, all wavefronts of the workgroup share
 // the tile's. F16 2048 x 2048, 33 tokens, us (a lane per sum, walking the row alone | this | the row kernel): one infinity 178 | 24 | 42, one
 // in every token 818 | 63 | 42, every value a NaN 10 | 16 | 41; F32 4096 x 4096, 33 tokens, one infinity 383 | 59 | 177; Q8_0 1024 -> 3584,
@@ -378,7 +391,7 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
       for (u32 v = 0; v < 4; v++)
         if (mb + v < tokens) {
           const size_t at = (size_t)(mb + v) * out_dim + n;
-          const float r = p[0][v];
+          const float r = p[0][v] * W::UNSCALE;   // exact, but for one rounding of a subnormal result
           if (__builtin_isfinite(r)) out[at] = residual ? residual[at] + r : r;
           else again |= 1u << (4 * j + v);
         }

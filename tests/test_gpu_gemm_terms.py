@@ -200,3 +200,34 @@ def test_infinite_weights_leave_the_other_rows_alone(gpu, oracle, t, in_dim, out
     for kind in (np.isfinite, np.isposinf, np.isneginf, np.isnan):
         assert np.array_equal(kind(got[:, touched]), kind(want)), kind.__name__
         assert np.array_equal(kind(added[:, touched]), kind(want)), kind.__name__
+
+
+@pytest.mark.parametrize("t", [F32, F16, Q8_0, IQ4_NL])
+@pytest.mark.parametrize("x_exp,w_exp", [(-112, 0), (-120, 10), (-128, 10), (-140, 15), (60, -130)])
+def test_activations_near_the_bottom_of_the_fp32_range(gpu, oracle, t, x_exp, w_exp):
+    """Values whose bfloat16 terms, some or all, are below the smallest normal one (the values themselves below it, too), against
+    weights of any size: the error bound of every other input, and half a last place where the result is subnormal."""
+    in_dim, out_dim, tokens = 544, 70, 33
+    if t != F32 and w_exp < 0:
+        pytest.skip("binary16 weights and block scales do not reach that far down")
+    rng = np.random.default_rng(t + 1000 - x_exp)
+    raw = synth.make_weights(rng, t, out_dim, in_dim)
+    if t == F32:
+        raw = (raw.view(np.float32) * np.float32(2.0) ** w_exp).astype(np.float32).view(np.uint8)
+    elif t == F16:
+        raw = (raw.view(np.float16) * np.float16(2.0) ** min(w_exp, 10)).astype(np.float16).view(np.uint8)
+    x = (synth.make_activations(rng, tokens, in_dim).astype(np.float64) * 2.0 ** x_exp).astype(np.float32).reshape(tokens, in_dim)
+    row = raw.size // out_dim
+    dense = np.stack([oracle.dequantize(raw[r * row:(r + 1) * row], t, in_dim) for r in range(out_dim)]).astype(np.float64)
+    want, mags = x.astype(np.float64) @ dense.T, np.abs(x.astype(np.float64)) @ np.abs(dense).T
+    # as in test_terms_kernels_match_the_oracle (17 steps of 32)
+    bound = (2.0 ** -6 + 34 + 17 / 8 + 1 + 3 + 1) * 2.0 ** -24 * mags + 2.0 ** -150
+    w, xd, od = DevArray(raw), DevArray(x), DevArray(nbytes=4 * tokens * out_dim)
+    try:
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        got = od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim).astype(np.float64)
+    finally:
+        for a in (w, xd, od):
+            a.close()
+    assert np.all(np.abs(got - want) <= bound), (np.abs(got - want) / mags).max()
+    assert np.linalg.norm(got - want) <= 2.0 ** -22 * np.linalg.norm(want) + 2.0 ** -150 * np.sqrt(want.size)
