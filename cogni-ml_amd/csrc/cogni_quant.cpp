@@ -1401,7 +1401,8 @@ static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w
   if (packed_bytes > GEMM_STREAM_MAX_PACKED) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": packed activations of 2 GiB or more");
   uint64_t rows = 0;
   for (uint32_t i = 0; i < count; i++) rows += out_dims[i];
-  // planes that fit behind the packed activations (one matrix only)
+  // planes that fit behind the packed activations (one matrix only). cogni_gemm_workspace_bytes_split sizes a workspace for the tile
+  // kernels' split of the shape: what they do not split has no room for planes here either
   uint32_t planes_max = 1;
   if (count == 1) {
     const size_t fit = (workspace_bytes - packed_bytes) / ((size_t)tokens * out_dims[0] * sizeof(float));
@@ -1501,7 +1502,8 @@ int cogni_matmul_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias,
       return cogni_gemv_packed16_dev(&w_raw, w_type, workspace, 0, &out, &out_dim, 1, in_dim, tokens, stream);
     }
     // the short-prefill kernels from eighteen tokens: they add in another order than cogni_gemm_dev, whose bits this entry
-    // point gives at seventeen (what its test holds it to)
+    // point has always given at seventeen. That is the only reason: they are ahead there, too (2048 -> 520, tile kernel | these, us
+    // behind the pack: Q4_K 8.5 | 4.9, Q5_K 9.7 | 5.7, Q6_K 9.5 | 6.4), and the resident runners take them
     if (tokens > 17 && in_dim % 256 == 0 && gemm_stream_take(w_type, tokens, in_dim, out_dim)) {
       if (!w_raw || !x || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_matmul_dev: null device pointer");
       if (int rc = gemm_check("cogni_matmul_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;

@@ -39,8 +39,9 @@ GEMV_MFMA_Q5K_ENTRY(q5_k_gemv_mfma_f32_tbatch3, 3)
 GEMV_MFMA_Q5K_ENTRY(q5_k_gemv_mfma_f32_tbatch4, 4)
 GEMV_MFMA_Q5K_ADD_ENTRY(q5_k_gemv_mfma_add_f32_tbatch3, 3)
 GEMV_MFMA_Q5K_ADD_ENTRY(q5_k_gemv_mfma_add_f32_tbatch4, 4)
-// Behind the decode kernels, whose distances in the code object stay what they were: in front of and among them these cost the
-// projections of eight tokens 0.6 us (58.0 -> 58.7; 58.4 here), with the same instructions in every kernel that runs.
+// Behind the decode kernels, whose distances in the code object stay what they were: with these in front of and among them the
+// projections of eight tokens took 58.7 us, with them here 58.4 (58.0 without), in one session each and with the same instructions
+// in every kernel that runs. Why is not known, and the difference is hardly more than that of two sessions.
 GEMV_TOP1_LOGITS_ENTRY(q4_k_gemv_top1_logits_partial_f32, FmtQ4K, 1)
 GEMV_TOP1_LOGITS_ENTRY(q4_k_gemv_top1_logits_partial_f32_tbatch2, FmtQ4K, 2)
 GEMV_TOP1_LOGITS_ENTRY(q5_k_gemv_top1_logits_partial_f32, FmtQ5K, 1)

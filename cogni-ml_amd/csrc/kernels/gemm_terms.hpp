@@ -2,7 +2,7 @@
 //   out[m][o] = (residual ? residual[m][o] : 0) + sum_j x[m][j] * w(o, j)
 // These types have no fp16-precision prefill form (the reference computes them in full precision at every token count,
 // src/ml/gguf/quant_matmul.cr:216-368), so every operand is split into bfloat16 terms that lose nothing: an fp32 value is
-// exactly three of them (8 + 8 + 8 significand bits, by truncation; bfloat16 has the exponent range of fp32, so no scaling),
+// exactly three of them (8 + 8 + 8 significand bits, by truncation),
 // a binary16 weight two, a Q8_0 or IQ4_NL code one (the block scale is applied to the 32-value sum in fp32). Truncated terms are
 // below 2^-7 and 2^-15 of the value and have its sign, so what is left out of a product is a bias: all term products are taken
 // but the last one of fp32 weights, x2 w2, below 2^-30. 3 instructions of v_mfma_f32_16x16x32_bf16 per 16 x 16 x 32 for the
@@ -20,9 +20,10 @@
 // IQ4_NL, 64 tokens: 34 us against 18.7; with four steps in flight instead of one 40), so a wavefront loads its steps with
 // neighbouring lanes on neighbouring bytes of a row, up to two ahead, and turns them through a region of LDS that no other
 // wavefront uses: no barrier in the loop.
-// What bounds it: small calls the chain load - LDS - sums (4 us), large ones the vector instructions that split x (6.5 per
-// value and 64 rows, one of them the scale: Q8_0 1024 -> 3584, 200 tokens 14.2 us without it, 14.7 with) beside the waits of two wavefronts
-// per SIMD (4096 x 4096 Q8_0, 256 tokens, 41 us = 207 TFLOP/s of results, 620 of matrix instructions).
+// What bounds it: small calls the chain load - LDS - sums (4 us), large ones no single unit. Q8_0 1024 -> 3584, 200 tokens, 14.7 us:
+// 3900 vector instructions per working SIMD (6.8 us; two fifths of them split x, 6.5 per value and 64 rows, one of them the scale: 14.2 us
+// without it), 2.7 us of matrix instructions, and two wavefronts per SIMD that wait 36 % of their time for loads and LDS and 31 % for
+// an issue slot.
 // Measured, row kernels (Q8_0: one-pass launches of eight tokens) -> these: Q8_0 1024 -> 3584, 9 / 48 / 200 tokens 9.6 / 35 /
 // 143 -> 4.6 / 7.1 / 14.3 us; F16 2048 -> 2048, 33 tokens 39.9 -> 8.3; F32 4096 -> 4096, 33 tokens 173 -> 23; IQ4_NL 4096 ->
 // 4096, 1 / 64 tokens 39 / 1923 -> 9.5 / 19.

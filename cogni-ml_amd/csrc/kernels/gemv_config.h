@@ -335,7 +335,10 @@ static inline int gemm_terms_take(unsigned type, unsigned tokens, unsigned in_di
 }
 // The tile (16 tm tokens x 16 tn rows) that takes the least time when the launch runs in rounds of 256 workgroups: a round
 // of 1 x 1 tiles is the unit, the others measured against it (4096 columns of Q8_0, one round each: 6.4 / 8.8 / 13.9 / 21.2 /
-// 34.6 us above an empty launch).
+// 34.6 us above an empty launch). By LDS and registers two or three of the smaller tiles share a compute unit, but a second round
+// still costs a tile its time (Q8_0 4096 columns, 1 x 1: 256 workgroups 10.2 us, 448 15.7, 896 28.0). Of all five tiles, timed for the
+// four types at 1024 / 2048 / 4096 columns, 1024 / 3584 rows and 17 / 33 / 64 / 100 / 200 / 256 tokens, this picks the fastest one 144
+// times out of 144 (Q8_0 4096 -> 3584 at 100 tokens: 44.8 / 36.9 / 28.7 / 23.5 / 38.8 us).
 static inline unsigned gemm_terms_plan(unsigned tokens, unsigned out_dim, unsigned* tm, unsigned* tn) {
   static const unsigned shape[5][3] = {{1, 1, 100}, {1, 2, 140}, {2, 2, 220}, {2, 4, 335}, {4, 4, 545}};
   unsigned best = 0;
@@ -359,9 +362,14 @@ typedef struct {
 } GemmStreamPlan;
 static inline unsigned gemm_stream_tokens(unsigned tokens) { return tokens <= 32u ? 1u : 2u; }
 // Rows of a workgroup and k splits: the cheapest of (super-blocks a wavefront walks) x (time of one, by type and tile) x
-// (load), plus the plane sum. The load is what workgroups that share a compute unit cost each other: 1 up to one workgroup per
-// unit, 1.7 more for every further one (Q4_K, 64 tokens x 32 rows, 4096 columns: 128 workgroups 9.2 us, 256 10.0, 384 19.5, 960
-// 39.1; 64 rows: 192 workgroups 16.9, 480 31.9). Q6_K at 64 tokens x 64 rows does not fit the registers.
+// (load), plus the plane sum. The load is what workgroups that share a compute unit cost each other, charged as 1 up to 180
+// workgroups and 1.7 more for every 256 from there: steeper than it measures (Q4_K, 64 tokens x 32 rows, 4096 columns, 128 / 256 / 384 /
+// 960 workgroups: 9.2 / 10.0 / 19.5 / 39.1 us = 1 / 1.09 / 2.1 / 4.3, charged 1 / 1.5 / 2.4 / 6.2); the plane sum counts 3 us (4.0 to 6.4
+// behind a profiler). So the picks were checked, every tile and split by name, 12 shapes of 1024 to 12288 columns and 17 to 512 tokens
+// with weights from memory, us: Q4_K picks the fastest but once (12288 -> 4096 at 32 tokens 15.2, fastest 14.6), Q6_K is at most 5 % off
+// (4096 -> 12288 at 24 tokens 19.5 | 18.5), Q5_K takes 64 rows too early: 4096 -> 4096 at 48 tokens 12.0 where 32 rows without a split
+// take 10.0, 4096 -> 12288 at 24 tokens 16.7 | 15.4, 12288 -> 4096 at 32 and 48 tokens 6 % off, the rest level. (Its 64 tokens x 64
+// rows need more than the 256 registers and spill three; Q6_K has no such kernel.)
 static inline GemmStreamPlan gemm_stream_plan(unsigned type, unsigned tokens, unsigned in_dim, unsigned long long rows, unsigned planes_max) {
   static const unsigned us100[3][2][2] = {{{100, 160}, {150, 260}}, {{170, 260}, {200, 320}}, {{200, 420}, {260, 0}}};   // [type][t][rt]
   const unsigned ty = type == 14u ? 2u : (type == 13u ? 1u : 0u), t = gemm_stream_tokens(tokens), nkb = in_dim >> 8;

@@ -3,8 +3,10 @@
 //   out[m][o] = (residual ? residual[m][o] : 0) + sum_j x[m][j] * w(o, j)
 // with w(o, j) the float itself, the binary16 value widened, or d * table[q] of an 18-byte IQ4_NL block (d: f16, then 16
 // bytes: element e < 16 of the block is the low nibble of byte e, element 16 + e its high nibble; the last block of a row
-// is clipped to in_dim, quant_matmul.cr:296-312). cogni_gemv_dev takes them for one token of F32 and F16 (and the first few
-// of a short row); several tokens and IQ4_NL go to the matrix cores (gemm_terms.hpp; gemm_terms_take in gemv_config.h).
+// is clipped to in_dim, quant_matmul.cr:296-312). cogni_gemv_dev takes the F32 and F16 kernels for one token (and the first few
+// of a short row); several tokens, and IQ4_NL at any count, go to the matrix cores (gemm_terms.hpp; gemm_terms_take in
+// gemv_config.h). Nothing in the library launches the IQ4_NL kernel: it is for hosts that launch by name, and what the error of the
+// matrix-core kernel is measured against.
 // The kernels are plain: fp32 accumulation, no staging.
 //
 // Kernel ABI: (w_raw, x, residual, out, in_dim:u32, out_dim:u32, tokens:u32); residual may be null. Block 256 = four
@@ -86,7 +88,7 @@ extern "C" __global__ __launch_bounds__(GEMV_PLAIN_BLOCK) void f16_gemv_plain_f3
   gemv_plain_core<PlainF16>(w, x, residual, out, in_dim, out_dim, tokens);
 }
 
-// IQ4_NL (for hosts that launch by name; cogni_gemv_dev takes gemm_terms.hpp): two lanes per 32-element block, lane parity = half of the block (low nibbles: elements 0..15, high nibbles:
+// IQ4_NL: two lanes per 32-element block, lane parity = half of the block (low nibbles: elements 0..15, high nibbles:
 // 16..31), 32 blocks per step of a wavefront. The block scale is applied once per block half: d * sum(x * table[q]).
 extern "C" __global__ __launch_bounds__(GEMV_PLAIN_BLOCK) void iq4_nl_gemv_plain_f32(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                                                                     const float* __restrict__ residual, float* __restrict__ out,

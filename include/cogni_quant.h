@@ -122,11 +122,12 @@ int cogni_dequantize_dev(uint64_t w_raw, uint32_t w_type, uint64_t n_elements, u
  * bin/cuda_q4k_gemv_probe.cr:125); Q8_0 accepts any in_dim >= 1 (its last block is clipped, quant_matmul.cr:241,259).
  * Types: Q8_0, Q4_K, Q5_K, Q6_K on the kernels above; F32, F16 and IQ4_NL (the remaining arms of
  * QuantMatmul.matmul_add, quant_matmul.cr:30-32, 272-368), any in_dim >= 1: one token of F32 and F16 (and the first few of a
- * short row) on plain row kernels "f32_gemv_plain_f32" | "f16_gemv_plain_f32" | "iq4_nl_gemv_plain_f32" (w_raw, x, residual,
- * out, in_dim:u32, out_dim:u32, tokens:u32), block 256 (a wavefront per output row, any token count in one launch). More
+ * short row) on plain row kernels "f32_gemv_plain_f32" | "f16_gemv_plain_f32" (w_raw, x, residual, out, in_dim:u32,
+ * out_dim:u32, tokens:u32), block 256 (a wavefront per output row, any token count in one launch). More
  * tokens of F32 and F16, IQ4_NL at any token count, and Q8_0 with more than eight tokens (or with rows that are no multiple of
  * 256 from three) take the matrix cores in one launch to the same precision, operands as exact bfloat16 terms:
- * "<type>_gemm_terms_f32_<TM>x<TN>". Every other ggml type is refused with COGNI_ERR_UNSUPPORTED_TYPE and the reference's
+ * "<type>_gemm_terms_f32_<TM>x<TN>". The code object also holds "iq4_nl_gemv_plain_f32", a row kernel of the same parameters that
+ * only hosts launching by name reach. Every other ggml type is refused with COGNI_ERR_UNSUPPORTED_TYPE and the reference's
  * message. */
 int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residual, uint64_t out,
                    uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream);
