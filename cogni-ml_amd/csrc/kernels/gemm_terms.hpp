@@ -24,9 +24,9 @@
 // 3900 vector instructions per working SIMD (6.8 us; two fifths of them split x, 6.5 per value and 64 rows, one of them the scale: 14.2 us
 // without it), 2.7 us of matrix instructions, and two wavefronts per SIMD that wait 36 % of their time for loads and LDS and 31 % for
 // an issue slot.
-// Measured, row kernels (Q8_0: one-pass launches of eight tokens) -> these: Q8_0 1024 -> 3584, 9 / 48 / 200 tokens 9.6 / 35 /
-// 143 -> 4.6 / 7.1 / 14.3 us; F16 2048 -> 2048, 33 tokens 39.9 -> 8.3; F32 4096 -> 4096, 33 tokens 173 -> 23; IQ4_NL 4096 ->
-// 4096, 1 / 64 tokens 39 / 1923 -> 9.5 / 19.
+// Measured, weights from memory, row kernels (Q8_0: one-pass launches of eight tokens) -> these: Q8_0 1024 -> 3584, 9 / 48 / 200
+// tokens 9.6 / 35 / 143 -> 5.0 / 7.8 / 15.4 us; F16 2048 -> 2048, 33 tokens 41.8 -> 9.1; F32 4096 -> 4096, 33 tokens 174 -> 26; IQ4_NL
+// 4096 -> 4096, 1 / 64 tokens 40 / 1926 -> 10.5 / 21.
 #pragma once
 #include "common.hpp"
 #include "dequant.hpp"

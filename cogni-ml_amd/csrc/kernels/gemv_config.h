@@ -322,10 +322,11 @@ static inline GEMV_HD void gemm_terms_tile(unsigned id, unsigned mtiles, unsigne
   *nt = (l / mtiles) * GEMM_XCD_COUNT + x;
 }
 // Which calls take these kernels. F16 and F32: the row kernels re-read a row per four tokens and are level for the first few
-// of a short row (F16, us, row kernel | tile: 512 -> 512 at 4 tokens 3.3 | 3.5, at 8 4.6 | 3.5; 2048 -> 2048 at 2 tokens
-// 6.2 | 6.3, at 3 7.5 | 6.4; 4096 -> 4096 at 2 13.5 | 10.0). IQ4_NL: always (one token of 1024 -> 3584 11.6 | 4.4). Q8_0: what
-// the one-pass kernels leave - more than eight tokens (9 of 1024 -> 3584: 9.6 | 4.6), and rows that are no multiple of 256 from
-// three (4000 -> 4096 at 2 tokens 10.0 | 9.1, at 3 12.3 | 9.1; 1000 -> 2041 at 2 4.5 | 4.7, at 3 5.3 | 4.7).
+// of a short row (F16, weights from memory, us, row kernel | tile: 512 -> 512 at 4 tokens 3.3 | 3.6, at 8 4.7 | 3.6; 2048 -> 2048 at 2
+// tokens 7.8 | 7.0, from the cache level, at 3 9.7 | 7.1; 4096 -> 4096 at 2 16.1 | 11.9; F32 512 -> 512 at 4 3.4 | 3.8, at 5 4.1 | 3.9).
+// IQ4_NL: always (one token of 1024 -> 3584 11.5 | 4.5). Q8_0: what the one-pass kernels leave - more than eight tokens (9 of 1024 ->
+// 3584: 9.6 | 5.0), and rows that are no multiple of 256 from three (at 2 tokens 4000 -> 4096 11.1 | 10.2, 1000 -> 2041 4.7 | 5.2; a third
+// costs the row kernels 2.3 and 0.8 more, the tiles nothing).
 #define GEMM_TERMS_Q80_FROM 3u
 static inline int gemm_terms_take(unsigned type, unsigned tokens, unsigned in_dim) {
   if (type == 20) return 1;
