@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -365,10 +366,19 @@ int cogni_gemv_image_stats(uint32_t* slots, uint32_t* in_use, uint32_t* pinned, 
   return 0;
 }
 
+// Tokens a launch of the term kernels may have: it has fewer than 2^32 threads, counted for the smallest tile (16 tokens x 16 rows), and
+// larger tiles are fewer workgroups. 0 from 2^27 rows on: such a matrix stays with the kernels whose workgroups walk the rows.
+static uint32_t gemm_terms_launch_tokens(uint32_t out_dim) {
+  const uint64_t ntiles = ((out_dim + 15ull) / 16 + GEMM_XCD_COUNT - 1) / GEMM_XCD_COUNT * GEMM_XCD_COUNT;
+  return (uint32_t)(0xFFFFFFFFull / (64 * GEMM_TERMS_WAVES) / ntiles * 16);
+}
+
 // Passes over the weights cogni_gemv_dev makes for one call (with an image slot at hand): the same rules as the call itself.
 int32_t cogni_gemv_passes(uint32_t w_type, uint32_t tokens, uint32_t in_dim, uint32_t out_dim) {
   if ((!gemv_type(w_type) && !plain_type(w_type)) || tokens == 0 || in_dim == 0 || out_dim == 0) return -1;
-  if (plain_type(w_type) || gemm_terms_take(w_type, tokens, in_dim)) return 1;
+  const uint32_t terms = gemm_terms_take(w_type, tokens, in_dim) ? gemm_terms_launch_tokens(out_dim) : 0;
+  if (terms) return (int32_t)(((uint64_t)tokens + terms - 1) / terms);
+  if (plain_type(w_type)) return 1;
   if (k_quant(w_type) && (in_dim % 256) != 0) return -1;
   const uint32_t from = gemv_mt_from(w_type, in_dim, out_dim);
   if (from && tokens >= from) return (int32_t)((tokens + GEMV_MT_MAX_TOKENS - 1) / GEMV_MT_MAX_TOKENS);
@@ -577,16 +587,24 @@ int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residua
     return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for fused matmul: ") + type_name(w_type));
   if (!w_raw || !x || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_dev: null device pointer");
   if (in_dim == 0 || out_dim == 0 || tokens == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_dev: zero dimension");
-  if (gemm_terms_take(w_type, tokens, in_dim)) {   // several tokens of F32, F16, IQ4_NL or Q8_0 on the matrix cores
-    uint32_t tm, tn;
-    const uint32_t grid = gemm_terms_plan(tokens, out_dim, &tm, &tn);
-    char name[48];
-    std::snprintf(name, sizeof name, "%s_gemm_terms_f32_%ux%u", type_prefix(w_type), tm, tn);
-    void* params[] = {&w_raw, &x, &residual, &out, &in_dim, &out_dim, &tokens};
-    return launch(name, grid, 64 * GEMM_TERMS_WAVES, 0, params, stream);
+  const uint32_t terms = gemm_terms_take(w_type, tokens, in_dim) ? gemm_terms_launch_tokens(out_dim) : 0;
+  if (terms) {   // several tokens of F32, F16, IQ4_NL or Q8_0 on the matrix cores
+    uint32_t m = 0;
+    for (uint32_t t0 = 0; t0 < tokens; t0 += m) {
+      m = std::min(tokens - t0, terms);
+      uint32_t tm, tn;
+      const uint32_t grid = gemm_terms_plan(m, out_dim, &tm, &tn);
+      char name[48];
+      std::snprintf(name, sizeof name, "%s_gemm_terms_f32_%ux%u", type_prefix(w_type), tm, tn);
+      uint64_t xm = x + (uint64_t)t0 * in_dim * 4, om = out + (uint64_t)t0 * out_dim * 4;
+      uint64_t rm = residual ? residual + (uint64_t)t0 * out_dim * 4 : 0;
+      void* params[] = {&w_raw, &xm, &rm, &om, &in_dim, &out_dim, &m};
+      if (int rc = launch(name, grid, 64 * GEMM_TERMS_WAVES, 0, params, stream)) return rc;
+    }
+    return 0;
   }
   if (plain_type(w_type)) {   // any token count in one launch: a wavefront per row, the workgroups walk the rows
-    const char* name = w_type == COGNI_TYPE_F32 ? "f32_gemv_plain_f32" : "f16_gemv_plain_f32";
+    const char* name = w_type == COGNI_TYPE_F32 ? "f32_gemv_plain_f32" : (w_type == COGNI_TYPE_F16 ? "f16_gemv_plain_f32" : "iq4_nl_gemv_plain_f32");
     const uint32_t groups = (out_dim + 3) / 4;
     void* params[] = {&w_raw, &x, &residual, &out, &in_dim, &out_dim, &tokens};
     return launch(name, groups < 65536u ? groups : 65536u, 256, 0, params, stream);

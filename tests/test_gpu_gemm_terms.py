@@ -231,3 +231,32 @@ def test_activations_near_the_bottom_of_the_fp32_range(gpu, oracle, t, x_exp, w_
             a.close()
     assert np.all(np.abs(got - want) <= bound), (np.abs(got - want) / mags).max()
     assert np.linalg.norm(got - want) <= 2.0 ** -22 * np.linalg.norm(want) + 2.0 ** -150 * np.sqrt(want.size)
+
+
+@pytest.mark.parametrize("t", [F32, F16])
+def test_more_tokens_than_a_launch_has_threads_for(gpu, t):
+    """2^24 tokens of one tile of rows are 2^23 workgroups of 512 threads, and a launch has fewer than 2^32: the call goes in several.
+    The weights are powers of two and zeros, so every output is exact."""
+    in_dim, out_dim, tokens = 3, 2, (1 << 24) + 17
+    dense = np.array([[0, 0, -0.5], [2, 0, 0]], dtype=np.float32 if t == F32 else np.float16)
+    x = np.random.default_rng(t).standard_normal((tokens, in_dim), dtype=np.float32)
+    want = np.stack([x[:, 2] * np.float32(-0.5), x[:, 0] * np.float32(2)], axis=1)
+    w, xd, od = DevArray(dense), DevArray(x), DevArray(np.full((tokens, out_dim), np.nan, dtype=np.float32))
+    try:
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens)
+        assert np.array_equal(od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim), want)
+        quant.gemv_dev(w.ptr, t, xd.ptr, od.ptr, in_dim, out_dim, tokens, od.ptr)   # in place
+        assert np.array_equal(od.read(np.float32, tokens * out_dim).reshape(tokens, out_dim), want + want)
+        assert quant.gemv_passes(t, tokens, in_dim, out_dim) == 2 and quant.gemv_passes(t, 1 << 20, in_dim, out_dim) == 1
+    finally:
+        for a in (w, xd, od):
+            a.close()
+
+
+def test_token_limit_of_a_launch(gpu):
+    """The launches of one call, by the number of rows; matrices of 2^27 rows keep the kernels that walk them."""
+    for out_dim in (1, 129, 3584, 151936, 1 << 26):
+        tiles = -(-out_dim // 128) * 8
+        most = ((1 << 32) - 1) // 512 // tiles * 16
+        assert quant.gemv_passes(IQ4_NL, most, 32, out_dim) == 1 and quant.gemv_passes(IQ4_NL, most + 1, 32, out_dim) == 2
+    assert quant.gemv_passes(IQ4_NL, 100, 32, (1 << 27) + 1) == 1
