@@ -125,7 +125,8 @@ int cogni_dequantize_dev(uint64_t w_raw, uint32_t w_type, uint64_t n_elements, u
  * short row) on plain row kernels "f32_gemv_plain_f32" | "f16_gemv_plain_f32" (w_raw, x, residual, out, in_dim:u32,
  * out_dim:u32, tokens:u32), block 256 (a wavefront per output row, any token count in one launch). More
  * tokens of F32 and F16, IQ4_NL at any token count, and Q8_0 with more than eight tokens (or with rows that are no multiple of
- * 256 from three) take the matrix cores in one launch to the same precision, operands as exact bfloat16 terms:
+ * 256 from three) take the matrix cores in one launch (of fewer than 2^32 threads: from 2^24 tokens of up to 128 rows, or as many outputs
+ * of taller matrices, in several) to the same precision, operands as exact bfloat16 terms:
  * "<type>_gemm_terms_f32_<TM>x<TN>". The code object also holds "iq4_nl_gemv_plain_f32", a row kernel of the same parameters that
  * only hosts launching by name reach. Every other ggml type is refused with COGNI_ERR_UNSUPPORTED_TYPE and the reference's
  * message. */
