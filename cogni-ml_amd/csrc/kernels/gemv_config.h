@@ -272,44 +272,36 @@ static inline int gemm_q4k_use_wide(unsigned out_dim, unsigned tokens) {
 
 // ---- prefill GEMM: which tile a workgroup takes. Workgroups go to the 8 XCDs round-robin (id % 8), each XCD has its own
 // L2 and 32 compute units, and a GEMM workgroup has a compute unit to itself, so the workgroups id = 8 l + x with the
-// same l / 32 run side by side on XCD x. They are given a block of bnt x bmt = 32 neighbouring tiles (bmt token tiles of
-// bnt weight tiles each): a weight tile is then fetched into that L2 once for bmt workgroups and an x tile once for bnt,
-// where one token tile per XCD (every workgroup of an XCD on the same x, each on weights of its own) made every L2 fill
-// with all the weights. One token tile: the blocks degenerate to that older numbering, which is kept as it is.
+// same l / 32 run side by side on XCD x. Every XCD gets an equal share of the tiles (they are numbered in one line and it takes
+// a contiguous piece of it), so that none has a round of workgroups more than the others, and the line winds through the
+// matrix so that 32 neighbours on it are a compact block: gn weight tiles of one token tile after each other, then the
+// same of the next token tile, then the next gn weight tiles. A weight tile is then fetched into that L2 once for the token tiles
+// of its block and an x tile once for gn weight tiles. (Whole blocks of 4 token tiles x 8 weight tiles dealt round-robin, as this was
+// before, left XCDs idle where the token tiles do not divide by four; us before -> now: Q4_K 4096 -> 30720 in 192-row tiles, 384 tokens
+// 140.9 -> 105.9, 640 tokens 269 -> 197; Q6_K 12288 -> 4096 in 128-row tiles, 640 tokens 190 -> 97.5; 512, 1024, 2048 tokens level.)
 #define GEMM_XCD_COUNT 8u
 #define GEMM_XCD_UNITS 32u
-static inline GEMV_HD unsigned gemm_block_mt(unsigned mtiles) { return mtiles >= 4u ? 4u : (mtiles >= 2u ? 2u : 1u); }
-// A block is bnt weight tiles x bmt token tiles: 32 tiles where there are enough of them, fewer when the launch has
-// fewer than 256 tiles, so that the blocks still go round all 8 XCDs.
-static inline GEMV_HD void gemm_block_shape(unsigned mtiles, unsigned ntiles, unsigned* bmt, unsigned* bnt) {
-  *bmt = gemm_block_mt(mtiles);
-  const unsigned per_xcd = (mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT;   // tiles an XCD gets when they are dealt evenly
-  const unsigned want = (per_xcd + *bmt - 1u) / *bmt, cap = GEMM_XCD_UNITS / *bmt;
-  *bnt = want < 1u ? 1u : (want > cap ? cap : want);
+// weight tiles of a block: 32 tiles of up to 4 token tiles where there are enough of them, fewer when the launch has fewer
+// than 256 tiles
+static inline GEMV_HD unsigned gemm_block_nt(unsigned mtiles, unsigned ntiles) {
+  const unsigned bmt = mtiles >= 4u ? 4u : mtiles;
+  const unsigned per_xcd = (mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT;
+  const unsigned want = (per_xcd + bmt - 1u) / bmt, cap = GEMM_XCD_UNITS / bmt;
+  return want < 1u ? 1u : (want > cap ? cap : want);
 }
 static inline GEMV_HD unsigned gemm_grid_x(unsigned mtiles, unsigned ntiles) {
-  if (mtiles < 2u) return GEMM_XCD_COUNT * ((mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT);
-  unsigned bmt, bnt;
-  gemm_block_shape(mtiles, ntiles, &bmt, &bnt);
-  const unsigned nb = ((ntiles + bnt - 1u) / bnt) * ((mtiles + bmt - 1u) / bmt);
-  return GEMM_XCD_COUNT * bmt * bnt * ((nb + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT);
+  return GEMM_XCD_COUNT * ((mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT);
 }
-// false: this workgroup has no tile (the grid is rounded up to whole blocks)
+// false: this workgroup has no tile (the grid is rounded up to equal shares)
 static inline GEMV_HD bool gemm_tile_of(unsigned id, unsigned mtiles, unsigned ntiles, unsigned* mt, unsigned* nt) {
-  const unsigned x = id % GEMM_XCD_COUNT, l = id / GEMM_XCD_COUNT;
-  if (mtiles < 2u) {
-    const unsigned per = (mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT, vt = x * per + l;
-    *mt = vt / ntiles;
-    *nt = vt - *mt * ntiles;
-    return vt < mtiles * ntiles;
-  }
-  unsigned bmt, bnt;
-  gemm_block_shape(mtiles, ntiles, &bmt, &bnt);
-  const unsigned units = bmt * bnt, nbn = (ntiles + bnt - 1u) / bnt, nb = nbn * ((mtiles + bmt - 1u) / bmt);
-  const unsigned b = (l / units) * GEMM_XCD_COUNT + x, i = l % units;
-  *nt = (b % nbn) * bnt + i / bmt;
-  *mt = (b / nbn) * bmt + i % bmt;
-  return b < nb && *nt < ntiles && *mt < mtiles;
+  const unsigned total = mtiles * ntiles, per = (total + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT;
+  const unsigned vt = (id % GEMM_XCD_COUNT) * per + id / GEMM_XCD_COUNT;
+  if (vt >= total) return false;
+  const unsigned gn = gemm_block_nt(mtiles, ntiles), g = vt / (gn * mtiles), i = vt - g * gn * mtiles;
+  const unsigned left = ntiles - g * gn, n = left < gn ? left : gn;   // (the last group of weight tiles may be a smaller one)
+  *mt = i / n;
+  *nt = g * gn + i % n;
+  return true;
 }
 
 // ---- several tokens of F32, F16, IQ4_NL or Q8_0 weights (gemm_terms.hpp): eight wavefronts = eight k-slices per tile.
