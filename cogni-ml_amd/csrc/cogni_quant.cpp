@@ -1146,39 +1146,39 @@ static uint32_t gemm_splits_of(uint32_t tiles, uint32_t in_dim) {
   if (s > nkb / 2) s = nkb / 2;
   return s < 2 ? 1 : s;
 }
-// Rows of the workgroup tile and k splits of a launch. Every type has two tile heights, 192 and 128 rows (<type>_gemm_f16 and
-// <type>_gemm_n128_f16), Q4_K also the 256-row tile of the eight-wavefront kernel (no k split). A launch runs in rounds of
-// 256 workgroups and a workgroup walks ceil(super-blocks / splits) super-blocks; per super-block a 128-row tile costs
-// GEMM_N128_COST_X100 per cent of a 192-row one and a 256-row tile GEMM_WIDE_ROUND_COST_X100 per cent; the cheapest plan wins
+// Rows of the workgroup tile and k splits of a launch. Every type has tiles of 192 and 128 rows (<type>_gemm_f16 and
+// <type>_gemm_n128_f16), Q4_K and Q6_K also the 256-row tile of the eight-wavefront kernels (<type>_gemm_wide_f16, taken without a
+// k split). A launch runs in rounds of 256 workgroups and a workgroup walks ceil(super-blocks / splits) super-blocks; what a tile
+// costs per super-block against one of 192 rows is gemm_tile_cost (gemv_config.h), and the cheapest plan wins
 // (the 4096-row projections at 512 tokens: 88 tiles x 2 splits = 176 workgroups of 192 rows, or 128 x 2 = 256 of the
 // smaller ones). `split` false: the plan for a workspace without planes. COGNI_GEMM_N128=0 | 1 and COGNI_GEMM_WIDE=0 | 1
 // override the choice (measurement knobs: 1 takes that tile wherever its kernel can run).
-#define GEMM_N128_COST_X100 75u
 struct GemmShape {
   uint32_t bn, splits;
 };
 static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, bool split = true) {
   const uint32_t mtiles = (tokens + 127) / 128, nkb = in_dim / 256;
-  auto eval = [&](uint32_t bn, uint32_t cost_x100, uint32_t* cost) {
+  auto eval = [&](uint32_t bn, uint64_t* cost) {
     const uint32_t tiles = mtiles * ((out_dim + bn - 1) / bn), s = split && bn != 256 ? gemm_splits_of(tiles, in_dim) : 1u;
-    *cost = ((tiles * s + 255u) / 256u) * ((nkb + s - 1) / s) * cost_x100;
+    *cost = (uint64_t)((tiles * s + 255u) / 256u) * ((nkb + s - 1) / s) * gemm_tile_cost(w_type, bn);
     return s;
   };
-  uint32_t cost192 = 0, cost128 = 0, cost256 = 0;
-  const uint32_t s192 = eval(192, 100u, &cost192), s128 = eval(128, GEMM_N128_COST_X100, &cost128);
+  uint64_t cost192 = 0, cost128 = 0, cost256 = 0;
+  const uint32_t s192 = eval(192, &cost192), s128 = eval(128, &cost128);
   bool n128 = cost128 < cost192;
   if (const char* e = std::getenv("COGNI_GEMM_N128")) {
     if (e[0] == '0') n128 = false;
     if (e[0] == '1') n128 = true;
   }
   GemmShape best = n128 ? GemmShape{128, s128} : GemmShape{192, s192};
-  // the eight-wavefront kernel: Q4_K launches that are not split and fill whole rounds of its tiles
-  if (w_type == COGNI_TYPE_Q4_K && best.splits == 1) {
-    (void)eval(256, GEMM_WIDE_ROUND_COST_X100, &cost256);
-    bool wide = gemm_q4k_use_wide(out_dim, tokens) && cost256 < (n128 ? cost128 : cost192);
+  // the eight-wavefront kernels: more tokens than the 64-token tiles have (Q6_K: and activations of a token tile below 4 GiB, which
+  // its 32-bit offsets reach)
+  if (w_type != COGNI_TYPE_Q5_K && tokens > 64 && (w_type != COGNI_TYPE_Q6_K || nkb < 65536u)) {
+    (void)eval(256, &cost256);
+    bool wide = cost256 < (n128 ? cost128 : cost192);
     if (const char* e = std::getenv("COGNI_GEMM_WIDE")) {
       if (e[0] == '0') wide = false;
-      if (e[0] == '1') wide = true;
+      if (e[0] == '1' && best.splits == 1) wide = true;
     }
     if (wide) best = GemmShape{256, 1};
   }
@@ -1249,7 +1249,7 @@ static GemmPlan gemm_plan(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, ui
       {{"q4_k_gemm_f16", "q4_k_gemm_n128_f16"}, {"q4_k_gemm_m64_f16", "q4_k_gemm_m64_n128_f16"}},
       {{"q5_k_gemm_f16", "q5_k_gemm_n128_f16"}, {"q5_k_gemm_m64_f16", "q5_k_gemm_m64_n128_f16"}},
       {{"q6_k_gemm_f16", "q6_k_gemm_n128_f16"}, {"q6_k_gemm_m64_f16", "q6_k_gemm_m64_n128_f16"}}};
-  p.kernel = wide ? "q4_k_gemm_wide_f16" : names[w_type == COGNI_TYPE_Q6_K ? 2 : (w_type == COGNI_TYPE_Q5_K ? 1 : 0)][m64][n128];
+  p.kernel = wide ? (w_type == COGNI_TYPE_Q6_K ? "q6_k_gemm_wide_f16" : "q4_k_gemm_wide_f16") : names[w_type == COGNI_TYPE_Q6_K ? 2 : (w_type == COGNI_TYPE_Q5_K ? 1 : 0)][m64][n128];
   const uint32_t ntiles = (out_dim + shape.bn - 1) / shape.bn;
   p.grid_x = gemm_grid_x(mtiles, ntiles);
   p.block = wide ? 512 : 256;
@@ -1311,15 +1311,17 @@ int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
     return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the fused gate/up SwiGLU GEMM: ") + type_name(w_type));
   if (!w_gate || !w_up || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemm_packed_swiglu_dev: null device pointer");
   if (int rc = gemm_check("cogni_gemm_packed_swiglu_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;
-  // a tile is 128 tokens x 96 rows of each matrix
-  const uint32_t mtiles = (tokens + 127) / 128, ntiles = (out_dim + 95) / 96;
+  const uint32_t mtiles = (tokens + 127) / 128;
+  const bool wide = gemm_swiglu_use_wide(out_dim, tokens);
+  const uint32_t rows = wide ? 128 : 96;   // a tile is 128 tokens x `rows` rows of each matrix
   void* params[] = {&w_gate, &w_up, &workspace, &out, &in_dim, &out_dim, &tokens};
-  return launch(tokens <= 64 ? "q4_k_gemm_swiglu_m64_f16" : "q4_k_gemm_swiglu_f16", gemm_grid_x(mtiles, ntiles), 256, 0, params, stream);
+  return launch(wide ? "q4_k_gemm_swiglu_wide_f16" : (tokens <= 64 ? "q4_k_gemm_swiglu_m64_f16" : "q4_k_gemm_swiglu_f16"),
+                gemm_grid_x(mtiles, (out_dim + rows - 1) / rows), wide ? 512 : 256, 0, params, stream);
 }
 
 // Several matrices of one type and row length against one block of packed activations, as one launch: no k split (the list
-// is what fills the chip), the tile height that needs fewer rounds of 256 workgroups (a 128-row tile costs
-// GEMM_N128_COST_X100 per cent of a 192-row one), the 64-token kernels for up to 64 tokens.
+// is what fills the chip), the tile whose rounds of 256 workgroups cost least (gemm_tile_cost; the 256-row tile: Q4_K), the 64-token
+// kernels for up to 64 tokens.
 namespace {
 struct GemmManyArgs {   // the kernels' first parameter (kernels/gemm_q4k.hpp)
   uint64_t w[6];
@@ -1339,46 +1341,35 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
     if (!w_raw[i] || !outs[i]) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
     if (int rc = gemm_check(who, w_type, in_dim, out_dims[i], tokens, workspace, workspace_bytes)) return rc;
   }
-  const uint32_t mtiles = (tokens + 127) / 128, nkb = in_dim / 256;
-  const size_t packed_bytes = cogni_gemm_workspace_bytes(w_type, in_dim, tokens);
-  // a matrix that alone gets the 256-row tiles of the eight-wavefront kernel (many tokens, many rows) keeps them: it is
-  // launched by itself, unsplit as the list is; the others form the list
-  uint32_t listed[6], nlisted = 0;
-  for (uint32_t i = 0; i < count; i++) {
-    if (gemm_shape(w_type, in_dim, out_dims[i], tokens, false).bn == 256) {
-      if (int rc = gemm_packed_launch(who, w_raw[i], w_type, workspace, packed_bytes, 0, 0, outs[i], in_dim, out_dims[i], tokens, stream)) return rc;
-    } else {
-      listed[nlisted++] = i;
-    }
+  if (count == 1)
+    return gemm_packed_launch(who, w_raw[0], w_type, workspace, cogni_gemm_workspace_bytes(w_type, in_dim, tokens), 0, 0, outs[0], in_dim,
+                              out_dims[0], tokens, stream);
+  const uint64_t mtiles = (tokens + 127) / 128;
+  const bool m64 = tokens <= 64;
+  uint32_t bn = 0;
+  uint64_t least = ~0ull;
+  for (uint32_t rows : {192u, 128u, 256u}) {
+    if (rows == 256 && (w_type != COGNI_TYPE_Q4_K || m64)) continue;
+    uint64_t tiles = 0;
+    for (uint32_t i = 0; i < count; i++) tiles += (out_dims[i] + rows - 1) / rows;
+    const uint64_t cost = (mtiles * tiles + 255) / 256 * gemm_tile_cost(w_type, rows);
+    if (cost < least) least = cost, bn = rows;
   }
-  if (nlisted == 0) return 0;
-  if (nlisted == 1) {
-    const uint32_t i = listed[0];
-    return gemm_packed_launch(who, w_raw[i], w_type, workspace, packed_bytes, 0, 0, outs[i], in_dim, out_dims[i], tokens, stream);
-  }
-  uint64_t tiles[2] = {0, 0};   // 192-row, 128-row
-  for (uint32_t k = 0; k < nlisted; k++) {
-    tiles[0] += (out_dims[listed[k]] + 191) / 192;
-    tiles[1] += (out_dims[listed[k]] + 127) / 128;
-  }
-  const uint64_t cost192 = ((mtiles * tiles[0] + 255) / 256) * nkb * 100, cost128 = ((mtiles * tiles[1] + 255) / 256) * nkb * GEMM_N128_COST_X100;
-  const bool n128 = cost128 < cost192, m64 = tokens <= 64;
-  const uint32_t bn = n128 ? 128 : 192;
   GemmManyArgs list{};
   uint32_t end = 0;
-  for (uint32_t k = 0; k < nlisted; k++) {
-    const uint32_t i = listed[k];
-    list.w[k] = w_raw[i];
-    list.out[k] = outs[i];
-    list.out_dim[k] = out_dims[i];
-    list.tile_end[k] = end += (out_dims[i] + bn - 1) / bn;
+  for (uint32_t i = 0; i < count; i++) {
+    list.w[i] = w_raw[i];
+    list.out[i] = outs[i];
+    list.out_dim[i] = out_dims[i];
+    list.tile_end[i] = end += (out_dims[i] + bn - 1) / bn;
   }
-  list.count = nlisted;
+  list.count = count;
   static const char* const names[2][2][2] = {
       {{"q4_k_gemm_many_f16", "q4_k_gemm_many_n128_f16"}, {"q4_k_gemm_many_m64_f16", "q4_k_gemm_many_m64_n128_f16"}},
       {{"q5_k_gemm_many_f16", "q5_k_gemm_many_n128_f16"}, {"q5_k_gemm_many_m64_f16", "q5_k_gemm_many_m64_n128_f16"}}};
   void* params[] = {&list, &workspace, &in_dim, &tokens};
-  return launch(names[w_type == COGNI_TYPE_Q5_K][m64][n128], gemm_grid_x(mtiles, end), 256, 0, params, stream);
+  if (bn == 256) return launch("q4_k_gemm_many_wide_f16", gemm_grid_x((uint32_t)mtiles, end), 512, 0, params, stream);
+  return launch(names[w_type == COGNI_TYPE_Q5_K][m64][bn == 128], gemm_grid_x((uint32_t)mtiles, end), 256, 0, params, stream);
 }
 
 static int swiglu_pack_check(const char* who, uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes,
@@ -1403,11 +1394,14 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
   if (int rc = swiglu_pack_check("cogni_gemm_packed_swiglu_pack_dev", w_gate, w_up, w_type, workspace, workspace_bytes, next_type, next_workspace,
                                  next_workspace_bytes, in_dim, out_dim, tokens))
     return rc;
-  const uint32_t mtiles = (tokens + 127) / 128, ntiles = (out_dim + 95) / 96;
+  const uint32_t mtiles = (tokens + 127) / 128;
+  const bool wide = gemm_swiglu_use_wide(out_dim, tokens);
+  const uint32_t rows = wide ? 128 : 96;   // a tile is 128 tokens x `rows` rows of each matrix
   void* params[] = {&w_gate, &w_up, &workspace, &out, &next_workspace, &in_dim, &out_dim, &tokens};
-  static const char* const names[2][2] = {{"q4_k_gemm_swiglu_pack_q4k_f16", "q4_k_gemm_swiglu_pack_q4k_m64_f16"},
-                                          {"q4_k_gemm_swiglu_pack_q6k_f16", "q4_k_gemm_swiglu_pack_q6k_m64_f16"}};
-  return launch(names[next_type == COGNI_TYPE_Q6_K][tokens <= 64], gemm_grid_x(mtiles, ntiles), 256, 0, params, stream);
+  static const char* const names[2][3] = {{"q4_k_gemm_swiglu_pack_q4k_f16", "q4_k_gemm_swiglu_pack_q4k_m64_f16", "q4_k_gemm_swiglu_pack_q4k_wide_f16"},
+                                          {"q4_k_gemm_swiglu_pack_q6k_f16", "q4_k_gemm_swiglu_pack_q6k_m64_f16", "q4_k_gemm_swiglu_pack_q6k_wide_f16"}};
+  return launch(names[next_type == COGNI_TYPE_Q6_K][wide ? 2 : tokens <= 64], gemm_grid_x(mtiles, (out_dim + rows - 1) / rows), wide ? 512 : 256, 0,
+                params, stream);
 }
 
 // Short prefills: the weights streamed through workgroups of four wavefronts (kernels/gemm_stream.hpp). The same packed

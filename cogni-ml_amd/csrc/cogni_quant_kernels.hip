@@ -10,6 +10,7 @@
 #include "kernels/gemm_q4k.hpp"
 #include "kernels/gemm_q4k_wide.hpp"
 #include "kernels/gemm_q6k.hpp"
+#include "kernels/gemm_q6k_wide.hpp"
 #include "kernels/norm.hpp"
 
 GEMV_MFMA_ENTRY(q4_k_gemv_mfma_f32_tbatch2, 2)

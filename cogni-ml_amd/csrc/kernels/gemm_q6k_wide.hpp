@@ -1,0 +1,240 @@
+// Prefill GEMM over raw Q6_K weights with eight wavefronts per workgroup: the wavefront roles of gemm_q4k_wide.hpp with the
+// operands of gemm_q6k.hpp (block layout, element order and assembly of the codes there).
+//
+//   q6_k_gemm_wide_f16 (w_raw, xp, bias|null, out:f32 [m][out_dim], in_dim:u32, out_dim:u32, m:u32, bias_stride:u32)
+//                      block 512, grid (gemm_grid_x(ceil(m/128), ceil(out_dim/256)), k splits), no dynamic LDS (112 KiB static);
+//                      with k splits > 1 `out` is `splits` planes of [m][out_dim] and bias is null, as for q6_k_gemm_f16
+//
+// A workgroup owns 128 tokens x 256 rows; wavefront (row quarter nh, k half kh) accumulates 128 tokens x 64 rows over half
+// kh of every super-block and copies the bytes that it decodes itself, so no two wavefronts share weights. Those are, of each
+// row, ql[64 kh, +64) and qh[32 kh, +32): six pieces of 16 bytes, 6 KiB = six copies a super-block into a region of its own;
+// the eight scale bytes of the half and d go from global memory to the lanes that need them.
+// Two x tiles of a whole super-block (128 KiB) and these 48 KiB do not fit LDS. So x is staged by half super-blocks, the
+// k-steps 0..3 and 4..7 of both k halves (32 KiB each, always in the same buffer): while one is consumed the other is filled,
+// copies issued three k-steps ahead of the barrier that hands them over. Every load goes through a buffer descriptor: as 64-bit
+// addresses the offsets of the copies cost 14 more registers, which spilled, and the compiler waited for all loads in flight in front
+// of the operand reads. 12288 -> 4096 at 2048 tokens: 211 us = 0.98 PFLOP/s, 237 on 128 x 128 tiles.
+#pragma once
+#include "gemm_q4k_wide.hpp"
+#include "gemm_q6k.hpp"
+
+__shared__ uint4 gemm_q6w_x0[2048];        // [kh][k-step 0..3][k-group][128 tokens]
+__shared__ uint4 gemm_q6w_x1[2048];        // the same of k-steps 4..7
+__shared__ uint4 gemm_q6w_wbuf[8 * 384];   // [wavefront][64 rows][ql 4 pieces, qh 2 pieces]
+
+extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void q6_k_gemm_wide_f16(
+    const uint8_t* w, const uint4* xp, const float* bias, float* out, u32 in_dim, u32 out_dim, u32 m, u32 bias_stride) {
+  constexpr u32 BS = 210;
+  const u32 tid = threadIdx.x, lane = tid & 63;
+  const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const u32 nh = wave & 3, kh = wave >> 2;
+  const u32 j = lane & 31, kg = lane >> 5;
+  // k split: super-blocks [kb0, kb0 + nkb) into plane blockIdx.y behind `out`
+  const u32 nkb_all = in_dim >> 8;
+  const u32 kb0 = blockIdx.y * nkb_all / gridDim.y, nkb = (blockIdx.y + 1) * nkb_all / gridDim.y - kb0;
+  out += (size_t)blockIdx.y * m * out_dim;
+  const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM, ntiles = (out_dim + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN;
+  u32 mt, nt;
+  if (!gemm_tile_of(blockIdx.x, mtiles, ntiles, &mt, &nt)) return;
+  const size_t row_bytes = (size_t)nkb_all * BS;
+  // constants of the code assembly, kept in registers (as literals each (a & mask) | b would be two instructions): the masks
+  // in scalar ones, of which an instruction takes one
+  u32 mask_lo = 0x000F000Fu, mask_hi = 0x00F000F0u, magic_lo = 0x64006400u, magic_hi = 0x54005400u, m3_lo = 0x00300030u, m3_hi = 0x03000300u;
+  asm volatile("" : "+s"(mask_lo), "+s"(mask_hi), "+s"(m3_lo), "+s"(m3_hi));
+  asm volatile("" : "+v"(magic_lo), "+v"(magic_hi));
+
+  const u32 row0 = nt * GEMM_WIDE_BN + nh * 64;        // first weight row of this wavefront
+  const u32 base_row = min(row0, out_dim - 1);
+  // loads through a buffer descriptor: scalar base, scalar offset of the super-block, a 32-bit offset per lane
+  const __amdgpu_buffer_rsrc_t wrsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + (size_t)base_row * row_bytes + (size_t)kb0 * BS), 0, 0xFFFFFFFFu, 0x00027000);
+  // copy i of this wavefront: piece p = 64 i + lane is piece p % 6 of wave-local row p / 6
+  u32 woff[6];
+#pragma unroll
+  for (int i = 0; i < 6; i++) {
+    const u32 p = 64u * i + lane, r = p / 6u, part = p - 6u * r;
+    woff[i] = (min(row0 + r, out_dim - 1) - base_row) * (u32)row_bytes + (part < 4u ? 64u * kh + 16u * part : 128u + 32u * kh + 16u * (part - 4u));
+  }
+  u32 soff[2];   // scales of the half, row c of this lane (d is 16 - 8 kh bytes further)
+#pragma unroll
+  for (int c = 0; c < 2; c++) soff[c] = (min(row0 + 32 * c + j, out_dim - 1) - base_row) * (u32)row_bytes + 192u + 8u * kh;
+  const u32 wrow = wave * 384 + j * 6 + kg;   // the lane's first ql piece of its row c = 0 (c = 1: 192 further)
+  const __amdgpu_buffer_rsrc_t xrsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(xp + ((size_t)mt * nkb_all + kb0) * 4096), 0, 0xFFFFFFFFu, 0x00027000);
+
+  float16_t acc[4][2];
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[r][c][v] = 0.0f;
+
+  auto copy_w = [&](u32 kb, int i) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(wrsrc, (lds_void*)(gemm_q6w_wbuf + wave * 384 + i * 64), 16, woff[i], kb * BS, 0, 0);
+  };
+  uint2 nsc[2];
+  u32 nd[2];
+  auto load_sc = [&](u32 kb, int c) {
+    nsc[c] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(wrsrc, soff[c], kb * BS, 0));
+    nd[c] = (u32)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(wrsrc, soff[c], kb * BS + (16u - 8u * kh), 0);
+  };
+  // copy i of half `hs` of a super-block's x: KiB 8 i + wave of the buffer, 16 of each kh
+  const u32 xw = (wave & 7u) * 64;
+  auto copy_x = [&](u32 kb, int hs, int i) {
+    const u32 src = kb * 65536u + ((i >> 1) * 2048 + hs * 1024 + (i & 1) * 512 + xw) * 16u;   // uniform
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lds_void*)((hs ? gemm_q6w_x1 : gemm_q6w_x0) + i * 512 + xw), 16, lane * 16, src, 0, 0);
+  };
+
+  GemmRaw6 cur[2];
+  u32 S[2][4];
+  uint4 A[2][4];
+  half8_t B[2][2];
+  auto take_raw = [&]() {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      cur[c].qa = gemm_q6w_wbuf[wrow + 192 * c];
+      cur[c].qb = gemm_q6w_wbuf[wrow + 192 * c + 2];
+      cur[c].qh = gemm_q6w_wbuf[wrow + 192 * c + 4];
+    }
+  };
+  // d * sc of the four 16-value sub-blocks of the lane's group (scale bytes kg, kg + 2, kg + 4, kg + 6 of the half's eight)
+  auto decode_scales = [&]() {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const float d = h2f(nd[c]);
+      const u32 lo = nsc[c].x >> (8 * kg), hi = nsc[c].y >> (8 * kg);
+      S[c][0] = h2_dup(d * (float)(int)(signed char)(lo & 0xFFu));
+      S[c][1] = h2_dup(d * (float)(int)(signed char)((lo >> 16) & 0xFFu));
+      S[c][2] = h2_dup(d * (float)(int)(signed char)(hi & 0xFFu));
+      S[c][3] = h2_dup(d * (float)(int)(signed char)((hi >> 16) & 0xFFu));
+    }
+  };
+  auto build_b = [&](half8_t (&Bd)[2], int t) {   // as in gemm_q6k_core
+    const int qd = t >> 1, h8 = t & 1, hi = qd >> 1;
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const uint4 Q = (qd & 1) ? cur[c].qb : cur[c].qa;
+      const u32 qa = h8 ? Q.z : Q.x, qb = h8 ? Q.w : Q.y;
+      const u32 ha = h8 ? cur[c].qh.z : cur[c].qh.x, hb = h8 ? cur[c].qh.w : cur[c].qh.y;
+      const u32 mask = hi ? mask_hi : mask_lo, magic = hi ? magic_hi : magic_lo, m3 = hi ? m3_hi : m3_lo;
+      const u32 off = hi ? 0xD600D600u : 0xE420E420u;   // half2(-96) : half2(-1056)
+      const int sl = (qd & 1) ? 2 : 4, sr = (qd & 1) ? 6 : 4;
+      const u32 sc = S[c][qd];
+      u32 n0 = (qa & mask) | magic, n1 = ((qa >> 8) & mask) | magic, n2 = (qb & mask) | magic, n3 = ((qb >> 8) & mask) | magic;
+      asm("" : "+v"(n0), "+v"(n1), "+v"(n2), "+v"(n3));
+      uint4 bw;
+      bw.x = h2_sub_mul(((ha << sl) & m3) | n0, off, sc);
+      bw.y = h2_sub_mul(((ha >> sr) & m3) | n1, off, sc);
+      bw.z = h2_sub_mul(((hb << sl) & m3) | n2, off, sc);
+      bw.w = h2_sub_mul(((hb >> sr) & m3) | n3, off, sc);
+      Bd[c] = *reinterpret_cast<const half8_t*>(&bw);
+    }
+  };
+  const u32 xrow = kh * 1024 + kg * 128 + j;
+  auto read_a = [&](uint4 (&Ad)[4], int t) {   // 32 lanes read 512 contiguous bytes
+    const uint4* arow = ((t & 4) ? gemm_q6w_x1 : gemm_q6w_x0) + xrow + (t & 3) * 256;
+#pragma unroll
+    for (int r = 0; r < 4; r++) Ad[r] = arow[r * 32];
+  };
+
+#pragma unroll
+  for (int i = 0; i < 6; i++) copy_w(0, i);
+#pragma unroll
+  for (int c = 0; c < 2; c++) load_sc(0, c);
+#pragma unroll
+  for (int i = 0; i < 4; i++) copy_x(0, 0, i);
+#pragma unroll
+  for (int i = 0; i < 4; i++) copy_x(0, 1, i);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  take_raw();
+  read_a(A[0], 0);
+  decode_scales();
+  build_b(B[0], 0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+
+  for (u32 kb = 0; kb < nkb; kb++) {
+    const u32 kn = min(kb + 1, nkb - 1);   // the last iteration copies its own tile again; it is not used
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      const int p = t & 1;
+      // The raw bytes were taken into registers in the last k-step of the iteration before, so the region is free. x: half 0
+      // is free behind the barrier of k-step 2, half 1 behind that of k-step 6; the copies into one follow the first reads of the
+      // other, in front of which the compiler waits for every load in flight.
+      if (t == 0) {
+#pragma unroll
+        for (int i = 0; i < 6; i++) copy_w(kn, i);
+      }
+      if (t == 3) {
+        read_a(A[p ^ 1], t + 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) copy_x(kn, 0, i);
+      }
+      if (t == 5) {
+        load_sc(kn, 0);
+        load_sc(kn, 1);
+      }
+      if (t < 7) {
+        if (t != 3) read_a(A[p ^ 1], t + 1);
+        build_b(B[p ^ 1], t + 1);
+      } else {
+        take_raw();
+        read_a(A[0], 0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) copy_x(kn, 1, i);
+        decode_scales();
+        build_b(B[0], 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const half8_t Ar = *reinterpret_cast<const half8_t*>(&A[p][r]);
+#pragma unroll
+        for (int c = 0; c < 2; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(B[p][c], Ar, acc[r][c], 0, 0, 0);
+      }
+#pragma unroll
+      for (int c = 0; c < 2; c++) asm volatile("" : "+v"(B[p ^ 1][c]));
+      if (t < 7) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 7, 0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+        }
+      } else {
+        __builtin_amdgcn_sched_group_barrier(0x020, 4, 0);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (t == 2) {
+        // half 1 of this super-block (copies of the last k-step before; the six weight copies of k-step 0 are younger) is there
+        // and half 0 has been read, for every wavefront
+        asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (t == 6) {
+        // half 0 of the next super-block and this wavefront's next weights are there, half 1 has been read
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // the raw bytes are in registers before the next copies overwrite the region
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last (unused) copies
+  __syncthreads();
+  float4* const h0 = reinterpret_cast<float4*>(gemm_q6w_x0);
+  float4* const h1 = reinterpret_cast<float4*>(gemm_q6w_x1);
+  if (kh == 0) gemm_wide_epilogue_half<0, 2>(acc, h0, h1, bias, out, out_dim, m, mt, nt, nh, j, kg, lane, bias_stride);
+  else gemm_wide_epilogue_half<1, 2>(acc, h1, h0, bias, out, out_dim, m, mt, nt, nh, j, kg, lane, bias_stride);
+}

@@ -254,20 +254,21 @@ static inline unsigned long long gemv_mt_image_bytes(unsigned type, unsigned in_
   return (unsigned long long)gemv_mt_padded_sb(in_dim) * (8192u + 1024u);
 }
 
-// ---- prefill GEMM: which Q4_K kernel an unsplit launch takes (gemm_q4k.hpp: 128 x 192 tiles, four wavefronts;
-// gemm_q4k_wide.hpp: 128 x 256 tiles, eight wavefronts). One workgroup per compute unit either way, so a launch runs in
-// rounds of 256 tiles. A round of wide tiles measures 1.24 times a round of the narrower ones (a third more work, done
-// with 25 % fewer activation bytes copied per flop and two wavefronts per SIMD), so the wide kernel is taken where it
-// saves enough whole rounds: 2048 x 12288 is 3 rounds instead of 4, 512 x 12288 (192 wide tiles: a quarter of the
-// compute units idle) and 1024 x 12288 (2 rounds either way) stay with the narrow tiles.
+// ---- prefill GEMM: what a tile costs. A workgroup has a compute unit to itself, so a launch runs in rounds of 256 tiles; a round
+// of 192-row tiles is 100, of 128-row tiles 75, of the 256-row tiles of the eight-wavefront kernels 131 (Q4_K; a third more work with 25 %
+// fewer activation bytes copied per flop and two wavefronts per SIMD) or 107 (Q6_K, whose 192-row tile copies no raw blocks). Measured,
+// Q4_K lists of 4096 columns, us a round: 47 to 53 | 37 to 39 | 61 to 69; so 30720 rows take, in 192 | 128 | 256-row tiles, 151.7 | 151.9 |
+// 134.7 at 512 tokens, 94.2 | 78.1 | 69.5 at 256, 105.9 | 113.1 | 121.4 at 384, 562 | 581 | 532 at 2048. Q6_K 12288 -> 4096: 314 | 237 | 211 at
+// 2048 tokens, 151 | 120 | 155 at 1024.
 #define GEMM_ROUND_TILES 256u
-#define GEMM_WIDE_ROUND_COST_X100 124u
-static inline int gemm_q4k_use_wide(unsigned out_dim, unsigned tokens) {
-  const unsigned mtiles = (tokens + 127u) / 128u;
-  const unsigned narrow = mtiles * ((out_dim + 191u) / 192u), wide = mtiles * ((out_dim + 255u) / 256u);
-  if (wide < GEMM_ROUND_TILES) return 0;
-  const unsigned rn = (narrow + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES, rw = (wide + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
-  return rw * GEMM_WIDE_ROUND_COST_X100 < rn * 100u;
+static inline unsigned gemm_tile_cost(unsigned type, unsigned rows) { return rows == 192u ? 100u : (rows == 128u ? 75u : (type == 14u ? 107u : 131u)); }
+// gate | up with SwiGLU: tiles of 96 rows of both matrices (four wavefronts) or of 128 (eight). 4096 -> 12288, us: 441 | 410 at 2048
+// tokens, 225 | 208 at 1024, 114 | 123 at 512, 58 | 59 at 256; 2048 -> 4096 at 1024 61.6 | 41.3; 3072 -> 8192 at 300 76.7 | 45.5.
+static inline int gemm_swiglu_use_wide(unsigned out_dim, unsigned tokens) {
+  const unsigned long long mtiles = (tokens + 127u) / 128u;
+  const unsigned long long rn = (mtiles * ((out_dim + 95u) / 96u) + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
+  const unsigned long long rw = (mtiles * ((out_dim + 127u) / 128u) + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
+  return tokens > 64u && rw * gemm_tile_cost(12u, 256u) < rn * gemm_tile_cost(12u, 192u);
 }
 
 // ---- prefill GEMM: which tile a workgroup takes. Workgroups go to the 8 XCDs round-robin (id % 8), each XCD has its own
