@@ -510,6 +510,20 @@ int cogni_gemv_packed16_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_ty
                 gemv_mt_lds_bytes(w_type) + GEMV_MT_X16_LDS_EXTRA, params, stream);
 }
 
+int cogni_gemv_packed16_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t image, uint64_t out, uint32_t next_type,
+                                        uint64_t next_image, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemv_packed16_swiglu_pack_dev";
+  if (!w_gate || !w_up || !image || !next_image) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  if (w_type != COGNI_TYPE_Q4_K || !gemv16_shape(w_type, in_dim, tokens))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": Q4_K, 1..16 tokens, in_dim a multiple of 256 up to 12288");
+  if (next_type != COGNI_TYPE_Q6_K || !gemv_mt_supported(next_type, 2, out_dim))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": the next matrix is Q6_K, out_dim a multiple of 256 up to 12288");
+  const uint32_t groups = out_dim / 16;
+  void* params[] = {&w_gate, &w_up, &image, &out, &next_image, &in_dim, &out_dim, &tokens};
+  return launch("q4_k_gemv_mt16_swiglu_pack_q6k_f32", groups < 256u ? groups : 256u, GEMV_MT_WAVES * 64,
+                gemv_mt_lds_bytes(w_type) + GEMV_MT_X16_LDS_EXTRA, params, stream);
+}
+
 int cogni_gemv_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t image, uint64_t out, uint32_t in_dim,
                                  uint32_t out_dim, uint32_t tokens, void* stream) {
   if (!w_gate || !w_up || !image || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_swiglu_dev: null device pointer");

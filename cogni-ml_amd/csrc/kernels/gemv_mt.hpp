@@ -20,6 +20,8 @@
 //     contract, src/ml/cuda/kernels/q4k_gemv_probe.ptx:437-768, q5k_gemv_probe.ptx:237 and q6k_gemv_probe.ptx:977: x rows at stride in_dim, outs
 //     at stride out_dim; these kernels handle eight tokens where those handle four).
 //   q4_k_gemv_mt_swiglu_f32 (w_gate, w_up, image, out, in_dim, out_dim, tokens)
+//   q4_k_gemv_mt16_swiglu_pack_q6k_f32 (w_gate, w_up, image, out | null, next_image, in_dim, out_dim, tokens): up to sixteen tokens, and the
+//     products written as the sixteen-token image a Q6_K matrix of out_dim columns reads (what pack_x_mt16_q6k_f16 makes of them)
 //
 // Arithmetic. The matrix cores multiply 16 activation rows x K values by K x 16 weight rows. The weights stay exact: a
 // masked pair of codes read as two binary16 numbers is code * 2^-24 (code * 2^-20 for codes left four bits up), the
@@ -622,10 +624,16 @@ struct MtArgs {
 // that row's index (out[0][m * gridDim.x + blockIdx.x], top_ids[same]; of equal values the lowest row wins): the partial
 // results top1_reduce_f32 finishes, as q6_k_gemv_top1_partial_f32 writes them for one token. With `logits` the row values are
 // stored as well (logits[m * rows + row]).
-template <class F, int SBW, int T, bool SWIGLU = false, bool TOP1 = false>
+// NEXT (SWIGLU, sixteen tokens): the products also go to `next` as the sixteen-token Q6_K image of the matrix behind (out[0] may be
+// null then; rows[0] a multiple of 256 up to GEMV_MT_MAX_IN_DIM): single binary16 terms need no scale of a whole super-block, and the
+// sixteen rows of a group are one of its sub-blocks, so a workgroup has all that it takes. The FFN half of a layer, 4096 -> 12288 -> 4096,
+// 13 tokens, without the pack launch 36.6 -> 35.2 us.
+template <class F, int SBW, int T, bool SWIGLU = false, bool TOP1 = false, bool NEXT = false>
 __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __restrict__ image,
                                              const float* __restrict__ residual, u32 in_dim, u32 tokens,
-                                             u32* __restrict__ top_ids = nullptr, float* __restrict__ logits = nullptr) {
+                                             u32* __restrict__ top_ids = nullptr, float* __restrict__ logits = nullptr,
+                                             uint8_t* __restrict__ next = nullptr) {
+  static_assert(!NEXT || (SWIGLU && F::NTOK == 16), "the image of the next matrix: sixteen tokens, gate | up");
   constexpr bool STREAM = SBW > 2;
   constexpr int NTOK = F::NTOK;   // token rows of the partial sums: 8, or 16 single-term tokens
   static_assert(NTOK == 8 || (NTOK == 16 && !TOP1), "sixteen tokens: rows or SwiGLU, no top-1");
@@ -657,6 +665,13 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
 
   u32 grp = blockIdx.x;
   if (grp >= ngroups) return;
+  if constexpr (NEXT) {   // the super-blocks past the row's end that fill the next image up to a multiple of 8 (there are more groups than those)
+    const u32 nsb2 = a.rows[0] >> 8, nsbp2 = gemv_mt_padded_sb(a.rows[0]), sb = nsb2 + blockIdx.x;
+    if (sb < nsbp2) {
+      *reinterpret_cast<uint4*>(next + (size_t)sb * 8192 + 16 * tid) = make_uint4(0u, 0u, 0u, 0u);
+      if (tid < 64) *reinterpret_cast<uint4*>(next + (size_t)nsbp2 * 8192 + (size_t)sb * 1024 + 16 * tid) = make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
   float top_v = -__builtin_inff();   // TOP1: the best row this thread has seen in its place of the row groups
   u32 top_i = 0xFFFFFFFFu;
 
@@ -737,7 +752,41 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if constexpr (SWIGLU) {
+    if constexpr (NEXT) {
+      // sixteen lanes are the rows of a token: one sub-block of the next matrix's super-block, the absent tokens as zeros
+      const u32 r = tid & 15, m = (u32)tid >> 4, row = grp * 16 + r;
+      if (m < 16u) {
+        float v = 0.f;
+        if (m < tokens) {
+          float g = 0.f, u = 0.f;
+#pragma unroll
+          for (u32 k = 0; k < GEMV_MT_WAVES; k++) {
+            g += part[((k * GEMV_MT_TMAX + 0) * NTOK + m) * 16 + r];
+            u += part[((k * GEMV_MT_TMAX + 1) * NTOK + m) * 16 + r];
+          }
+          v = swiglu_one(g, u);
+          if (a.out[0]) a.out[0][(size_t)m * a.rows[0] + row] = v;
+        }
+        const float h = (float)(_Float16)v;
+        const u32 sb = row >> 8, s = (row >> 4) & 15;
+        // halves 0, 2, 1, 3 of the quad as eight bytes (mt_pack16_store_q6k), its sum in that function's order
+        const float h1 = MT_DPP(h, 0x55), h2 = MT_DPP(h, 0xAA), h3 = MT_DPP(h, 0xFF);   // quad_perm: lane 1, 2, 3 of the quad
+        if ((r & 3) == 0)
+          *reinterpret_cast<mt_half4*>(next + ((size_t)(sb * 8 + (s >> 1)) * 64 + (r >> 2) * 16 + m) * 16 + 8 * (s & 1)) =
+              (mt_half4){(_Float16)h, (_Float16)h2, (_Float16)h1, (_Float16)h3};
+        float sm = h + MT_DPP(h, MT_QUAD_1032);
+        sm += MT_DPP(sm, MT_QUAD_2301);
+        sm += MT_DPP(sm, MT_ROW_HALF_MIRROR);
+        sm += MT_DPP(sm, MT_ROW_ROR8);
+        const float s16 = 0.0625f;
+        const _Float16 sh = (_Float16)(sm * s16), sl = (_Float16)fmaf(sm, s16, -(float)sh);
+        if (r == 0) {
+          _Float16* ap = reinterpret_cast<_Float16*>(next + (size_t)gemv_mt_padded_sb(a.rows[0]) * 8192 + (size_t)sb * 1024 + ((s >> 2) * 16 + m) * 16) + (s & 3);
+          ap[0] = sh;
+          ap[4] = sl;
+        }
+      }
+    } else if constexpr (SWIGLU) {
       for (u32 o = tid; o < 16u * tokens; o += GEMV_MT_WAVES * 64) {
         const u32 r = o & 15, m = o >> 4;
         float g = 0.f, u = 0.f;
@@ -981,17 +1030,17 @@ GEMV_MT_TOP1_ENTRY(q6_k_gemv_mt_top1_partial_f32, MtQ6K)
 // (w_gate, w_up, image, out, in_dim, out_dim, tokens): out[m][o] = silu(gate . x) * (up . x); block 512, grid = min(256,
 // ceil(out_dim / 16)), dynamic shared memory as q4_k_gemv_mt_f32. The parameter list of q4_k_dual_gemv_swiglu_f32 with the
 // image in the place of x and the token count behind.
-template <class F>
+template <class F, bool NEXT = false>
 __device__ __forceinline__ void gemv_mt_swiglu_dispatch(const uint8_t* w_gate, const uint8_t* w_up, const uint8_t* image, float* out,
-                                                        u32 in_dim, u32 out_dim, u32 tokens) {
+                                                        u32 in_dim, u32 out_dim, u32 tokens, uint8_t* next = nullptr) {
   const MtArgs a = {{w_gate, w_up, nullptr}, {out, nullptr, nullptr}, {out_dim, out_dim, 0u}};
   switch (gemv_mt_padded_sb(in_dim) >> 3) {
-    case 1: gemv_mt_core<F, 1, 2, true>(a, image, nullptr, in_dim, tokens); break;
-    case 2: gemv_mt_core<F, 2, 2, true>(a, image, nullptr, in_dim, tokens); break;
-    case 3: gemv_mt_core<F, 3, 1, true>(a, image, nullptr, in_dim, tokens); break;
-    case 4: gemv_mt_core<F, 4, 1, true>(a, image, nullptr, in_dim, tokens); break;
-    case 5: gemv_mt_core<F, 5, 1, true>(a, image, nullptr, in_dim, tokens); break;
-    default: gemv_mt_core<F, 6, 1, true>(a, image, nullptr, in_dim, tokens); break;
+    case 1: gemv_mt_core<F, 1, 2, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
+    case 2: gemv_mt_core<F, 2, 2, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
+    case 3: gemv_mt_core<F, 3, 1, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
+    case 4: gemv_mt_core<F, 4, 1, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
+    case 5: gemv_mt_core<F, 5, 1, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
+    default: gemv_mt_core<F, 6, 1, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
   }
 }
 extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void q4_k_gemv_mt_swiglu_f32(
@@ -1002,4 +1051,9 @@ extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void q4_k_gemv_mt_sw
 extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void q4_k_gemv_mt16_swiglu_f32(
     const uint8_t* w_gate, const uint8_t* w_up, const uint8_t* image, float* out, u32 in_dim, u32 out_dim, u32 tokens) {
   gemv_mt_swiglu_dispatch<MtQ4Kx16>(w_gate, w_up, image, out, in_dim, out_dim, tokens);
+}
+// the same with the products as the image of the Q6_K matrix behind it: out_dim a multiple of 256 up to GEMV_MT_MAX_IN_DIM
+extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void q4_k_gemv_mt16_swiglu_pack_q6k_f32(
+    const uint8_t* w_gate, const uint8_t* w_up, const uint8_t* image, float* out, uint8_t* next, u32 in_dim, u32 out_dim, u32 tokens) {
+  gemv_mt_swiglu_dispatch<MtQ4Kx16, true>(w_gate, w_up, image, out, in_dim, out_dim, tokens, next);
 }

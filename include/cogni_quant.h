@@ -221,6 +221,12 @@ int cogni_add_rmsnorm_pack16_dev(uint64_t x, uint64_t add, uint64_t norm, uint64
                                  uint64_t image, uint32_t dim, uint32_t tokens, float eps, void* stream);
 int cogni_gemv_packed16_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t image, uint64_t out, uint32_t in_dim,
                                    uint32_t out_dim, uint32_t tokens, void* stream);
+/* The same with the products also (out = 0: only) written as the sixteen-token image of the matrix behind them: next_type Q6_K,
+ * out_dim a multiple of 256 up to 12288, next_image as large as cogni_gemv_image_bytes(next_type, out_dim, 8) - byte for byte what
+ * cogni_gemv_pack16_dev makes of them. Kernel "q4_k_gemv_mt16_swiglu_pack_q6k_f32" (w_gate, w_up, image, out, next_image, in_dim, out_dim,
+ * tokens), grid, block and dynamic shared memory of "q4_k_gemv_mt16_swiglu_f32". */
+int cogni_gemv_packed16_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t image, uint64_t out, uint32_t next_type,
+                                        uint64_t next_image, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream);
 int cogni_gemv_packed16_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t image, uint64_t residual, const uint64_t* out,
                             const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
 /* The gate and up projections and the SwiGLU against an image, one launch:
