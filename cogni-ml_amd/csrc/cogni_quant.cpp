@@ -1185,14 +1185,15 @@ static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, 
     if (e[0] == '1') n128 = true;
   }
   GemmShape best = n128 ? GemmShape{128, s128} : GemmShape{192, s192};
-  // the eight-wavefront kernels: more tokens than the 64-token tiles have (Q6_K: and activations of a token tile below 4 GiB, which
-  // its 32-bit offsets reach)
-  if (w_type != COGNI_TYPE_Q5_K && tokens > 64 && (w_type != COGNI_TYPE_Q6_K || nkb < 65536u)) {
+  // the eight-wavefront kernels, for more tokens than the 64-token tiles have and launches that are not split: Q4_K by
+  // gemm_q4k_use_wide; Q6_K where the 192-row tiles are not the better of the two others (and the activations of a token tile stay
+  // below 4 GiB, which its 32-bit offsets reach)
+  if (best.splits == 1 && tokens > 64 && (w_type == COGNI_TYPE_Q4_K || (w_type == COGNI_TYPE_Q6_K && nkb < 65536u))) {
     (void)eval(256, &cost256);
-    bool wide = cost256 < (n128 ? cost128 : cost192);
+    bool wide = (w_type == COGNI_TYPE_Q4_K ? gemm_q4k_use_wide(out_dim, tokens) != 0 : n128) && cost256 < (n128 ? cost128 : cost192);
     if (const char* e = std::getenv("COGNI_GEMM_WIDE")) {
       if (e[0] == '0') wide = false;
-      if (e[0] == '1' && best.splits == 1) wide = true;
+      if (e[0] == '1') wide = true;
     }
     if (wide) best = GemmShape{256, 1};
   }
@@ -1244,7 +1245,7 @@ int cogni_gemm_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias, u
 // of 8, y = k splits), block.
 struct GemmPlan {
   const char* kernel;
-  uint32_t grid_x, splits, block;
+  uint32_t tiles_x, grid_x, splits, block;   // workgroups launched and grid reported, in x
 };
 static GemmPlan gemm_plan(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, size_t workspace_bytes) {
   const uint32_t mtiles = (tokens + 127) / 128;
@@ -1265,6 +1266,7 @@ static GemmPlan gemm_plan(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, ui
       {{"q6_k_gemm_f16", "q6_k_gemm_n128_f16"}, {"q6_k_gemm_m64_f16", "q6_k_gemm_m64_n128_f16"}}};
   p.kernel = wide ? (w_type == COGNI_TYPE_Q6_K ? "q6_k_gemm_wide_f16" : "q4_k_gemm_wide_f16") : names[w_type == COGNI_TYPE_Q6_K ? 2 : (w_type == COGNI_TYPE_Q5_K ? 1 : 0)][m64][n128];
   const uint32_t ntiles = (out_dim + shape.bn - 1) / shape.bn;
+  p.tiles_x = gemm_tiles_grid(mtiles, ntiles);
   p.grid_x = gemm_grid_x(mtiles, ntiles);
   p.block = wide ? 512 : 256;
   return p;
@@ -1294,13 +1296,13 @@ static int gemm_packed_launch(const char* who, uint64_t w_raw, uint32_t w_type, 
   uint32_t splits = p.splits;
   if (splits == 1) {
     void* params[] = {&w_raw, &workspace, &add, &out, &in_dim, &out_dim, &tokens, &add_stride};
-    return launch(p.kernel, p.grid_x, p.block, 0, params, stream);
+    return launch(p.kernel, p.tiles_x, p.block, 0, params, stream);
   }
   uint64_t planes = workspace + need, none = 0;
   uint32_t total = tokens * out_dim, zero = 0;
   {
     void* params[] = {&w_raw, &workspace, &none, &planes, &in_dim, &out_dim, &tokens, &zero};
-    int rc = launch(p.kernel, p.grid_x, p.block, 0, params, stream, splits);
+    int rc = launch(p.kernel, p.tiles_x, p.block, 0, params, stream, splits);
     if (rc != 0) return rc;
   }
   void* params[] = {&planes, &add, &out, &total, &out_dim, &splits, &add_stride};
@@ -1330,7 +1332,7 @@ int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
   const uint32_t rows = wide ? 128 : 96;   // a tile is 128 tokens x `rows` rows of each matrix
   void* params[] = {&w_gate, &w_up, &workspace, &out, &in_dim, &out_dim, &tokens};
   return launch(wide ? "q4_k_gemm_swiglu_wide_f16" : (tokens <= 64 ? "q4_k_gemm_swiglu_m64_f16" : "q4_k_gemm_swiglu_f16"),
-                gemm_grid_x(mtiles, (out_dim + rows - 1) / rows), wide ? 512 : 256, 0, params, stream);
+                gemm_tiles_grid(mtiles, (out_dim + rows - 1) / rows), wide ? 512 : 256, 0, params, stream);
 }
 
 // Several matrices of one type and row length against one block of packed activations, as one launch: no k split (the list
@@ -1382,8 +1384,8 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
       {{"q4_k_gemm_many_f16", "q4_k_gemm_many_n128_f16"}, {"q4_k_gemm_many_m64_f16", "q4_k_gemm_many_m64_n128_f16"}},
       {{"q5_k_gemm_many_f16", "q5_k_gemm_many_n128_f16"}, {"q5_k_gemm_many_m64_f16", "q5_k_gemm_many_m64_n128_f16"}}};
   void* params[] = {&list, &workspace, &in_dim, &tokens};
-  if (bn == 256) return launch("q4_k_gemm_many_wide_f16", gemm_grid_x((uint32_t)mtiles, end), 512, 0, params, stream);
-  return launch(names[w_type == COGNI_TYPE_Q5_K][m64][bn == 128], gemm_grid_x((uint32_t)mtiles, end), 256, 0, params, stream);
+  if (bn == 256) return launch("q4_k_gemm_many_wide_f16", gemm_tiles_grid((uint32_t)mtiles, end), 512, 0, params, stream);
+  return launch(names[w_type == COGNI_TYPE_Q5_K][m64][bn == 128], gemm_tiles_grid((uint32_t)mtiles, end), 256, 0, params, stream);
 }
 
 static int swiglu_pack_check(const char* who, uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes,
@@ -1414,7 +1416,7 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
   void* params[] = {&w_gate, &w_up, &workspace, &out, &next_workspace, &in_dim, &out_dim, &tokens};
   static const char* const names[2][3] = {{"q4_k_gemm_swiglu_pack_q4k_f16", "q4_k_gemm_swiglu_pack_q4k_m64_f16", "q4_k_gemm_swiglu_pack_q4k_wide_f16"},
                                           {"q4_k_gemm_swiglu_pack_q6k_f16", "q4_k_gemm_swiglu_pack_q6k_m64_f16", "q4_k_gemm_swiglu_pack_q6k_wide_f16"}};
-  return launch(names[next_type == COGNI_TYPE_Q6_K][wide ? 2 : tokens <= 64], gemm_grid_x(mtiles, (out_dim + rows - 1) / rows), wide ? 512 : 256, 0,
+  return launch(names[next_type == COGNI_TYPE_Q6_K][wide ? 2 : tokens <= 64], gemm_tiles_grid(mtiles, (out_dim + rows - 1) / rows), wide ? 512 : 256, 0,
                 params, stream);
 }
 

@@ -261,6 +261,14 @@ static inline unsigned long long gemv_mt_image_bytes(unsigned type, unsigned in_
 // 134.7 at 512 tokens, 94.2 | 78.1 | 69.5 at 256, 105.9 | 113.1 | 121.4 at 384, 562 | 581 | 532 at 2048. Q6_K 12288 -> 4096: 314 | 237 | 211 at
 // 2048 tokens, 151 | 120 | 155 at 1024.
 #define GEMM_ROUND_TILES 256u
+// A single Q4_K matrix takes the 256-row tiles where they fill whole rounds and save enough of the 192-row ones' (its plan
+// is what cogni_gemm_plan names; lists and gate | up go by the costs alone).
+static inline int gemm_q4k_use_wide(unsigned out_dim, unsigned tokens) {
+  const unsigned mtiles = (tokens + 127u) / 128u;
+  const unsigned narrow = mtiles * ((out_dim + 191u) / 192u), wide = mtiles * ((out_dim + 255u) / 256u);
+  const unsigned rn = (narrow + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES, rw = (wide + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
+  return wide >= GEMM_ROUND_TILES && rw * 124u < rn * 100u;
+}
 static inline unsigned gemm_tile_cost(unsigned type, unsigned rows) { return rows == 192u ? 100u : (rows == 128u ? 75u : (type == 14u ? 107u : 131u)); }
 // gate | up with SwiGLU: tiles of 96 rows of both matrices (four wavefronts) or of 128 (eight). 4096 -> 12288, us: 441 | 410 at 2048
 // tokens, 225 | 208 at 1024, 114 | 123 at 512, 58 | 59 at 256; 2048 -> 4096 at 1024 61.6 | 41.3; 3072 -> 8192 at 300 76.7 | 45.5.
@@ -284,20 +292,30 @@ static inline int gemm_swiglu_use_wide(unsigned out_dim, unsigned tokens) {
 #define GEMM_XCD_UNITS 32u
 // weight tiles of a block: 32 tiles of up to 4 token tiles where there are enough of them, fewer when the launch has fewer
 // than 256 tiles
+static inline GEMV_HD unsigned gemm_block_mt(unsigned mtiles) { return mtiles >= 4u ? 4u : (mtiles >= 2u ? 2u : 1u); }
 static inline GEMV_HD unsigned gemm_block_nt(unsigned mtiles, unsigned ntiles) {
-  const unsigned bmt = mtiles >= 4u ? 4u : mtiles;
+  const unsigned bmt = gemm_block_mt(mtiles);
   const unsigned per_xcd = (mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT;
   const unsigned want = (per_xcd + bmt - 1u) / bmt, cap = GEMM_XCD_UNITS / bmt;
   return want < 1u ? 1u : (want > cap ? cap : want);
 }
-static inline GEMV_HD unsigned gemm_grid_x(unsigned mtiles, unsigned ntiles) {
+// The workgroups the library launches: one per tile, rounded up to equal shares.
+static inline GEMV_HD unsigned gemm_tiles_grid(unsigned mtiles, unsigned ntiles) {
   return GEMM_XCD_COUNT * ((mtiles * ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT);
 }
-// false: this workgroup has no tile (the grid is rounded up to equal shares)
+// The grid cogni_gemm_plan gives hosts that launch by name: rounded up to whole blocks for every XCD, as it always was (any grid of
+// gemm_tiles_grid or more is valid: the surplus workgroups leave).
+static inline GEMV_HD unsigned gemm_grid_x(unsigned mtiles, unsigned ntiles) {
+  if (mtiles < 2u) return gemm_tiles_grid(mtiles, ntiles);
+  const unsigned bmt = gemm_block_mt(mtiles), bnt = gemm_block_nt(mtiles, ntiles);
+  const unsigned nb = ((ntiles + bnt - 1u) / bnt) * ((mtiles + bmt - 1u) / bmt);
+  return GEMM_XCD_COUNT * bmt * bnt * ((nb + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT);
+}
+// false: this workgroup has no tile
 static inline GEMV_HD bool gemm_tile_of(unsigned id, unsigned mtiles, unsigned ntiles, unsigned* mt, unsigned* nt) {
   const unsigned total = mtiles * ntiles, per = (total + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT;
-  const unsigned vt = (id % GEMM_XCD_COUNT) * per + id / GEMM_XCD_COUNT;
-  if (vt >= total) return false;
+  const unsigned l = id / GEMM_XCD_COUNT, vt = (id % GEMM_XCD_COUNT) * per + l;
+  if (l >= per || vt >= total) return false;
   const unsigned gn = gemm_block_nt(mtiles, ntiles), g = vt / (gn * mtiles), i = vt - g * gn * mtiles;
   const unsigned left = ntiles - g * gn, n = left < gn ? left : gn;   // (the last group of weight tiles may be a smaller one)
   *mt = i / n;
