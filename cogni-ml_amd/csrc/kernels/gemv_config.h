@@ -224,20 +224,25 @@ static inline unsigned gemv_mt_multi_from(unsigned type, unsigned in_dim) {
   if (!gemv_mt_supported(type, 2, in_dim)) return 0;
   return 4u * (in_dim >> 8) < 3u * gemv_mt_padded_sb(in_dim) ? 5u : 2u;
 }
-// tiles per wavefront: rows of more than 4096 values one (the operands are streamed); else as many as keep 256 workgroups
-// busy, at most three (Q4_K, Q5_K) or two (Q6_K, Q8_0: their units are larger). Host and kernel use the same rule.
+// tiles per wavefront: rows of more than 4096 values one (the operands are streamed); else the count, up to three (Q4_K, Q5_K) or
+// two (Q6_K, Q8_0: their units are larger), whose rounds of 256 workgroups take least. In hundredths of a us, 4096 columns of Q4_K:
+// one round 564 | 755 | 950, more of them 460 + 170 | 580 + 308 | 680 + 480 a round. Of the counts timed for the four types at 20 row counts of
+// 1024 to 4096 columns this takes the fastest or one within 3 %; as many tiles as keep 256 workgroups busy, the rule before, cost up to
+// 31 % more (Q4_K 16384 rows 15.0 us with three tiles, 11.4 with one; 10240 rows 11.0 with two, 8.9 with three; Q6_K 12288 rows 16.2 | 13.7).
+// Host and kernel use the same rule.
 static inline GEMV_HD unsigned gemv_mt_tiles(unsigned type, unsigned in_dim, unsigned ntiles) {
   if (in_dim > 4096u) return 1;
-  const unsigned tmax = (type == 14 || type == 8) ? 2u : (unsigned)GEMV_MT_TMAX;
-  unsigned t = ntiles / 256u;
-  if (t < 1) t = 1;
-  if (t > tmax) t = tmax;
-  return t;
+  const unsigned r1 = (ntiles + 255u) / 256u, r2 = ((ntiles + 1u) / 2u + 255u) / 256u, r3 = ((ntiles + 2u) / 3u + 255u) / 256u;
+  const unsigned c1 = r1 <= 1u ? 564u : 460u + 170u * r1, c2 = r2 <= 1u ? 755u : 580u + 308u * r2, c3 = r3 <= 1u ? 950u : 680u + 480u * r3;
+  const int three = type != 14 && type != 8 && c3 < c1 && c3 < c2;
+  return three ? (unsigned)GEMV_MT_TMAX : (c2 < c1 ? 2u : 1u);
 }
+// One workgroup per compute unit at most; they walk the row groups (a workgroup that has none leaves at once).
 static inline unsigned gemv_mt_grid(unsigned type, unsigned in_dim, unsigned total_rows) {
-  const unsigned ntiles = (total_rows + 15) / 16, t = gemv_mt_tiles(type, in_dim, ntiles);
-  const unsigned groups = (ntiles + t - 1) / t;
-  return groups < 256u ? groups : 256u;   // more groups than compute units: the workgroups walk them
+  const unsigned ntiles = (total_rows + 15) / 16;
+  (void)type;
+  (void)in_dim;
+  return ntiles < 256u ? ntiles : 256u;
 }
 // the k-slices' partial sums, then per wavefront the slots of its units: 6 x (16 rows x 144 B) for Q4_K, 6 x (16 rows x
 // 176 B) for Q5_K, 4 x (16 rows x 240 B) for Q6_K, 4 x (16 rows x 272 B) for Q8_0

@@ -664,7 +664,15 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
   const u32 rg = lane >> 4;
 
   u32 grp = blockIdx.x;
-  if (grp >= ngroups) return;
+  if (grp >= ngroups) {
+    if constexpr (TOP1) {   // no rows: a partial result that never wins
+      if ((u32)tid < tokens) {
+        a.out[0][(size_t)tid * gridDim.x + blockIdx.x] = -__builtin_inff();
+        top_ids[(size_t)tid * gridDim.x + blockIdx.x] = 0xFFFFFFFFu;
+      }
+    }
+    return;
+  }
   if constexpr (NEXT) {   // the super-blocks past the row's end that fill the next image up to a multiple of 8 (there are more groups than those)
     const u32 nsb2 = a.rows[0] >> 8, nsbp2 = gemv_mt_padded_sb(a.rows[0]), sb = nsb2 + blockIdx.x;
     if (sb < nsbp2) {
