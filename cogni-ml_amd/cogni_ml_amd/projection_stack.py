@@ -58,6 +58,7 @@ class QwenProjectionStackRunner:
         self.weights, self.tokens, self.hidden = weights, tokens, weights.hidden
         self._xs = np.ascontiguousarray(xs, dtype=np.float32)
         self._buffers = []
+        self._rounds = self._rounds_of(weights.entries)
         self._w = {}
         self._images = {}   # (input name, weight type) -> packed activation image shared by every list that reads that input
         self._act = {"x": self._alloc(4 * tokens * self.hidden)}
@@ -102,49 +103,69 @@ class QwenProjectionStackRunner:
     def _reset_sequence(self):
         hip.copy_htod(self._act["x"].ptr, self._xs, self._xs.nbytes, "sequence input")
 
+    @staticmethod
+    def _rounds_of(entries):
+        """The projections in rounds: one that reads another's output is in a later round than that, so the projections of a round
+        are independent of each other. A round is a list of groups of up to six that share input, type and row length (q | k | v |
+        gate | up), each group one launch."""
+        depth, rounds = {"x": 0}, []
+        for e in entries:
+            name, src, t, out_dim, in_dim, raw = e
+            if src not in depth or name in depth:   # reads what a later one writes, or writes a buffer again: strictly in order
+                return [[[e]] for e in entries]
+            d = depth[name] = depth[src] + 1
+            while len(rounds) < d:
+                rounds.append([])
+            for grp in rounds[d - 1]:
+                if len(grp) < 6 and (grp[0][1], int(grp[0][2]), grp[0][4]) == (src, int(t), in_dim):
+                    grp.append(e)
+                    break
+            else:
+                rounds[d - 1].append([e])
+        return rounds
+
+    @staticmethod
+    def _pack_each(jobs, one, two):
+        """The activation blocks of `jobs`, two to a launch."""
+        for i in range(0, len(jobs) - 1, 2):
+            two(*jobs[i], *jobs[i + 1])
+        if len(jobs) % 2:
+            one(*jobs[-1])
+
     def _launch(self, tok0, count):
         stream = hip.current_stream_handle()
-        ents = self.weights.entries
-        packed = set()
-        i = 0
-        while i < len(ents):
-            name, src, t, out_dim, in_dim, raw = ents[i]
-            nxt = ents[i + 1] if i + 1 < len(ents) else None
-            # up to three consecutive projections of one input, type and row length (q | k | v, gate | up) go to the
-            # library as one list (the qmatvec_many seam), which stages the input once for them
-            j = i + 1
-            while j < len(ents) and j - i < 3 and (ents[j][1], ents[j][2], ents[j][4]) == (src, t, in_dim):
-                j += 1
-            if j - i >= 2 and 0 < quant.gemv_one_pass_multi_from(t, in_dim) <= count:
-                # several tokens of a shape the one-pass kernel takes: the input is packed once per sequence step and
-                # every list that reads it (q | k | v, then gate | up) goes against that one image
-                grp = ents[i:j]
-                key = (src, int(t))
-                if key not in packed:
-                    quant.gemv_pack_dev(self._act[src].ptr + 4 * tok0 * in_dim, t, in_dim, count, self._images[key].ptr, stream)
-                    packed.add(key)
-                quant.gemv_packed_dev([self._w[e[0]].ptr for e in grp], t, self._images[key].ptr,
-                                      [self._act[e[0]].ptr + 4 * tok0 * e[3] for e in grp], [e[3] for e in grp], in_dim,
-                                      count, 0, stream)
-                i = j
-                continue
-            if j - i >= 2:
-                grp = ents[i:j]
-                quant.gemv_many_dev([self._w[e[0]].ptr for e in grp], t, self._act[src].ptr + 4 * tok0 * in_dim,
-                                    [self._act[e[0]].ptr + 4 * tok0 * e[3] for e in grp], [e[3] for e in grp], in_dim,
-                                    count, stream)
-                i = j
-                continue
-            if nxt is not None and nxt[1:5] == (src, t, out_dim, in_dim):
-                # two projections of one shape on the same input (k | v, gate | up) share one launch
-                quant.gemv_dual_dev(self._w[name].ptr, self._w[nxt[0]].ptr, t, self._act[src].ptr + 4 * tok0 * in_dim,
-                                    self._act[name].ptr + 4 * tok0 * out_dim, self._act[nxt[0]].ptr + 4 * tok0 * out_dim,
-                                    in_dim, out_dim, count, stream)
-                i += 2
-                continue
-            quant.gemv_dev(self._w[name].ptr, t, self._act[src].ptr + 4 * tok0 * in_dim,
-                           self._act[name].ptr + 4 * tok0 * out_dim, in_dim, out_dim, count, 0, stream)
-            i += 1
+
+        def act(name, dim):
+            return self._act[name].ptr + 4 * tok0 * dim
+
+        for groups in self._rounds:
+            # several tokens of a shape the one-pass kernel takes: every input is packed once, and what reads it goes against that
+            # image; the others through the library, which picks their kernels
+            imaged, singles, jobs = [], [], {}
+            for grp in groups:
+                name, src, t, out_dim, in_dim, raw = grp[0]
+                start = quant.gemv_one_pass_multi_from(t, in_dim) if len(grp) >= 2 else quant.gemv_one_pass_from(t, in_dim, out_dim)
+                if 1 < count and 0 < start <= count:
+                    jobs.setdefault((src, int(t)), (act(src, in_dim), t, in_dim, self._images[(src, int(t))].ptr))
+                    imaged.append(grp)
+                elif len(grp) >= 2:
+                    most = 6 if count == 1 else 3   # matrices in a launch of the kernels for one and for several tokens
+                    for part in (grp[i:i + most] for i in range(0, len(grp), most)):
+                        quant.gemv_many_dev([self._w[e[0]].ptr for e in part], t, act(src, in_dim), [act(e[0], e[3]) for e in part],
+                                            [e[3] for e in part], in_dim, count, stream)
+                else:
+                    singles.append((self._w[name].ptr, t, act(src, in_dim), act(name, out_dim), in_dim, out_dim))
+            self._pack_each(list(jobs.values()), lambda x, t, k, image: quant.gemv_pack_dev(x, t, k, count, image, stream),
+                            lambda *ab: quant.gemv_pack_two_dev(*ab, count, stream))
+            for grp in imaged:
+                name, src, t, out_dim, in_dim, raw = grp[0]
+                quant.gemv_packed_dev([self._w[e[0]].ptr for e in grp], t, self._images[(src, int(t))].ptr, [act(e[0], e[3]) for e in grp],
+                                      [e[3] for e in grp], in_dim, count, 0, stream)
+            for i in range(0, len(singles) - 1, 2):
+                quant.gemv_two_dev(*singles[i], *singles[i + 1], count, stream)
+            if len(singles) % 2:
+                w, t, x, out, in_dim, out_dim = singles[-1]
+                quant.gemv_dev(w, t, x, out, in_dim, out_dim, count, 0, stream)
 
     @staticmethod
     def _family(t):
@@ -163,44 +184,39 @@ class QwenProjectionStackRunner:
         """All `count` tokens through the GEMMs: one pack per (input, layout), one GEMM per list of projections that share
         their input, type and row length (or per projection)."""
         stream = hip.current_stream_handle()
-        ents = self.weights.entries
-        packed, done = set(), set()
         list_types = (int(TensorType.Q4_K), int(TensorType.Q5_K))
-        for idx, (name, src, t, out_dim, in_dim, raw) in enumerate(ents):
-            if name in done:
-                continue
-            if count <= 16 and self._one_pass16(t, in_dim):
-                # up to sixteen tokens: the one-pass decode kernels with sixteen single-term tokens, one image per input,
-                # every projection of that input, type and row length in the same call
-                key16 = (src, self._family(t))
-                img = self._images16[key16]
-                if key16 + ("x16",) not in packed:
-                    quant.gemv_pack16_dev(self._act[src].ptr, t, in_dim, count, img.ptr, stream)
-                    packed.add(key16 + ("x16",))
-                grp = [e for e in ents[idx:] if e[0] not in done and (e[1], int(e[2]), e[4]) == (src, int(t), in_dim)][:8]
-                quant.gemv_packed16_dev([self._w[e[0]].ptr for e in grp], t, img.ptr, [self._act[e[0]].ptr for e in grp],
-                                        [e[3] for e in grp], in_dim, count, 0, stream)
-                done.update(e[0] for e in grp)
-                continue
-            key = (src, self._family(t))
-            ws, nbytes = self._prefill_ws[key]
-            if key not in packed:
-                quant.gemm_pack_dev(self._act[src].ptr, t, in_dim, count, ws.ptr, nbytes, stream)
-                packed.add(key)
-            # every projection still to come of the same input, type and row length joins this launch (q | k | v | gate | up:
-            # their input is this one's, so it exists already) - the prefill counterpart of the qmatvec_many seam
-            grp = [e for e in ents[idx:] if e[0] not in done and (e[1], int(e[2]), e[4]) == (src, int(t), in_dim)][:6]
-            if quant.gemm_stream_takes(t, in_dim, sum(e[3] for e in grp), count):
-                quant.gemm_stream_dev([self._w[e[0]].ptr for e in grp], t, ws.ptr, nbytes, [self._act[e[0]].ptr for e in grp],
-                                      [e[3] for e in grp], in_dim, count, 0, stream)
-                done.update(e[0] for e in grp)
-            elif len(grp) >= 2 and int(t) in list_types:
-                quant.gemm_packed_many_dev([self._w[e[0]].ptr for e in grp], t, ws.ptr, nbytes, [self._act[e[0]].ptr for e in grp],
-                                           [e[3] for e in grp], in_dim, count, stream)
-                done.update(e[0] for e in grp)
-            else:
-                quant.gemm_packed_dev(self._w[name].ptr, t, ws.ptr, nbytes, self._act[name].ptr, in_dim, out_dim, count, 0, stream)
-                done.add(name)
+        for groups in self._rounds:
+            # the inputs of the round, packed once each, two to a launch
+            jobs16, jobs = {}, {}
+            for grp in groups:
+                name, src, t, out_dim, in_dim, raw = grp[0]
+                key = (src, self._family(t))
+                if count <= 16 and self._one_pass16(t, in_dim):
+                    jobs16.setdefault(key, (self._act[src].ptr, t, in_dim, self._images16[key].ptr))
+                else:
+                    jobs.setdefault(key, (self._act[src].ptr, t, in_dim, self._prefill_ws[key][0].ptr, self._prefill_ws[key][1]))
+            self._pack_each(list(jobs16.values()), lambda x, t, k, image: quant.gemv_pack16_dev(x, t, k, count, image, stream),
+                            lambda *ab: quant.gemv_pack16_two_dev(*ab, count, stream))
+            self._pack_each(list(jobs.values()), lambda x, t, k, ws, nbytes: quant.gemm_pack_dev(x, t, k, count, ws, nbytes, stream),
+                            lambda *ab: quant.gemm_pack_two_dev(*ab, count, stream))
+            for grp in groups:
+                name, src, t, out_dim, in_dim, raw = grp[0]
+                key = (src, self._family(t))
+                w, out, dims = [self._w[e[0]].ptr for e in grp], [self._act[e[0]].ptr for e in grp], [e[3] for e in grp]
+                if key in jobs16:
+                    # up to sixteen tokens: the one-pass decode kernels with sixteen single-term tokens
+                    quant.gemv_packed16_dev(w, t, self._images16[key].ptr, out, dims, in_dim, count, 0, stream)
+                    continue
+                ws, nbytes = self._prefill_ws[key]
+                while dims:   # (the prefill counterpart of the qmatvec_many seam)
+                    if quant.gemm_stream_takes(t, in_dim, sum(dims), count):
+                        quant.gemm_stream_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, 0, stream)
+                        break
+                    if len(dims) >= 2 and int(t) in list_types:
+                        quant.gemm_packed_many_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, stream)
+                        break
+                    quant.gemm_packed_dev(w[0], t, ws.ptr, nbytes, out[0], in_dim, dims[0], count, 0, stream)
+                    w, out, dims = w[1:], out[1:], dims[1:]
 
     def _run_token(self, tok):
         self._launch(tok, 1)

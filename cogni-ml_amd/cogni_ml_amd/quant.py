@@ -378,6 +378,37 @@ def gemv_packed16_swiglu_dev(w_gate_ptr, w_up_ptr, w_type, image_ptr, out_ptr, i
                                                     ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
 
 
+def gemv_two_dev(w_a, type_a, x_a, out_a, in_dim_a, out_dim_a, w_b, type_b, x_b, out_b, in_dim_b, out_dim_b, tokens=1, stream=None):
+    """Two matrices with an input each (o and down of a layer): one launch for one token of Q4_K or Q5_K beside Q4_K or Q6_K, else
+    gemv_dev for the one and the other."""
+    U64, U32 = ctypes.c_uint64, ctypes.c_uint32
+    _check(hip.lib().cogni_gemv_two_dev(U64(w_a), U32(int(type_a)), U64(x_a), U64(out_a), U32(in_dim_a), U32(out_dim_a), U64(w_b),
+                                        U32(int(type_b)), U64(x_b), U64(out_b), U32(in_dim_b), U32(out_dim_b), U32(tokens), stream))
+
+
+def _pack_two(name, x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream):
+    U64, U32 = ctypes.c_uint64, ctypes.c_uint32
+    _check(getattr(hip.lib(), name)(U64(x_a), U32(int(type_a)), U32(in_dim_a), U64(image_a), U64(x_b), U32(int(type_b)), U32(in_dim_b),
+                                    U64(image_b), U32(tokens), stream))
+
+
+def gemv_pack_two_dev(x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream=None):
+    """gemv_pack_dev of two activation blocks in one launch."""
+    _pack_two("cogni_gemv_pack_two_dev", x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream)
+
+
+def gemv_pack16_two_dev(x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream=None):
+    """gemv_pack16_dev of two activation blocks in one launch."""
+    _pack_two("cogni_gemv_pack16_two_dev", x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream)
+
+
+def gemm_pack_two_dev(x_a, type_a, in_dim_a, ws_a, ws_bytes_a, x_b, type_b, in_dim_b, ws_b, ws_bytes_b, tokens, stream=None):
+    """gemm_pack_dev of two activation blocks in one launch."""
+    U64, U32, SZ = ctypes.c_uint64, ctypes.c_uint32, ctypes.c_size_t
+    _check(hip.lib().cogni_gemm_pack_two_dev(U64(x_a), U32(int(type_a)), U32(in_dim_a), U64(ws_a), SZ(ws_bytes_a), U64(x_b), U32(int(type_b)),
+                                             U32(in_dim_b), U64(ws_b), SZ(ws_bytes_b), U32(tokens), stream))
+
+
 def gemv_packed16_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, image_ptr, out_ptr, next_type, next_image_ptr, in_dim, out_dim, tokens,
                                   stream=None):
     """The same with the products handed on as the sixteen-token image of the (Q6_K) matrix behind them; out_ptr may be 0."""

@@ -130,6 +130,16 @@ lib LibCogniHIP
                               count : UInt32, in_dim : UInt32, tokens : UInt32, stream : Void*) : Int32
   fun cogni_gemv_packed16_swiglu_dev(w_gate : UInt64, w_up : UInt64, w_type : UInt32, image : UInt64, out : UInt64, in_dim : UInt32,
                                      out_dim : UInt32, tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemv_two_dev(w_a : UInt64, type_a : UInt32, x_a : UInt64, out_a : UInt64, in_dim_a : UInt32, out_dim_a : UInt32,
+                         w_b : UInt64, type_b : UInt32, x_b : UInt64, out_b : UInt64, in_dim_b : UInt32, out_dim_b : UInt32,
+                         tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemv_pack_two_dev(x_a : UInt64, type_a : UInt32, in_dim_a : UInt32, image_a : UInt64, x_b : UInt64, type_b : UInt32,
+                              in_dim_b : UInt32, image_b : UInt64, tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemv_pack16_two_dev(x_a : UInt64, type_a : UInt32, in_dim_a : UInt32, image_a : UInt64, x_b : UInt64, type_b : UInt32,
+                                in_dim_b : UInt32, image_b : UInt64, tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemm_pack_two_dev(x_a : UInt64, type_a : UInt32, in_dim_a : UInt32, workspace_a : UInt64, bytes_a : LibC::SizeT,
+                              x_b : UInt64, type_b : UInt32, in_dim_b : UInt32, workspace_b : UInt64, bytes_b : LibC::SizeT,
+                              tokens : UInt32, stream : Void*) : Int32
   fun cogni_gemv_packed16_swiglu_pack_dev(w_gate : UInt64, w_up : UInt64, w_type : UInt32, image : UInt64, out : UInt64, next_type : UInt32,
                                           next_image : UInt64, in_dim : UInt32, out_dim : UInt32, tokens : UInt32, stream : Void*) : Int32
   fun cogni_gemm_packed_many_dev(w_raw : UInt64*, w_type : UInt32, workspace : UInt64, workspace_bytes : LibC::SizeT, outs : UInt64*,

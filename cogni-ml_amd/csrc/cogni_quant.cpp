@@ -419,6 +419,62 @@ int cogni_gemv_pack_dev(uint64_t x, uint32_t w_type, uint32_t in_dim, uint32_t t
   return launch(w_type == COGNI_TYPE_Q6_K ? "pack_x_mt_q6k_f16" : "pack_x_mt_q4k_f16", 2 * gemv_mt_padded_sb(in_dim), 256, 0, params, stream);
 }
 
+// The images of two activation blocks in one launch.
+static int gemv_pack_two(const char* who, bool x16, uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t image_a, uint64_t x_b,
+                         uint32_t type_b, uint32_t in_dim_b, uint64_t image_b, uint32_t tokens, void* stream) {
+  if (!x_a || !image_a || !x_b || !image_b) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  uint32_t q6_a = type_a == COGNI_TYPE_Q6_K, q6_b = type_b == COGNI_TYPE_Q6_K;
+  const uint32_t per = x16 ? 4 : 2;
+  void* params[] = {&x_a, &image_a, &in_dim_a, &q6_a, &x_b, &image_b, &in_dim_b, &q6_b, &tokens};
+  return launch(x16 ? "pack_x_mt16_two_f16" : "pack_x_mt_two_f16", per * (gemv_mt_padded_sb(in_dim_a) + gemv_mt_padded_sb(in_dim_b)), 256, 0, params,
+                stream);
+}
+int cogni_gemv_pack_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t image_a, uint64_t x_b, uint32_t type_b, uint32_t in_dim_b,
+                            uint64_t image_b, uint32_t tokens, void* stream) {
+  if (!gemv_mt_supported(type_a, (int)tokens, in_dim_a) || !gemv_mt_supported(type_b, (int)tokens, in_dim_b))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_pack_two_dev: no one-pass kernel for this type, token count and in_dim "
+                                            "(cogni_gemv_image_bytes is 0)");
+  return gemv_pack_two("cogni_gemv_pack_two_dev", false, x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream);
+}
+
+// Matrices against an image: up to `most` of them per launch, as one matrix of all their rows; a matrix whose row count is not a
+// multiple of 16 ends its launch (a tile of 16 rows is of one matrix). Three at most have their own kernel parameters, more (Q4_K,
+// Q5_K) go as a list.
+namespace {
+struct GemvListArgs {   // GemvList<6> and MtArgs<6> (kernels/gemv.hpp, gemv_mt.hpp)
+  uint64_t w[6];
+  uint64_t out[6];
+  uint32_t rows[6];
+};
+}   // namespace
+static int gemv_mt_lists(const char* who, bool x16, const uint64_t* w_raw, uint32_t w_type, uint64_t image, uint64_t residual, const uint64_t* out,
+                         const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
+  const uint32_t most = (w_type == COGNI_TYPE_Q4_K || w_type == COGNI_TYPE_Q5_K) ? 6u : 3u;
+  for (uint32_t i0 = 0; i0 < count;) {
+    GemvListArgs l{};
+    uint32_t n = 0;
+    uint64_t total = 0;
+    while (n < most && i0 + n < count) {
+      if (n >= 3 && total + out_dims[i0 + n] > 0x7FFFFFFFull) break;
+      l.w[n] = w_raw[i0 + n], l.out[n] = out[i0 + n], l.rows[n] = out_dims[i0 + n];
+      total += l.rows[n];
+      n++;
+      if (l.rows[n - 1] % 16 != 0) break;
+    }
+    if (total > 0x7FFFFFFFull) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": too many rows");
+    uint64_t res = i0 == 0 ? residual : 0;
+    char name[48];
+    std::snprintf(name, sizeof name, "%s_gemv_mt%s%s_f32", type_prefix(w_type), x16 ? "16" : "", n > 3 ? "_list" : "");
+    void* three[] = {&l.w[0], &l.w[1], &l.w[2], &image, &res, &l.out[0], &l.out[1], &l.out[2], &in_dim, &l.rows[0], &l.rows[1], &l.rows[2], &tokens};
+    void* list[] = {&l, &image, &in_dim, &tokens};
+    const int rc = launch(name, gemv_mt_grid(w_type, in_dim, (uint32_t)total), GEMV_MT_WAVES * 64,
+                          gemv_mt_lds_bytes(w_type) + (x16 ? GEMV_MT_X16_LDS_EXTRA : 0u), n > 3 ? list : three, stream);
+    if (rc != 0) return rc;
+    i0 += n;
+  }
+  return 0;
+}
+
 int cogni_gemv_packed_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t image, uint64_t residual, const uint64_t* out,
                           const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
   if (!w_raw || !out || !out_dims || !image) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_dev: null argument");
@@ -428,28 +484,7 @@ int cogni_gemv_packed_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t image
   if (residual && count != 1) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_dev: a residual goes with a single matrix");
   for (uint32_t i = 0; i < count; i++)
     if (!w_raw[i] || !out[i] || out_dims[i] == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_dev: null pointer or zero rows");
-  // up to three matrices per launch, as one matrix of all their rows; a matrix whose row count is not a multiple of 16
-  // ends its launch (a tile of 16 rows is of one matrix)
-  for (uint32_t i0 = 0; i0 < count;) {
-    uint64_t w[3] = {0, 0, 0}, o[3] = {0, 0, 0};
-    uint32_t rows[3] = {0, 0, 0}, n = 0;
-    uint64_t total = 0;
-    while (n < 3 && i0 + n < count) {
-      w[n] = w_raw[i0 + n], o[n] = out[i0 + n], rows[n] = out_dims[i0 + n];
-      total += rows[n];
-      n++;
-      if (rows[n - 1] % 16 != 0) break;
-    }
-    if (total > 0x7FFFFFFFull) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_dev: too many rows");
-    uint64_t res = i0 == 0 ? residual : 0;
-    void* params[] = {&w[0], &w[1], &w[2], &image, &res, &o[0], &o[1], &o[2], &in_dim, &rows[0], &rows[1], &rows[2], &tokens};
-    const char* kernel = w_type == COGNI_TYPE_Q6_K ? "q6_k_gemv_mt_f32" : (w_type == COGNI_TYPE_Q5_K ? "q5_k_gemv_mt_f32" : (w_type == COGNI_TYPE_Q8_0 ? "q8_0_gemv_mt_f32" : "q4_k_gemv_mt_f32"));
-    const int rc = launch(kernel, gemv_mt_grid(w_type, in_dim, (uint32_t)total),
-                          GEMV_MT_WAVES * 64, gemv_mt_lds_bytes(w_type), params, stream);
-    if (rc != 0) return rc;
-    i0 += n;
-  }
-  return 0;
+  return gemv_mt_lists("cogni_gemv_packed_dev", false, w_raw, w_type, image, residual, out, out_dims, count, in_dim, tokens, stream);
 }
 
 // Nine to sixteen tokens in one pass over the weights: the one-pass kernels with their sixteen activation rows as sixteen
@@ -465,6 +500,12 @@ int cogni_gemv_pack16_dev(uint64_t x, uint32_t w_type, uint32_t in_dim, uint32_t
   void* params[] = {&x, &image, &tokens, &in_dim};
   return launch(w_type == COGNI_TYPE_Q6_K ? "pack_x_mt16_q6k_f16" : "pack_x_mt16_q4k_f16", 4 * gemv_mt_padded_sb(in_dim), 256, 0, params, stream);
 }
+int cogni_gemv_pack16_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t image_a, uint64_t x_b, uint32_t type_b, uint32_t in_dim_b,
+                              uint64_t image_b, uint32_t tokens, void* stream) {
+  if (!gemv16_shape(type_a, in_dim_a, tokens) || !gemv16_shape(type_b, in_dim_b, tokens))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_pack16_two_dev: Q4_K, Q5_K, Q6_K or Q8_0, 1..16 tokens, in_dim a multiple of 256 up to 12288");
+  return gemv_pack_two("cogni_gemv_pack16_two_dev", true, x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream);
+}
 int cogni_gemv_packed16_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t image, uint64_t residual, const uint64_t* out,
                             const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
   const char* who = "cogni_gemv_packed16_dev";
@@ -475,26 +516,7 @@ int cogni_gemv_packed16_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t ima
   if (residual && count != 1) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": a residual goes with a single matrix");
   for (uint32_t i = 0; i < count; i++)
     if (!w_raw[i] || !out[i] || out_dims[i] == 0) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null pointer or zero rows");
-  // up to three matrices per launch, as cogni_gemv_packed_dev
-  for (uint32_t i0 = 0; i0 < count;) {
-    uint64_t w[3] = {0, 0, 0}, o[3] = {0, 0, 0}, none = residual;
-    uint32_t rows[3] = {0, 0, 0}, n = 0;
-    uint64_t total = 0;
-    while (n < 3 && i0 + n < count) {
-      w[n] = w_raw[i0 + n], o[n] = out[i0 + n], rows[n] = out_dims[i0 + n];
-      total += rows[n];
-      n++;
-      if (rows[n - 1] % 16 != 0) break;
-    }
-    if (total > 0x7FFFFFFFull) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": too many rows");
-    void* params[] = {&w[0], &w[1], &w[2], &image, &none, &o[0], &o[1], &o[2], &in_dim, &rows[0], &rows[1], &rows[2], &tokens};
-    const char* kernel = w_type == COGNI_TYPE_Q6_K ? "q6_k_gemv_mt16_f32" : (w_type == COGNI_TYPE_Q5_K ? "q5_k_gemv_mt16_f32" : (w_type == COGNI_TYPE_Q8_0 ? "q8_0_gemv_mt16_f32" : "q4_k_gemv_mt16_f32"));
-    const int rc = launch(kernel, gemv_mt_grid(w_type, in_dim, (uint32_t)total),
-                          GEMV_MT_WAVES * 64, gemv_mt_lds_bytes(w_type) + GEMV_MT_X16_LDS_EXTRA, params, stream);
-    if (rc != 0) return rc;
-    i0 += n;
-  }
-  return 0;
+  return gemv_mt_lists(who, true, w_raw, w_type, image, residual, out, out_dims, count, in_dim, tokens, stream);
 }
 
 int cogni_gemv_packed16_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t image, uint64_t out, uint32_t in_dim,
@@ -747,25 +769,27 @@ int cogni_gemv_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t x, cons
     int rc = 0;
     if (try_one_pass(w_raw, w_type, x, 0, out, out_dims, count, in_dim, tokens, from, stream, &rc)) return rc;
   }
-  if (count == 2 && out_dims[0] == out_dims[1])
+  if (count == 2 && out_dims[0] == out_dims[1] && !(tokens == 1 && w_type == COGNI_TYPE_Q5_K && (in_dim % 256) == 0))
     return cogni_gemv_dual_dev(w_raw[0], w_raw[1], w_type, x, out[0], out[1], in_dim, out_dims[0], tokens, stream);
-  // one token of several Q4_K matrices: up to three per launch as one matrix of all their rows (q | k | v: one launch and
-  // one staging of x instead of three)
-  if (tokens == 1 && w_type == COGNI_TYPE_Q4_K && (in_dim % 256) == 0 && total <= 0x7FFFFFFFull) {
-    for (uint32_t i0 = 0; i0 < count; i0 += 3) {
-      const uint32_t n = count - i0 < 3 ? count - i0 : 3;
+  // one token of several Q4_K or Q5_K matrices: up to six per launch as one matrix of all their rows (q | k | v | gate | up: one
+  // launch and one staging of x instead of five); up to three of Q4_K have their own kernel parameters
+  if (tokens == 1 && (w_type == COGNI_TYPE_Q4_K || w_type == COGNI_TYPE_Q5_K) && (in_dim % 256) == 0 && total <= 0x7FFFFFFFull) {
+    for (uint32_t i0 = 0; i0 < count; i0 += 6) {
+      const uint32_t n = count - i0 < 6 ? count - i0 : 6;
       int rc;
       if (n == 1) {
         rc = cogni_gemv_dev(w_raw[i0], w_type, x, 0, out[i0], in_dim, out_dims[i0], 1, stream);
       } else {
-        uint64_t w[3] = {w_raw[i0], w_raw[i0 + 1], n > 2 ? w_raw[i0 + 2] : 0};
-        uint64_t o[3] = {out[i0], out[i0 + 1], n > 2 ? out[i0 + 2] : 0};
-        uint32_t rows[3] = {out_dims[i0], out_dims[i0 + 1], n > 2 ? out_dims[i0 + 2] : 0};
-        uint32_t grid = 0, block = 0, shmem = 0;
-        rc = cogni_gemv_launch_dims(w_type, 1, in_dim, rows[0] + rows[1] + rows[2], &grid, &block, &shmem);
+        GemvListArgs l{};
+        uint32_t grid = 0, block = 0, shmem = 0, rows = 0;
+        for (uint32_t i = 0; i < n; i++) l.w[i] = w_raw[i0 + i], l.out[i] = out[i0 + i], rows += l.rows[i] = out_dims[i0 + i];
+        rc = cogni_gemv_launch_dims(w_type, 1, in_dim, rows, &grid, &block, &shmem);
         if (rc != 0) return rc;
-        void* params[] = {&w[0], &w[1], &w[2], &x, &o[0], &o[1], &o[2], &in_dim, &rows[0], &rows[1], &rows[2]};
-        rc = launch("q4_k_many_gemv_f32", grid, block, shmem, params, stream);
+        void* three[] = {&l.w[0], &l.w[1], &l.w[2], &x, &l.out[0], &l.out[1], &l.out[2], &in_dim, &l.rows[0], &l.rows[1], &l.rows[2]};
+        void* list[] = {&l, &x, &in_dim};
+        const bool own = n <= 3 && w_type == COGNI_TYPE_Q4_K;
+        rc = launch(own ? "q4_k_many_gemv_f32" : (w_type == COGNI_TYPE_Q4_K ? "q4_k_list_gemv_f32" : "q5_k_list_gemv_f32"), grid, block, shmem,
+                    own ? three : list, stream);
       }
       if (rc != 0) return rc;
     }
@@ -805,6 +829,29 @@ int cogni_gemv_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t x, cons
     if (rc != 0) return rc;
   }
   return 0;
+}
+
+// One token of two matrices with an input each: one launch for Q4_K or Q5_K beside Q4_K or Q6_K, else one after the other.
+int cogni_gemv_two_dev(uint64_t w_a, uint32_t type_a, uint64_t x_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a, uint64_t w_b,
+                       uint32_t type_b, uint64_t x_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens, void* stream) {
+  auto a_type = [](uint32_t t) { return t == COGNI_TYPE_Q4_K || t == COGNI_TYPE_Q5_K; };
+  auto b_type = [](uint32_t t) { return t == COGNI_TYPE_Q4_K || t == COGNI_TYPE_Q6_K; };
+  // the kernels' b is the one whose workgroups start first: the longer rows where the types leave the choice
+  if (!(a_type(type_a) && b_type(type_b)) || (a_type(type_b) && b_type(type_a) && in_dim_a > in_dim_b))
+    std::swap(w_a, w_b), std::swap(type_a, type_b), std::swap(x_a, x_b), std::swap(out_a, out_b), std::swap(in_dim_a, in_dim_b), std::swap(out_dim_a, out_dim_b);
+  if (tokens == 1 && a_type(type_a) && b_type(type_b) && w_a && x_a && out_a && w_b && x_b && out_b && in_dim_a && in_dim_b && out_dim_a && out_dim_b &&
+      (in_dim_a % 256) == 0 && (in_dim_b % 256) == 0) {
+    const bool r1 = gemv_rows_m1(type_a, out_dim_a) == 1 && gemv_rows_m1(type_b, out_dim_b) == 1;
+    auto wgs = [&](uint32_t t, uint32_t out_dim) { return r1 ? (out_dim + GEMV_WAVES - 1) / GEMV_WAVES : gemv_grid(t, 1, out_dim); };
+    uint32_t wgs_b = wgs(type_b, out_dim_b);
+    const uint32_t shmem = std::max(gemv_lds_bytes(type_a, 1, in_dim_a), gemv_lds_bytes(type_b, 1, in_dim_b));
+    char name[48];
+    std::snprintf(name, sizeof name, "%s_and_%s_gemv_f32%s", type_prefix(type_a), type_prefix(type_b), r1 ? "_r1" : "");
+    void* params[] = {&w_a, &x_a, &out_a, &in_dim_a, &out_dim_a, &w_b, &x_b, &out_b, &in_dim_b, &out_dim_b, &wgs_b};
+    return launch(name, wgs(type_a, out_dim_a) + wgs_b, GEMV_BLOCK, shmem, params, stream);
+  }
+  if (int rc = cogni_gemv_dev(w_a, type_a, x_a, 0, out_a, in_dim_a, out_dim_a, tokens, stream)) return rc;
+  return cogni_gemv_dev(w_b, type_b, x_b, 0, out_b, in_dim_b, out_dim_b, tokens, stream);
 }
 
 int cogni_swiglu_dev(uint64_t gate, uint64_t up, uint64_t out, uint32_t n, void* stream) {
@@ -1231,6 +1278,22 @@ int cogni_gemm_pack_dev(uint64_t x, uint32_t w_type, uint32_t in_dim, uint32_t t
   void* params[] = {&x, &workspace, &tokens, &in_dim};
   // 8 tokens x one super-block per workgroup
   return launch(w_type == COGNI_TYPE_Q6_K ? "pack_x_f16_q6k" : "pack_x_f16_q4k", mtiles * 16 * (in_dim / 256), 256, 0, params, stream);
+}
+
+int cogni_gemm_pack_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t workspace_a, size_t bytes_a, uint64_t x_b, uint32_t type_b,
+                            uint32_t in_dim_b, uint64_t workspace_b, size_t bytes_b, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_pack_two_dev";
+  if (!x_a || !x_b) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  if (int rc = gemm_check(who, type_a, in_dim_a, 1, tokens, workspace_a, bytes_a)) return rc;
+  if (int rc = gemm_check(who, type_b, in_dim_b, 1, tokens, workspace_b, bytes_b)) return rc;
+  const uint64_t wgs = (uint64_t)((tokens + 127) / 128) * 16 * (in_dim_a / 256 + in_dim_b / 256);
+  if (wgs > 0x7FFFFFull) {   // (fewer than 2^31 threads in a launch)
+    if (int rc = cogni_gemm_pack_dev(x_a, type_a, in_dim_a, tokens, workspace_a, bytes_a, stream)) return rc;
+    return cogni_gemm_pack_dev(x_b, type_b, in_dim_b, tokens, workspace_b, bytes_b, stream);
+  }
+  uint32_t q6_a = type_a == COGNI_TYPE_Q6_K, q6_b = type_b == COGNI_TYPE_Q6_K;
+  void* params[] = {&x_a, &workspace_a, &in_dim_a, &q6_a, &x_b, &workspace_b, &in_dim_b, &q6_b, &tokens};
+  return launch("pack_x_two_f16", (uint32_t)wgs, 256, 0, params, stream);
 }
 
 int cogni_gemm_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias, uint64_t out, uint32_t in_dim,

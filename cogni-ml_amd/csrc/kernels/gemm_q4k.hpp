@@ -78,15 +78,16 @@ __device__ __forceinline__ u32 gemm_k_element(u32 ks, u32 kg, u32 e) {
 #define PACK_TOK 8
 #endif
 // Q6: the element order of the Q6_K kernel (gemm_q6k.hpp) instead of the Q4_K one.
+// bid: the workgroup's number, where it is not the launch's (two blocks in one launch).
 template <bool Q6>
-__device__ __forceinline__ void pack_x_core(const float* __restrict__ x, uint4* __restrict__ xp, u32 m, u32 in_dim) {
+__device__ __forceinline__ void pack_x_core(const float* __restrict__ x, uint4* __restrict__ xp, u32 m, u32 in_dim, u32 bid = blockIdx.x) {
   // [32 (k-step, k-group)][32 tokens] uint4, each (k-step, k-group) row padded by one uint4 so that the
   // transposing 8-byte writes of a wavefront (same token, 32 different rows) spread over the banks
   __shared__ uint2 img[32 * (PACK_TOK + 1) * 2];
   const u32 nkb = in_dim >> 8;
   const u32 tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr u32 NQ = GEMM_BM / PACK_TOK;
-  const u32 kb = blockIdx.x % nkb, tq = (blockIdx.x / nkb) % NQ, mt = blockIdx.x / (NQ * nkb);
+  const u32 kb = bid % nkb, tq = (bid / nkb) % NQ, mt = bid / (NQ * nkb);
   // lane -> 4 consecutive k = 4 lane .. 4 lane + 3 of the super-block; their place in the image (inverse of
   // gemm_k_element): Q4_K: group g = k / 64, high-nibble half, 16-byte half h, upper-8-bytes bit, slot 0 or 4;
   // Q6_K: 128-half n, quadrant qd, 16-run u, upper-8 bit, slot 0 or 4 (gemm_k_element_q6k)
@@ -123,6 +124,17 @@ __device__ __forceinline__ void pack_x_core(const float* __restrict__ x, uint4* 
 }
 extern "C" __global__ __launch_bounds__(256) void pack_x_f16_q4k(const float* x, uint4* xp, u32 m, u32 in_dim) {
   pack_x_core<false>(x, xp, m, in_dim);
+}
+
+// Two blocks of m tokens in one launch: (x_a, xp_a, in_dim_a, q6_a, x_b, xp_b, in_dim_b, q6_b, m), the workgroups of pack_x_f16_q4k | q6k for
+// a (wgs_a = 16 ceil(m/128) in_dim_a/256 of them), then those for b.
+extern "C" __global__ __launch_bounds__(256) void pack_x_two_f16(const float* x_a, uint4* xp_a, u32 in_dim_a, u32 q6_a, const float* x_b, uint4* xp_b,
+                                                                 u32 in_dim_b, u32 q6_b, u32 m) {
+  const u32 wgs_a = (m + GEMM_BM - 1) / GEMM_BM * (GEMM_BM / PACK_TOK) * (in_dim_a >> 8);
+  const bool b = blockIdx.x >= wgs_a;
+  const u32 bid = blockIdx.x - (b ? wgs_a : 0u);
+  if (b ? q6_b : q6_a) pack_x_core<true>(b ? x_b : x_a, b ? xp_b : xp_a, m, b ? in_dim_b : in_dim_a, bid);
+  else pack_x_core<false>(b ? x_b : x_a, b ? xp_b : xp_a, m, b ? in_dim_b : in_dim_a, bid);
 }
 
 __device__ __forceinline__ u32 h2_dup(float v) {

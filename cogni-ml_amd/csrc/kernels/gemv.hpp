@@ -45,22 +45,39 @@
 // q6_k_gemv_top1_partial_f32 (src/ml/cuda/kernels/q6k_gemv_probe.ptx:1331-1580) for the output head. With `logits` the row
 // values are stored there as well (logits[m * out_dim + row], the bits of the plain kernel), so that a head that wants both
 // reads its weights once: the Q6_K 151936 x 4096 head with norm and reduce, one token, 190 us as two passes, 103 as one.
-// LIST (with DUAL, M = 1): up to three matrices of one row length and any row counts as one matrix of all their rows
-// (q | k | v of a decoder layer: the reference's qmatvec_many seam, src/ml/gguf/qwen35_cpu.cr:1419-1445); `list` names
-// them, w / w_b / out / out_b / out_dim are not used.
+// LIST (with DUAL, M = 1): up to LIST matrices of one row length and any row counts (zero: not there) as one matrix of all their
+// rows (q | k | v of a decoder layer, or all that read one input: the reference's qmatvec_many seam,
+// src/ml/gguf/qwen35_cpu.cr:1419-1445); `list` names them, w / w_b / out / out_b / out_dim are not used.
+template <int N>
 struct GemvList {
-  const uint8_t* w[3];
-  float* out[3];
-  u32 rows[3];
+  const uint8_t* w[N];
+  float* out[N];
+  u32 rows[N];
+  // the pointer of the matrix that row `row` of all of them belongs to, and that matrix's first row
+  template <class P, int I = 0>
+  __device__ __forceinline__ P pick(u32 row, P const (&of)[N], u32& first, u32 begin = 0) const {
+    if constexpr (I + 1 < N) {
+      if (row >= begin + rows[I]) return pick<P, I + 1>(row, of, first, begin + rows[I]);
+    }
+    first = begin;
+    return of[I];
+  }
+  template <int I = 0>
+  __device__ __forceinline__ u32 total() const {
+    if constexpr (I + 1 < N) return rows[I] + total<I + 1>();
+    return rows[I];
+  }
 };
+// bid, nwg: this workgroup's number and their count, where they are not the launch's (two matrices in one launch, gemv_two).
 // RO (one token, plain kernels): rows per wavefront where they differ from F::rows(M) - the variants for matrices of few
 // rows (gemv_rows_m1 in gemv_config.h), 0 = F::rows(M).
-template <class F, int M, bool ADD, bool DUAL = false, bool SWIGLU = false, bool TOP1 = false, bool LIST = false, int RO = 0>
+template <class F, int M, bool ADD, bool DUAL = false, bool SWIGLU = false, bool TOP1 = false, int LIST = 0, int RO = 0>
 __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const float* __restrict__ x,
                                           const float* __restrict__ residual, float* __restrict__ out,
                                           u32 in_dim, u32 out_dim, const uint8_t* __restrict__ w_b = nullptr,
                                           float* __restrict__ out_b = nullptr, u32* __restrict__ top_ids = nullptr,
-                                          const GemvList* list = nullptr, float* __restrict__ logits = nullptr) {
+                                          const GemvList<LIST ? LIST : 1>* list = nullptr, float* __restrict__ logits = nullptr,
+                                          u32 bid = blockIdx.x, u32 nwg = gridDim.x) {
   constexpr int R = RO ? RO : F::rows(M);
   constexpr int MG = M < F::MG_MAX ? M : F::MG_MAX;   // tokens held in registers at a time
   constexpr int NG = (M + MG - 1) / MG;
@@ -82,12 +99,15 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
   static_assert(!SWIGLU || (DUAL && M == 1 && !ADD && R % 2 == 0), "SWIGLU is a one-token mode of the matrix pair");
   static_assert(!TOP1 || (!DUAL && !ADD), "TOP1 is a mode of the plain GEMV");
   static_assert(!LIST || (DUAL && M == 1 && !ADD && !SWIGLU), "LIST is a one-token mode of several matrices");
-  const u32 total_rows = LIST ? list->rows[0] + list->rows[1] + list->rows[2] : (DUAL ? 2 * out_dim : out_dim);
-  // A workgroup takes the row groups blockIdx.x, blockIdx.x + gridDim.x, ... (GEMV_WAVES * R rows each; with SWIGLU
+  u32 total_rows = DUAL ? 2 * out_dim : out_dim;
+  if constexpr (LIST != 0) {
+    total_rows = list->total();
+  }
+  // A workgroup takes the row groups bid, bid + nwg, ... (GEMV_WAVES * R rows each; with SWIGLU
   // half as many rows of each matrix); a grid of one workgroup per group is the plain case.
   const u32 group_rows = SWIGLU ? GEMV_WAVES * R / 2 : GEMV_WAVES * R;
   const u32 ngroups = ((SWIGLU ? out_dim : total_rows) + group_rows - 1) / group_rows;
-  u32 row0 = (blockIdx.x * GEMV_WAVES + wave) * R;
+  u32 row0 = (bid * GEMV_WAVES + wave) * R;
   const uint8_t* rowp[R];
   auto set_group = [&](u32 grp) {
     row0 = (grp * GEMV_WAVES + wave) * R;
@@ -99,16 +119,16 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
       } else {
         const u32 row = min(row0 + r, total_rows - 1);
         if constexpr (LIST) {
-          const u32 r0 = list->rows[0], r01 = r0 + list->rows[1];
-          rowp[r] = row < r0 ? list->w[0] + (size_t)row * row_bytes
-                             : (row < r01 ? list->w[1] + (size_t)(row - r0) * row_bytes : list->w[2] + (size_t)(row - r01) * row_bytes);
+          u32 first;
+          const uint8_t* const wm = list->pick(row, list->w, first);   // (row is the same for the whole wavefront: scalar selects)
+          rowp[r] = wm + (size_t)(row - first) * row_bytes;
         } else {
           rowp[r] = (DUAL && row >= out_dim) ? w_b + (size_t)(row - out_dim) * row_bytes : w + (size_t)row * row_bytes;
         }
       }
     }
   };
-  set_group(blockIdx.x);
+  set_group(bid);
 
   float acc[R][M];
 #pragma unroll
@@ -300,10 +320,9 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
           const u32 row = row0 + r;
           if (lane == 0 && row < total_rows) {
             if constexpr (LIST) {   // (one token: m = 0)
-              const u32 r0 = list->rows[0], r01 = r0 + list->rows[1];
-              if (row < r0) list->out[0][row] = v;
-              else if (row < r01) list->out[1][row - r0] = v;
-              else list->out[2][row - r01] = v;
+              u32 first;
+              float* const om = list->pick(row, list->out, first);
+              om[row - first] = v;
             } else if (DUAL && row >= out_dim) {
               out_b[(size_t)m * out_dim + (row - out_dim)] = v;
             } else {
@@ -332,8 +351,8 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
 #pragma unroll
       for (int wv = 1; wv < GEMV_WAVES; wv++)
         if (top_v[tid][wv] > best || (top_v[tid][wv] == best && top_i[tid][wv] < best_id)) best = top_v[tid][wv], best_id = top_i[tid][wv];
-      out[(size_t)tid * gridDim.x + blockIdx.x] = best;
-      top_ids[(size_t)tid * gridDim.x + blockIdx.x] = best_id;
+      out[(size_t)tid * nwg + bid] = best;
+      top_ids[(size_t)tid * nwg + bid] = best_id;
     }
   };
 
@@ -387,8 +406,8 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
     // between the request for the activations and their way into LDS); a later group requests them at the top of the
     // loop, after staging its first chunk of activations again if the row is longer than one chunk (otherwise the
     // activations stay where they are).
-    for (u32 grp = blockIdx.x;;) {
-      if (grp != blockIdx.x) {
+    for (u32 grp = bid;;) {
+      if (grp != bid) {
         if (ncs > CH) {
           __builtin_amdgcn_s_barrier();   // every wavefront has read the last chunk into registers
           stage_chunk_serial(0);
@@ -398,7 +417,7 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
       }
       for (u32 s = 0; s + 1 < ncs; s++) column_set(s, gemv_false{});
       column_set(ncs - 1, gemv_true{});
-      grp += gridDim.x;
+      grp += nwg;
       if (grp >= ngroups) break;
       finish(row0);
 #pragma unroll
@@ -409,12 +428,12 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
     }
   }
   // Column sets are taken F::SPI at a time: all their weight loads are issued before the first is consumed. Directly
-  // staged activations of one token group (two tokens of a K-quant): the workgroup walks the row groups blockIdx.x,
-  // blockIdx.x + gridDim.x, ... and stages the activations again only if the row is longer than one chunk.
+  // staged activations of one token group (two tokens of a K-quant): the workgroup walks the row groups bid,
+  // bid + nwg, ... and stages the activations again only if the row is longer than one chunk.
   if constexpr (!PIPE) {
     constexpr bool WALK = DIRECT && NG == 1;
-    for (u32 grp = blockIdx.x;;) {
-      const bool first = grp == blockIdx.x;
+    for (u32 grp = bid;;) {
+      const bool first = grp == bid;
       for (u32 s = 0; s < ncs; s += F::SPI) {
         const bool restage = NG == 1 && (s % CH) == 0 && (first || ncs > CH);   // CH is a multiple of SPI or covers the whole row
         typename F::template Stage<R> stA, stB;
@@ -439,7 +458,7 @@ __device__ __forceinline__ void gemv_core(const uint8_t* __restrict__ w, const f
         if (two) step(stB, s + 1);
       }
       if (!WALK) break;
-      grp += gridDim.x;
+      grp += nwg;
       if (grp >= ngroups) break;
       finish(row0);
 #pragma unroll
@@ -519,7 +538,7 @@ __device__ __forceinline__ void gemv_entry(const uint8_t* w, const float* x, con
       return;
     }
   }
-  gemv_core<F, M, ADD, false, false, false, false, RO>(w, x, residual, out, in_dim, out_dim);
+  gemv_core<F, M, ADD, false, false, false, 0, RO>(w, x, residual, out, in_dim, out_dim);
 }
 
 // ---- entry points ---------------------------------------------------------------------------
@@ -669,9 +688,45 @@ extern "C" __global__ __launch_bounds__(GEMV_BLOCK) GEMV_OCC(1) void q4_k_dual_g
 extern "C" __global__ __launch_bounds__(GEMV_BLOCK) GEMV_OCC(1) void q4_k_many_gemv_f32(
     const uint8_t* w0, const uint8_t* w1, const uint8_t* w2, const float* x, float* out0, float* out1, float* out2, u32 in_dim,
     u32 rows0, u32 rows1, u32 rows2) {
-  const GemvList list = {{w0, w1, w2}, {out0, out1, out2}, {rows0, rows1, rows2}};
-  gemv_core<FmtQ4K, 1, false, true, false, false, true>(nullptr, x, nullptr, nullptr, in_dim, 0, nullptr, nullptr, nullptr, &list);
+  const GemvList<3> list = {{w0, w1, w2}, {out0, out1, out2}, {rows0, rows1, rows2}};
+  gemv_core<FmtQ4K, 1, false, true, false, false, 3>(nullptr, x, nullptr, nullptr, in_dim, 0, nullptr, nullptr, nullptr, &list);
 }
+
+// (list: six weight addresses, six outputs, six row counts by value, x, in_dim): one token against up to six matrices of one type and
+// row length; block, dynamic shared memory and grid as <type>_gemv_f32 for a matrix of all their rows, every row computed as there.
+// A launch costs its start (dispatch, activations, first rows) and its end whatever it reads, so the projections of a layer that
+// read one input (q | k | v | gate | up) are one: 4096 -> 30720 rows of Q4_K 20.7 us as q | k | v and gate | up, 16.6 as one (71 MB at 4.3 TB/s);
+// of Q5_K, which had no lists, 30.5 as five launches and 22.1; 1024 -> 7680 8.2 | 5.2 and 16.2 | 7.0.
+#define GEMV_LIST_ENTRY(NAME, FMT)                                                                                              \
+  extern "C" __global__ __launch_bounds__(GEMV_BLOCK) GEMV_OCC(1) void NAME(const GemvList<6> list, const float* x, u32 in_dim) { \
+    gemv_core<FMT, 1, false, true, false, false, 6>(nullptr, x, nullptr, nullptr, in_dim, 0, nullptr, nullptr, nullptr, &list);  \
+  }
+GEMV_LIST_ENTRY(q4_k_list_gemv_f32, FmtQ4K)
+GEMV_LIST_ENTRY(q5_k_list_gemv_f32, FmtQ5K)
+
+// (w_a, x_a, out_a, in_dim_a, out_dim_a, w_b, x_b, out_b, in_dim_b, out_dim_b, wgs_b): one token of two matrices with an input each in one
+// launch (o and down of a layer). Workgroups 0 .. wgs_b - 1 are those of <type_b>_gemv_f32[_r1] for its matrix, the ones behind those
+// of <type_a>_gemv_f32[_r1]: the longer rows start first and the others fill the compute units as they come free. Dynamic shared memory: the
+// larger of the two. Every row is computed as in those kernels. Q4_K 4096 -> 4096 and Q6_K 12288 -> 4096: 14.2 us one after the other, 11.7 as one (50.7 MB at
+// 4.3 TB/s); 1024 -> 1024 and 3072 -> 1024 5.7 | 3.5.
+#define GEMV_TWO_ENTRY(NAME, FMT_A, FMT_B, RO)                                                                                   \
+  extern "C" __global__ __launch_bounds__(GEMV_BLOCK) GEMV_OCC(1) void NAME(                                                      \
+      const uint8_t* w_a, const float* x_a, float* out_a, u32 in_dim_a, u32 out_dim_a, const uint8_t* w_b, const float* x_b,      \
+      float* out_b, u32 in_dim_b, u32 out_dim_b, u32 wgs_b) {                                                                    \
+    if (blockIdx.x < wgs_b)                                                                                                      \
+      gemv_core<FMT_B, 1, false, false, false, false, 0, RO>(w_b, x_b, nullptr, out_b, in_dim_b, out_dim_b, nullptr, nullptr, nullptr, \
+                                                             nullptr, nullptr, blockIdx.x, wgs_b);                               \
+    else                                                                                                                         \
+      gemv_core<FMT_A, 1, false, false, false, false, 0, RO>(w_a, x_a, nullptr, out_a, in_dim_a, out_dim_a, nullptr, nullptr, nullptr, \
+                                                             nullptr, nullptr, blockIdx.x - wgs_b, gridDim.x - wgs_b);           \
+  }
+#define GEMV_TWO_ENTRIES(A, FMT_A, B, FMT_B)             \
+  GEMV_TWO_ENTRY(A##_and_##B##_gemv_f32, FMT_A, FMT_B, 0) \
+  GEMV_TWO_ENTRY(A##_and_##B##_gemv_f32_r1, FMT_A, FMT_B, 1)
+GEMV_TWO_ENTRIES(q4_k, FmtQ4K, q4_k, FmtQ4K)
+GEMV_TWO_ENTRIES(q4_k, FmtQ4K, q6_k, FmtQ6K)
+GEMV_TWO_ENTRIES(q5_k, FmtQ5K, q4_k, FmtQ4K)
+GEMV_TWO_ENTRIES(q5_k, FmtQ5K, q6_k, FmtQ6K)
 
 // (gate, up, out, n): out[i] = silu(gate[i]) * up[i], the reference's swiglu_f32 (bin/cuda_ffn_sequence_probe.cr:46-84).
 // block = 256, grid = ceil(n / 256).

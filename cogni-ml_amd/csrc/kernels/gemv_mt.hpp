@@ -281,6 +281,40 @@ extern "C" __global__ __launch_bounds__(256) void pack_x_mt_q6k_f16(const float*
   mt_pack_store_q6k(image, nsbp, sb, tok, lane, v, present);
 }
 
+// The images of two activation blocks of `tokens` tokens in one launch: workgroups 0 .. 2 * padded super-blocks of a - 1 (4 * for
+// sixteen tokens) are those of the pack kernel of a's order, the ones behind those of b's. A short launch costs about 1.5 us in a stream
+// whatever it does. (x_a, image_a, in_dim_a, q6_a, x_b, image_b, in_dim_b, q6_b, tokens), q6: the Q6_K order
+template <bool X16>
+__device__ __forceinline__ void pack_mt_two(const float* __restrict__ x_a, uint8_t* __restrict__ image_a, u32 in_dim_a, u32 q6_a,
+                                            const float* __restrict__ x_b, uint8_t* __restrict__ image_b, u32 in_dim_b, u32 q6_b, u32 tokens) {
+  constexpr u32 SLOTS = X16 ? 16 : 8;
+  const u32 lane = threadIdx.x & 63, wgs_a = SLOTS / 4 * gemv_mt_padded_sb(in_dim_a);
+  const bool b = blockIdx.x >= wgs_a;   // the same for the whole workgroup
+  const float* const x = b ? x_b : x_a;
+  uint8_t* const image = b ? image_b : image_a;
+  const u32 in_dim = b ? in_dim_b : in_dim_a, q6 = b ? q6_b : q6_a;
+  const u32 unit = (blockIdx.x - (b ? wgs_a : 0u)) * 4 + (threadIdx.x >> 6);
+  const u32 nsb = in_dim >> 8, nsbp = gemv_mt_padded_sb(in_dim), sb = unit / SLOTS, tok = unit % SLOTS;
+  if (sb >= nsbp) return;
+  const bool present = tok < tokens && sb < nsb;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (present) __builtin_memcpy(&v, x + (size_t)tok * in_dim + (size_t)sb * 256 + 4 * lane, 16);
+  if constexpr (X16) {
+    if (q6) mt_pack16_store_q6k(image, nsbp, sb, tok, lane, v);
+    else mt_pack16_store_q4k(image, nsbp, sb, tok, lane, v);
+  } else {
+    if (q6) mt_pack_store_q6k(image, nsbp, sb, tok, lane, v, present);
+    else mt_pack_store_q4k(image, nsbp, sb, tok, lane, v, present);
+  }
+}
+#define PACK_MT_TWO_ENTRY(NAME, X16)                                                                                                   \
+  extern "C" __global__ __launch_bounds__(256) void NAME(const float* x_a, uint8_t* image_a, u32 in_dim_a, u32 q6_a, const float* x_b, \
+                                                         uint8_t* image_b, u32 in_dim_b, u32 q6_b, u32 tokens) {                       \
+    pack_mt_two<X16>(x_a, image_a, in_dim_a, q6_a, x_b, image_b, in_dim_b, q6_b, tokens);                                              \
+  }
+PACK_MT_TWO_ENTRY(pack_x_mt_two_f16, false)
+PACK_MT_TWO_ENTRY(pack_x_mt16_two_f16, true)
+
 // ---- loads in assembly ---------------------------------------------------------------------------------------------------
 // The compiler knows neither that these are loads nor when they land. A value loaded this way must not be touched before
 // mt_wait<N> has said that it is there and mt_pin has tied it to that wait.
@@ -607,10 +641,26 @@ typedef MtQ6KT<false> MtQ6K;
 typedef MtQ6KT<true> MtQ6Kx16;
 
 // ---- the GEMV ------------------------------------------------------------------------------------------------------------
+template <int N>
 struct MtArgs {
-  const uint8_t* w[3];
-  float* out[3];
-  u32 rows[3];
+  const uint8_t* w[N];
+  float* out[N];
+  u32 rows[N];
+  // the pointer of the matrix that row `row` of all of them belongs to, that matrix's first row and its row count
+  template <class P, int I = 0>
+  __device__ __forceinline__ P pick(u32 row, P const (&of)[N], u32& first, u32& count, u32 begin = 0) const {
+    if constexpr (I + 1 < N) {
+      if (row >= begin + rows[I]) return pick<P, I + 1>(row, of, first, count, begin + rows[I]);
+    }
+    first = begin;
+    count = rows[I];
+    return of[I];
+  }
+  template <int I = 0>
+  __device__ __forceinline__ u32 total() const {
+    if constexpr (I + 1 < N) return rows[I] + total<I + 1>();
+    return rows[I];
+  }
 };
 
 // (mt_stream_wait, the number a streamed unit waits with, lives in gemv_config.h: host code can test it there)
@@ -628,8 +678,8 @@ struct MtArgs {
 // null then; rows[0] a multiple of 256 up to GEMV_MT_MAX_IN_DIM): single binary16 terms need no scale of a whole super-block, and the
 // sixteen rows of a group are one of its sub-blocks, so a workgroup has all that it takes. The FFN half of a layer, 4096 -> 12288 -> 4096,
 // 13 tokens, without the pack launch 36.6 -> 35.2 us.
-template <class F, int SBW, int T, bool SWIGLU = false, bool TOP1 = false, bool NEXT = false>
-__device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __restrict__ image,
+template <class F, int SBW, int T, bool SWIGLU = false, bool TOP1 = false, bool NEXT = false, int N = 3>
+__device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* __restrict__ image,
                                              const float* __restrict__ residual, u32 in_dim, u32 tokens,
                                              u32* __restrict__ top_ids = nullptr, float* __restrict__ logits = nullptr,
                                              uint8_t* __restrict__ next = nullptr) {
@@ -648,7 +698,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
   const int tid = threadIdx.x, lane = tid & 63;
   const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const u32 nsb = in_dim >> 8, nsbp = gemv_mt_padded_sb(in_dim);   // super-blocks of a row, and of the image
-  const u32 total_rows = a.rows[0] + a.rows[1] + a.rows[2];
+  const u32 total_rows = a.total();
   const u32 ntiles = (total_rows + 15) >> 4;
   const u32 ngroups = SWIGLU ? (a.rows[0] + 15) >> 4 : (ntiles + T - 1) / T;
   // LDS: partial[wave][GEMV_MT_TMAX][NTOK tokens][16 rows] f32 | slots[wave][NSLOT units]
@@ -724,17 +774,17 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
   auto set_rows = [&](u32 g, int mat = 0) {   // (mat: with SWIGLU and streamed operands, gate (0) and up (1) take turns)
 #pragma unroll
     for (int t = 0; t < T; t++) {
+      // the tile's matrix (rows of all but the last are multiples of 16, so a tile is of one matrix), uniform over the workgroup
+      u32 first = 0, count = a.rows[0];
+      const u32 tile_row = (SWIGLU ? g : g * T + (u32)t) * 16;
+      const uint8_t* wm;
+      if constexpr (SWIGLU) wm = a.w[STREAM ? mat : t];
+      else wm = a.pick(min(tile_row, total_rows - 1), a.w, first, count);
 #pragma unroll
       for (int m = 0; m < NC; m++) {
         const u32 p = 64u * m + lane;
         const u32 pr = min(p / (u32)F::P, 15u), piece = p - (u32)F::P * (p / (u32)F::P);
-        const u32 vr = SWIGLU ? min(g * 16 + pr, a.rows[0] - 1) : min((g * T + (u32)t) * 16 + pr, total_rows - 1);
-        const uint8_t* rp;
-        if constexpr (SWIGLU) rp = a.w[STREAM ? mat : t] + (size_t)vr * row_bytes;
-        else if (vr < a.rows[0]) rp = a.w[0] + (size_t)vr * row_bytes;
-        else if (vr < a.rows[0] + a.rows[1]) rp = a.w[1] + (size_t)(vr - a.rows[0]) * row_bytes;
-        else rp = a.w[2] + (size_t)(vr - a.rows[0] - a.rows[1]) * row_bytes;
-        cptr[t][m] = rp + F::piece_offset(piece);
+        cptr[t][m] = wm + (size_t)min(tile_row - first + pr, count - 1) * row_bytes + F::piece_offset(piece);
       }
     }
   };
@@ -819,14 +869,12 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
           const bool real = row < a.rows[0];
           top1_take(top_v, top_i, real ? v : -__builtin_inff(), real ? row : 0xFFFFFFFFu);
           if (logits && real) logits[(size_t)m * a.rows[0] + row] = v;
-        } else if (row < a.rows[0]) {
-          const size_t oi = (size_t)m * a.rows[0] + row;
-          if (residual) v += residual[oi];
-          a.out[0][oi] = v;
-        } else if (row < a.rows[0] + a.rows[1]) {
-          a.out[1][(size_t)m * a.rows[1] + (row - a.rows[0])] = v;
         } else if (row < total_rows) {
-          a.out[2][(size_t)m * a.rows[2] + (row - a.rows[0] - a.rows[1])] = v;
+          u32 first, count;
+          float* const om = a.pick(row, a.out, first, count);
+          const size_t oi = (size_t)m * count + (row - first);
+          if (residual && first == 0) v += residual[oi];   // (the first matrix's)
+          om[oi] = v;
         }
       }
     }
@@ -966,26 +1014,25 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs& a, const uint8_t* __r
 // The tile count per wavefront follows from the row count (gemv_mt_tiles, the rule the host sizes the grid with); tile
 // count and super-blocks per k-slice are template parameters so that register use and loads in flight are compile-time
 // constants. Shapes outside gemv_mt_supported() must not be launched.
-template <class F, bool TOP1 = false>
-__device__ __forceinline__ void gemv_mt_dispatch(const MtArgs& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens,
+template <class F, bool TOP1 = false, int N = 3>
+__device__ __forceinline__ void gemv_mt_dispatch(const MtArgs<N>& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens,
                                                  u32* top_ids = nullptr, float* logits = nullptr) {
-  const u32 ntiles = (a.rows[0] + a.rows[1] + a.rows[2] + 15) >> 4;
-  const u32 t = gemv_mt_tiles(F::TYPE, in_dim, ntiles);
+  const u32 t = gemv_mt_tiles(F::TYPE, in_dim, (a.total() + 15) >> 4);
   switch (gemv_mt_padded_sb(in_dim) >> 3) {
     case 1:
-      if (t <= 1) gemv_mt_core<F, 1, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if (t == 2) gemv_mt_core<F, 1, 2, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 1, 3, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
+      if (t <= 1) gemv_mt_core<F, 1, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if (t == 2) gemv_mt_core<F, 1, 2, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 1, 3, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
       break;
     case 2:
-      if (t <= 1) gemv_mt_core<F, 2, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if (t == 2) gemv_mt_core<F, 2, 2, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 2, 3, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits);
+      if (t <= 1) gemv_mt_core<F, 2, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if (t == 2) gemv_mt_core<F, 2, 2, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 2, 3, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
       break;
-    case 3: gemv_mt_core<F, 3, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
-    case 4: gemv_mt_core<F, 4, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
-    case 5: gemv_mt_core<F, 5, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
-    default: gemv_mt_core<F, 6, 1, false, TOP1>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 3: gemv_mt_core<F, 3, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 4: gemv_mt_core<F, 4, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 5: gemv_mt_core<F, 5, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    default: gemv_mt_core<F, 6, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
   }
 }
 
@@ -993,7 +1040,7 @@ __device__ __forceinline__ void gemv_mt_dispatch(const MtArgs& a, const uint8_t*
   extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void NAME(                                                 \
       const uint8_t* w0, const uint8_t* w1, const uint8_t* w2, const uint8_t* image, const float* residual, float* out0, \
       float* out1, float* out2, u32 in_dim, u32 rows0, u32 rows1, u32 rows2, u32 tokens) {                               \
-    const MtArgs a = {{w0, w1, w2}, {out0, out1, out2}, {rows0, rows1, rows2}};                                          \
+    const MtArgs<3> a = {{w0, w1, w2}, {out0, out1, out2}, {rows0, rows1, rows2}};                                          \
     gemv_mt_dispatch<FMT>(a, image, residual, in_dim, tokens);                                                           \
   }
 GEMV_MT_ENTRY(q4_k_gemv_mt_f32, MtQ4K)
@@ -1007,6 +1054,17 @@ GEMV_MT_ENTRY(q5_k_gemv_mt16_f32, MtQ5Kx16)
 GEMV_MT_ENTRY(q6_k_gemv_mt16_f32, MtQ6Kx16)
 GEMV_MT_ENTRY(q8_0_gemv_mt16_f32, MtQ80x16)
 
+// (list: six weight addresses, six outputs, six row counts by value, image, in_dim, tokens): up to six matrices against one image in one
+// launch (q | k | v | gate | up), everything else as in the three-matrix kernels above
+#define GEMV_MT_LIST_ENTRY(NAME, FMT)                                                                                              \
+  extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void NAME(const MtArgs<6> list, const uint8_t* image, u32 in_dim, u32 tokens) { \
+    gemv_mt_dispatch<FMT>(list, image, nullptr, in_dim, tokens);                                                                 \
+  }
+GEMV_MT_LIST_ENTRY(q4_k_gemv_mt_list_f32, MtQ4K)
+GEMV_MT_LIST_ENTRY(q5_k_gemv_mt_list_f32, MtQ5K)
+GEMV_MT_LIST_ENTRY(q4_k_gemv_mt16_list_f32, MtQ4Kx16)
+GEMV_MT_LIST_ENTRY(q5_k_gemv_mt16_list_f32, MtQ5Kx16)
+
 // (w, image, partial_ids, partial_values, in_dim, out_dim, tokens): the output head's arg-max for 2..8 tokens in one pass
 // over the weights. Grid, block and dynamic shared memory as q4_k_gemv_mt_f32 | q6_k_gemv_mt_f32 for out_dim rows;
 // partial_*[token * gridDim.x + workgroup], finished by top1_reduce_f32 with count = gridDim.x. The one-token kernel's
@@ -1018,7 +1076,7 @@ GEMV_MT_ENTRY(q8_0_gemv_mt16_f32, MtQ80x16)
   /* of a row's matrix away, and this release of the compiler crashes in its control-flow simplification doing so)    */  \
   u32 none;                                                                                                               \
   asm volatile("s_mov_b32 %0, 0" : "=s"(none));                                                                           \
-  const MtArgs a = {{w, w, w}, {partial_values, partial_values, partial_values}, {out_dim, none, none}};                  \
+  const MtArgs<3> a = {{w, w, w}, {partial_values, partial_values, partial_values}, {out_dim, none, none}};                  \
   gemv_mt_dispatch<FMT, true>(a, image, nullptr, in_dim, tokens, partial_ids, LOGITS);
 #define GEMV_MT_TOP1_ENTRY(NAME, FMT)                                                                                    \
   extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void NAME(const uint8_t* w, const uint8_t* image,          \
@@ -1041,7 +1099,7 @@ GEMV_MT_TOP1_ENTRY(q6_k_gemv_mt_top1_partial_f32, MtQ6K)
 template <class F, bool NEXT = false>
 __device__ __forceinline__ void gemv_mt_swiglu_dispatch(const uint8_t* w_gate, const uint8_t* w_up, const uint8_t* image, float* out,
                                                         u32 in_dim, u32 out_dim, u32 tokens, uint8_t* next = nullptr) {
-  const MtArgs a = {{w_gate, w_up, nullptr}, {out, nullptr, nullptr}, {out_dim, out_dim, 0u}};
+  const MtArgs<3> a = {{w_gate, w_up, nullptr}, {out, nullptr, nullptr}, {out_dim, out_dim, 0u}};
   switch (gemv_mt_padded_sb(in_dim) >> 3) {
     case 1: gemv_mt_core<F, 1, 2, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;
     case 2: gemv_mt_core<F, 2, 2, true, false, NEXT>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, next); break;

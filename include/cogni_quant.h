@@ -151,7 +151,9 @@ int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residua
  *                           "q6_k_gemv_mt_f32" | "q8_0_gemv_mt_f32" (w0, w1, w2,
  *                           image, residual, out0, out1, out2, in_dim, rows0, rows1, rows2, tokens), block 512, up to three
  *                           matrices per launch as one matrix of all their rows (a matrix whose row count is not a multiple
- *                           of 16 ends its launch), geometry from cogni_gemv_packed_launch_dims.
+ *                           of 16 ends its launch), geometry from cogni_gemv_packed_launch_dims. Four to six of Q4_K or Q5_K:
+ *                           "<type>_gemv_mt_list_f32" (six weight pointers, six output pointers, six row counts by value, image,
+ *                           in_dim, tokens).
  * The image is caller-owned device memory; pack and GEMV are ordered by the stream. Accuracy: about 5e-7 of max|out|
  * (22-bit activations, exact weights, fp32 accumulation).
  * cogni_gemv_dev (from 3 to 5 tokens on, by type and row length), cogni_gemv_dual_dev and cogni_gemv_many_dev (2 tokens
@@ -202,7 +204,7 @@ int cogni_gemv_packed_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t image
  * cogni_gemv_pack16_dev writes the image (cogni_gemv_image_bytes(type, in_dim, 8) bytes: the same size; Q4_K and Q5_K
  * share one, Q6_K has its own; kernels "pack_x_mt16_q4k_f16" | "pack_x_mt16_q6k_f16" (x, image, tokens:u32, in_dim:u32), block
  * 256, grid 4 * ceil(in_dim / 2048) * 8); cogni_gemv_packed16_dev runs up to eight matrices of one type and row length
- * against it, three per launch, a [tokens][out_dim] residual (may be 0) with a single matrix (kernels "q4_k_gemv_mt16_f32" |
+ * against it, three per launch (Q4_K, Q5_K: six, "<type>_gemv_mt16_list_f32"), a [tokens][out_dim] residual (may be 0) with a single matrix (kernels "q4_k_gemv_mt16_f32" |
  * "q5_k_gemv_mt16_f32" | "q6_k_gemv_mt16_f32" | "q8_0_gemv_mt16_f32" - Q8_0 reads the Q4_K image -, parameters, grid and block of "<type>_gemv_mt_f32", 12 KiB more dynamic
  * shared memory). The reference has no counterpart: its router sends every M > 8 to the prefill GEMM
  * (src/ml/gguf/qwen35_cpu.cr:1478-1490); cogni_matmul_dev takes this path by itself for 9..16 tokens of a K-quant matrix without a bias (Q8_0, whose reference path stays in
@@ -252,6 +254,19 @@ int cogni_gemv_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
 int cogni_gemv_dual_dev(uint64_t w_raw_a, uint64_t w_raw_b, uint32_t w_type, uint64_t x, uint64_t out_a, uint64_t out_b,
                         uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream);
 
+/* cogni_gemv_pack_dev | cogni_gemv_pack16_dev of two activation blocks of `tokens` tokens in one launch (the inputs of o and down of a
+ * layer), each byte for byte what that call writes. Kernels "pack_x_mt_two_f16" | "pack_x_mt16_two_f16" (x_a, image_a, in_dim_a, q6_a:u32, x_b,
+ * image_b, in_dim_b, q6_b:u32, tokens; q6: 1 for the Q6_K order), block 256, grid the sum of the two. */
+int cogni_gemv_pack_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t image_a, uint64_t x_b, uint32_t type_b, uint32_t in_dim_b,
+                            uint64_t image_b, uint32_t tokens, void* stream);
+int cogni_gemv_pack16_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t image_a, uint64_t x_b, uint32_t type_b, uint32_t in_dim_b,
+                              uint64_t image_b, uint32_t tokens, void* stream);
+/* Two matrices with an input each (o and down of a layer): out[m*out_dim + o] = sum_j x[m*in_dim + j] * deq(W[o][j]) for a and for b. One
+ * token of a Q4_K or Q5_K matrix beside a Q4_K or Q6_K one is one launch of "<type_a>_and_<type_b>_gemv_f32[_r1]" (w_a, x_a, out_a, in_dim_a,
+ * out_dim_a, w_b, x_b, out_b, in_dim_b, out_dim_b, workgroups of b:u32), block and shared memory (the larger) as cogni_gemv_plan gives
+ * them for the two, every row bit for bit as from cogni_gemv_dev; anything else is cogni_gemv_dev for the one and the other. */
+int cogni_gemv_two_dev(uint64_t w_a, uint32_t type_a, uint64_t x_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a, uint64_t w_b,
+                       uint32_t type_b, uint64_t x_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens, void* stream);
 /* Several matrices of one type and in_dim against the same activations (q | k | v, gate | up) on device pointers: the
  * reference's qmatvec_many seam (src/ml/gguf/qwen35_cpu.cr:1419-1445), which hands a list of weights and one x to the
  * GPU arm.  out[i][m*out_dims[i] + o] = sum_j x[m*in_dim + j] * deq(W_i[o][j]).
@@ -259,8 +274,9 @@ int cogni_gemv_dual_dev(uint64_t w_raw_a, uint64_t w_raw_b, uint32_t w_type, uin
  * kernel takes: one launch per group of up to four tokens of "q4_k_many_gemv_mfma_f32_tbatchM"
  * (w0, w1, w2, x, out0, out1, out2, in_dim, rows0, rows1, rows2), block 512, grid and shared memory of one matrix with
  * the sum of the rows (cogni_gemv_plan), the activations staged once for all of them. Two matrices of one shape: as
- * cogni_gemv_dual_dev. One token of Q4_K matrices: up to three per launch of "q4_k_many_gemv_f32" (the same parameter
- * list), block, shared memory and grid as cogni_gemv_launch_dims gives one token of a matrix with the sum of the rows; each
+ * cogni_gemv_dual_dev. One token of Q4_K or Q5_K matrices: up to six per launch of "<type>_list_gemv_f32" (six weight pointers, six
+ * output pointers, six row counts by value, x, in_dim; two or three of Q4_K "q4_k_many_gemv_f32", the same parameter
+ * list as above), block, shared memory and grid as cogni_gemv_launch_dims gives one token of a matrix with the sum of the rows; each
  * row comes out bit for bit as from cogni_gemv_dev. Everything else: one cogni_gemv_dev per matrix. count in 1..8. */
 int cogni_gemv_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t x, const uint64_t* out, const uint32_t* out_dims,
                         uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
@@ -428,6 +444,10 @@ size_t cogni_gemm_workspace_bytes_split(uint32_t w_type, uint32_t in_dim, uint32
  * converts x inside the kernel (gemm_q4k.metal:678-686). */
 int cogni_gemm_pack_dev(uint64_t x, uint32_t w_type, uint32_t in_dim, uint32_t tokens, uint64_t workspace, size_t workspace_bytes,
                         void* stream);
+/* Two activation blocks of `tokens` tokens in one launch, each byte for byte what cogni_gemm_pack_dev writes: kernel "pack_x_two_f16" (x_a,
+ * workspace_a, in_dim_a, q6_a:u32, x_b, workspace_b, in_dim_b, q6_b:u32, tokens; q6: 1 for the Q6_K order), block 256, grid the sum of the two. */
+int cogni_gemm_pack_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t workspace_a, size_t bytes_a, uint64_t x_b, uint32_t type_b,
+                            uint32_t in_dim_b, uint64_t workspace_b, size_t bytes_b, uint32_t tokens, void* stream);
 int cogni_gemm_packed_dev(uint64_t w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t bias, uint64_t out,
                           uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream);
 int cogni_gemm_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias, uint64_t out, uint32_t in_dim,
@@ -452,9 +472,8 @@ int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
  * a prefill layer, the counterpart for M > 8 of cogni_gemv_many_dev (the reference issues one qmatmul_nobias per weight,
  * src/ml/gguf/qwen35_cpu.cr:1478-1490): out_i[m][o] = sum_j x[m][j] * deq(W_i[o][j]), every output bit for bit what
  * cogni_gemm_packed_dev gives for that matrix with a workspace that holds the packed activations only (no k split). One to
- * six matrices, Q4_K or Q5_K, no bias. A matrix that alone gets the 256-row tiles of q4_k_gemm_wide_f16 (cogni_gemm_plan)
- * keeps them and is launched by itself; the others form the list. Kernels "<type>_gemm_many[_m64][_n128]_f16" (list by value: six weight pointers, six
- * output pointers, six row counts, six cumulative tile counts, the count; workspace; in_dim:u32; tokens:u32), block 256,
+ * six matrices, Q4_K or Q5_K, no bias. Kernels "<type>_gemm_many[_m64][_n128]_f16", "q4_k_gemm_many_wide_f16" (list by value: six weight pointers, six
+ * output pointers, six row counts, six cumulative tile counts, the count; workspace; in_dim:u32; tokens:u32), block 256 (wide: 512),
  * grid as cogni_gemm_plan gives it for a matrix of all the tiles. */
 int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
                                const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);

@@ -33,3 +33,97 @@ def test_swiglu_that_writes_the_next_image(gpu, in_dim, out_dim, tokens):
         quant.gemv_packed16_swiglu_pack_dev(wg.ptr, wu.ptr, Q4_K, image.ptr, 0, Q6_K, pc.ptr, in_dim, out_dim - 16, tokens)
     for a in (wg, wu, xd, image, want, got, pa, pb, pc):
         a.close()
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q5_K])
+@pytest.mark.parametrize("in_dim,dims", [(4096, [4096, 1024, 1024, 12288, 12288]), (256, [1, 7, 3, 2]), (12288, [40, 9, 300, 5, 17, 2]),
+                                         (2048, [9000, 1, 1, 1, 1, 1, 33])])
+def test_lists_of_one_token(gpu, t, in_dim, dims):
+    """Up to six matrices in a launch: each row as cogni_gemv_dev computes it."""
+    rng = np.random.default_rng(in_dim + len(dims))
+    xd = DevArray(synth.make_activations(rng, 1, in_dim))
+    wd = [DevArray(synth.make_weights(rng, t, d, in_dim)) for d in dims]
+    one, lst = ([DevArray(np.full(d, np.float32(5.0))) for d in dims] for _ in range(2))
+    for w, o, d in zip(wd, one, dims):
+        quant.gemv_dev(w.ptr, t, xd.ptr, o.ptr, in_dim, d)
+    quant.gemv_many_dev([w.ptr for w in wd], t, xd.ptr, [o.ptr for o in lst], dims, in_dim)
+    for a, b, d in zip(one, lst, dims):
+        assert np.array_equal(a.read(np.float32, d), b.read(np.float32, d)), d
+    for a in [xd] + wd + one + lst:
+        a.close()
+
+
+# both orders, both row counts per wavefront, rows of one and of several column sets, types without the kernel
+@pytest.mark.parametrize("a,b", [((Q4_K, 4096, 4096), (Q6_K, 12288, 4096)), ((Q6_K, 3072, 1024), (Q5_K, 1024, 1024)), ((Q4_K, 8192, 3), (Q4_K, 256, 5000)),
+                                 ((Q5_K, 2560, 2041), (Q4_K, 256, 2048)), ((Q6_K, 512, 40), (Q6_K, 256, 33)), ((Q4_K, 256, 1), (Q6_K, 256, 12300))])
+def test_two_matrices_with_an_input_each(gpu, a, b):
+    rng = np.random.default_rng(a[2] + b[2])
+    mats = []
+    for t, in_dim, out_dim in (a, b):
+        mats.append((DevArray(synth.make_weights(rng, t, out_dim, in_dim)), t, DevArray(synth.make_activations(rng, 1, in_dim)),
+                     DevArray(np.full(out_dim, np.float32(5.0))), DevArray(np.full(out_dim, np.float32(6.0))), in_dim, out_dim))
+    for w, t, x, one, two, in_dim, out_dim in mats:
+        quant.gemv_dev(w.ptr, t, x.ptr, one.ptr, in_dim, out_dim)
+    quant.gemv_two_dev(*[v for w, t, x, one, two, in_dim, out_dim in mats for v in (w.ptr, t, x.ptr, two.ptr, in_dim, out_dim)])
+    for w, t, x, one, two, in_dim, out_dim in mats:
+        assert np.array_equal(one.read(np.float32, out_dim), two.read(np.float32, out_dim)), (t, in_dim, out_dim)
+    w, t, x, one, two, in_dim, out_dim = mats[0]
+    with pytest.raises(quant.QuantError, match="null device pointer"):
+        quant.gemv_two_dev(w.ptr, t, 0, two.ptr, in_dim, out_dim, w.ptr, t, x.ptr, two.ptr, in_dim, out_dim)
+    for m in mats:
+        for i in (0, 2, 3, 4):
+            m[i].close()
+
+
+# lists whose tile counts take one, two and three tiles per wavefront, a ragged last matrix, streamed operands, sixteen tokens
+@pytest.mark.parametrize("t", [Q4_K, Q5_K])
+@pytest.mark.parametrize("tokens,in_dim,dims", [(8, 4096, [4096, 1024, 1024, 12288, 12288]), (2, 2048, [16, 32, 48, 5]), (5, 1024, [4096, 16, 6000, 160, 11]),
+                                                (3, 6144, [16, 160, 32, 48, 64, 9]), (16, 2048, [1024, 256, 256, 9008, 7]), (9, 12288, [16, 16, 16, 40])])
+def test_lists_of_several_tokens(gpu, t, tokens, in_dim, dims):
+    """Four to six matrices against one image: each output as the image and that matrix alone give it."""
+    rng = np.random.default_rng(in_dim + tokens)
+    pack, packed = (quant.gemv_pack16_dev, quant.gemv_packed16_dev) if tokens > 8 else (quant.gemv_pack_dev, quant.gemv_packed_dev)
+    xd, image = DevArray(synth.make_activations(rng, tokens, in_dim)), DevArray(nbytes=quant.gemv_image_bytes(t, in_dim, 8))
+    wd = [DevArray(synth.make_weights(rng, t, d, in_dim)) for d in dims]
+    one, lst = ([DevArray(np.full(tokens * d, np.float32(5.0))) for d in dims] for _ in range(2))
+    pack(xd.ptr, t, in_dim, tokens, image.ptr)
+    for w, o, d in zip(wd, one, dims):
+        packed([w.ptr], t, image.ptr, [o.ptr], [d], in_dim, tokens)
+    packed([w.ptr for w in wd], t, image.ptr, [o.ptr for o in lst], dims, in_dim, tokens)
+    for a, b, d in zip(one, lst, dims):
+        assert np.array_equal(a.read(np.float32, tokens * d), b.read(np.float32, tokens * d)), d
+    for a in [xd, image] + wd + one + lst:
+        a.close()
+
+
+@pytest.mark.parametrize("kind", ["gemv", "gemv16", "gemm"])
+@pytest.mark.parametrize("a,b", [((Q4_K, 4096), (Q6_K, 12288)), ((Q6_K, 256), (Q5_K, 2816)), ((Q4_K, 512), (Q4_K, 256))])
+def test_two_activation_blocks_in_one_launch(gpu, kind, a, b):
+    tokens = {"gemv": 5, "gemv16": 13, "gemm": 130}[kind]
+    rng = np.random.default_rng(a[1] + b[1])
+    args, blocks = [], []
+    for t, in_dim in (a, b):
+        x = DevArray(synth.make_activations(rng, tokens, in_dim))
+        nb = quant.gemm_workspace_bytes(t, in_dim, tokens) if kind == "gemm" else quant.gemv_image_bytes(t, in_dim, 8)
+        p, q = (DevArray(np.full(nb, 0xFF, np.uint8)) for _ in range(2))
+        if kind == "gemm":
+            quant.gemm_pack_dev(x.ptr, t, in_dim, tokens, p.ptr, nb)
+            args += [x.ptr, t, in_dim, q.ptr, nb]
+        else:
+            (quant.gemv_pack_dev if kind == "gemv" else quant.gemv_pack16_dev)(x.ptr, t, in_dim, tokens, p.ptr)
+            args += [x.ptr, t, in_dim, q.ptr]
+        blocks.append((x, p, q, nb))
+    {"gemv": quant.gemv_pack_two_dev, "gemv16": quant.gemv_pack16_two_dev, "gemm": quant.gemm_pack_two_dev}[kind](*args, tokens)
+    for x, p, q, nb in blocks:
+        assert np.array_equal(p.read(np.uint8, nb), q.read(np.uint8, nb))
+        for d in (x, p, q):
+            d.close()
+
+
+def test_rounds_of_a_stack():
+    """What reads an output comes in a later round; what cannot be put into rounds stays in its order."""
+    from cogni_ml_amd.projection_stack import QWEN_LAYER_4096, QwenProjectionStackRunner
+    rounds = QwenProjectionStackRunner._rounds_of([e + (None,) for e in QWEN_LAYER_4096])
+    assert [[[e[0] for e in g] for g in r] for r in rounds] == [[["q", "k", "v", "gate", "up"]], [["o"], ["down"]]]
+    for odd in ([("a", "b", Q4_K, 256, 256, None), ("b", "x", Q4_K, 256, 256, None)], [("a", "x", Q4_K, 256, 256, None), ("a", "x", Q4_K, 256, 256, None)]):
+        assert QwenProjectionStackRunner._rounds_of(odd) == [[[e]] for e in odd]
