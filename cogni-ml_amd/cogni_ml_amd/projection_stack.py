@@ -199,7 +199,20 @@ class QwenProjectionStackRunner:
                             lambda *ab: quant.gemv_pack16_two_dev(*ab, count, stream))
             self._pack_each(list(jobs.values()), lambda x, t, k, ws, nbytes: quant.gemm_pack_dev(x, t, k, count, ws, nbytes, stream),
                             lambda *ab: quant.gemm_pack_two_dev(*ab, count, stream))
+            # single matrices of short prefills: two to a launch (o and down)
+            streamed = [g[0] for g in groups if len(g) == 1 and (g[0][1], self._family(g[0][2])) not in jobs16 and
+                        quant.gemm_stream_takes(g[0][2], g[0][4], g[0][3], count)]
+            streamed = streamed[:len(streamed) // 2 * 2]
+            for i in range(0, len(streamed), 2):
+                args = []
+                for name, src, t, out_dim, in_dim, raw in streamed[i:i + 2]:
+                    ws, nbytes = self._prefill_ws[(src, self._family(t))]
+                    args += [self._w[name].ptr, t, ws.ptr, nbytes, self._act[name].ptr, in_dim, out_dim]
+                quant.gemm_stream_two_dev(*args, count, stream)
+            done = {e[0] for e in streamed}
             for grp in groups:
+                if grp[0][0] in done:
+                    continue
                 name, src, t, out_dim, in_dim, raw = grp[0]
                 key = (src, self._family(t))
                 w, out, dims = [self._w[e[0]].ptr for e in grp], [self._act[e[0]].ptr for e in grp], [e[3] for e in grp]

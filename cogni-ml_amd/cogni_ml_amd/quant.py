@@ -455,6 +455,15 @@ def gemm_stream_dev(w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, ou
                                            ctypes.c_uint32(tokens), stream))
 
 
+def gemm_stream_two_dev(w_a, type_a, ws_a, ws_bytes_a, out_a, in_dim_a, out_dim_a, w_b, type_b, ws_b, ws_bytes_b, out_b, in_dim_b, out_dim_b,
+                        tokens, stream=None):
+    """gemm_stream_dev of two matrices with an input each (o and down of a layer), in one launch where both go in tiles of 32 rows."""
+    U64, U32, SZ = ctypes.c_uint64, ctypes.c_uint32, ctypes.c_size_t
+    _check(hip.lib().cogni_gemm_stream_two_dev(U64(w_a), U32(int(type_a)), U64(ws_a), SZ(ws_bytes_a), U64(out_a), U32(in_dim_a),
+                                               U32(out_dim_a), U64(w_b), U32(int(type_b)), U64(ws_b), SZ(ws_bytes_b), U64(out_b),
+                                               U32(in_dim_b), U32(out_dim_b), U32(tokens), stream))
+
+
 def gemm_stream_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, workspace_bytes, out_ptr, next_type, next_workspace_ptr,
                                 next_workspace_bytes, in_dim, out_dim, tokens, stream=None):
     """gemm_packed_swiglu_pack_dev for short prefills (weights streamed)."""

@@ -1485,6 +1485,18 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
 
 // Short prefills: the weights streamed through workgroups of four wavefronts (kernels/gemm_stream.hpp). The same packed
 // activations, planes and precision as the tile kernels above.
+// Planes of [tokens][out_dim] that fit behind the packed activations. cogni_gemm_workspace_bytes_split sizes a workspace for the tile
+// kernels' split of the shape: what they do not split has no room for planes here either.
+static uint32_t gemm_stream_planes(size_t packed_bytes, size_t workspace_bytes, uint32_t tokens, uint32_t out_dim) {
+  const size_t fit = (workspace_bytes - packed_bytes) / ((size_t)tokens * out_dim * sizeof(float));
+  return fit < 2 ? 1u : (fit < GEMM_STREAM_MAX_SPLITS ? (uint32_t)fit : GEMM_STREAM_MAX_SPLITS);
+}
+static int gemm_stream_sum(uint64_t planes, uint64_t add, uint32_t add_stride, uint64_t out, uint32_t out_dim, uint32_t tokens, uint32_t splits,
+                           void* stream) {
+  uint32_t total = tokens * out_dim;
+  void* sum[] = {&planes, &add, &out, &total, &out_dim, &splits, &add_stride};
+  return launch("gemm_sum_splits_f32", (total + 1023) / 1024, 256, 0, sum, stream);
+}
 static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t add,
                               uint32_t add_stride, const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim,
                               uint32_t tokens, void* stream) {
@@ -1492,13 +1504,7 @@ static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w
   if (packed_bytes > GEMM_STREAM_MAX_PACKED) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": packed activations of 2 GiB or more");
   uint64_t rows = 0;
   for (uint32_t i = 0; i < count; i++) rows += out_dims[i];
-  // planes that fit behind the packed activations (one matrix only). cogni_gemm_workspace_bytes_split sizes a workspace for the tile
-  // kernels' split of the shape: what they do not split has no room for planes here either
-  uint32_t planes_max = 1;
-  if (count == 1) {
-    const size_t fit = (workspace_bytes - packed_bytes) / ((size_t)tokens * out_dims[0] * sizeof(float));
-    planes_max = fit < 2 ? 1u : (fit < GEMM_STREAM_MAX_SPLITS ? (uint32_t)fit : GEMM_STREAM_MAX_SPLITS);
-  }
+  const uint32_t planes_max = count == 1 ? gemm_stream_planes(packed_bytes, workspace_bytes, tokens, out_dims[0]) : 1u;   // (one matrix only)
   const GemmStreamPlan p = gemm_stream_plan(w_type, tokens, in_dim, rows, planes_max);
   GemmManyArgs list{};
   uint32_t end = 0;
@@ -1515,10 +1521,7 @@ static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w
   void* params[] = {&list, &workspace, &kadd, &add_stride, &in_dim, &tokens};
   if (int rc = launch(name, gemm_stream_grid(tokens, p.t, end), 256, 0, params, stream, p.splits)) return rc;
   if (p.splits == 1) return 0;
-  uint64_t planes = workspace + packed_bytes, out = outs[0];
-  uint32_t out_dim = out_dims[0], total = tokens * out_dim, splits = p.splits;
-  void* sum[] = {&planes, &add, &out, &total, &out_dim, &splits, &add_stride};
-  return launch("gemm_sum_splits_f32", (total + 1023) / 1024, 256, 0, sum, stream);
+  return gemm_stream_sum(workspace + packed_bytes, add, add_stride, outs[0], out_dims[0], tokens, p.splits, stream);
 }
 
 int cogni_gemm_stream_takes(uint32_t w_type, uint32_t in_dim, uint32_t rows, uint32_t tokens) {
@@ -1536,6 +1539,46 @@ int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t works
   }
   return gemm_stream_launch(who, w_raw, w_type, workspace, workspace_bytes, residual, residual ? out_dims[0] : 0, outs, out_dims, count, in_dim,
                             tokens, stream);
+}
+
+// Two matrices with an input each: one launch where both go in tiles of 32 rows (with 64 rows a matrix fills the chip by itself).
+// 4096 -> 4096 of Q4_K and 12288 -> 4096 of Q6_K at 48 tokens are 128 and 256 workgroups, each launch half of what the chip holds.
+int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a, size_t bytes_a, uint64_t out_a, uint32_t in_dim_a,
+                              uint32_t out_dim_a, uint64_t w_b, uint32_t type_b, uint64_t workspace_b, size_t bytes_b, uint64_t out_b,
+                              uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_stream_two_dev";
+  if (!w_a || !w_b || !out_a || !out_b) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  if (int rc = gemm_check(who, type_a, in_dim_a, out_dim_a, tokens, workspace_a, bytes_a)) return rc;
+  if (int rc = gemm_check(who, type_b, in_dim_b, out_dim_b, tokens, workspace_b, bytes_b)) return rc;
+  auto first = [](uint32_t t) { return t == COGNI_TYPE_Q4_K || t == COGNI_TYPE_Q5_K; };
+  auto second = [](uint32_t t) { return t == COGNI_TYPE_Q4_K || t == COGNI_TYPE_Q6_K; };
+  if ((!first(type_a) || !second(type_b)) && first(type_b) && second(type_a)) {
+    std::swap(w_a, w_b), std::swap(type_a, type_b), std::swap(workspace_a, workspace_b), std::swap(bytes_a, bytes_b);
+    std::swap(out_a, out_b), std::swap(in_dim_a, in_dim_b), std::swap(out_dim_a, out_dim_b);
+  }
+  const size_t packed_a = cogni_gemm_workspace_bytes(type_a, in_dim_a, tokens), packed_b = cogni_gemm_workspace_bytes(type_b, in_dim_b, tokens);
+  if (first(type_a) && second(type_b) && packed_a <= GEMM_STREAM_MAX_PACKED && packed_b <= GEMM_STREAM_MAX_PACKED) {
+    GemmStreamPlan pa = gemm_stream_plan(type_a, tokens, in_dim_a, out_dim_a, gemm_stream_planes(packed_a, bytes_a, tokens, out_dim_a));
+    GemmStreamPlan pb = gemm_stream_plan(type_b, tokens, in_dim_b, out_dim_b, gemm_stream_planes(packed_b, bytes_b, tokens, out_dim_b));
+    const uint32_t tiles_a = (out_dim_a + 31) / 32, tiles_b = (out_dim_b + 31) / 32;
+    const uint64_t grid = (uint64_t)pa.splits * gemm_stream_grid(tokens, pa.t, tiles_a) + (uint64_t)pb.splits * gemm_stream_grid(tokens, pb.t, tiles_b);
+    if (pa.rt == 1 && pb.rt == 1 && grid < (1u << 24)) {
+      GemmManyArgs list_a{}, list_b{};
+      list_a.w[0] = w_a, list_a.out[0] = pa.splits > 1 ? workspace_a + packed_a : out_a;
+      list_a.out_dim[0] = out_dim_a, list_a.tile_end[0] = tiles_a, list_a.count = 1;
+      list_b.w[0] = w_b, list_b.out[0] = pb.splits > 1 ? workspace_b + packed_b : out_b;
+      list_b.out_dim[0] = out_dim_b, list_b.tile_end[0] = tiles_b, list_b.count = 1;
+      char name[64];
+      std::snprintf(name, sizeof name, "%s_and_%s_gemm_stream_f16_%ux1", type_prefix(type_a), type_prefix(type_b), pa.t);
+      void* params[] = {&list_a, &workspace_a, &in_dim_a, &pa.splits, &list_b, &workspace_b, &in_dim_b, &pb.splits, &tokens};
+      if (int rc = launch(name, (uint32_t)grid, 256, 0, params, stream)) return rc;
+      if (pa.splits > 1)
+        if (int rc = gemm_stream_sum(workspace_a + packed_a, 0, 0, out_a, out_dim_a, tokens, pa.splits, stream)) return rc;
+      return pb.splits > 1 ? gemm_stream_sum(workspace_b + packed_b, 0, 0, out_b, out_dim_b, tokens, pb.splits, stream) : 0;
+    }
+  }
+  if (int rc = gemm_stream_launch(who, &w_a, type_a, workspace_a, bytes_a, 0, 0, &out_a, &out_dim_a, 1, in_dim_a, tokens, stream)) return rc;
+  return gemm_stream_launch(who, &w_b, type_b, workspace_b, bytes_b, 0, 0, &out_b, &out_dim_b, 1, in_dim_b, tokens, stream);
 }
 
 int cogni_gemm_stream_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,

@@ -10,6 +10,8 @@
 //   q4_k_gemm_stream_swiglu_pack_q4k|q6k_f16_<T>x2   (list of the gate matrix (out may be null), w_up, xp, xq, in_dim, m): a gate
 //                                     tile and the up tile of the same 32 rows per wavefront; silu(gate) * up to out and as the packed input
 //                                     of the next GEMM to xq (the absent tokens of a 32-token tile as zeros)
+//   <type_a>_and_<type_b>_gemm_stream_f16_<T>x1 (list_a, xp_a, in_dim_a, splits_a, list_b, xp_b, in_dim_b, splits_b, m): two matrices
+//                                     with an input each (o and down of a layer) in one launch, grid = splits x gemm_stream_grid of both
 //
 // What bounds it: a compute unit returns loads in order, so the activations, L2 hits, wait behind weights that come from
 // memory, and it keeps about 64 KB in flight: some 47 KB/us whatever the mix (Q4_K 30720 rows x 4096, 64 tokens: 250 MB of
@@ -126,32 +128,37 @@ struct StreamQ6K {   // pieces 0..12 from the block's start, the last sixteen by
   }
 };
 
-// T: token tiles of 32; RT: row tiles of 32. PACK (with SWIGLU; 12 or 14): as in gemm_epilogue_swiglu_half.
+// uint4 of LDS: the wavefronts' weights, then the k-slices' sums in their place
+template <class W, int T, int RT>
+constexpr u32 gemm_stream_lds() {
+  constexpr u32 weights = GEMM_STREAM_WAVES * 32 * RT * W::STRIDE, sums = GEMM_STREAM_WAVES * RT * T * 256;
+  return weights > sums ? weights : sums;
+}
+// T: token tiles of 32; RT: row tiles of 32. PACK (with SWIGLU; 12 or 14): as in gemm_epilogue_swiglu_half. bid, split, nsplits: the
+// workgroup's number, its k split and their count, where they are not the launch's.
 template <class W, int T, int RT, bool SWIGLU = false, int PACK = 0>
-__device__ __forceinline__ void gemm_stream_core(const GemmManyArgs& list, const uint4* xp, const float* add, u32 add_stride, u32 in_dim, u32 m,
-                                                 const uint8_t* w_up = nullptr, uint2* xq = nullptr) {
+__device__ __forceinline__ void gemm_stream_core(uint4* lds, const GemmManyArgs& list, const uint4* xp, const float* add, u32 add_stride, u32 in_dim,
+                                                 u32 m, const uint8_t* w_up = nullptr, uint2* xq = nullptr, u32 bid = blockIdx.x,
+                                                 u32 split = blockIdx.y, u32 nsplits = gridDim.y) {
   static_assert(!SWIGLU || RT == 2, "a gate tile and the up tile of the same rows");
   constexpr int NM = SWIGLU ? 2 : 1;                             // matrices the workgroup's row tiles come from
   constexpr u32 PIECES = 32 * RT / NM * W::PPR;                  // 16-byte pieces of a matrix's rows per super-block
   constexpr int NL = (int)((PIECES + 63) / 64);                  // loads of them per lane
   constexpr u32 ROWS = SWIGLU ? 32 : 32 * RT;                    // rows of a matrix a workgroup covers
   constexpr u32 WAVE_U4 = 32 * RT * W::STRIDE;                   // a wavefront's weights in LDS
-  constexpr u32 PART_U4 = GEMM_STREAM_WAVES * RT * T * 256;      // the k-slices' sums, behind the loop
-  constexpr u32 LDS_U4 = GEMM_STREAM_WAVES * WAVE_U4 > PART_U4 ? GEMM_STREAM_WAVES * WAVE_U4 : PART_U4;
-  __shared__ uint4 lds[LDS_U4];
   const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const u32 j = lane & 31, kg = lane >> 5;
   u32 mt, nt;
-  gemm_terms_tile(blockIdx.x, (m + 32 * T - 1) / (32 * T), &mt, &nt);
+  gemm_terms_tile(bid, (m + 32 * T - 1) / (32 * T), &mt, &nt);
   if (nt >= list.tile_end[list.count - 1]) return;   // (the grid is rounded up to whole rows of tiles per XCD)
   u32 mi = 0, first = 0;
   while (mi + 1 < list.count && nt >= list.tile_end[mi]) first = list.tile_end[mi++];
   nt -= first;
   const uint8_t* const w = list.w[mi];
   const u32 out_dim = list.out_dim[mi];
-  float* const out = list.out[mi] + (size_t)blockIdx.y * m * out_dim;   // k split: one plane per blockIdx.y
+  float* const out = list.out[mi] + (size_t)split * m * out_dim;   // one plane per k split
   const u32 nkb_all = in_dim >> 8;
-  const u32 kb0 = blockIdx.y * nkb_all / gridDim.y, kb1 = (blockIdx.y + 1) * nkb_all / gridDim.y;
+  const u32 kb0 = split * nkb_all / nsplits, kb1 = (split + 1) * nkb_all / nsplits;
   const u32 n0 = nt * ROWS;
   const size_t row_bytes = (size_t)nkb_all * W::BS;
   u32 magic_lo = 0x64006400u, magic_hi = 0x54005400u;   // in registers: (q & mask) | magic is one instruction
@@ -358,7 +365,8 @@ __device__ __forceinline__ void gemm_stream_core(const GemmManyArgs& list, const
 #define GEMM_STREAM_ENTRY(PREFIX, W, T, RT, OCC)                                                                                     \
   extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void PREFIX##_gemm_stream_f16_##T##x##RT( \
       const GemmManyArgs list, const uint4* xp, const float* add, u32 add_stride, u32 in_dim, u32 m) {                                \
-    gemm_stream_core<W, T, RT>(list, xp, add, add_stride, in_dim, m);                                                                 \
+    __shared__ uint4 lds[gemm_stream_lds<W, T, RT>()];                                                                                \
+    gemm_stream_core<W, T, RT>(lds, list, xp, add, add_stride, in_dim, m);                                                            \
   }
 #define GEMM_STREAM_TYPE(PREFIX, W)    \
   GEMM_STREAM_ENTRY(PREFIX, W, 1, 1, 3) \
@@ -372,9 +380,37 @@ GEMM_STREAM_ENTRY(q5_k, StreamQ5K, 2, 2, 2)
 #define GEMM_STREAM_SWIGLU_ENTRY(T, OCC, NEXT, PACK)                                                                                  \
   extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void q4_k_gemm_stream_swiglu_pack_##NEXT##_f16_##T##x2( \
       const GemmManyArgs list, const uint8_t* w_up, const uint4* xp, uint2* xq, u32 in_dim, u32 m) {                                  \
-    gemm_stream_core<StreamQ4K, T, 2, true, PACK>(list, xp, nullptr, 0, in_dim, m, w_up, xq);                                         \
+    __shared__ uint4 lds[gemm_stream_lds<StreamQ4K, T, 2>()];                                                                         \
+    gemm_stream_core<StreamQ4K, T, 2, true, PACK>(lds, list, xp, nullptr, 0, in_dim, m, w_up, xq);                                    \
   }
 GEMM_STREAM_SWIGLU_ENTRY(1, 2, q4k, 12)
 GEMM_STREAM_SWIGLU_ENTRY(2, 2, q4k, 12)
 GEMM_STREAM_SWIGLU_ENTRY(1, 2, q6k, 14)
 GEMM_STREAM_SWIGLU_ENTRY(2, 2, q6k, 14)
+
+// Two matrices with an input each. b's workgroups come first: it is the one with the longer rows in a layer (down beside o), so its
+// chains start at once and a's, which are shorter, fill the units in between.
+// (Q4_K 4096 -> 4096 and Q6_K 12288 -> 4096 at 48 tokens are 128 and 256 workgroups of a chip that holds 512: 12 and 27 us behind a
+// profiler one after the other; the projections of a layer in 63.5 us, 70.1 with two launches.)
+#define GEMM_STREAM_TWO_ENTRY(PREFIX_A, WA, PREFIX_B, WB, T, OCC)                                                                      \
+  extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void PREFIX_A##_and_##PREFIX_B##_gemm_stream_f16_##T##x1( \
+      const GemmManyArgs list_a, const uint4* xp_a, u32 in_dim_a, u32 splits_a, const GemmManyArgs list_b, const uint4* xp_b, u32 in_dim_b, \
+      u32 splits_b, u32 m) {                                                                                                          \
+    constexpr u32 LDS_A = gemm_stream_lds<WA, T, 1>(), LDS_B = gemm_stream_lds<WB, T, 1>();                                           \
+    __shared__ uint4 lds[LDS_A > LDS_B ? LDS_A : LDS_B];                                                                              \
+    const u32 wgs_a = gemm_stream_grid(m, T, list_a.tile_end[0]), wgs_b = gemm_stream_grid(m, T, list_b.tile_end[0]);                 \
+    const u32 first_a = wgs_b * splits_b;                                                                                             \
+    if (blockIdx.x < first_a) {                                                                                                       \
+      gemm_stream_core<WB, T, 1>(lds, list_b, xp_b, nullptr, 0, in_dim_b, m, nullptr, nullptr, blockIdx.x % wgs_b, blockIdx.x / wgs_b, splits_b); \
+    } else {                                                                                                                          \
+      const u32 id = blockIdx.x - first_a;                                                                                            \
+      gemm_stream_core<WA, T, 1>(lds, list_a, xp_a, nullptr, 0, in_dim_a, m, nullptr, nullptr, id % wgs_a, id / wgs_a, splits_a);     \
+    }                                                                                                                                 \
+  }
+#define GEMM_STREAM_TWO(PREFIX_A, WA, PREFIX_B, WB)    \
+  GEMM_STREAM_TWO_ENTRY(PREFIX_A, WA, PREFIX_B, WB, 1, 3) \
+  GEMM_STREAM_TWO_ENTRY(PREFIX_A, WA, PREFIX_B, WB, 2, 2)
+GEMM_STREAM_TWO(q4_k, StreamQ4K, q6_k, StreamQ6K)
+GEMM_STREAM_TWO(q4_k, StreamQ4K, q4_k, StreamQ4K)
+GEMM_STREAM_TWO(q5_k, StreamQ5K, q6_k, StreamQ6K)
+GEMM_STREAM_TWO(q5_k, StreamQ5K, q4_k, StreamQ4K)

@@ -406,7 +406,7 @@ static inline GemmStreamPlan gemm_stream_plan(unsigned type, unsigned tokens, un
     }
   return best;
 }
-static inline unsigned gemm_stream_grid(unsigned tokens, unsigned t, unsigned ntiles) {
+static inline GEMV_HD unsigned gemm_stream_grid(unsigned tokens, unsigned t, unsigned ntiles) {
   const unsigned mt = (tokens + 32u * t - 1u) / (32u * t);
   return mt * ((ntiles + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT) * GEMM_XCD_COUNT;
 }

@@ -499,10 +499,15 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
  * it may be the output) goes with one matrix. The k range is split as far as planes fit behind the packed activations
  * (cogni_gemm_workspace_bytes_split). cogni_gemm_stream_swiglu_pack_dev: as cogni_gemm_packed_swiglu_pack_dev (Q4_K; `out` may be
  * null); of the absent tokens of the packed block only those of the last tile of 32 are written (zeros). Any token count is taken
- * as long as the packed activations are below 2 GiB. */
+ * as long as the packed activations are below 2 GiB. cogni_gemm_stream_two_dev: two matrices with an input each (o and down of a layer),
+ * the values of cogni_gemm_stream_dev for the one and the other; a Q4_K or Q5_K matrix beside a Q4_K or Q6_K one that both go in tiles of
+ * 32 rows are one launch of "<type_a>_and_<type_b>_gemm_stream_f16_<T>x1". Neither workspace may overlap the other. */
 int cogni_gemm_stream_takes(uint32_t w_type, uint32_t in_dim, uint32_t rows, uint32_t tokens);
 int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t residual,
                           const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
+int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a, size_t bytes_a, uint64_t out_a, uint32_t in_dim_a,
+                              uint32_t out_dim_a, uint64_t w_b, uint32_t type_b, uint64_t workspace_b, size_t bytes_b, uint64_t out_b,
+                              uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens, void* stream);
 int cogni_gemm_stream_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                       uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
                                       uint32_t out_dim, uint32_t tokens, void* stream);

@@ -149,3 +149,32 @@ def test_gate_up_swiglu_pack(gpu, in_dim, out_dim, tokens, next_type):
     finally:
         for a in (g, u, xd, ws, nx, nx2, ref, out):
             a.close()
+
+
+# both orders, both token tiles, with and without k splits, uneven rows; a pair that takes 64 rows and a pair without the kernel go one by one
+@pytest.mark.parametrize("tokens", [18, 48, 70])
+@pytest.mark.parametrize("a,b", [((Q4_K, 4096, 4096), (Q6_K, 12288, 4096)), ((Q6_K, 3072, 1030), (Q5_K, 1024, 130)), ((Q4_K, 256, 1), (Q4_K, 2816, 33)),
+                                 ((Q5_K, 512, 4096), (Q4_K, 1280, 515)), ((Q4_K, 1024, 12288), (Q6_K, 256, 70)), ((Q6_K, 512, 40), (Q6_K, 256, 33))])
+def test_two_matrices_with_an_input_each(gpu, a, b, tokens):
+    """The launch of two matrices: each output as cogni_gemm_stream_dev gives it, bit for bit."""
+    rng = np.random.default_rng(a[1] + b[1] + tokens)
+    mats = []
+    for t, in_dim, out_dim in (a, b):
+        x, nb = DevArray(synth.make_activations(rng, tokens, in_dim)), quant.gemm_workspace_bytes(t, in_dim, tokens, out_dim)
+        ws, w = DevArray(nbytes=nb), DevArray(synth.make_weights(rng, t, out_dim, in_dim))
+        one, two = (DevArray(np.full(tokens * out_dim + 64, np.float32(v))) for v in (5.0, 6.0))
+        quant.gemm_pack_dev(x.ptr, t, in_dim, tokens, ws.ptr, nb)
+        quant.gemm_stream_dev([w.ptr], t, ws.ptr, nb, [one.ptr], [out_dim], in_dim, tokens)
+        mats.append((w, t, ws, nb, two, in_dim, out_dim, one, x))
+    print("case", a, b, tokens, flush=True)
+    args = [v for w, t, ws, nb, two, in_dim, out_dim, one, x in mats for v in (w.ptr, t, ws.ptr, nb, two.ptr, in_dim, out_dim)]
+    quant.gemm_stream_two_dev(*args, tokens)
+    for w, t, ws, nb, two, in_dim, out_dim, one, x in mats:
+        got = two.read(np.float32, tokens * out_dim + 64)
+        assert np.array_equal(got[:tokens * out_dim], one.read(np.float32, tokens * out_dim)), (t, in_dim, out_dim)
+        assert (got[tokens * out_dim:] == 6.0).all()
+    with pytest.raises(quant.QuantError, match="null device pointer"):
+        quant.gemm_stream_two_dev(*args[:4], 0, *args[5:], tokens)
+    for m in mats:
+        for i in (0, 2, 4, 7, 8):
+            m[i].close()
