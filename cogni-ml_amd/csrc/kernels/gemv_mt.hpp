@@ -367,6 +367,7 @@ struct MtK45 {
   static constexpr int NTOK = X16 ? 16 : 8;   // tokens a launch covers
   static constexpr int BB = Q5 ? 176 : 144, P = BB / 16, NCOPY = 3, LAST = 16 * P - 128, NAUX = 1, NSLOT = 6, TMAX = 3;
   static constexpr int QOFF = Q5 ? 48 : 16;   // where qs starts in the block
+  static constexpr bool SHIFTED = false;      // (blocks start on 16 bytes)
   static constexpr u32 UNIT_BYTES = 16 * P * 16, AUX_SB_BYTES = 64 * 16;
   // byte offset, inside the row's block, of the piece that goes to place `piece` of the row in LDS
   static __device__ __forceinline__ u32 piece_offset(u32 piece) { return piece * 16; }
@@ -486,6 +487,7 @@ struct MtQ80T {
   static constexpr unsigned TYPE = 8;
   static constexpr int NTOK = X16 ? 16 : 8;
   static constexpr int BB = 272, P = 17, NCOPY = 5, LAST = 16, NAUX = 1, NSLOT = 4, TMAX = 2;
+  static constexpr bool SHIFTED = false;
   static constexpr u32 UNIT_BYTES = 16 * P * 16, AUX_SB_BYTES = 64 * 16;
   static __device__ __forceinline__ u32 piece_offset(u32 piece) { return piece * 16; }
   static __device__ __forceinline__ u32 aux_offset(u32 lane) { return lane * 16; }
@@ -548,19 +550,22 @@ typedef MtQ80T<true> MtQ80x16;
 
 // Q6_K (210 B: ql[128], qh[64], scales:i8[16], d). Element 128 n + 32 k + l (half n, quarter k, l < 32) has its low four bits
 // in nibble k / 2 of ql[64 n + 32 (k % 2) + l] and its high two in bits 2 k, 2 k + 1 of qh[32 n + l]; sub-block
-// s = 8 n + 2 k + l / 16. A row's block starts at a multiple of 2 bytes only; it is copied from exactly its start (the
-// memory pipeline takes unaligned 16-byte loads), so inside LDS every field sits at its natural alignment. A row in LDS
-// is 15 pieces (240 bytes: rows 60 dwords apart hit 16 different bank groups): pieces 0..12 are bytes 0..207 of the block,
-// piece 13 is bytes 194..209 (shifted back so that nothing past the end of the matrix is read: d sits at byte 222 of
-// the row) and piece 14 repeats piece 13.
+// s = 8 n + 2 k + l / 16. A row's block starts at a multiple of 2 bytes only. It is copied as the 14 aligned pieces of 16 bytes that
+// hold it (210 bytes from an even start are never in more), and the lanes read its fields at the block's shift, 0 to 14 bytes: a
+// copy from inside a dword takes the memory pipeline about twice as long, and a read of LDS from there costs more than that, so
+// the fields of a block that starts inside a dword (every other one) are put together from two dwords. Head of 151936 x 4096 at six
+// tokens with its norm and reduce, us: copied from the start as it lies 120.4, like this 112.5, without the shift of odd blocks (wrong) 104.
+// Every piece holds a byte of the block, so what is read beside it lies in the same 16 aligned bytes as one of the matrix's, never in
+// another page. A row in LDS is 15 pieces (240 bytes: rows 60 dwords apart hit 16 different bank groups), piece 14 a copy of piece 13.
 // (X16: sixteen single-term tokens, as MtK45's)
 template <bool X16 = false>
 struct MtQ6KT {
   static constexpr int NTOK = X16 ? 16 : 8;
   static constexpr unsigned TYPE = 14;
-  static constexpr int BB = 210, P = 15, NCOPY = 4, LAST = 48, NAUX = 1, NSLOT = 4, TMAX = 2;
+  static constexpr int BB = 210, P = 15, NCOPY = 4, LAST = 16 * P - 192, NAUX = 1, NSLOT = 4, TMAX = 2;
+  static constexpr bool SHIFTED = true;
   static constexpr u32 UNIT_BYTES = 16 * P * 16, AUX_SB_BYTES = 64 * 16;
-  static __device__ __forceinline__ u32 piece_offset(u32 piece) { return piece < 13 ? piece * 16 : 194u; }
+  static __device__ __forceinline__ u32 piece_offset(u32 piece) { return min(piece, 13u) * 16; }
   static __device__ __forceinline__ u32 aux_offset(u32 lane) { return lane * 16; }   // 16 bytes of its own per lane
 
   // the scales of the lane's two tokens and, as the matrix-core operand of lane (kg, row), the sums of sub-blocks
@@ -575,20 +580,36 @@ struct MtQ6KT {
   }
   // [2 n + hh]: ql dword of quarters 0/2, of quarters 1/3, qh dword; sck: the scale bytes of sub-blocks 4 kg .. 4 kg + 3
   struct Raw { u32 a[4], b[4], h[4]; uint4 sc; u32 d, sck; };
-  static __device__ __forceinline__ Raw read(const char* row, u32 kg) {
+  // SH: the block may start inside a dword (of LDS), sh = by how many bytes
+  template <bool SH>
+  static __device__ __forceinline__ Raw fields(const char* row, u32 kg, u32 sh) {
     Raw w;
+    // four bytes of the block, from the two dwords they are in
+    auto at = [&](u32 b) {
+      const u32* d = reinterpret_cast<const u32*>(row + b);
+      return SH ? __builtin_amdgcn_alignbyte(d[1], d[0], sh) : d[0];
+    };
 #pragma unroll
     for (int n = 0; n < 2; n++)
 #pragma unroll
       for (int hh = 0; hh < 2; hh++) {
-        w.a[2 * n + hh] = *reinterpret_cast<const u32*>(row + 64 * n + 16 * hh + 4 * kg);
-        w.b[2 * n + hh] = *reinterpret_cast<const u32*>(row + 64 * n + 32 + 16 * hh + 4 * kg);
-        w.h[2 * n + hh] = *reinterpret_cast<const u32*>(row + 128 + 32 * n + 16 * hh + 4 * kg);
+        w.a[2 * n + hh] = at(64 * n + 16 * hh + 4 * kg);
+        w.b[2 * n + hh] = at(64 * n + 32 + 16 * hh + 4 * kg);
+        w.h[2 * n + hh] = at(128 + 32 * n + 16 * hh + 4 * kg);
       }
-    w.sc = *reinterpret_cast<const uint4*>(row + 192);
-    w.sck = *reinterpret_cast<const u32*>(row + 192 + 4 * kg);
-    w.d = *reinterpret_cast<const unsigned short*>(row + 222);
+    const u32* const sc = reinterpret_cast<const u32*>(row + 192);
+    const u32 s0 = sc[0], s1 = sc[1], s2 = sc[2], s3 = sc[3], s4 = sc[4];   // (d is behind the scales)
+    w.sc = SH ? make_uint4(__builtin_amdgcn_alignbyte(s1, s0, sh), __builtin_amdgcn_alignbyte(s2, s1, sh), __builtin_amdgcn_alignbyte(s3, s2, sh),
+                           __builtin_amdgcn_alignbyte(s4, s3, sh))
+              : make_uint4(s0, s1, s2, s3);
+    w.sck = at(192 + 4 * kg);
+    w.d = SH ? s4 >> (8 * sh) : s4;
     return w;
+  }
+  static __device__ __forceinline__ Raw read(const char* start, u32 kg) {
+    const u32 sh = (u32)(uintptr_t)start & 3u;
+    if (__builtin_amdgcn_ballot_w64(sh != 0) == 0) return fields<false>(start, kg, 0);
+    return fields<true>(start - sh, kg, sh);
   }
   static __device__ __forceinline__ float sbyte_f(u32 v, int k) { return (float)(int)(signed char)((v >> (8 * k)) & 0xFFu); }
   static __device__ __forceinline__ void unit(const Raw& w, const mt_u32x4 (&b)[8], const Aux& ax, float (&acc)[4]) {
@@ -697,6 +718,9 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
   char* lds = reinterpret_cast<char*>(mt_lds4);
   const int tid = threadIdx.x, lane = tid & 63;
   const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // The k-slice of this wavefront. SHIFTED: odd super-blocks take more instructions, so the wavefronts w and w + 4 of a SIMD get one kind
+  // each.
+  const u32 slice = F::SHIFTED ? wave ^ (wave >> 2) : wave;
   const u32 nsb = in_dim >> 8, nsbp = gemv_mt_padded_sb(in_dim);   // super-blocks of a row, and of the image
   const u32 total_rows = a.total();
   const u32 ntiles = (total_rows + 15) >> 4;
@@ -738,7 +762,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
   const uint8_t* aux = image + (size_t)nsbp * 8192;
   // (uniform bases and two lane offsets: no address registers per load)
   const u32 lane16 = lane * 16u, rg_off = F::aux_offset(lane);
-  auto slice_sb = [&](int i) -> u32 { return GEMV_MT_CONTIGUOUS_SLICES ? wave * (u32)SBW + (u32)i : wave + 8u * (u32)i; };
+  auto slice_sb = [&](int i) -> u32 { return GEMV_MT_CONTIGUOUS_SLICES ? slice * (u32)SBW + (u32)i : slice + 8u * (u32)i; };
   auto issue_set = [&](int i, int set) {
     const u32 sb = slice_sb(i);
     u64 ob = mt_sbase(image + (size_t)sb * 8192), ob2 = mt_sbase(image + (size_t)sb * 8192 + 4096);
@@ -771,6 +795,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
   // ---- the copies of a row group's units. Copy m of a unit: piece p = 64 m + lane (< 16 P), row p / P of the tile.
   const size_t row_bytes = (size_t)nsb * F::BB;
   const uint8_t* cptr[T][NC];   // where this lane's piece of copy m of tile t starts, without the super-block offset
+  [[maybe_unused]] u32 copied15[T], read15[T];   // SHIFTED: address of row ar of tile t, modulo 16: of the group copied, of the one read
   auto set_rows = [&](u32 g, int mat = 0) {   // (mat: with SWIGLU and streamed operands, gate (0) and up (1) take turns)
 #pragma unroll
     for (int t = 0; t < T; t++) {
@@ -786,24 +811,41 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
         const u32 pr = min(p / (u32)F::P, 15u), piece = p - (u32)F::P * (p / (u32)F::P);
         cptr[t][m] = wm + (size_t)min(tile_row - first + pr, count - 1) * row_bytes + F::piece_offset(piece);
       }
+      if constexpr (F::SHIFTED) copied15[t] = (u32)(uintptr_t)wm + min(tile_row - first + ar, count - 1) * (u32)row_bytes;
     }
+  };
+  auto aligned = [](const uint8_t* p) {
+    if constexpr (F::SHIFTED) return reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(p) & ~(uintptr_t)15);
+    else return p;
   };
   auto issue_unit = [&](int i, int t, int slot) {
     // (a super-block past the row's end: the row's last block stands in; its operands in the image are zeros)
     const u32 off = min(slice_sb(i), nsb - 1u) * F::BB, dst = slots_lds + (u32)slot * F::UNIT_BYTES;
 #pragma unroll
-    for (int m = 0; m + 1 < NC; m++) mt_copy16(dst + 1024u * m, cptr[t][m] + off);
-    if (lane < F::LAST) mt_copy16(dst + 1024u * (NC - 1), cptr[t][NC - 1] + off);
+    for (int m = 0; m + 1 < NC; m++) mt_copy16(dst + 1024u * m, aligned(cptr[t][m] + off));
+    if (lane < F::LAST) mt_copy16(dst + 1024u * (NC - 1), aligned(cptr[t][NC - 1] + off));
+  };
+  // where row ar of super-block i, tile t starts in its slot
+  auto row_at = [&](int i, int t, int slot) -> const char* {
+    const char* row = slots + slot * F::UNIT_BYTES + ar * (F::P * 16);
+    if constexpr (F::SHIFTED) row += (read15[t] + min(slice_sb(i), nsb - 1u) * F::BB) & 15u;
+    return row;
+  };
+  auto start_reading = [&]() {   // the group copied last is the one that is read now
+    if constexpr (F::SHIFTED) {
+#pragma unroll
+      for (int t = 0; t < T; t++) read15[t] = copied15[t];
+    }
   };
 
   // k-slices through LDS in wavefront order: partial[wave][tile][token][row]; hi + lo of a token first
   auto store_part = [&](int t, const float (&acc)[4]) {
     if constexpr (NTOK == 16) {
 #pragma unroll
-      for (int k = 0; k < 4; k++) part[((wave * GEMV_MT_TMAX + t) * 16 + 4 * rg + k) * 16 + ar] = acc[k];
+      for (int k = 0; k < 4; k++) part[((slice * GEMV_MT_TMAX + t) * 16 + 4 * rg + k) * 16 + ar] = acc[k];
     } else {
-      part[((wave * GEMV_MT_TMAX + t) * 8 + 2 * rg) * 16 + ar] = acc[0] + acc[1];
-      part[((wave * GEMV_MT_TMAX + t) * 8 + 2 * rg + 1) * 16 + ar] = acc[2] + acc[3];
+      part[((slice * GEMV_MT_TMAX + t) * 8 + 2 * rg) * 16 + ar] = acc[0] + acc[1];
+      part[((slice * GEMV_MT_TMAX + t) * 8 + 2 * rg + 1) * 16 + ar] = acc[2] + acc[3];
     }
   };
   auto finish = [&]() {
@@ -908,6 +950,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
       float acc[T][4];
 #pragma unroll
       for (int t = 0; t < T; t++) acc[t][0] = acc[t][1] = acc[t][2] = acc[t][3] = 0.f;
+      start_reading();
       if constexpr (walk) set_rows(grp + gridDim.x);
       auto unit = [&](auto utag) {
         constexpr int u = decltype(utag)::value, i = u / T, t = u % T;
@@ -915,7 +958,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
         // the unit has landed when at most the copies behind it are outstanding: all NU - 1 other units while slots are
         // being refilled, else the ones after it in this group (other loads or stores in between only make the wait longer)
         mt_wait<walk ? NC * (NU - 1) : NC * (NU - 1 - u)>();
-        const typename F::Raw w = F::read(slots + u * F::UNIT_BYTES + ar * (F::P * 16), kg);
+        const typename F::Raw w = F::read(row_at(i, t, u), kg);
         if constexpr (walk) {
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot has been read
           issue_unit(i, t, u);
@@ -949,6 +992,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
 #pragma unroll 1
      for (int mat = 0; mat < (SWIGLU ? 2 : 1); mat++) {
       set_rows(grp, mat);
+      start_reading();
 #pragma unroll
       for (int u = 0; u < NSLOT; u++) {
         if (u < NS) issue_set(u, u);
@@ -961,7 +1005,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
         mt_wait<mt_stream_wait(S, NSLOT, NS, NA, NC, i)>();
         pin_set(i % NS);
         const typename F::Aux ax = F::aux(auxr[i % NS]);
-        const typename F::Raw w = F::read(slots + (i % NSLOT) * F::UNIT_BYTES + ar * (F::P * 16), kg);
+        const typename F::Raw w = F::read(row_at(i, 0, i % NSLOT), kg);
         F::unit(w, breg[i % NS], ax, acc);
         asm volatile("" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
         __builtin_amdgcn_sched_barrier(0);

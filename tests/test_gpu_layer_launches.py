@@ -127,3 +127,25 @@ def test_rounds_of_a_stack():
     assert [[[e[0] for e in g] for g in r] for r in rounds] == [[["q", "k", "v", "gate", "up"]], [["o"], ["down"]]]
     for odd in ([("a", "b", Q4_K, 256, 256, None), ("b", "x", Q4_K, 256, 256, None)], [("a", "x", Q4_K, 256, 256, None), ("a", "x", Q4_K, 256, 256, None)]):
         assert QwenProjectionStackRunner._rounds_of(odd) == [[[e]] for e in odd]
+
+
+@pytest.mark.parametrize("in_dim", [256, 768, 2048, 3328, 4096, 12288])
+@pytest.mark.parametrize("first", [0, 2, 4, 10, 14])
+def test_q6_k_blocks_at_every_shift(gpu, oracle, first, in_dim):
+    """The one-pass kernels copy a Q6_K block as the aligned 16-byte pieces that hold it: rows of odd and even numbers of blocks (blocks
+    inside and at the start of a dword), and a matrix that starts `first` bytes behind 16 aligned ones."""
+    out_dim, tokens = 37, 5
+    rng = np.random.default_rng(in_dim + first)
+    raw, x = synth.make_weights(rng, Q6_K, out_dim, in_dim), synth.make_activations(rng, tokens, in_dim)
+    w = DevArray(np.concatenate([np.full(first, 0x5A, np.uint8), np.frombuffer(raw, np.uint8), np.full(16, 0xA5, np.uint8)]))
+    xd, image = DevArray(x), DevArray(nbytes=quant.gemv_image_bytes(Q6_K, in_dim, 8))
+    od = DevArray(np.full(tokens * out_dim, np.nan, dtype=np.float32))
+    quant.gemv_pack_dev(xd.ptr, Q6_K, in_dim, tokens, image.ptr)
+    quant.gemv_packed_dev([w.ptr + first], Q6_K, image.ptr, [od.ptr], [out_dim], in_dim, tokens)
+    got = od.read(np.float32, tokens * out_dim)
+    want = oracle.matmul_add(x, tokens, in_dim, raw, Q6_K, out_dim, np.zeros(out_dim, dtype=np.float32))
+    # the bound of smoke(): 22-bit activations and fp32 sums against 64 bits
+    tol = 1e-4 * np.linalg.norm(x.reshape(tokens, -1), axis=1).max() * np.abs(oracle.dequantize(raw, Q6_K, out_dim * in_dim)).max()
+    assert np.abs(got - want).max() <= tol and np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    for d in (w, xd, image, od):
+        d.close()
