@@ -132,6 +132,14 @@ class QwenProjectionStackRunner:
         if len(jobs) % 2:
             one(*jobs[-1])
 
+    @staticmethod
+    def _pairs(entries, two):
+        """Entries that are launched alone go two to a launch; the names that have been."""
+        n = len(entries) // 2 * 2
+        for i in range(0, n, 2):
+            two(entries[i], entries[i + 1])
+        return {e[0] for e in entries[:n]}
+
     def _launch(self, tok0, count):
         stream = hip.current_stream_handle()
 
@@ -157,7 +165,15 @@ class QwenProjectionStackRunner:
                     singles.append((self._w[name].ptr, t, act(src, in_dim), act(name, out_dim), in_dim, out_dim))
             self._pack_each(list(jobs.values()), lambda x, t, k, image: quant.gemv_pack_dev(x, t, k, count, image, stream),
                             lambda *ab: quant.gemv_pack_two_dev(*ab, count, stream))
+            def one_image(e):
+                name, src, t, out_dim, in_dim, raw = e
+                return self._w[name].ptr, t, self._images[(src, int(t))].ptr, act(name, out_dim), in_dim, out_dim
+
+            done = self._pairs([g[0] for g in imaged if len(g) == 1],
+                               lambda a, b: quant.gemv_packed_two_dev(*one_image(a), *one_image(b), count, stream))
             for grp in imaged:
+                if grp[0][0] in done:
+                    continue
                 name, src, t, out_dim, in_dim, raw = grp[0]
                 quant.gemv_packed_dev([self._w[e[0]].ptr for e in grp], t, self._images[(src, int(t))].ptr, [act(e[0], e[3]) for e in grp],
                                       [e[3] for e in grp], in_dim, count, 0, stream)
@@ -199,17 +215,22 @@ class QwenProjectionStackRunner:
                             lambda *ab: quant.gemv_pack16_two_dev(*ab, count, stream))
             self._pack_each(list(jobs.values()), lambda x, t, k, ws, nbytes: quant.gemm_pack_dev(x, t, k, count, ws, nbytes, stream),
                             lambda *ab: quant.gemm_pack_two_dev(*ab, count, stream))
-            # single matrices of short prefills: two to a launch (o and down)
-            streamed = [g[0] for g in groups if len(g) == 1 and (g[0][1], self._family(g[0][2])) not in jobs16 and
-                        quant.gemm_stream_takes(g[0][2], g[0][4], g[0][3], count)]
-            streamed = streamed[:len(streamed) // 2 * 2]
-            for i in range(0, len(streamed), 2):
-                args = []
-                for name, src, t, out_dim, in_dim, raw in streamed[i:i + 2]:
-                    ws, nbytes = self._prefill_ws[(src, self._family(t))]
-                    args += [self._w[name].ptr, t, ws.ptr, nbytes, self._act[name].ptr, in_dim, out_dim]
-                quant.gemm_stream_two_dev(*args, count, stream)
-            done = {e[0] for e in streamed}
+            # single matrices of up to sixteen tokens, or of short prefills: two to a launch (o and down)
+            def one_image(e):
+                name, src, t, out_dim, in_dim, raw = e
+                return self._w[name].ptr, t, self._images16[(src, self._family(t))].ptr, self._act[name].ptr, in_dim, out_dim
+
+            def one_packed(e):
+                name, src, t, out_dim, in_dim, raw = e
+                ws, nbytes = self._prefill_ws[(src, self._family(t))]
+                return self._w[name].ptr, t, ws.ptr, nbytes, self._act[name].ptr, in_dim, out_dim
+
+            alone = [g[0] for g in groups if len(g) == 1]
+            done = self._pairs([e for e in alone if (e[1], self._family(e[2])) in jobs16],
+                               lambda a, b: quant.gemv_packed16_two_dev(*one_image(a), *one_image(b), count, stream))
+            done |= self._pairs([e for e in alone if (e[1], self._family(e[2])) not in jobs16 and
+                                 quant.gemm_stream_takes(e[2], e[4], e[3], count)],
+                                lambda a, b: quant.gemm_stream_two_dev(*one_packed(a), *one_packed(b), count, stream))
             for grp in groups:
                 if grp[0][0] in done:
                     continue

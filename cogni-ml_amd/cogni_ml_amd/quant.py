@@ -386,6 +386,25 @@ def gemv_two_dev(w_a, type_a, x_a, out_a, in_dim_a, out_dim_a, w_b, type_b, x_b,
                                         U32(int(type_b)), U64(x_b), U64(out_b), U32(in_dim_b), U32(out_dim_b), U32(tokens), stream))
 
 
+def _packed_two(name, w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b, in_dim_b, out_dim_b, tokens, stream):
+    U64, U32 = ctypes.c_uint64, ctypes.c_uint32
+    _check(getattr(hip.lib(), name)(U64(w_a), U32(int(type_a)), U64(image_a), U64(out_a), U32(in_dim_a), U32(out_dim_a), U64(w_b),
+                                    U32(int(type_b)), U64(image_b), U64(out_b), U32(in_dim_b), U32(out_dim_b), U32(tokens), stream))
+
+
+def gemv_packed_two_dev(w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b, in_dim_b, out_dim_b, tokens, stream=None):
+    """gemv_packed_dev of two matrices with an image each (o and down of a layer), in one launch where there is a kernel for the pair."""
+    _packed_two("cogni_gemv_packed_two_dev", w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b, in_dim_b,
+                out_dim_b, tokens, stream)
+
+
+def gemv_packed16_two_dev(w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b, in_dim_b, out_dim_b, tokens,
+                          stream=None):
+    """gemv_packed16_dev of two matrices with an image each."""
+    _packed_two("cogni_gemv_packed16_two_dev", w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b, in_dim_b,
+                out_dim_b, tokens, stream)
+
+
 def _pack_two(name, x_a, type_a, in_dim_a, image_a, x_b, type_b, in_dim_b, image_b, tokens, stream):
     U64, U32 = ctypes.c_uint64, ctypes.c_uint32
     _check(getattr(hip.lib(), name)(U64(x_a), U32(int(type_a)), U32(in_dim_a), U64(image_a), U64(x_b), U32(int(type_b)), U32(in_dim_b),

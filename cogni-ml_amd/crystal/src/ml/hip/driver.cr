@@ -133,6 +133,12 @@ lib LibCogniHIP
   fun cogni_gemv_two_dev(w_a : UInt64, type_a : UInt32, x_a : UInt64, out_a : UInt64, in_dim_a : UInt32, out_dim_a : UInt32,
                          w_b : UInt64, type_b : UInt32, x_b : UInt64, out_b : UInt64, in_dim_b : UInt32, out_dim_b : UInt32,
                          tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemv_packed_two_dev(w_a : UInt64, type_a : UInt32, image_a : UInt64, out_a : UInt64, in_dim_a : UInt32, out_dim_a : UInt32,
+                                w_b : UInt64, type_b : UInt32, image_b : UInt64, out_b : UInt64, in_dim_b : UInt32, out_dim_b : UInt32,
+                                tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemv_packed16_two_dev(w_a : UInt64, type_a : UInt32, image_a : UInt64, out_a : UInt64, in_dim_a : UInt32, out_dim_a : UInt32,
+                                  w_b : UInt64, type_b : UInt32, image_b : UInt64, out_b : UInt64, in_dim_b : UInt32, out_dim_b : UInt32,
+                                  tokens : UInt32, stream : Void*) : Int32
   fun cogni_gemv_pack_two_dev(x_a : UInt64, type_a : UInt32, in_dim_a : UInt32, image_a : UInt64, x_b : UInt64, type_b : UInt32,
                               in_dim_b : UInt32, image_b : UInt64, tokens : UInt32, stream : Void*) : Int32
   fun cogni_gemv_pack16_two_dev(x_a : UInt64, type_a : UInt32, in_dim_a : UInt32, image_a : UInt64, x_b : UInt64, type_b : UInt32,

@@ -519,6 +519,46 @@ int cogni_gemv_packed16_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t ima
   return gemv_mt_lists(who, true, w_raw, w_type, image, residual, out, out_dims, count, in_dim, tokens, stream);
 }
 
+// Two matrices with an image each: one launch where a wavefront of either takes one tile and the pair has a kernel.
+static int gemv_packed_two(const char* who, bool x16, uint64_t w_a, uint32_t type_a, uint64_t image_a, uint64_t out_a, uint32_t in_dim_a,
+                           uint32_t out_dim_a, uint64_t w_b, uint32_t type_b, uint64_t image_b, uint64_t out_b, uint32_t in_dim_b,
+                           uint32_t out_dim_b, uint32_t tokens, void* stream) {
+  if (!w_a || !image_a || !out_a || !w_b || !image_b || !out_b || out_dim_a == 0 || out_dim_b == 0)
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null pointer or zero rows");
+  auto first = [](uint32_t t) { return t == COGNI_TYPE_Q4_K || t == COGNI_TYPE_Q5_K; };
+  auto second = [](uint32_t t) { return t == COGNI_TYPE_Q4_K || t == COGNI_TYPE_Q6_K; };
+  if ((!first(type_a) || !second(type_b)) && first(type_b) && second(type_a)) {
+    std::swap(w_a, w_b), std::swap(type_a, type_b), std::swap(image_a, image_b), std::swap(out_a, out_b);
+    std::swap(in_dim_a, in_dim_b), std::swap(out_dim_a, out_dim_b);
+  }
+  if (first(type_a) && second(type_b) && out_dim_a <= 0x7FFFFFFFu && out_dim_b <= 0x7FFFFFFFu &&
+      gemv_mt_tiles(type_a, in_dim_a, (out_dim_a + 15) / 16) == 1 && gemv_mt_tiles(type_b, in_dim_b, (out_dim_b + 15) / 16) == 1) {
+    char name[48];
+    std::snprintf(name, sizeof name, "%s_and_%s_gemv_mt%s_f32", type_prefix(type_a), type_prefix(type_b), x16 ? "16" : "");
+    void* params[] = {&w_a, &image_a, &out_a, &in_dim_a, &out_dim_a, &w_b, &image_b, &out_b, &in_dim_b, &out_dim_b, &tokens};
+    return launch(name, gemv_mt_grid(type_a, in_dim_a, out_dim_a) + gemv_mt_grid(type_b, in_dim_b, out_dim_b), GEMV_MT_WAVES * 64,
+                  std::max(gemv_mt_lds_bytes(type_a), gemv_mt_lds_bytes(type_b)) + (x16 ? GEMV_MT_X16_LDS_EXTRA : 0u), params, stream);
+  }
+  if (int rc = gemv_mt_lists(who, x16, &w_a, type_a, image_a, 0, &out_a, &out_dim_a, 1, in_dim_a, tokens, stream)) return rc;
+  return gemv_mt_lists(who, x16, &w_b, type_b, image_b, 0, &out_b, &out_dim_b, 1, in_dim_b, tokens, stream);
+}
+int cogni_gemv_packed_two_dev(uint64_t w_a, uint32_t type_a, uint64_t image_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a, uint64_t w_b,
+                              uint32_t type_b, uint64_t image_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens,
+                              void* stream) {
+  if (!gemv_mt_supported(type_a, (int)tokens, in_dim_a) || !gemv_mt_supported(type_b, (int)tokens, in_dim_b))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed_two_dev: no one-pass kernel for this type, token count and in_dim");
+  return gemv_packed_two("cogni_gemv_packed_two_dev", false, w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b,
+                         in_dim_b, out_dim_b, tokens, stream);
+}
+int cogni_gemv_packed16_two_dev(uint64_t w_a, uint32_t type_a, uint64_t image_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a, uint64_t w_b,
+                                uint32_t type_b, uint64_t image_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens,
+                                void* stream) {
+  if (!gemv16_shape(type_a, in_dim_a, tokens) || !gemv16_shape(type_b, in_dim_b, tokens))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemv_packed16_two_dev: Q4_K, Q5_K, Q6_K or Q8_0, 1..16 tokens, in_dim a multiple of 256 up to 12288");
+  return gemv_packed_two("cogni_gemv_packed16_two_dev", true, w_a, type_a, image_a, out_a, in_dim_a, out_dim_a, w_b, type_b, image_b, out_b,
+                         in_dim_b, out_dim_b, tokens, stream);
+}
+
 int cogni_gemv_packed16_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t image, uint64_t out, uint32_t in_dim,
                                    uint32_t out_dim, uint32_t tokens, void* stream) {
   const char* who = "cogni_gemv_packed16_swiglu_dev";

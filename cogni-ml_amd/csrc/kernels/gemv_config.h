@@ -238,7 +238,7 @@ static inline GEMV_HD unsigned gemv_mt_tiles(unsigned type, unsigned in_dim, uns
   return three ? (unsigned)GEMV_MT_TMAX : (c2 < c1 ? 2u : 1u);
 }
 // One workgroup per compute unit at most; they walk the row groups (a workgroup that has none leaves at once).
-static inline unsigned gemv_mt_grid(unsigned type, unsigned in_dim, unsigned total_rows) {
+static inline GEMV_HD unsigned gemv_mt_grid(unsigned type, unsigned in_dim, unsigned total_rows) {
   const unsigned ntiles = (total_rows + 15) / 16;
   (void)type;
   (void)in_dim;

@@ -695,6 +695,7 @@ struct MtArgs {
 // that row's index (out[0][m * gridDim.x + blockIdx.x], top_ids[same]; of equal values the lowest row wins): the partial
 // results top1_reduce_f32 finishes, as q6_k_gemv_top1_partial_f32 writes them for one token. With `logits` the row values are
 // stored as well (logits[m * rows + row]).
+// bid, nwg: this workgroup's number and their count, where they are not the launch's (two matrices in one launch).
 // NEXT (SWIGLU, sixteen tokens): the products also go to `next` as the sixteen-token Q6_K image of the matrix behind (out[0] may be
 // null then; rows[0] a multiple of 256 up to GEMV_MT_MAX_IN_DIM): single binary16 terms need no scale of a whole super-block, and the
 // sixteen rows of a group are one of its sub-blocks, so a workgroup has all that it takes. The FFN half of a layer, 4096 -> 12288 -> 4096,
@@ -703,7 +704,7 @@ template <class F, int SBW, int T, bool SWIGLU = false, bool TOP1 = false, bool 
 __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* __restrict__ image,
                                              const float* __restrict__ residual, u32 in_dim, u32 tokens,
                                              u32* __restrict__ top_ids = nullptr, float* __restrict__ logits = nullptr,
-                                             uint8_t* __restrict__ next = nullptr) {
+                                             uint8_t* __restrict__ next = nullptr, u32 bid = blockIdx.x, u32 nwg = gridDim.x) {
   static_assert(!NEXT || (SWIGLU && F::NTOK == 16), "the image of the next matrix: sixteen tokens, gate | up");
   constexpr bool STREAM = SBW > 2;
   constexpr int NTOK = F::NTOK;   // token rows of the partial sums: 8, or 16 single-term tokens
@@ -737,7 +738,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
   const u32 ar = lane & 15, kg = lane >> 4;
   const u32 rg = lane >> 4;
 
-  u32 grp = blockIdx.x;
+  u32 grp = bid;
   if (grp >= ngroups) {
     if constexpr (TOP1) {   // no rows: a partial result that never wins
       if ((u32)tid < tokens) {
@@ -951,7 +952,7 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
 #pragma unroll
       for (int t = 0; t < T; t++) acc[t][0] = acc[t][1] = acc[t][2] = acc[t][3] = 0.f;
       start_reading();
-      if constexpr (walk) set_rows(grp + gridDim.x);
+      if constexpr (walk) set_rows(grp + nwg);
       auto unit = [&](auto utag) {
         constexpr int u = decltype(utag)::value, i = u / T, t = u % T;
         __builtin_amdgcn_sched_barrier(0);   // (unit after unit: interleaved, their operands do not fit the register file)
@@ -979,9 +980,9 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
       for (int t = 0; t < T; t++) store_part(t, acc[t]);
       finish();
     };
-    while (grp + gridDim.x < ngroups) {
+    while (grp + nwg < ngroups) {
       group(std::true_type{});
-      grp += gridDim.x;
+      grp += nwg;
       between_groups();
     }
     group(std::false_type{});
@@ -1026,8 +1027,8 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
       store_part(mat, acc);
      }
       finish();
-      if (grp + gridDim.x >= ngroups) break;
-      grp += gridDim.x;
+      if (grp + nwg >= ngroups) break;
+      grp += nwg;
       between_groups();
     }
   }
@@ -1108,6 +1109,40 @@ GEMV_MT_LIST_ENTRY(q4_k_gemv_mt_list_f32, MtQ4K)
 GEMV_MT_LIST_ENTRY(q5_k_gemv_mt_list_f32, MtQ5K)
 GEMV_MT_LIST_ENTRY(q4_k_gemv_mt16_list_f32, MtQ4Kx16)
 GEMV_MT_LIST_ENTRY(q5_k_gemv_mt16_list_f32, MtQ5Kx16)
+
+// (w_a, image_a, out_a, in_dim_a, rows_a, w_b, image_b, out_b, in_dim_b, rows_b, tokens): two matrices with an image each (o and down of a
+// layer) in one launch, of row counts that give a wavefront one tile (gemv_mt_tiles). Workgroups 0 .. gemv_mt_grid(b) - 1 are those of
+// b, whose rows are the longer ones in a layer, the ones behind those of a. A launch of few tiles leaves compute units idle, and every
+// launch costs its start and its end. Every row is computed as in <type>_gemv_mt_f32 | <type>_gemv_mt16_f32, dynamic shared memory the larger of the two.
+template <class F>
+__device__ __forceinline__ void gemv_mt_one_tile(const uint8_t* w, const uint8_t* image, float* out, u32 in_dim, u32 rows, u32 tokens, u32 bid,
+                                                 u32 nwg) {
+  const MtArgs<1> a = {{w}, {out}, {rows}};
+  switch (gemv_mt_padded_sb(in_dim) >> 3) {
+    case 1: gemv_mt_core<F, 1, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+    case 2: gemv_mt_core<F, 2, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+    case 3: gemv_mt_core<F, 3, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+    case 4: gemv_mt_core<F, 4, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+    case 5: gemv_mt_core<F, 5, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+    default: gemv_mt_core<F, 6, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+  }
+}
+#define GEMV_MT_TWO_ENTRY(NAME, FMT_A, FMT_B)                                                                                     \
+  extern "C" __global__ __launch_bounds__(GEMV_MT_WAVES * 64) void NAME(                                                          \
+      const uint8_t* w_a, const uint8_t* image_a, float* out_a, u32 in_dim_a, u32 rows_a, const uint8_t* w_b, const uint8_t* image_b, \
+      float* out_b, u32 in_dim_b, u32 rows_b, u32 tokens) {                                                                       \
+    const u32 wgs_b = gemv_mt_grid(FMT_B::TYPE, in_dim_b, rows_b);                                                                \
+    if (blockIdx.x < wgs_b) gemv_mt_one_tile<FMT_B>(w_b, image_b, out_b, in_dim_b, rows_b, tokens, blockIdx.x, wgs_b);            \
+    else gemv_mt_one_tile<FMT_A>(w_a, image_a, out_a, in_dim_a, rows_a, tokens, blockIdx.x - wgs_b, gridDim.x - wgs_b);           \
+  }
+GEMV_MT_TWO_ENTRY(q4_k_and_q4_k_gemv_mt_f32, MtQ4K, MtQ4K)
+GEMV_MT_TWO_ENTRY(q4_k_and_q6_k_gemv_mt_f32, MtQ4K, MtQ6K)
+GEMV_MT_TWO_ENTRY(q5_k_and_q4_k_gemv_mt_f32, MtQ5K, MtQ4K)
+GEMV_MT_TWO_ENTRY(q5_k_and_q6_k_gemv_mt_f32, MtQ5K, MtQ6K)
+GEMV_MT_TWO_ENTRY(q4_k_and_q4_k_gemv_mt16_f32, MtQ4Kx16, MtQ4Kx16)
+GEMV_MT_TWO_ENTRY(q4_k_and_q6_k_gemv_mt16_f32, MtQ4Kx16, MtQ6Kx16)
+GEMV_MT_TWO_ENTRY(q5_k_and_q4_k_gemv_mt16_f32, MtQ5Kx16, MtQ4Kx16)
+GEMV_MT_TWO_ENTRY(q5_k_and_q6_k_gemv_mt16_f32, MtQ5Kx16, MtQ6Kx16)
 
 // (w, image, partial_ids, partial_values, in_dim, out_dim, tokens): the output head's arg-max for 2..8 tokens in one pass
 // over the weights. Grid, block and dynamic shared memory as q4_k_gemv_mt_f32 | q6_k_gemv_mt_f32 for out_dim rows;

@@ -261,6 +261,16 @@ int cogni_gemv_pack_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, ui
                             uint64_t image_b, uint32_t tokens, void* stream);
 int cogni_gemv_pack16_two_dev(uint64_t x_a, uint32_t type_a, uint32_t in_dim_a, uint64_t image_a, uint64_t x_b, uint32_t type_b, uint32_t in_dim_b,
                               uint64_t image_b, uint32_t tokens, void* stream);
+/* Two matrices against an image each (o and down of a layer): the values of cogni_gemv_packed_dev | cogni_gemv_packed16_dev for the one and the
+ * other. A Q4_K or Q5_K matrix beside a Q4_K or Q6_K one of up to 4096 rows (more where a wavefront takes one tile of 16 all the same) are
+ * one launch of "<type_a>_and_<type_b>_gemv_mt_f32" | "..._gemv_mt16_f32" (w_a, image_a, out_a, in_dim_a, rows_a, w_b, image_b, out_b, in_dim_b,
+ * rows_b, tokens), the sum of the two grids, the larger shared memory. */
+int cogni_gemv_packed_two_dev(uint64_t w_a, uint32_t type_a, uint64_t image_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a, uint64_t w_b,
+                              uint32_t type_b, uint64_t image_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens,
+                              void* stream);
+int cogni_gemv_packed16_two_dev(uint64_t w_a, uint32_t type_a, uint64_t image_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a, uint64_t w_b,
+                                uint32_t type_b, uint64_t image_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens,
+                                void* stream);
 /* Two matrices with an input each (o and down of a layer): out[m*out_dim + o] = sum_j x[m*in_dim + j] * deq(W[o][j]) for a and for b. One
  * token of a Q4_K or Q5_K matrix beside a Q4_K or Q6_K one is one launch of "<type_a>_and_<type_b>_gemv_f32[_r1]" (w_a, x_a, out_a, in_dim_a,
  * out_dim_a, w_b, x_b, out_b, in_dim_b, out_dim_b, workgroups of b:u32), block and shared memory (the larger) as cogni_gemv_plan gives

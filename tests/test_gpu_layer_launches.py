@@ -129,6 +129,38 @@ def test_rounds_of_a_stack():
         assert QwenProjectionStackRunner._rounds_of(odd) == [[[e]] for e in odd]
 
 
+# both orders, one and six super-blocks per k-slice, rows past the grid's 256 tiles, a ragged end, pairs without a kernel (two tiles a wavefront, types)
+@pytest.mark.parametrize("tokens", [2, 7, 8, 9, 16])
+@pytest.mark.parametrize("a,b", [((Q4_K, 4096, 4096), (Q6_K, 12288, 4096)), ((Q6_K, 2816, 1000), (Q5_K, 1024, 1024)), ((Q4_K, 256, 1), (Q4_K, 8192, 5000)),
+                                 ((Q5_K, 5376, 33), (Q4_K, 2560, 16)), ((Q4_K, 1024, 12288), (Q6_K, 256, 70)), ((Q6_K, 512, 40), (Q6_K, 256, 33))])
+def test_two_matrices_with_an_image_each(gpu, a, b, tokens):
+    """The launch of two matrices: each output as its image and that matrix alone give it, bit for bit."""
+    x16 = tokens > 8
+    pack, packed, two = (quant.gemv_pack16_dev, quant.gemv_packed16_dev, quant.gemv_packed16_two_dev) if x16 else \
+        (quant.gemv_pack_dev, quant.gemv_packed_dev, quant.gemv_packed_two_dev)
+    rng = np.random.default_rng(a[1] + b[1] + tokens)
+    args, mats = [], []
+    for t, in_dim, out_dim in (a, b):
+        x, image = DevArray(synth.make_activations(rng, tokens, in_dim)), DevArray(nbytes=quant.gemv_image_bytes(t, in_dim, 8))
+        w = DevArray(synth.make_weights(rng, t, out_dim, in_dim))
+        one, both = (DevArray(np.full(tokens * out_dim + 64, np.float32(v))) for v in (5.0, 6.0))
+        pack(x.ptr, t, in_dim, tokens, image.ptr)
+        packed([w.ptr], t, image.ptr, [one.ptr], [out_dim], in_dim, tokens)
+        args += [w.ptr, t, image.ptr, both.ptr, in_dim, out_dim]
+        mats.append((x, image, w, one, both, out_dim))
+    print("case", a, b, tokens, flush=True)
+    two(*args, tokens)
+    for x, image, w, one, both, out_dim in mats:
+        got = both.read(np.float32, tokens * out_dim + 64)
+        assert np.array_equal(got[:tokens * out_dim], one.read(np.float32, tokens * out_dim)), out_dim
+        assert (got[tokens * out_dim:] == 6.0).all()
+    with pytest.raises(quant.QuantError, match="null pointer"):
+        two(*args[:3], 0, *args[4:], tokens)
+    for m in mats:
+        for d in m[:5]:
+            d.close()
+
+
 @pytest.mark.parametrize("in_dim", [256, 768, 2048, 3328, 4096, 12288])
 @pytest.mark.parametrize("first", [0, 2, 4, 10, 14])
 def test_q6_k_blocks_at_every_shift(gpu, oracle, first, in_dim):
