@@ -43,6 +43,12 @@ def lib():
         L.cogni_data_bytes.argtypes = [ctypes.c_uint32, ctypes.c_int64]
         L.cogni_weight_device_ptr.restype = ctypes.c_uint64
         L.cogni_weight_device_ptr.argtypes = [ctypes.c_void_p]
+        # the calls a program issues one by one: with the types declared ctypes converts plain integers itself (0.3 us a call less than
+        # with an object per argument, of 3.7)
+        U64, U32 = ctypes.c_uint64, ctypes.c_uint32
+        L.cogni_matmul_dev.argtypes = [U64, U32, U64, U64, U64, U32, U32, U32, U64, ctypes.c_size_t, ctypes.c_void_p]
+        L.cogni_gemv_dev.argtypes = [U64, U32, U64, U64, U64, U32, U32, U32, ctypes.c_void_p]
+        L.cogni_dequantize_dev.argtypes = [U64, U32, U64, U64, ctypes.c_void_p]
         L.mlhip_mem_alloc.argtypes = [ctypes.POINTER(ctypes.c_uint64), ctypes.c_size_t]
         L.mlhip_mem_free.argtypes = [ctypes.c_uint64]
         L.mlhip_memcpy_htod.argtypes = [ctypes.c_uint64, ctypes.c_void_p, ctypes.c_size_t]

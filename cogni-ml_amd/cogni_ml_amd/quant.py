@@ -63,14 +63,11 @@ def gemv_plan(w_type, tokens, in_dim, out_dim, add=False):
 
 
 def dequantize_dev(w_ptr, w_type, n_elements, out_ptr, stream=None):
-    _check(hip.lib().cogni_dequantize_dev(ctypes.c_uint64(w_ptr), ctypes.c_uint32(int(w_type)),
-                                          ctypes.c_uint64(n_elements), ctypes.c_uint64(out_ptr), stream))
+    _check(hip.lib().cogni_dequantize_dev(w_ptr, int(w_type), n_elements, out_ptr, stream))
 
 
 def gemv_dev(w_ptr, w_type, x_ptr, out_ptr, in_dim, out_dim, tokens=1, residual_ptr=0, stream=None):
-    _check(hip.lib().cogni_gemv_dev(ctypes.c_uint64(w_ptr), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(x_ptr),
-                                    ctypes.c_uint64(residual_ptr), ctypes.c_uint64(out_ptr), ctypes.c_uint32(in_dim),
-                                    ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
+    _check(hip.lib().cogni_gemv_dev(w_ptr, int(w_type), x_ptr, residual_ptr, out_ptr, in_dim, out_dim, tokens, stream))
 
 
 def gemv_many_dev(w_ptrs, w_type, x_ptr, out_ptrs, out_dims, in_dim, tokens=1, stream=None):
@@ -495,10 +492,8 @@ def gemm_stream_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, wor
 def matmul_dev(w_ptr, w_type, x_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr=0, workspace_bytes=0, bias_ptr=0,
                stream=None):
     """The GEMV/GEMM router (tokens > threshold and Q4_K -> GEMM)."""
-    _check(hip.lib().cogni_matmul_dev(ctypes.c_uint64(w_ptr), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(x_ptr),
-                                      ctypes.c_uint64(bias_ptr), ctypes.c_uint64(out_ptr), ctypes.c_uint32(in_dim),
-                                      ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens),
-                                      ctypes.c_uint64(workspace_ptr), ctypes.c_size_t(workspace_bytes), stream))
+    _check(hip.lib().cogni_matmul_dev(w_ptr, int(w_type), x_ptr, bias_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr,
+                                      workspace_bytes, stream))
 
 
 def set_gemm_threshold(tokens):
