@@ -1602,7 +1602,11 @@ int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_
     GemmStreamPlan pb = gemm_stream_plan(type_b, tokens, in_dim_b, out_dim_b, gemm_stream_planes(packed_b, bytes_b, tokens, out_dim_b));
     const uint32_t tiles_a = (out_dim_a + 31) / 32, tiles_b = (out_dim_b + 31) / 32;
     const uint64_t grid = (uint64_t)pa.splits * gemm_stream_grid(tokens, pa.t, tiles_a) + (uint64_t)pb.splits * gemm_stream_grid(tokens, pb.t, tiles_b);
-    if (pa.rt == 1 && pb.rt == 1 && grid < (1u << 24)) {
+    // (two matrices of one input may share its workspace: then the planes of both would be the same memory)
+    const uint64_t end_a = workspace_a + packed_a + (uint64_t)pa.splits * tokens * out_dim_a * sizeof(float);
+    const uint64_t end_b = workspace_b + packed_b + (uint64_t)pb.splits * tokens * out_dim_b * sizeof(float);
+    const bool apart = pa.splits == 1 || pb.splits == 1 || end_a <= workspace_b + packed_b || end_b <= workspace_a + packed_a;
+    if (pa.rt == 1 && pb.rt == 1 && apart && grid < (1u << 24)) {
       GemmManyArgs list_a{}, list_b{};
       list_a.w[0] = w_a, list_a.out[0] = pa.splits > 1 ? workspace_a + packed_a : out_a;
       list_a.out_dim[0] = out_dim_a, list_a.tile_end[0] = tiles_a, list_a.count = 1;

@@ -511,7 +511,8 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
  * null); of the absent tokens of the packed block only those of the last tile of 32 are written (zeros). Any token count is taken
  * as long as the packed activations are below 2 GiB. cogni_gemm_stream_two_dev: two matrices with an input each (o and down of a layer),
  * the values of cogni_gemm_stream_dev for the one and the other; a Q4_K or Q5_K matrix beside a Q4_K or Q6_K one that both go in tiles of
- * 32 rows are one launch of "<type_a>_and_<type_b>_gemm_stream_f16_<T>x1". Neither workspace may overlap the other. */
+ * 32 rows are one launch of "<type_a>_and_<type_b>_gemm_stream_f16_<T>x1". One workspace may serve two matrices of one
+ * input (they then go one after the other if both split their k range), two must not overlap. */
 int cogni_gemm_stream_takes(uint32_t w_type, uint32_t in_dim, uint32_t rows, uint32_t tokens);
 int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t residual,
                           const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);

@@ -178,3 +178,26 @@ def test_two_matrices_with_an_input_each(gpu, a, b, tokens):
     for m in mats:
         for i in (0, 2, 4, 7, 8):
             m[i].close()
+
+
+@pytest.mark.parametrize("a,b", [((Q4_K, 96), (Q5_K, 1024)), ((Q5_K, 1024), (Q4_K, 1024))])
+def test_two_matrices_of_one_workspace(gpu, a, b):
+    """Both read the same packed activations and put the planes of their k splits behind them: each output as alone, bit for bit."""
+    in_dim, tokens = 12288, 48   # (rows long enough for a k split)
+    rng = np.random.default_rng(a[1] + b[1])
+    x, nb = DevArray(synth.make_activations(rng, tokens, in_dim)), max(quant.gemm_workspace_bytes(t, in_dim, tokens, d) for t, d in (a, b))
+    assert nb >= quant.gemm_workspace_bytes(Q4_K, in_dim, tokens) + 2 * 4 * tokens * max(a[1], b[1])   # room for planes
+    ws = DevArray(nbytes=nb)
+    quant.gemm_pack_dev(x.ptr, Q4_K, in_dim, tokens, ws.ptr, nb)
+    mats = []
+    for t, d in (a, b):
+        w, one, two = DevArray(synth.make_weights(rng, t, d, in_dim)), DevArray(nbytes=4 * tokens * d), DevArray(nbytes=4 * tokens * d)
+        quant.gemm_stream_dev([w.ptr], t, ws.ptr, nb, [one.ptr], [d], in_dim, tokens)
+        mats.append((w, t, two, d, one))
+    quant.gemm_stream_two_dev(*[v for w, t, two, d, one in mats for v in (w.ptr, t, ws.ptr, nb, two.ptr, in_dim, d)], tokens)
+    for w, t, two, d, one in mats:
+        assert np.array_equal(two.read(np.float32, tokens * d), one.read(np.float32, tokens * d)), (t, d)
+        for dev in (w, two, one):
+            dev.close()
+    x.close()
+    ws.close()
