@@ -550,13 +550,14 @@ typedef MtQ80T<true> MtQ80x16;
 
 // Q6_K (210 B: ql[128], qh[64], scales:i8[16], d). Element 128 n + 32 k + l (half n, quarter k, l < 32) has its low four bits
 // in nibble k / 2 of ql[64 n + 32 (k % 2) + l] and its high two in bits 2 k, 2 k + 1 of qh[32 n + l]; sub-block
-// s = 8 n + 2 k + l / 16. A row's block starts at a multiple of 2 bytes only. It is copied as the 14 aligned pieces of 16 bytes that
-// hold it (210 bytes from an even start are never in more), and the lanes read its fields at the block's shift, 0 to 14 bytes: a
+// s = 8 n + 2 k + l / 16. A row's block starts at a multiple of 2 bytes from the matrix's start only. It is copied as the 14 aligned
+// pieces of 16 bytes that hold it (15 from the last byte of such a piece), and the lanes read its fields at the block's shift, 0 to 15 bytes: a
 // copy from inside a dword takes the memory pipeline about twice as long, and a read of LDS from there costs more than that, so
 // the fields of a block that starts inside a dword (every other one) are put together from two dwords. Head of 151936 x 4096 at six
 // tokens with its norm and reduce, us: copied from the start as it lies 120.4, like this 112.5, without the shift of odd blocks (wrong) 104.
 // Every piece holds a byte of the block, so what is read beside it lies in the same 16 aligned bytes as one of the matrix's, never in
-// another page. A row in LDS is 15 pieces (240 bytes: rows 60 dwords apart hit 16 different bank groups), piece 14 a copy of piece 13.
+// another page. A row in LDS is 15 pieces (240 bytes: rows 60 dwords apart hit 16 different bank groups); piece 14 is the one with the block's last
+// byte, mostly piece 13 again.
 // (X16: sixteen single-term tokens, as MtK45's)
 template <bool X16 = false>
 struct MtQ6KT {
@@ -565,7 +566,7 @@ struct MtQ6KT {
   static constexpr int BB = 210, P = 15, NCOPY = 4, LAST = 16 * P - 192, NAUX = 1, NSLOT = 4, TMAX = 2;
   static constexpr bool SHIFTED = true;
   static constexpr u32 UNIT_BYTES = 16 * P * 16, AUX_SB_BYTES = 64 * 16;
-  static __device__ __forceinline__ u32 piece_offset(u32 piece) { return min(piece, 13u) * 16; }
+  static __device__ __forceinline__ u32 piece_offset(u32 piece) { return min(piece * 16, 209u); }
   static __device__ __forceinline__ u32 aux_offset(u32 lane) { return lane * 16; }   // 16 bytes of its own per lane
 
   // the scales of the lane's two tokens and, as the matrix-core operand of lane (kg, row), the sums of sub-blocks
@@ -609,7 +610,12 @@ struct MtQ6KT {
   static __device__ __forceinline__ Raw read(const char* start, u32 kg) {
     const u32 sh = (u32)(uintptr_t)start & 3u;
     if (__builtin_amdgcn_ballot_w64(sh != 0) == 0) return fields<false>(start, kg, 0);
-    return fields<true>(start - sh, kg, sh);
+    Raw w = fields<true>(start - sh, kg, sh);
+    if (__builtin_amdgcn_readfirstlane(sh) & 1u) {   // a matrix at an odd address (all its blocks are): d may be in two dwords
+      const u32* const d = reinterpret_cast<const u32*>(start - sh + 208);
+      w.d = __builtin_amdgcn_alignbyte(d[1], d[0], sh);
+    }
+    return w;
   }
   static __device__ __forceinline__ float sbyte_f(u32 v, int k) { return (float)(int)(signed char)((v >> (8 * k)) & 0xFFu); }
   static __device__ __forceinline__ void unit(const Raw& w, const mt_u32x4 (&b)[8], const Aux& ax, float (&acc)[4]) {

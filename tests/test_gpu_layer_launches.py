@@ -162,7 +162,7 @@ def test_two_matrices_with_an_image_each(gpu, a, b, tokens):
 
 
 @pytest.mark.parametrize("in_dim", [256, 768, 2048, 3328, 4096, 12288])
-@pytest.mark.parametrize("first", [0, 2, 4, 10, 14])
+@pytest.mark.parametrize("first", [0, 1, 2, 3, 4, 10, 14, 15])
 def test_q6_k_blocks_at_every_shift(gpu, oracle, first, in_dim):
     """The one-pass kernels copy a Q6_K block as the aligned 16-byte pieces that hold it: rows of odd and even numbers of blocks (blocks
     inside and at the start of a dword), and a matrix that starts `first` bytes behind 16 aligned ones."""
