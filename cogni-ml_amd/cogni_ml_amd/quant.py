@@ -63,11 +63,15 @@ def gemv_plan(w_type, tokens, in_dim, out_dim, add=False):
 
 
 def dequantize_dev(w_ptr, w_type, n_elements, out_ptr, stream=None):
-    _check(hip.lib().cogni_dequantize_dev(w_ptr, int(w_type), n_elements, out_ptr, stream))
+    if type(stream) is int:
+        stream = ctypes.c_void_p(stream)
+    _check(hip.lib().typed_dequantize_dev(w_ptr, int(w_type), n_elements, out_ptr, stream))
 
 
 def gemv_dev(w_ptr, w_type, x_ptr, out_ptr, in_dim, out_dim, tokens=1, residual_ptr=0, stream=None):
-    _check(hip.lib().cogni_gemv_dev(w_ptr, int(w_type), x_ptr, residual_ptr, out_ptr, in_dim, out_dim, tokens, stream))
+    if type(stream) is int:
+        stream = ctypes.c_void_p(stream)
+    _check(hip.lib().typed_gemv_dev(w_ptr, int(w_type), x_ptr, residual_ptr, out_ptr, in_dim, out_dim, tokens, stream))
 
 
 def gemv_many_dev(w_ptrs, w_type, x_ptr, out_ptrs, out_dims, in_dim, tokens=1, stream=None):
@@ -492,7 +496,9 @@ def gemm_stream_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, wor
 def matmul_dev(w_ptr, w_type, x_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr=0, workspace_bytes=0, bias_ptr=0,
                stream=None):
     """The GEMV/GEMM router (tokens > threshold and Q4_K -> GEMM)."""
-    _check(hip.lib().cogni_matmul_dev(w_ptr, int(w_type), x_ptr, bias_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr,
+    if type(stream) is int:
+        stream = ctypes.c_void_p(stream)
+    _check(hip.lib().typed_matmul_dev(w_ptr, int(w_type), x_ptr, bias_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr,
                                       workspace_bytes, stream))
 
 

@@ -285,6 +285,17 @@ def test_runner_rejects_invalid_active_counts():
     assert r.active_tokens == 4
 
 
+@pytest.mark.parametrize("stream", [None, 1 << 40, ctypes.c_void_p(1 << 40), ctypes.c_uint64(1 << 40), ctypes.c_size_t(1 << 40)])
+def test_single_operators_take_a_stream_in_any_form(stream):
+    """The calls reach the library (which refuses the null pointers before it looks at the stream), typed and as the raw symbols."""
+    for call in (lambda: quant.matmul_dev(0, 12, 0, 0, 256, 16, 1, stream=stream), lambda: quant.gemv_dev(0, 12, 0, 0, 256, 16, 1, stream=stream),
+                 lambda: quant.dequantize_dev(0, 12, 256, 0, stream=stream)):
+        with pytest.raises(quant.QuantError, match="null device pointer"):
+            call()
+    null, u32 = ctypes.c_void_p(0), ctypes.c_uint32
+    assert hip.lib().cogni_gemv_dev(null, u32(12), null, null, null, ctypes.c_int(256), u32(16), u32(1), ctypes.c_void_p(0)) != 0
+
+
 def test_one_pass_geometry_and_thresholds():
     """Pack + one pass over the weights: which shapes have a kernel, the size of the activation image (8 KiB of operands
     per super-block, then the scales and the sub-block sums), where gemv_dev switches to it,
