@@ -1259,13 +1259,13 @@ struct GemmShape {
 };
 static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, bool split = true) {
   const uint32_t mtiles = (tokens + 127) / 128, nkb = in_dim / 256;
-  auto eval = [&](uint32_t bn, uint64_t* cost) {
+  auto eval = [&](uint32_t bn, uint32_t tile_cost, uint64_t* cost) {
     const uint32_t tiles = mtiles * ((out_dim + bn - 1) / bn), s = split && bn != 256 ? gemm_splits_of(tiles, in_dim) : 1u;
-    *cost = (uint64_t)((tiles * s + 255u) / 256u) * ((nkb + s - 1) / s) * gemm_tile_cost(w_type, bn);
+    *cost = (uint64_t)((tiles * s + 255u) / 256u) * ((nkb + s - 1) / s) * tile_cost;
     return s;
   };
   uint64_t cost192 = 0, cost128 = 0, cost256 = 0;
-  const uint32_t s192 = eval(192, &cost192), s128 = eval(128, &cost128);
+  const uint32_t s192 = eval(192, gemm_tile_cost(w_type, 192), &cost192), s128 = eval(128, gemm_tile_cost(w_type, 128), &cost128);
   bool n128 = cost128 < cost192;
   if (const char* e = std::getenv("COGNI_GEMM_N128")) {
     if (e[0] == '0') n128 = false;
@@ -1276,7 +1276,7 @@ static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, 
   // gemm_q4k_use_wide; Q6_K where the 192-row tiles are not the better of the two others (and the activations of a token tile stay
   // below 4 GiB, which its 32-bit offsets reach)
   if (best.splits == 1 && tokens > 64 && (w_type == COGNI_TYPE_Q4_K || (w_type == COGNI_TYPE_Q6_K && nkb < 65536u))) {
-    (void)eval(256, &cost256);
+    (void)eval(256, w_type == COGNI_TYPE_Q4_K ? GEMM_Q4K_WIDE_COST : gemm_tile_cost(w_type, 256), &cost256);
     bool wide = (w_type == COGNI_TYPE_Q4_K ? gemm_q4k_use_wide(out_dim, tokens) != 0 : n128) && cost256 < (n128 ? cost128 : cost192);
     if (const char* e = std::getenv("COGNI_GEMM_WIDE")) {
       if (e[0] == '0') wide = false;

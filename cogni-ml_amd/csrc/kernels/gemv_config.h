@@ -266,13 +266,18 @@ static inline unsigned long long gemv_mt_image_bytes(unsigned type, unsigned in_
 // 134.7 at 512 tokens, 94.2 | 78.1 | 69.5 at 256, 105.9 | 113.1 | 121.4 at 384, 562 | 581 | 532 at 2048. Q6_K 12288 -> 4096: 314 | 237 | 211 at
 // 2048 tokens, 151 | 120 | 155 at 1024.
 #define GEMM_ROUND_TILES 256u
-// A single Q4_K matrix takes the 256-row tiles where they fill whole rounds and save enough of the 192-row ones' (its plan
-// is what cogni_gemm_plan names; lists and gate | up go by the costs alone).
+// A single Q4_K matrix (cogni_gemm_plan) takes the 256-row tiles where they fill whole rounds and those cost less, at 124, than
+// the 192- and the 128-row ones'. 4096 columns, weights from memory, us in 192 | 128 | 256-row tiles: three rounds against four and five, 12288
+// rows at 2048 tokens 205 | 218 | 202, 10240 at 2048 188 | 182 | 180, 20480 at 1024 189 | 187 | 181, 32000 at 640 193 | 190 | 185; four
+// against five and seven, 14336 at 2048 246 | 256 | 247, 28672 at 1024 248 | 261 | 246; seven against nine and eleven, 27648 at 2048 460 | 497 | 452.
+// (12288 columns, 28672 rows at 1024: 683 | 715 | 690.) Up to 64 tokens never: 151936 rows at 64 in the 64-token kernels 153, in 256-row tiles 184.
+// Lists and gate | up go by the costs above alone.
+#define GEMM_Q4K_WIDE_COST 124u
 static inline int gemm_q4k_use_wide(unsigned out_dim, unsigned tokens) {
   const unsigned mtiles = (tokens + 127u) / 128u;
   const unsigned narrow = mtiles * ((out_dim + 191u) / 192u), wide = mtiles * ((out_dim + 255u) / 256u);
   const unsigned rn = (narrow + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES, rw = (wide + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
-  return wide >= GEMM_ROUND_TILES && rw * 124u < rn * 100u;
+  return wide >= GEMM_ROUND_TILES && rw * GEMM_Q4K_WIDE_COST < rn * 100u;
 }
 static inline unsigned gemm_tile_cost(unsigned type, unsigned rows) { return rows == 192u ? 100u : (rows == 128u ? 75u : (type == 14u ? 107u : 131u)); }
 // gate | up with SwiGLU: tiles of 96 rows of both matrices (four wavefronts) or of 128 (eight). 4096 -> 12288, us: 441 | 410 at 2048

@@ -176,6 +176,9 @@ def test_gemm_plan_picks_tile_and_split_for_the_shape():
     assert quant.gemm_plan(12, 4096, 12288, 2048, big) == ("q4_k_gemm_wide_f16", 768, 1, 512)
     assert quant.gemm_plan(12, 4096, 12288, 1024, big) == ("q4_k_gemm_f16", 512, 1, 256)       # two rounds either way
     assert quant.gemm_plan(12, 4096, 12288, 4096, big) == ("q4_k_gemm_wide_f16", 1536, 1, 512)  # 6 rounds instead of 8
+    # a quarter of the rounds saved or a fifth, and 128-row tiles that would take five for its three
+    for out_dim, tokens in ((14336, 2048), (28672, 1024), (27648, 2048), (13824, 4096), (10240, 2048), (20480, 1024), (32000, 640)):
+        assert quant.gemm_plan(12, 4096, out_dim, tokens, big)[0] == "q4_k_gemm_wide_f16", (out_dim, tokens)
     # the grid is whole blocks of 32 tiles (8 weight tiles x 4 token tiles), 8 blocks at a time: a clipped shape rounds up
     assert quant.gemm_plan(12, 4096, 12288 + 192, 512, big)[1] == 8 * 32 * 2 and quant.gemm_plan(12, 256, 400, 130, big)[1:3] == (16, 1)
     # the 12288 -> 4096 down projection at M = 512: 88 tiles of 192 rows with the k range split in two are 176 workgroups,
