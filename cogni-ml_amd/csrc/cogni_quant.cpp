@@ -1253,10 +1253,14 @@ static uint32_t gemm_splits_of(uint32_t tiles, uint32_t in_dim) {
 // costs per super-block against one of 192 rows is gemm_tile_cost (gemv_config.h), and the cheapest plan wins
 // (the 4096-row projections at 512 tokens: 88 tiles x 2 splits = 176 workgroups of 192 rows, or 128 x 2 = 256 of the
 // smaller ones). `split` false: the plan for a workspace without planes. COGNI_GEMM_N128=0 | 1 and COGNI_GEMM_WIDE=0 | 1
-// override the choice (measurement knobs: 1 takes that tile wherever its kernel can run).
+// override the choice (measurement knobs: 1 takes that tile wherever its kernel can run; COGNI_GEMM_WIDE also of lists and gate | up).
 struct GemmShape {
   uint32_t bn, splits;
 };
+static int gemm_wide_knob() {
+  const char* e = std::getenv("COGNI_GEMM_WIDE");
+  return e && (e[0] == '0' || e[0] == '1') ? e[0] - '0' : -1;
+}
 static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, bool split = true) {
   const uint32_t mtiles = (tokens + 127) / 128, nkb = in_dim / 256;
   auto eval = [&](uint32_t bn, uint32_t tile_cost, uint64_t* cost) {
@@ -1275,13 +1279,10 @@ static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, 
   // the eight-wavefront kernels, for more tokens than the 64-token tiles have and launches that are not split: Q4_K by
   // gemm_q4k_use_wide; Q6_K where the 192-row tiles are not the better of the two others (and the activations of a token tile stay
   // below 4 GiB, which its 32-bit offsets reach)
-  if (best.splits == 1 && tokens > 64 && (w_type == COGNI_TYPE_Q4_K || (w_type == COGNI_TYPE_Q6_K && nkb < 65536u))) {
+  if (best.splits == 1 && (w_type == COGNI_TYPE_Q4_K || (w_type == COGNI_TYPE_Q6_K && nkb < 65536u))) {
     (void)eval(256, w_type == COGNI_TYPE_Q4_K ? GEMM_Q4K_WIDE_COST : gemm_tile_cost(w_type, 256), &cost256);
-    bool wide = (w_type == COGNI_TYPE_Q4_K ? gemm_q4k_use_wide(out_dim, tokens) != 0 : n128) && cost256 < (n128 ? cost128 : cost192);
-    if (const char* e = std::getenv("COGNI_GEMM_WIDE")) {
-      if (e[0] == '0') wide = false;
-      if (e[0] == '1') wide = true;
-    }
+    bool wide = tokens > 64 && (w_type == COGNI_TYPE_Q4_K ? gemm_q4k_use_wide(out_dim, tokens) != 0 : n128) && cost256 < (n128 ? cost128 : cost192);
+    if (const int knob = gemm_wide_knob(); knob >= 0) wide = knob != 0;
     if (wide) best = GemmShape{256, 1};
   }
   return best;
@@ -1431,7 +1432,7 @@ int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
   if (!w_gate || !w_up || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_gemm_packed_swiglu_dev: null device pointer");
   if (int rc = gemm_check("cogni_gemm_packed_swiglu_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;
   const uint32_t mtiles = (tokens + 127) / 128;
-  const bool wide = gemm_swiglu_use_wide(out_dim, tokens);
+  const bool wide = gemm_swiglu_use_wide(out_dim, tokens, gemm_wide_knob());
   const uint32_t rows = wide ? 128 : 96;   // a tile is 128 tokens x `rows` rows of each matrix
   void* params[] = {&w_gate, &w_up, &workspace, &out, &in_dim, &out_dim, &tokens};
   return launch(wide ? "q4_k_gemm_swiglu_wide_f16" : (tokens <= 64 ? "q4_k_gemm_swiglu_m64_f16" : "q4_k_gemm_swiglu_f16"),
@@ -1465,15 +1466,7 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
                               out_dims[0], tokens, stream);
   const uint64_t mtiles = (tokens + 127) / 128;
   const bool m64 = tokens <= 64;
-  uint32_t bn = 0;
-  uint64_t least = ~0ull;
-  for (uint32_t rows : {192u, 128u, 256u}) {
-    if (rows == 256 && (w_type != COGNI_TYPE_Q4_K || m64)) continue;
-    uint64_t tiles = 0;
-    for (uint32_t i = 0; i < count; i++) tiles += (out_dims[i] + rows - 1) / rows;
-    const uint64_t cost = (mtiles * tiles + 255) / 256 * gemm_tile_cost(w_type, rows);
-    if (cost < least) least = cost, bn = rows;
-  }
+  const uint32_t bn = gemm_list_rows(w_type, out_dims, count, tokens, gemm_wide_knob());
   GemmManyArgs list{};
   uint32_t end = 0;
   for (uint32_t i = 0; i < count; i++) {
@@ -1514,7 +1507,7 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
                                  next_workspace_bytes, in_dim, out_dim, tokens))
     return rc;
   const uint32_t mtiles = (tokens + 127) / 128;
-  const bool wide = gemm_swiglu_use_wide(out_dim, tokens);
+  const bool wide = gemm_swiglu_use_wide(out_dim, tokens, gemm_wide_knob());
   const uint32_t rows = wide ? 128 : 96;   // a tile is 128 tokens x `rows` rows of each matrix
   void* params[] = {&w_gate, &w_up, &workspace, &out, &next_workspace, &in_dim, &out_dim, &tokens};
   static const char* const names[2][3] = {{"q4_k_gemm_swiglu_pack_q4k_f16", "q4_k_gemm_swiglu_pack_q4k_m64_f16", "q4_k_gemm_swiglu_pack_q4k_wide_f16"},

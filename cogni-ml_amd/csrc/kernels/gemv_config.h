@@ -280,13 +280,28 @@ static inline int gemm_q4k_use_wide(unsigned out_dim, unsigned tokens) {
   return wide >= GEMM_ROUND_TILES && rw * GEMM_Q4K_WIDE_COST < rn * 100u;
 }
 static inline unsigned gemm_tile_cost(unsigned type, unsigned rows) { return rows == 192u ? 100u : (rows == 128u ? 75u : (type == 14u ? 107u : 131u)); }
+// knob: COGNI_GEMM_WIDE, 0 | 1 where it is set (no 256-row tiles | those wherever there is a kernel for them), else -1.
 // gate | up with SwiGLU: tiles of 96 rows of both matrices (four wavefronts) or of 128 (eight). 4096 -> 12288, us: 441 | 410 at 2048
 // tokens, 225 | 208 at 1024, 114 | 123 at 512, 58 | 59 at 256; 2048 -> 4096 at 1024 61.6 | 41.3; 3072 -> 8192 at 300 76.7 | 45.5.
-static inline int gemm_swiglu_use_wide(unsigned out_dim, unsigned tokens) {
+static inline int gemm_swiglu_use_wide(unsigned out_dim, unsigned tokens, int knob) {
   const unsigned long long mtiles = (tokens + 127u) / 128u;
   const unsigned long long rn = (mtiles * ((out_dim + 95u) / 96u) + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
   const unsigned long long rw = (mtiles * ((out_dim + 127u) / 128u) + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
-  return tokens > 64u && rw * gemm_tile_cost(12u, 256u) < rn * gemm_tile_cost(12u, 192u);
+  return knob >= 0 ? knob : tokens > 64u && rw * gemm_tile_cost(12u, 256u) < rn * gemm_tile_cost(12u, 192u);
+}
+// A list of Q4_K or Q5_K matrices as one launch: rows of its tiles. The 256-row ones: Q4_K, more tokens than the 64-token kernels take.
+static inline unsigned gemm_list_rows(unsigned type, const unsigned* out_dims, unsigned count, unsigned tokens, int knob) {
+  const unsigned of[3] = {192u, 128u, 256u};
+  unsigned long long least = ~0ull;
+  unsigned best = 192u, k, i;
+  if (type == 12u && knob == 1) return 256u;
+  for (k = 0; k < (type == 12u && tokens > 64u && knob != 0 ? 3u : 2u); k++) {
+    unsigned long long tiles = 0, cost;
+    for (i = 0; i < count; i++) tiles += ((unsigned long long)out_dims[i] + of[k] - 1u) / of[k];
+    cost = ((tokens + 127u) / 128u * tiles + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES * gemm_tile_cost(type, of[k]);
+    if (cost < least) least = cost, best = of[k];
+  }
+  return best;
 }
 
 // ---- prefill GEMM: which tile a workgroup takes. Workgroups go to the 8 XCDs round-robin (id % 8), each XCD has its own

@@ -1,4 +1,6 @@
 """Session set-up shared by the GPU parity tests (all of them call through libcogni_hip.so)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -34,3 +36,25 @@ class DevArray:
 
     def close(self):
         self.buf.close()
+
+
+def launched_blocks(issue):
+    """Workgroup sizes (x) of the kernels that issue(stream handle) launches, in no particular order: captured, not run."""
+    L, stream = hip.lib(), hip.HIPStream()
+    stream.begin_capture()
+    try:
+        issue(stream.handle)
+    finally:
+        graph = stream.end_capture()
+    count = ctypes.c_size_t(0)
+    hip.check(L.hipGraphGetNodes(graph._handle, None, ctypes.byref(count)), "hipGraphGetNodes")
+    nodes = (ctypes.c_void_p * count.value)()
+    hip.check(L.hipGraphGetNodes(graph._handle, nodes, ctypes.byref(count)), "hipGraphGetNodes")
+    blocks = []
+    for node in nodes:
+        params = (ctypes.c_uint32 * 64)()   # hipKernelNodeParams, which starts with the block's dimensions
+        hip.check(L.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), params), "hipGraphKernelNodeGetParams")
+        blocks.append(params[0])
+    graph.close()
+    stream.close()
+    return blocks

@@ -288,7 +288,7 @@ def test_gate_up_swiglu_hands_on_packed_activations(gpu, tokens, out_dim, in_dim
 @pytest.mark.parametrize("t,tokens,in_dim,dims", [
     (Q4_K, 130, 512, [200, 96, 1000]), (Q4_K, 64, 4096, [4096, 1024, 1024, 12288, 12288]), (Q5_K, 9, 256, [7]),
     (Q5_K, 300, 768, [129, 128, 192, 193, 5, 640]), (Q4_K, 512, 4096, [4096, 1024, 1024]), (Q4_K, 33, 1024, [191, 385]),
-    (Q4_K, 2048, 512, [1024, 12288, 1024])])          # (the 12288-row member gets the eight-wavefront kernel, by itself)
+    (Q4_K, 2048, 512, [1024, 12288, 1024])])          # (the 12288-row member alone gets the eight-wavefront kernel, the list 192-row tiles)
 def test_lists_of_matrices_in_one_gemm(gpu, t, tokens, in_dim, dims):
     """cogni_gemm_packed_many_dev: up to six matrices of one type and row length against one packed activation block in one
     launch; every output bit for bit what cogni_gemm_packed_dev gives for that matrix alone without a k split (row counts that

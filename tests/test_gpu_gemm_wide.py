@@ -4,30 +4,43 @@ import numpy as np
 import pytest
 
 from cogni_ml_amd import quant, synth
-from gpu_common import DevArray, gpu  # noqa: F401
+from gpu_common import DevArray, gpu, launched_blocks  # noqa: F401
 from helpers import Q4_K, Q6_K
 from test_gpu_gemm import check, run_gemm
 
 pytestmark = pytest.mark.gpu
 
 
-# row counts whose 128-row tiles need two rounds of 256 workgroups and whose 256-row tiles need one; super-blocks odd and even
-@pytest.mark.parametrize("tokens,in_dim,dims", [(130, 256, [16001, 4101, 1000]), (255, 768, [8192, 8192 + 37]), (257, 512, [300, 7, 14000])])
-def test_lists(gpu, tokens, in_dim, dims, monkeypatch):
+# the first three: 192-row tiles in one round of 256 workgroups. The others: two rounds of those and of the 128-row ones, one of 256-row
+# tiles; whole and clipped tiles, a row count that is no multiple of four, matrices that end inside a tile, super-blocks odd and even
+@pytest.mark.parametrize("tokens,in_dim,dims,block", [
+    (130, 256, [16001, 4101, 1000], 256), (255, 768, [8192, 8192 + 37], 256), (257, 512, [300, 7, 14000], 256),
+    (255, 256, [24001, 4101, 1000], 512), (130, 768, [16384, 8192 + 37, 300], 512), (257, 512, [300, 7, 20000], 512)])
+def test_lists(gpu, tokens, in_dim, dims, block, monkeypatch):
     rng = np.random.default_rng(tokens)
     raws = [synth.make_weights(rng, Q4_K, d, in_dim) for d in dims]
     x = synth.make_activations(rng, tokens, in_dim)
     wsb = quant.gemm_workspace_bytes(Q4_K, in_dim, tokens)
     ws, xd, wd = DevArray(nbytes=wsb), DevArray(x), [DevArray(r) for r in raws]
-    one, lst = ([DevArray(np.full(tokens * d, np.float32(-3.0))) for d in dims] for _ in range(2))
+    outs = [[DevArray(np.full(tokens * d, np.float32(-3.0))) for d in dims] for _ in range(4)]
     quant.gemm_pack_dev(xd.ptr, Q4_K, in_dim, tokens, ws.ptr, wsb)
     monkeypatch.setenv("COGNI_GEMM_WIDE", "0")
-    for w, o, d in zip(wd, one, dims):
+    for w, o, d in zip(wd, outs[0], dims):
         quant.gemm_packed_dev(w.ptr, Q4_K, ws.ptr, wsb, o.ptr, in_dim, d, tokens)
-    quant.gemm_packed_many_dev([w.ptr for w in wd], Q4_K, ws.ptr, wsb, [o.ptr for o in lst], dims, in_dim, tokens)
-    for a, b, d in zip(one, lst, dims):
-        assert np.array_equal(a.read(np.float32, tokens * d), b.read(np.float32, tokens * d)), d
-    for a in [ws, xd] + wd + one + lst:
+    want = [o.read(np.float32, tokens * d) for o, d in zip(outs[0], dims)]
+    for knob, expect, out in (("0", 256, outs[1]), ("1", 512, outs[2]), (None, block, outs[3])):
+        if knob is None:
+            monkeypatch.delenv("COGNI_GEMM_WIDE")
+        else:
+            monkeypatch.setenv("COGNI_GEMM_WIDE", knob)
+
+        def issue(stream=None):
+            quant.gemm_packed_many_dev([w.ptr for w in wd], Q4_K, ws.ptr, wsb, [o.ptr for o in out], dims, in_dim, tokens, stream)
+        assert launched_blocks(issue) == [expect], knob
+        issue()
+        for o, a, d in zip(out, want, dims):
+            assert np.array_equal(o.read(np.float32, tokens * d), a), (knob, d)
+    for a in [ws, xd] + wd + sum(outs, []):
         a.close()
 
 
@@ -48,8 +61,14 @@ def test_gate_up_swiglu(gpu, tokens, out_dim, in_dim, next_type, monkeypatch):
         quant.gemm_packed_dev(w.ptr, Q4_K, ws.ptr, wsb, o.ptr, in_dim, out_dim, tokens)
     quant.swiglu_dev(g.ptr, u.ptr, o1.ptr, tokens * out_dim)
     quant.gemm_pack_dev(o1.ptr, next_type, out_dim, tokens, p1.ptr, nxb)
-    quant.gemm_packed_swiglu_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, o2.ptr, in_dim, out_dim, tokens)
-    quant.gemm_packed_swiglu_pack_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, o3.ptr, next_type, p2.ptr, nxb, in_dim, out_dim, tokens)
+
+    def issue(stream=None):
+        quant.gemm_packed_swiglu_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, o2.ptr, in_dim, out_dim, tokens, stream)
+        quant.gemm_packed_swiglu_pack_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, o3.ptr, next_type, p2.ptr, nxb, in_dim, out_dim, tokens, stream)
+    assert launched_blocks(issue) == [256, 256]
+    monkeypatch.delenv("COGNI_GEMM_WIDE")
+    assert launched_blocks(issue) == [512, 512]
+    issue()
     want = o1.read(np.float32, tokens * out_dim)
     assert np.array_equal(o2.read(np.float32, want.size), want)
     assert np.array_equal(o3.read(np.float32, want.size), want)
