@@ -199,7 +199,8 @@ def test_gemm_plan_picks_tile_and_split_for_the_shape():
     assert (name, gx, block) == ("q4_k_gemm_m64_f16", 64, 256) and gy == 4
     # (unsplit, 96 tiles of 128 rows spread over more compute units than 64 of 192)
     assert quant.gemm_plan(12, 4096, 12288, 64, quant.gemm_workspace_bytes(12, 4096, 64)) == ("q4_k_gemm_m64_n128_f16", 96, 1, 256)
-    # the eight-wavefront kernel is Q4_K's alone
+    # the eight-wavefront kernels: Q5_K has none, Q6_K's is taken where the 192-row tiles are not the better of the other two
+    assert quant.gemm_plan(14, 12288, 4096, 2048, big) == ("q6_k_gemm_wide_f16", 256, 1, 512)
     assert quant.gemm_plan(13, 4096, 12288, 2048, big)[0] == "q5_k_gemm_f16" and quant.gemm_plan(14, 4096, 12288, 2048, big)[0] == "q6_k_gemm_f16"
     with pytest.raises(quant.QuantError, match="Unsupported quant type"):
         quant.gemm_plan(8, 4096, 12288, 512, big)
@@ -412,8 +413,9 @@ def test_matrix_core_gemv_grid_covers_every_row():
 
 
 def test_gemm_tile_numbering_covers_every_tile_once():
-    """gemm_tile_of / gemm_grid_x (gemv_config.h) through a small C++ program: every tile of a launch is taken by exactly
-    one workgroup, and the workgroups that share an XCD side by side hold a compact block of tiles."""
+    """gemm_tile_of (gemv_config.h) through a small C++ program, over the grid the library launches (gemm_tiles_grid) and the larger one that
+    hosts launching by name are given (gemm_grid_x): every tile is taken by exactly one workgroup, no XCD gets more than its equal share, and
+    the workgroups that share an XCD side by side hold a compact block of tiles."""
     import subprocess
     import tempfile
     src = r'''
@@ -425,14 +427,19 @@ int main() {
   int bad = 0;
   for (unsigned mt = 1; mt <= 40; mt++)
     for (unsigned nt = 1; nt <= 130; nt += (nt < 70 ? 1 : 7)) {
-      const unsigned grid = gemm_grid_x(mt, nt);
-      std::set<std::pair<unsigned, unsigned>> seen;
-      for (unsigned id = 0; id < grid; id++) {
-        unsigned a, b;
-        if (!gemm_tile_of(id, mt, nt, &a, &b)) continue;
-        if (a >= mt || b >= nt || !seen.insert({a, b}).second) bad++;
+      if (gemm_tiles_grid(mt, nt) > gemm_grid_x(mt, nt) || gemm_tiles_grid(mt, nt) >= mt * nt + 8) bad++;
+      for (const unsigned grid : {gemm_tiles_grid(mt, nt), gemm_grid_x(mt, nt)}) {
+        std::set<std::pair<unsigned, unsigned>> seen;
+        unsigned share[8] = {};
+        for (unsigned id = 0; id < grid; id++) {
+          unsigned a, b;
+          if (!gemm_tile_of(id, mt, nt, &a, &b)) continue;
+          share[id % 8]++;
+          if (a >= mt || b >= nt || !seen.insert({a, b}).second) bad++;
+        }
+        for (const unsigned n : share) if (n > (mt * nt + 7) / 8) bad++;
+        if (seen.size() != (size_t)mt * nt || grid % 8 != 0 || grid > 8 * (mt * nt + 32 * 8)) bad++;
       }
-      if (seen.size() != (size_t)mt * nt || grid % 8 != 0 || grid > 8 * (mt * nt + 32 * 8)) bad++;
     }
   // 512 x 12288 in 128 x 192 tiles: the first 32 workgroups of XCD 0 hold 8 weight tiles x 4 token tiles
   std::set<unsigned> ms, ns;
