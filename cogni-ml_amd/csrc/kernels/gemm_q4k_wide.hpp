@@ -240,7 +240,7 @@ __device__ __forceinline__ void gemm_wide_core(const uint8_t* w, const uint4* xp
   const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const u32 nh = wave & 3, kh = wave >> 2;
   const u32 j = lane & 31, kg = lane >> 5;
-  const u32 nkb = in_dim >> 8;   // (no k split: the host takes this kernel only for launches of whole rounds of tiles)
+  const u32 nkb = in_dim >> 8;   // (no k split: the host takes these kernels only for launches that fill the chip without)
   const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM;
   const u32 ntiles = many ? many->tile_end[many->count - 1] : (out_dim + TILE_ROWS - 1) / TILE_ROWS;
   // workgroup -> tile, XCD-aware (see q4_k_gemm_f16)

@@ -2,8 +2,7 @@
 // operands of gemm_q6k.hpp (block layout, element order and assembly of the codes there).
 //
 //   q6_k_gemm_wide_f16 (w_raw, xp, bias|null, out:f32 [m][out_dim], in_dim:u32, out_dim:u32, m:u32, bias_stride:u32)
-//                      block 512, grid (gemm_grid_x(ceil(m/128), ceil(out_dim/256)), k splits), no dynamic LDS (112 KiB static);
-//                      with k splits > 1 `out` is `splits` planes of [m][out_dim] and bias is null, as for q6_k_gemm_f16
+//                      block 512, grid gemm_grid_x(ceil(m/128), ceil(out_dim/256)), no dynamic LDS (112 KiB static); no k split
 //
 // A workgroup owns 128 tokens x 256 rows; wavefront (row quarter nh, k half kh) accumulates 128 tokens x 64 rows over half
 // kh of every super-block and copies the bytes that it decodes itself, so no two wavefronts share weights. Those are, of each
@@ -29,14 +28,11 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const u32 nh = wave & 3, kh = wave >> 2;
   const u32 j = lane & 31, kg = lane >> 5;
-  // k split: super-blocks [kb0, kb0 + nkb) into plane blockIdx.y behind `out`
-  const u32 nkb_all = in_dim >> 8;
-  const u32 kb0 = blockIdx.y * nkb_all / gridDim.y, nkb = (blockIdx.y + 1) * nkb_all / gridDim.y - kb0;
-  out += (size_t)blockIdx.y * m * out_dim;
+  const u32 nkb = in_dim >> 8;
   const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM, ntiles = (out_dim + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN;
   u32 mt, nt;
   if (!gemm_tile_of(blockIdx.x, mtiles, ntiles, &mt, &nt)) return;
-  const size_t row_bytes = (size_t)nkb_all * BS;
+  const size_t row_bytes = (size_t)nkb * BS;
   // constants of the code assembly, kept in registers (as literals each (a & mask) | b would be two instructions): the masks
   // in scalar ones, of which an instruction takes one
   u32 mask_lo = 0x000F000Fu, mask_hi = 0x00F000F0u, magic_lo = 0x64006400u, magic_hi = 0x54005400u, m3_lo = 0x00300030u, m3_hi = 0x03000300u;
@@ -47,7 +43,7 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   const u32 base_row = min(row0, out_dim - 1);
   // loads through a buffer descriptor: scalar base, scalar offset of the super-block, a 32-bit offset per lane
   const __amdgpu_buffer_rsrc_t wrsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + (size_t)base_row * row_bytes + (size_t)kb0 * BS), 0, 0xFFFFFFFFu, 0x00027000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + (size_t)base_row * row_bytes), 0, 0xFFFFFFFFu, 0x00027000);
   // copy i of this wavefront: piece p = 64 i + lane is piece p % 6 of wave-local row p / 6
   u32 woff[6];
 #pragma unroll
@@ -60,7 +56,7 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   for (int c = 0; c < 2; c++) soff[c] = (min(row0 + 32 * c + j, out_dim - 1) - base_row) * (u32)row_bytes + 192u + 8u * kh;
   const u32 wrow = wave * 384 + j * 6 + kg;   // the lane's first ql piece of its row c = 0 (c = 1: 192 further)
   const __amdgpu_buffer_rsrc_t xrsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(xp + ((size_t)mt * nkb_all + kb0) * 4096), 0, 0xFFFFFFFFu, 0x00027000);
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(xp + (size_t)mt * nkb * 4096), 0, 0xFFFFFFFFu, 0x00027000);
 
   float16_t acc[4][2];
 #pragma unroll
