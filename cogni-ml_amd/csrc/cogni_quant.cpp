@@ -805,7 +805,7 @@ int cogni_gemv_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t x, cons
     aligned = aligned && (out_dims[i] % 16) == 0;
   }
   if (const uint32_t from = gemv_mt_multi_from(w_type, in_dim); from && count >= 2 && tokens >= from) {
-    // the one-pass kernel: one image for all of them, up to three matrices per launch
+    // the one-pass kernel: one image for all of them, up to three matrices per launch (Q4_K, Q5_K: six)
     int rc = 0;
     if (try_one_pass(w_raw, w_type, x, 0, out, out_dims, count, in_dim, tokens, from, stream, &rc)) return rc;
   }

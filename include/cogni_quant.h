@@ -151,9 +151,12 @@ int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residua
  *                           "q6_k_gemv_mt_f32" | "q8_0_gemv_mt_f32" (w0, w1, w2,
  *                           image, residual, out0, out1, out2, in_dim, rows0, rows1, rows2, tokens), block 512, up to three
  *                           matrices per launch as one matrix of all their rows (a matrix whose row count is not a multiple
- *                           of 16 ends its launch), geometry from cogni_gemv_packed_launch_dims. Four to six of Q4_K or Q5_K:
+ *                           of 16 ends its launch: the kernels take a tile of 16 rows from one matrix, so a host that launches
+ *                           by name has to end it there too), geometry from cogni_gemv_packed_launch_dims. Four to six of Q4_K or Q5_K:
  *                           "<type>_gemv_mt_list_f32" (six weight pointers, six output pointers, six row counts by value, image,
  *                           in_dim, tokens).
+ * Q6_K weights are copied as the aligned pieces of 16 bytes that hold a block: up to 15 bytes before the first and behind the last
+ * block of a matrix are read with them and not used (of an aligned piece that holds a byte of the matrix, so never of another page).
  * The image is caller-owned device memory; pack and GEMV are ordered by the stream. Accuracy: about 5e-7 of max|out|
  * (22-bit activations, exact weights, fp32 accumulation).
  * cogni_gemv_dev (from 3 to 5 tokens on, by type and row length), cogni_gemv_dual_dev and cogni_gemv_many_dev (2 tokens
@@ -190,9 +193,10 @@ int cogni_gemv_image_stats(uint32_t* slots, uint32_t* in_use, uint32_t* pinned, 
  * type or shape the call refuses. No GPU needed. */
 int32_t cogni_gemv_passes(uint32_t w_type, uint32_t tokens, uint32_t in_dim, uint32_t out_dim);
 /* Launch geometry of the one-pass kernel for a launch of total_rows rows (all its matrices together): a workgroup's eight
- * wavefronts carry t tiles of 16 rows at a time (in_dim above 4096: t = 1; else t = clamp(tiles / 256, 1, 3), Q6_K at most 2),
- * a row group is t tiles, grid_x = min(256, row groups) and the workgroups walk the groups blockIdx.x, blockIdx.x +
- * grid_x, ...; block_x = 512; shared_mem_bytes 122880 (Q4_K) or 135168 (Q6_K). No GPU needed. */
+ * wavefronts carry t tiles of 16 rows at a time (in_dim above 4096: t = 1; else the count, up to 3 or for Q6_K and Q8_0 up to 2, whose
+ * rounds take least: the kernel works it out from the row count), a row group is t tiles, grid_x = min(256, tiles of 16 rows) and the
+ * workgroups walk the groups blockIdx.x, blockIdx.x + grid_x, ... (one that has none leaves); block_x = 512; shared_mem_bytes 122880 (Q4_K)
+ * or 135168 (Q6_K). No GPU needed. */
 int cogni_gemv_packed_launch_dims(uint32_t w_type, uint32_t in_dim, uint32_t total_rows, uint32_t* grid_x, uint32_t* block_x,
                                   uint32_t* shared_mem_bytes);
 int cogni_gemv_pack_dev(uint64_t x, uint32_t w_type, uint32_t in_dim, uint32_t tokens, uint64_t image, void* stream);
@@ -430,10 +434,11 @@ int cogni_gemv_top1_noalloc_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uin
  *          grid from cogni_gemm_plan (whole blocks of 32 tiles of 128 x 192, 8 XCDs at a time), no dynamic shared memory; or, where
  *          tiles of 128 x 192 times the k split would leave compute units idle (the 4096-row projections at 512 tokens),
  *          q4_k_gemm_n128_f16 | q5_k_gemm_n128_f16 | q6_k_gemm_n128_f16 (same arguments and block, tiles of 128 x 128); or,
- *          for Q4_K launches that fill whole rounds of 128 x 256 tiles, q4_k_gemm_wide_f16 (same arguments), block 512.
+ *          for Q4_K and Q6_K launches without a k split whose rounds of 128 x 256 tiles cost least, q4_k_gemm_wide_f16 |
+ *          q6_k_gemm_wide_f16 (same arguments), block 512.
  *          Launches of up to 64 tokens take the forms of the 192- and 128-row kernels that work on the first 64 tokens of
  *          the token tile, <type>_gemm_m64_f16 | <type>_gemm_m64_n128_f16 (same arguments and block).
- *          cogni_gemm_plan says which, with the grid; all of them give the same bits for the same k split.
+ *          cogni_gemm_plan says which, with the grid and the block; all of them give the same bits for the same k split.
  * (pack_x_f16_*: block 256, grid ceil(tokens/128)*16*(in_dim/256).) Other types: COGNI_ERR_UNSUPPORTED_TYPE. */
 size_t cogni_gemm_workspace_bytes(uint32_t w_type, uint32_t in_dim, uint32_t tokens);
 /* The workspace size with which cogni_gemm_dev may also split the k range: a launch with fewer than 128 tiles of
@@ -473,7 +478,10 @@ int cogni_gemm_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias, u
  *                                 out_dim rows; the sums as cogni_gemm_packed_dev gives them, silu as swiglu_f32): the
  *                                 gate and up matrices never exist in memory. Kernel q4_k_gemm_swiglu_f16 (w_gate, w_up,
  *                                 workspace, out, in_dim, out_dim, tokens), block 256, grid as cogni_gemm_plan gives it
- *                                 for a matrix of 2 * out_dim rows. Other types: COGNI_ERR_UNSUPPORTED_TYPE. */
+ *                                 for a matrix of 2 * out_dim rows in 192-row tiles (96 rows of each matrix); or, where tiles of 128
+ *                                 rows of each cost less, q4_k_gemm_swiglu_wide_f16 (same arguments and bits), block 512, grid
+ *                                 at least the number of tiles rounded up to a multiple of 8. Other types:
+ *                                 COGNI_ERR_UNSUPPORTED_TYPE. */
 int cogni_gemm_packed_add_dev(uint64_t w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t residual, uint64_t out,
                               uint32_t in_dim, uint32_t out_dim, uint32_t tokens, void* stream);
 int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
@@ -484,7 +492,7 @@ int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
  * cogni_gemm_packed_dev gives for that matrix with a workspace that holds the packed activations only (no k split). One to
  * six matrices, Q4_K or Q5_K, no bias. Kernels "<type>_gemm_many[_m64][_n128]_f16", "q4_k_gemm_many_wide_f16" (list by value: six weight pointers, six
  * output pointers, six row counts, six cumulative tile counts, the count; workspace; in_dim:u32; tokens:u32), block 256 (wide: 512),
- * grid as cogni_gemm_plan gives it for a matrix of all the tiles. */
+ * grid at least the number of tiles (128 tokens x 192, 128 or 256 rows) rounded up to a multiple of 8. */
 int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
                                const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
 /* cogni_gemm_packed_swiglu_dev that also hands its products on as the packed activations of the GEMM behind it - the down
@@ -495,7 +503,8 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
  * not stored at all. out_dim a multiple of 256; next_workspace_bytes >= cogni_gemm_workspace_bytes(next_type, out_dim,
  * tokens) (with the k-split planes behind it if the next GEMM is to split: cogni_gemm_workspace_bytes_split); the two
  * workspaces must not overlap. Kernels q4_k_gemm_swiglu_pack_q4k_f16 | q4_k_gemm_swiglu_pack_q6k_f16 (w_gate, w_up,
- * workspace, out | 0, next_workspace, in_dim, out_dim, tokens), launched as q4_k_gemm_swiglu_f16. Up to 64 tokens go to the
+ * workspace, out | 0, next_workspace, in_dim, out_dim, tokens), launched as q4_k_gemm_swiglu_f16, and q4_k_gemm_swiglu_pack_q4k_wide_f16 |
+ * q4_k_gemm_swiglu_pack_q6k_wide_f16, launched as q4_k_gemm_swiglu_wide_f16. Up to 64 tokens go to the
  * kernels of the same names with `_m64` in front of `_f16` (q4_k_gemm_swiglu_m64_f16, q4_k_gemm_swiglu_pack_q4k_m64_f16, ...:
  * two tiles of 32 tokens per wavefront, the same parameters and bits). */
 int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
@@ -522,9 +531,10 @@ int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_
 int cogni_gemm_stream_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                       uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
                                       uint32_t out_dim, uint32_t tokens, void* stream);
-/* The launch cogni_gemm_packed_dev makes for a shape and a workspace of `workspace_bytes`: kernel name, grid (x: tiles,
- * y: k splits; with y > 1 gemm_sum_splits_f32 follows) and block, for hosts that launch by name (level 1) and for
- * callers who want to know which of the two Q4_K tilings a shape gets. Any out pointer may be null. The counterpart of
+/* The launch cogni_gemm_packed_dev makes for a shape and a workspace of `workspace_bytes`: kernel name, grid (x: tiles, rounded up
+ * to whole blocks - any grid of the tiles rounded up to a multiple of 8 or more does, the library itself launches that; y: k
+ * splits; with y > 1 gemm_sum_splits_f32 follows) and block, for hosts that launch by name (level 1) and for
+ * callers who want to know which tiling a shape gets. Any out pointer may be null. The counterpart of
  * cogni_gemv_plan; the reference picks its Metal prefill pipeline by type only (qwen35_metal.cr:11035). */
 int cogni_gemm_plan(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens, size_t workspace_bytes, const char** kernel,
                     uint32_t* grid_x, uint32_t* grid_y, uint32_t* block_x);
