@@ -554,7 +554,8 @@ typedef MtQ80T<true> MtQ80x16;
 // pieces of 16 bytes that hold it (15 from the last byte of such a piece), and the lanes read its fields at the block's shift, 0 to 15 bytes: a
 // copy from inside a dword takes the memory pipeline about twice as long, and a read of LDS from there costs more than that, so
 // the fields of a block that starts inside a dword (every other one) are put together from two dwords. Head of 151936 x 4096 at six
-// tokens with its norm and reduce, us: copied from the start as it lies 120.4, like this 112.5, without the shift of odd blocks (wrong) 104.
+// tokens with its norm and reduce, us: copied from the start as it lies 120.4, like this 112.5, without the shift of odd blocks (wrong) 104
+// (on other boxes 121.3 and 114.9, 123.7 and 120.8).
 // Every piece holds a byte of the block, so what is read beside it lies in the same 16 aligned bytes as one of the matrix's, never in
 // another page. A row in LDS is 15 pieces (240 bytes: rows 60 dwords apart hit 16 different bank groups); piece 14 is the one with the block's last
 // byte, mostly piece 13 again.
