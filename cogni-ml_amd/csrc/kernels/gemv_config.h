@@ -225,17 +225,22 @@ static inline unsigned gemv_mt_multi_from(unsigned type, unsigned in_dim) {
   return 4u * (in_dim >> 8) < 3u * gemv_mt_padded_sb(in_dim) ? 5u : 2u;
 }
 // tiles per wavefront: rows of more than 4096 values one (the operands are streamed); else the count, up to three (Q4_K, Q5_K) or
-// two (Q6_K, Q8_0: their units are larger), whose rounds of 256 workgroups take least. In hundredths of a us, 4096 columns of Q4_K:
-// one round 564 | 755 | 950, more of them 460 + 170 | 580 + 308 | 680 + 480 a round. Of the counts timed for the four types at 20 row counts of
-// 1024 to 4096 columns this takes the fastest or one within 3 %; as many tiles as keep 256 workgroups busy, the rule before, cost up to
-// 31 % more (Q4_K 16384 rows 15.0 us with three tiles, 11.4 with one; 10240 rows 11.0 with two, 8.9 with three; Q6_K 12288 rows 16.2 | 13.7).
-// Host and kernel use the same rule.
+// two (Q6_K, Q8_0: their units are larger), whose rounds of 256 workgroups take least. Up to 256 tiles one. Else, in hundredths of a us fitted
+// to launches of 906 to 151936 rows, weights from memory, for one | two | three tiles (one round of two | three: 755 | 950, 392 | 468, 510):
+// 460 + 170 | 580 + 308 | 680 + 480 a round, rows of up to 2048 values of Q4_K and Q5_K 292 + 113 | 291 + 190 | 309 + 254, up to 1024 of Q6_K and Q8_0
+// 302 + 160 | 380 + 270: the shorter a row, the more a round's start and end weigh. As many tiles as keep 256 workgroups busy, the first rule, cost up to
+// 33 % more (Q4_K 4096 -> 16384 15.0 us with three tiles, 11.4 with one; -> 10240 11.0 with two, 8.9 with three), the long rows' line for all up to 19 %
+// more than that where rows are short (Q4_K 1024 -> 24576 8.0 with three, 9.5 with one; Q8_0 1024 -> 13386 8.1 | 8.9). This takes at most 3 % more than
+// the first rule (Q4_K 1024 -> 24576 at sixteen tokens 8.5 | 8.7), all told 7 % less. Host and kernel use the same rule.
 static inline GEMV_HD unsigned gemv_mt_tiles(unsigned type, unsigned in_dim, unsigned ntiles) {
-  if (in_dim > 4096u) return 1;
+  if (in_dim > 4096u || ntiles <= 256u) return 1;
+  const int two = type == 14 || type == 8;
   const unsigned r1 = (ntiles + 255u) / 256u, r2 = ((ntiles + 1u) / 2u + 255u) / 256u, r3 = ((ntiles + 2u) / 3u + 255u) / 256u;
-  const unsigned c1 = r1 <= 1u ? 564u : 460u + 170u * r1, c2 = r2 <= 1u ? 755u : 580u + 308u * r2, c3 = r3 <= 1u ? 950u : 680u + 480u * r3;
-  const int three = type != 14 && type != 8 && c3 < c1 && c3 < c2;
-  return three ? (unsigned)GEMV_MT_TMAX : (c2 < c1 ? 2u : 1u);
+  unsigned c1 = 460u + 170u * r1, c2 = r2 <= 1u ? 755u : 580u + 308u * r2, c3 = r3 <= 1u ? 950u : 680u + 480u * r3;
+  if (two && in_dim <= 1024u) c1 = 302u + 160u * r1, c2 = r2 <= 1u ? 510u : 380u + 270u * r2;
+  if (!two && in_dim <= 2048u)
+    c1 = 292u + 113u * r1, c2 = r2 <= 1u ? 392u : 291u + 190u * r2, c3 = r3 <= 1u ? 468u : 309u + 254u * r3;
+  return !two && c3 < c1 && c3 < c2 ? (unsigned)GEMV_MT_TMAX : (c2 < c1 ? 2u : 1u);
 }
 // One workgroup per compute unit at most; they walk the row groups (a workgroup that has none leaves at once).
 static inline GEMV_HD unsigned gemv_mt_grid(unsigned type, unsigned in_dim, unsigned total_rows) {

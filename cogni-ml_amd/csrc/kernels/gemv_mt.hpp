@@ -559,15 +559,21 @@ typedef MtQ80T<true> MtQ80x16;
 // Every piece holds a byte of the block, so what is read beside it lies in the same 16 aligned bytes as one of the matrix's, never in
 // another page. A row in LDS is 15 pieces (240 bytes: rows 60 dwords apart hit 16 different bank groups); piece 14 is the one with the block's last
 // byte, mostly piece 13 again.
+// SHIFT false: copied from exactly its start, the fields at their natural alignment, piece 13 shifted back to the block's last sixteen
+// bytes (d at byte 222) and piece 14 again. The better form for rows of up to 4096 values that are no multiple of 2048 (16 bytes) and for longer
+// ones of an odd number of blocks: there a block's shift changes from row to row, and every wavefront puts fields together. us, copied from
+// its start | as aligned pieces (gemv_mt_from_start), 6 tokens, weights from memory: 1536 -> 8192 5.7 | 6.4, -> 24576 12.6 | 14.4, 3328 -> 4096 6.3 | 7.1, -> 16384 16.2 | 17.4,
+// 5888 -> 2048 7.0 | 7.9, 7936 -> 906 8.3 | 9.0; but 4096 -> 20480 21.7 | 18.9, 2048 -> 151936 62.9 | 56.4, 5632 -> 16384 29.9 | 28.2, 12288 -> 16384 56.0 | 52.2.
 // (X16: sixteen single-term tokens, as MtK45's)
-template <bool X16 = false>
+template <bool X16 = false, bool SHIFT = true>
 struct MtQ6KT {
   static constexpr int NTOK = X16 ? 16 : 8;
   static constexpr unsigned TYPE = 14;
   static constexpr int BB = 210, P = 15, NCOPY = 4, LAST = 16 * P - 192, NAUX = 1, NSLOT = 4, TMAX = 2;
-  static constexpr bool SHIFTED = true;
+  static constexpr bool SHIFTED = SHIFT;
+  typedef MtQ6KT<X16, false> FromStart;
   static constexpr u32 UNIT_BYTES = 16 * P * 16, AUX_SB_BYTES = 64 * 16;
-  static __device__ __forceinline__ u32 piece_offset(u32 piece) { return min(piece * 16, 209u); }
+  static __device__ __forceinline__ u32 piece_offset(u32 piece) { return SHIFT ? min(piece * 16, 209u) : (piece < 13 ? piece * 16 : 194u); }
   static __device__ __forceinline__ u32 aux_offset(u32 lane) { return lane * 16; }   // 16 bytes of its own per lane
 
   // the scales of the lane's two tokens and, as the matrix-core operand of lane (kg, row), the sums of sub-blocks
@@ -609,6 +615,11 @@ struct MtQ6KT {
     return w;
   }
   static __device__ __forceinline__ Raw read(const char* start, u32 kg) {
+    if constexpr (!SHIFT) {
+      Raw w = fields<false>(start, kg, 0);
+      w.d = *reinterpret_cast<const unsigned short*>(start + 222);
+      return w;
+    }
     const u32 sh = (u32)(uintptr_t)start & 3u;
     if (__builtin_amdgcn_ballot_w64(sh != 0) == 0) return fields<false>(start, kg, 0);
     Raw w = fields<true>(start - sh, kg, sh);
@@ -1066,25 +1077,51 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
 // The tile count per wavefront follows from the row count (gemv_mt_tiles, the rule the host sizes the grid with); tile
 // count and super-blocks per k-slice are template parameters so that register use and loads in flight are compile-time
 // constants. Shapes outside gemv_mt_supported() must not be launched.
+// Rows whose blocks the format copies from their start (MtQ6KT). Of 2048 values also where there are up to 1280 tiles: 4096 rows 4.2 | 4.4 us,
+// 6144 5.3 | 5.5, 20480 11.3 | 11.4, but 32000 16.0 | 15.3.
+template <class F, int SBW>
+__device__ __forceinline__ bool gemv_mt_from_start(u32 in_dim, u32 ntiles) {
+  return F::SHIFTED && ((in_dim & (SBW <= 2 ? 2047u : 511u)) != 0 || (SBW == 1 && ntiles <= 1280u));
+}
+// one tile per wavefront
+template <class F, int SBW, bool TOP1, int N>
+__device__ __forceinline__ void gemv_mt_single(const MtArgs<N>& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens,
+                                               u32* top_ids = nullptr, float* logits = nullptr, u32 bid = blockIdx.x, u32 nwg = gridDim.x) {
+  if constexpr (F::SHIFTED) {
+    if (gemv_mt_from_start<F, SBW>(in_dim, (a.total() + 15) >> 4))
+      return gemv_mt_core<typename F::FromStart, SBW, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits, nullptr, bid, nwg);
+  }
+  gemv_mt_core<F, SBW, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits, nullptr, bid, nwg);
+}
+template <class F, int SBW, bool TOP1, int N>
+__device__ __forceinline__ void gemv_mt_tiled(const MtArgs<N>& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens, u32* top_ids,
+                                              float* logits, u32 t) {
+  if (t <= 1) gemv_mt_core<F, SBW, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+  else if (t == 2) gemv_mt_core<F, SBW, 2, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+  else if constexpr (F::TMAX >= 3) gemv_mt_core<F, SBW, 3, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
+}
+template <class F, int SBW, bool TOP1, int N>
+__device__ __forceinline__ void gemv_mt_resident(const MtArgs<N>& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens, u32* top_ids,
+                                                 float* logits) {
+  const u32 ntiles = (a.total() + 15) >> 4, t = gemv_mt_tiles(F::TYPE, in_dim, ntiles);
+  if constexpr (F::SHIFTED) {
+    if (gemv_mt_from_start<F, SBW>(in_dim, ntiles)) return gemv_mt_tiled<typename F::FromStart, SBW, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits, t);
+  }
+  gemv_mt_tiled<F, SBW, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits, t);
+}
 template <class F, bool TOP1 = false, int N = 3>
 __device__ __forceinline__ void gemv_mt_dispatch(const MtArgs<N>& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens,
                                                  u32* top_ids = nullptr, float* logits = nullptr) {
-  const u32 t = gemv_mt_tiles(F::TYPE, in_dim, (a.total() + 15) >> 4);
+  // (All arguments in one load: those that are first used behind the branches below would be waited for a second time there. 4096 ->
+  // 4096 of Q4_K, six tokens, 5.4 us with two waits, 5.1 with one.)
+  asm volatile("" : "+s"(in_dim), "+s"(tokens) : "s"(image), "s"(residual), "s"(a.w[0]), "s"(a.out[0]), "s"(a.rows[0]));
   switch (gemv_mt_padded_sb(in_dim) >> 3) {
-    case 1:
-      if (t <= 1) gemv_mt_core<F, 1, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if (t == 2) gemv_mt_core<F, 1, 2, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 1, 3, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
-      break;
-    case 2:
-      if (t <= 1) gemv_mt_core<F, 2, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if (t == 2) gemv_mt_core<F, 2, 2, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
-      else if constexpr (F::TMAX >= 3) gemv_mt_core<F, 2, 3, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits);
-      break;
-    case 3: gemv_mt_core<F, 3, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
-    case 4: gemv_mt_core<F, 4, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
-    case 5: gemv_mt_core<F, 5, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
-    default: gemv_mt_core<F, 6, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 1: gemv_mt_resident<F, 1, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 2: gemv_mt_resident<F, 2, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 3: gemv_mt_single<F, 3, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 4: gemv_mt_single<F, 4, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    case 5: gemv_mt_single<F, 5, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
+    default: gemv_mt_single<F, 6, TOP1, N>(a, image, residual, in_dim, tokens, top_ids, logits); break;
   }
 }
 
@@ -1126,12 +1163,12 @@ __device__ __forceinline__ void gemv_mt_one_tile(const uint8_t* w, const uint8_t
                                                  u32 nwg) {
   const MtArgs<1> a = {{w}, {out}, {rows}};
   switch (gemv_mt_padded_sb(in_dim) >> 3) {
-    case 1: gemv_mt_core<F, 1, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
-    case 2: gemv_mt_core<F, 2, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
-    case 3: gemv_mt_core<F, 3, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
-    case 4: gemv_mt_core<F, 4, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
-    case 5: gemv_mt_core<F, 5, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
-    default: gemv_mt_core<F, 6, 1, false, false, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, nullptr, bid, nwg); break;
+    case 1: gemv_mt_single<F, 1, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, bid, nwg); break;
+    case 2: gemv_mt_single<F, 2, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, bid, nwg); break;
+    case 3: gemv_mt_single<F, 3, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, bid, nwg); break;
+    case 4: gemv_mt_single<F, 4, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, bid, nwg); break;
+    case 5: gemv_mt_single<F, 5, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, bid, nwg); break;
+    default: gemv_mt_single<F, 6, false, 1>(a, image, nullptr, in_dim, tokens, nullptr, nullptr, bid, nwg); break;
   }
 }
 #define GEMV_MT_TWO_ENTRY(NAME, FMT_A, FMT_B)                                                                                     \

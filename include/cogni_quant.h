@@ -155,7 +155,7 @@ int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residua
  *                           by name has to end it there too), geometry from cogni_gemv_packed_launch_dims. Four to six of Q4_K or Q5_K:
  *                           "<type>_gemv_mt_list_f32" (six weight pointers, six output pointers, six row counts by value, image,
  *                           in_dim, tokens).
- * Q6_K weights are copied as the aligned pieces of 16 bytes that hold a block: up to 15 bytes before the first and behind the last
+ * Q6_K weights may be copied as the aligned pieces of 16 bytes that hold a block: up to 15 bytes before the first and behind the last
  * block of a matrix are read with them and not used (of an aligned piece that holds a byte of the matrix, so never of another page).
  * The image is caller-owned device memory; pack and GEMV are ordered by the stream. Accuracy: about 5e-7 of max|out|
  * (22-bit activations, exact weights, fp32 accumulation).

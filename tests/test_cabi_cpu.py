@@ -348,6 +348,30 @@ def test_one_pass_geometry_and_thresholds():
             quant.gemv_packed_launch_dims(*bad)
 
 
+def test_tiles_per_wavefront_are_among_the_fastest():
+    """gemv_mt_tiles (gemv_config.h) against times of the one-pass kernels with one, two and three tiles per wavefront (MI355X, us, 6 tokens,
+    weights from memory): never more than 5 % behind the fastest, one tile up to 256 of them and for rows of more than 4096 values."""
+    import subprocess
+    import tempfile
+    timed = [(12, 1024, 13386, 6.76, 6.14, 7.42), (12, 1024, 24576, 9.50, 8.39, 8.12), (12, 1024, 44000, 14.94, 13.65, 12.90),
+             (12, 1024, 151936, 43.16, 36.51, 33.64), (12, 1536, 24576, 9.54, 8.81, 8.96), (12, 2048, 44000, 14.82, 14.54, 14.28),
+             (13, 1024, 24576, 10.71, 9.71, 9.93), (13, 1536, 151936, 50.68, 44.49, 42.77), (14, 1024, 13386, 8.54, 8.61), (14, 1024, 24576, 12.54, 12.33),
+             (14, 1536, 10240, 7.65, 9.14), (14, 1536, 64000, 28.16, 26.87), (14, 3328, 20480, 18.38, 20.73), (14, 4096, 151936, 105.21, 101.09),
+             (8, 1024, 24576, 11.50, 10.84), (8, 1536, 16384, 8.92, 9.74), (8, 3328, 8192, 10.54, 9.85)]
+    src = '#include <cstdio>\n#include "gemv_config.h"\nint main() { unsigned t, k, r; while (std::scanf("%u %u %u", &t, &k, &r) == 3) ' \
+          'std::printf("%u\\n", gemv_mt_tiles(t, k, (r + 15) / 16)); }'
+    asked = [c[:3] for c in timed] + [(t, k, r) for t in (8, 12, 13, 14) for k, r in ((1024, 4096), (4096, 4096), (4352, 151936))]
+    with tempfile.TemporaryDirectory() as d:
+        open(os.path.join(d, "t.cpp"), "w").write(src)
+        subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "cogni-ml_amd", "csrc", "kernels"), "-o", os.path.join(d, "t"),
+                        os.path.join(d, "t.cpp")], check=True)
+        picks = subprocess.run([os.path.join(d, "t")], input="\n".join("%d %d %d" % c for c in asked), capture_output=True, text=True, check=True)
+    picks = [int(p) for p in picks.stdout.split()]
+    for c, t in zip(timed, picks):
+        assert c[2 + t] <= 1.05 * min(c[3:]), (c, t)
+    assert picks[len(timed):] == [1] * 12
+
+
 def test_one_pass_argument_errors_do_not_need_a_gpu():
     assert hip.lib().cogni_gemv_release_stream(None) == 0          # a stream without an image: nothing to do
     with pytest.raises(quant.QuantError, match="no one-pass kernel") as e:

@@ -4,7 +4,7 @@ import pytest
 
 from cogni_ml_amd import quant, synth
 from gpu_common import DevArray, gpu  # noqa: F401
-from helpers import Q4_K, Q5_K, Q6_K
+from helpers import Q4_K, Q5_K, Q6_K, Q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -180,4 +180,30 @@ def test_q6_k_blocks_at_every_shift(gpu, oracle, first, in_dim):
     tol = 1e-4 * np.linalg.norm(x.reshape(tokens, -1), axis=1).max() * np.abs(oracle.dequantize(raw, Q6_K, out_dim * in_dim)).max()
     assert np.abs(got - want).max() <= tol and np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
     for d in (w, xd, image, od):
+        d.close()
+
+
+# row counts on both sides of the rule's lines: one tile in several rounds, two and three tiles, a last group that is not full
+@pytest.mark.parametrize("rows", [4097, 8200, 13386, 24577])
+@pytest.mark.parametrize("t,in_dim", [(Q4_K, 1024), (Q5_K, 1536), (Q6_K, 768), (Q6_K, 1024), (Q6_K, 2048), (Q6_K, 3328), (Q8_0, 1024)])
+def test_rows_do_not_depend_on_the_tiles_per_wavefront(gpu, t, in_dim, rows):
+    """Every row as from launches of up to 256 tiles of 16 rows, which take one tile per wavefront; up to eight tokens and sixteen."""
+    rng = np.random.default_rng(rows + in_dim)
+    raw = synth.make_weights(rng, t, rows, in_dim)
+    row_bytes, part = len(raw) // rows, 4096
+    w, x = DevArray(raw), DevArray(synth.make_activations(rng, 13, in_dim))
+    image = DevArray(nbytes=quant.gemv_image_bytes(t, in_dim, 8))
+    for tokens, pack, gemv in ((7, quant.gemv_pack_dev, quant.gemv_packed_dev), (13, quant.gemv_pack16_dev, quant.gemv_packed16_dev)):
+        out = DevArray(np.full(tokens * rows, np.nan, np.float32))
+        pack(x.ptr, t, in_dim, tokens, image.ptr)
+        gemv([w.ptr], t, image.ptr, [out.ptr], [rows], in_dim, tokens)
+        got = out.read(np.float32, tokens * rows).reshape(tokens, rows)
+        for r0 in range(0, rows, part):
+            n = min(part, rows - r0)
+            piece = DevArray(np.full(tokens * n, np.nan, np.float32))
+            gemv([w.ptr + r0 * row_bytes], t, image.ptr, [piece.ptr], [n], in_dim, tokens)
+            assert np.array_equal(piece.read(np.float32, tokens * n).reshape(tokens, n), got[:, r0:r0 + n]), r0
+            piece.close()
+        out.close()
+    for d in (w, x, image):
         d.close()
