@@ -231,7 +231,7 @@ static inline unsigned gemv_mt_multi_from(unsigned type, unsigned in_dim) {
 // 302 + 160 | 380 + 270: the shorter a row, the more a round's start and end weigh. As many tiles as keep 256 workgroups busy, the first rule, cost up to
 // 33 % more (Q4_K 4096 -> 16384 15.0 us with three tiles, 11.4 with one; -> 10240 11.0 with two, 8.9 with three), the long rows' line for all up to 19 %
 // more than that where rows are short (Q4_K 1024 -> 24576 8.0 with three, 9.5 with one; Q8_0 1024 -> 13386 8.1 | 8.9). This takes at most 3 % more than
-// the first rule (Q4_K 1024 -> 24576 at sixteen tokens 8.5 | 8.7), all told 7 % less. Host and kernel use the same rule.
+// the first rule (Q4_K 1024 -> 24576 at sixteen tokens 8.5 | 8.7), all told 5 % less. Host and kernel use the same rule.
 static inline GEMV_HD unsigned gemv_mt_tiles(unsigned type, unsigned in_dim, unsigned ntiles) {
   if (in_dim > 4096u || ntiles <= 256u) return 1;
   const int two = type == 14 || type == 8;

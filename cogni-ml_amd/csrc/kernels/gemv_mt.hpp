@@ -1078,17 +1078,20 @@ __device__ __forceinline__ void gemv_mt_core(const MtArgs<N>& a, const uint8_t* 
 // count and super-blocks per k-slice are template parameters so that register use and loads in flight are compile-time
 // constants. Shapes outside gemv_mt_supported() must not be launched.
 // Rows whose blocks the format copies from their start (MtQ6KT). Of 2048 values also where there are up to 1280 tiles: 4096 rows 4.2 | 4.4 us,
-// 6144 5.3 | 5.5, 20480 11.3 | 11.4, but 32000 16.0 | 15.3.
-template <class F, int SBW>
+// 6144 5.3 | 5.5, 20480 11.3 | 11.4, but 32000 16.0 | 15.3; of more than 4096 in a single round of workgroups of a launch of
+// their own (PAIR: beside another matrix) for up to eight tokens: a pass of 12288 -> 4096 at eight with its pack launch 15.1 | 15.6; but the stack's o and
+// down as one launch at eight 49.0 | 48.6, the FFN block at thirteen 34.2 | 33.9.
+template <class F, int SBW, bool PAIR = false>
 __device__ __forceinline__ bool gemv_mt_from_start(u32 in_dim, u32 ntiles) {
-  return F::SHIFTED && ((in_dim & (SBW <= 2 ? 2047u : 511u)) != 0 || (SBW == 1 && ntiles <= 1280u));
+  return F::SHIFTED && ((in_dim & (SBW <= 2 ? 2047u : 511u)) != 0 || (SBW == 1 && ntiles <= 1280u) ||
+                        (SBW > 2 && F::NTOK == 8 && !PAIR && ntiles <= 256u));
 }
 // one tile per wavefront
 template <class F, int SBW, bool TOP1, int N>
 __device__ __forceinline__ void gemv_mt_single(const MtArgs<N>& a, const uint8_t* image, const float* residual, u32 in_dim, u32 tokens,
                                                u32* top_ids = nullptr, float* logits = nullptr, u32 bid = blockIdx.x, u32 nwg = gridDim.x) {
   if constexpr (F::SHIFTED) {
-    if (gemv_mt_from_start<F, SBW>(in_dim, (a.total() + 15) >> 4))
+    if (gemv_mt_from_start<F, SBW, N == 1>(in_dim, (a.total() + 15) >> 4))   // (a list of one: gemv_mt_one_tile)
       return gemv_mt_core<typename F::FromStart, SBW, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits, nullptr, bid, nwg);
   }
   gemv_mt_core<F, SBW, 1, false, TOP1, false, N>(a, image, residual, in_dim, tokens, top_ids, logits, nullptr, bid, nwg);
