@@ -20,10 +20,12 @@
 // IQ4_NL, 64 tokens: 34 us against 18.7; with four steps in flight instead of one 40), so a wavefront loads its steps with
 // neighbouring lanes on neighbouring bytes of a row, up to two ahead, and turns them through a region of LDS that no other
 // wavefront uses: no barrier in the loop.
-// What bounds it: small calls the chain load - LDS - sums (4 us), large ones no single unit. Q8_0 1024 -> 3584, 200 tokens, 14.7 us:
-// 3900 vector instructions per working SIMD (6.8 us; two fifths of them split x, 6.5 per value and 64 rows, one of them the scale: 14.2 us
-// without it), 2.7 us of matrix instructions, and two wavefronts per SIMD that wait 36 % of their time for loads and LDS and 31 % for
-// an issue slot.
+// What bounds it: small calls the chain load - LDS - sums (4 us), large ones the issue slots of a SIMD: Q8_0 4096 -> 4096, 256 tokens, 13300
+// instructions per SIMD, 82 % of its cycles, where a kernel without any load still takes 36 of the 42 us and one without the splitting of
+// x 39. A matrix instruction takes 7 to 8 clocks of issue, but its sum is there only 16 clocks later: the products of a token tile go out row tile by
+// row tile (TN independent sums), with the next tile's terms and the last one's sums in between, instead of one sum after the other: Q8_0 1024 ->
+// 3584, 200 tokens 15.1 -> 14.6 us, 4096 -> 4096, 256 tokens 43.5 -> 42.3; F16 2048 -> 2048, 33 tokens 8.65 -> 8.45; F32 4096 -> 4096, 256 tokens 79 -> 72.
+// Splitting by v_cvt_pk_bf16_f32 and v_dot2_f32_bf16, half the instructions, gained nothing: the second takes twice as long.
 // Measured, weights from memory, row kernels (Q8_0: one-pass launches of eight tokens) -> these: Q8_0 1024 -> 3584, 9 / 48 / 200
 // tokens 9.6 / 35 / 143 -> 5.0 / 7.8 / 15.4 us; F16 2048 -> 2048, 33 tokens 41.8 -> 9.1; F32 4096 -> 4096, 33 tokens 174 -> 26; IQ4_NL
 // 4096 -> 4096, 1 / 64 tokens 40 / 1926 -> 10.5 / 21.
@@ -315,34 +317,63 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
     for (int t = 0; t < TM; t++) r.x[t].put(mine + t * XD, lane);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the lanes read what other lanes of the wavefront wrote
   };
+  // One step. Token tile t's matrix instructions go out term product by term product across the TN row tiles (TN independent sums: one
+  // after the other the three to eight of a sum wait for each other), with tile t + 1's terms and tile t - 1's sums made in between.
   auto compute = [&]() {
-    bf16x8_t X[TM][3];
-#pragma unroll
-    for (int t = 0; t < TM; t++) {
-      float v[8];
-      TermsF32Tile::get(mine + t * XD, lane, v);
-      terms_split<3>(v, X[t]);
-    }
+    constexpr bool AHEAD = W::TERMS == 1 || TM < 4;   // room for two sets of terms of x
+    constexpr int XB = AHEAD ? 2 : 1;
+    bf16x8_t B[TN][W::TERMS], X[XB][3];
+    float d[TN];
+    terms_f4 p[2][TN];
+    float v[8];
+    TermsF32Tile::get(mine, lane, v);
+    if constexpr (TM * TN == 1) terms_split<3>(v, X[0]);
 #pragma unroll
     for (int c = 0; c < TN; c++) {
       const u32* wl = mine + TM * XD + c * W::LDS_DWORDS;
-      bf16x8_t B[W::TERMS];
-      W::terms(wl, lane, B);
-      const float d = W::scale(wl, lane);
+      W::terms(wl, lane, B[c]);
+      d[c] = W::scale(wl, lane);
+    }
+    if constexpr (TM * TN > 1) terms_split<3>(v, X[0]);
+    auto fold = [&](int t) {   // the sum over the step's 32 values joins the running sum in one rounding
 #pragma unroll
-      for (int t = 0; t < TM; t++) {
-        // term i of x against term j of w, i + j <= 3, smallest first; the sum over the step's 32 values joins the running sum
-        // in one rounding
-        terms_f4 p = {0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < TN; c++)
 #pragma unroll
-        for (int ij = 3; ij >= 0; ij--)
+        for (int e = 0; e < 4; e++) acc[t][c][e] = W::SCALED ? fmaf(d[c], p[t & 1][c][e], acc[t][c][e]) : acc[t][c][e] + p[t & 1][c][e];
+    };
 #pragma unroll
-          for (int j = 0; j < W::TERMS; j++)
-            if (ij - j >= 0 && ij - j < 3) p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t][ij - j], B[j], p, 0, 0, 0);
+    for (int t = 0; t < TM; t++) {
+      if (TM > 1) __builtin_amdgcn_sched_barrier(0);
+      if (AHEAD && t + 1 < TM) TermsF32Tile::get(mine + (t + 1) * XD, lane, v);
+      if (!AHEAD && t > 0) {
+        TermsF32Tile::get(mine + t * XD, lane, v);
+        terms_split<3>(v, X[0]);
+      }
 #pragma unroll
-        for (int v = 0; v < 4; v++) acc[t][c][v] = W::SCALED ? fmaf(d, p[v], acc[t][c][v]) : acc[t][c][v] + p[v];
+      for (int c = 0; c < TN; c++) p[t & 1][c] = terms_f4{0.f, 0.f, 0.f, 0.f};
+      // term i of x against term j of w, i + j <= 3, smallest first
+#pragma unroll
+      for (int ij = 3; ij >= 0; ij--)
+#pragma unroll
+        for (int j = 0; j < W::TERMS; j++)
+          if (ij - j >= 0 && ij - j < 3) {
+#pragma unroll
+            for (int c = 0; c < TN; c++) p[t & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t % XB][ij - j], B[c][j], p[t & 1][c], 0, 0, 0);
+          }
+      if (AHEAD && t + 1 < TM) terms_split<3>(v, X[(t + 1) % XB]);
+      if (t > 0) fold(t - 1);
+      if (AHEAD && TM > 1) {
+        constexpr int MFMAS = TN * (W::TERMS == 1 ? 3 : (W::TERMS == 2 ? 6 : 8)), VALU = (72 + 4 * TN + MFMAS - 1) / MFMAS;
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+        for (int i = 0; i < MFMAS; i++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+        }
       }
     }
+    if (TM > 1) __builtin_amdgcn_sched_barrier(0);
+    fold(TM - 1);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   };
   // whole steps: contiguous runs of them per wavefront; a last step that the row ends inside is added by the last wavefront
