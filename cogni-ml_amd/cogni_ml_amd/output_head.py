@@ -42,8 +42,8 @@ class QwenOutputHeadRunner:
         self._logits = self._alloc(4 * tokens * self.vocab) if read_logits else None
         # token groups that go through the one-pass kernel: the norm writes that kernel's activation image itself
         t = weights.output_type
-        self._from = quant.gemv_one_pass_from(t, self.hidden, self.vocab) if int(t) in (12, 14) and self.hidden <= 4096 else 0
-        self._image = self._alloc(quant.gemv_image_bytes(t, self.hidden, quant.MAX_GEMV_TOKENS)) if self._from else None
+        self._packed = [n > 0 and quant.gemv_top1_one_pass(t, n, self.hidden, self.vocab, read_logits) for n in range(self.GROUP + 1)]
+        self._image = self._alloc(quant.gemv_image_bytes(t, self.hidden, quant.MAX_GEMV_TOKENS)) if any(self._packed) else None
         self.top1_ids = np.zeros(tokens, dtype=np.int32)
         self.top1_values = np.zeros(tokens, dtype=np.float32)
         self.logits = None
@@ -76,7 +76,7 @@ class QwenOutputHeadRunner:
         h, t = self.hidden, self.weights.output_type
         normed = self._normed.ptr + 4 * tok0 * h
         lg = self._logits.ptr + 4 * tok0 * self.vocab if self._logits is not None else 0   # stored by the pass that finds the top-1
-        packed = self._from and count >= self._from
+        packed = self._packed[count]
         if packed:
             quant.rmsnorm_pack_dev(self._x.ptr + 4 * tok0 * h, self._norm.ptr, 0, t, self._image.ptr, h, count, self.eps, st)
         else:

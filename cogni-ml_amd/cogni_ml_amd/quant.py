@@ -100,6 +100,12 @@ def gemv_one_pass_multi_from(w_type, in_dim):
     return int(f(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(in_dim)))
 
 
+def gemv_top1_one_pass(w_type, tokens, in_dim, out_dim, logits=False):
+    """Whether the norm that writes the image and the one-pass kernel are the faster way for an output head of `tokens` tokens."""
+    return bool(hip.lib().cogni_gemv_top1_one_pass(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(tokens), ctypes.c_uint32(in_dim),
+                                                   ctypes.c_uint32(out_dim), ctypes.c_int32(bool(logits))))
+
+
 def gemv_image_stats():
     """(slots, in use, pinned by a capture, multi-token calls that found no slot) of the library's activation images."""
     a, b, c, d = ctypes.c_uint32(), ctypes.c_uint32(), ctypes.c_uint32(), ctypes.c_uint64()

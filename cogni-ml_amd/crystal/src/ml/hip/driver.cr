@@ -57,6 +57,7 @@ lib LibCogniHIP
   fun cogni_gemv_plan(type : UInt32, tokens : UInt32, add : Int32, in_dim : UInt32, out_dim : UInt32, kernel : UInt8**,
                       grid_x : UInt32*, block_x : UInt32*, shared_mem_bytes : UInt32*) : Int32
   fun cogni_gemv_one_pass_from(w_type : UInt32, in_dim : UInt32, out_dim : UInt32) : UInt32
+  fun cogni_gemv_top1_one_pass(w_type : UInt32, tokens : UInt32, in_dim : UInt32, out_dim : UInt32, logits : Int32) : Int32
   fun cogni_gemv_one_pass_multi_from(w_type : UInt32, in_dim : UInt32) : UInt32
   fun cogni_gemv_passes(w_type : UInt32, tokens : UInt32, in_dim : UInt32, out_dim : UInt32) : Int32
   fun cogni_gemv_image_stats(slots : UInt32*, in_use : UInt32*, pinned : UInt32*, calls_without_image : UInt64*) : Int32

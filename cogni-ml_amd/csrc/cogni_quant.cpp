@@ -334,6 +334,9 @@ size_t cogni_gemv_image_bytes(uint32_t w_type, uint32_t in_dim, uint32_t tokens)
 }
 
 uint32_t cogni_gemv_one_pass_from(uint32_t w_type, uint32_t in_dim, uint32_t out_dim) { return gemv_mt_from(w_type, in_dim, out_dim); }
+int32_t cogni_gemv_top1_one_pass(uint32_t w_type, uint32_t tokens, uint32_t in_dim, uint32_t out_dim, int32_t logits) {
+  return gemv_mt_head_takes(w_type, tokens, in_dim, out_dim, logits);
+}
 uint32_t cogni_gemv_one_pass_multi_from(uint32_t w_type, uint32_t in_dim) { return gemv_mt_multi_from(w_type, in_dim); }
 
 int cogni_gemv_release_stream(void* stream) {

@@ -218,6 +218,20 @@ static inline unsigned gemv_mt_from(unsigned type, unsigned in_dim, unsigned out
   if (in_dim <= 4096u && out_dim >= GEMV_MT_TALL_ROWS) return (type == 14 || out_dim >= GEMV_MT_VERY_TALL_ROWS) ? 2u : 3u;
   return type == 14 ? 3u : (in_dim >= 4096u ? 4u : 5u);
 }
+// The resident output head (a norm that writes the image in front, top-1 inside, with or without the logits): tokens of a group that go
+// through one pass. Beside the counts above, two and more tokens of at least GEMV_MT_HEAD_ROWS rows (the fewest timed), whatever the row
+// length: the other kernels take two tokens a pass there, or walk the weights once for the logits and once for the top-1. Q6_K, rows of 1024 | 1280 |
+// 2304 | 2816 values, 151936 rows, us a step, before -> one pass: 2 tokens 137 -> 62 | 138 -> 63 | 148 -> 109 | 152 -> 115, 3 tokens
+// with logits 132 -> 64 | 191 -> 65 | 336 -> 110 | 381 -> 117; 32000 rows, 2 tokens 42 -> 28 | 42 -> 28 | 43 -> 38 | 43 -> 38. Q4_K 109 -> 48 | 108 -> 48 |
+// 112 -> 70 | 112 -> 71 (32000 rows of 1024 35 -> 24, of 4096 39 -> 32); 3 tokens with logits 68 -> 48 | 105 -> 49 | 153 -> 74 | 168 -> 74. Not Q4_K rows of 1024 values,
+// three or four tokens, top-1 alone: the matrix-core kernel fills its k-slices there (151936 rows 43 | 48, 50000 27 | 30, 32000 24 | 25).
+#define GEMV_MT_HEAD_ROWS 32000u
+static inline int gemv_mt_head_takes(unsigned type, unsigned tokens, unsigned in_dim, unsigned out_dim, int logits) {
+  if ((type != 12 && type != 14) || in_dim > 4096u || tokens > (unsigned)GEMV_MT_MAX_TOKENS || !gemv_mt_supported(type, 2, in_dim)) return 0;
+  if (tokens >= gemv_mt_from(type, in_dim, out_dim)) return 1;
+  if (tokens < 2u || out_dim < GEMV_MT_HEAD_ROWS) return 0;
+  return !(type == 12 && in_dim <= 1024u && tokens >= 3u && !logits);
+}
 // The same for a pair, a list of matrices or the fused gate | up | SwiGLU: from two tokens (one pack serves all of them and
 // the weights are read once), from five on rows that fill less than three quarters of their k-slices.
 static inline unsigned gemv_mt_multi_from(unsigned type, unsigned in_dim) {

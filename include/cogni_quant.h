@@ -178,6 +178,9 @@ uint32_t cogni_gemv_one_pass_from(uint32_t w_type, uint32_t in_dim, uint32_t out
  * Rows that are not a multiple of 2048 values also wait for 5 tokens in cogni_gemv_one_pass_from when they fill less
  * than that. No GPU needed. */
 uint32_t cogni_gemv_one_pass_multi_from(uint32_t w_type, uint32_t in_dim);
+/* Whether an output head whose norm writes the image (cogni_rmsnorm_pack_dev, then cogni_gemv_packed_top1[_logits]_dev) is the faster way for
+ * `tokens` tokens: 1 or 0. Earlier than cogni_gemv_one_pass_from for vocabularies. */
+int32_t cogni_gemv_top1_one_pass(uint32_t w_type, uint32_t tokens, uint32_t in_dim, uint32_t out_dim, int32_t logits);
 /* Gives back the image the library keeps for `stream` (waits for the stream's work first; nothing to do and no error if it
  * has none). Call it before destroying a stream that ran multi-token GEMVs: the eight slots are otherwise used up by the
  * first eight streams of the process, and later streams run the per-token-group kernels. A graph captured on the stream

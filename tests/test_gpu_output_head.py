@@ -197,6 +197,35 @@ def test_output_head_runner(gpu, oracle, hidden, vocab, tokens):
         stream.close()
 
 
+@pytest.mark.parametrize("t,hidden,vocab,tokens,logits,packed", [
+    (Q6_K, 1024, 32003, 2, True, True), (Q6_K, 2304, 32000, 3, False, True), (Q6_K, 1280, 31999, 4, True, False),
+    (Q4_K, 2816, 32001, 2, False, True), (Q4_K, 1024, 32000, 4, True, True), (Q4_K, 1024, 32000, 3, False, False)])
+def test_output_head_runner_of_few_tokens(gpu, oracle, t, hidden, vocab, tokens, logits, packed):
+    """Two to four tokens of a vocabulary whose rows do not fill the k-slices: the norm writes the image and the one-pass kernel takes
+    them from GEMV_MT_HEAD_ROWS rows on. Top-1 and logits within the GEMV bar of the oracle, and the top-1 that of the logits."""
+    rng = np.random.default_rng(hidden + vocab + tokens)
+    w = Weights((1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32), synth.make_weights(rng, t, vocab, hidden), t, hidden, vocab)
+    xs = (rng.standard_normal(tokens * hidden) * 3).astype(np.float32)
+    assert quant.gemv_top1_one_pass(t, tokens, hidden, vocab, logits) == packed and not quant.gemv_top1_one_pass(t, 1, hidden, vocab, logits)
+    runner = QwenOutputHeadRunner.from_weights(w, tokens, xs, 1e-6, read_logits=logits)
+    try:
+        runner.upload_weights()
+        runner.reset_sequence()
+        runner.run_sequence()
+        runner.read_outputs()
+        for tok in range(tokens):
+            normed = oracle.rms_norm(xs[tok * hidden:(tok + 1) * hidden], w.norm, 1e-6)
+            want = oracle.matmul_add(normed, 1, hidden, w.output_raw, t, vocab, np.zeros(vocab, dtype=np.float32), threads=8)
+            bar = 2e-5 * float(np.abs(want).max())
+            assert abs(runner.top1_values[tok] - want.max()) <= bar and want[runner.top1_ids[tok]] >= want.max() - bar
+            if logits:
+                dev = runner.logits[tok * vocab:(tok + 1) * vocab]
+                assert np.abs(dev - want).max() <= bar
+                assert runner.top1_ids[tok] == first_max(dev) and runner.top1_values[tok] == dev.max()
+    finally:
+        runner.close()
+
+
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
 def test_embedding_row_from_a_device_token_id(gpu, oracle, t):
     """The reference's token embedder (bin/cuda_mixed_stack_probe.cr:900-947): row token_ids[0] of the embedding matrix,
