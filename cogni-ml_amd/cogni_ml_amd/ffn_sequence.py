@@ -75,6 +75,7 @@ class FFNSequenceRunner:
             na = quant.gemv_image_bytes(down_type, ffn_dim, quant.MAX_GEMV_TOKENS)
             if nx and na:
                 self._img16_x, self._img16_act = self._alloc(nx), self._alloc(na)
+        self._issued = {}   # prefill: the library calls of a token count
         self.combined = self.out = None
         self._runner = hip.ResidentSequenceRunner(tokens, self._upload_weights, self._reset_sequence, self._run_token,
                                                   self._read_outputs, self._run_sequence)
@@ -192,7 +193,7 @@ class FFNSequenceRunner:
 
     def _run_sequence(self, active_tokens):
         if self._ws_x is not None and active_tokens > quant.get_gemm_threshold():
-            self._launch_prefill(active_tokens)
+            hip.issue(self._issued, (active_tokens, self.keep_combined), lambda: self._launch_prefill(active_tokens), quant._check)
             return
         for tok0 in range(0, active_tokens, quant.MAX_GEMV_TOKENS):
             self._launch(tok0, min(quant.MAX_GEMV_TOKENS, active_tokens - tok0))

@@ -10,6 +10,12 @@ import contextlib
 import ctypes
 import enum
 import os
+import threading
+
+try:
+    from . import _calls as calls   # native entry points of quant's single-operator calls
+except ImportError:
+    calls = None
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_PKG), "lib", "libcogni_hip.so")
@@ -27,6 +33,8 @@ class HIPError(RuntimeError):
 def lib():
     """Load libcogni_hip.so. There is no fallback: a missing library is an error."""
     global _lib
+    if _recording_threads and getattr(_noting, "calls", None) is not None:
+        return _noting.lib
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError("%s is missing: build it with `make -C cogni-ml_amd/csrc` "
@@ -50,6 +58,8 @@ def lib():
         L.typed_matmul_dev = proto(ctypes.c_int, U64, U32, U64, U64, U64, U32, U32, U32, U64, ctypes.c_size_t)(("cogni_matmul_dev", L))
         L.typed_gemv_dev = proto(ctypes.c_int, U64, U32, U64, U64, U64, U32, U32, U32)(("cogni_gemv_dev", L))
         L.typed_dequantize_dev = proto(ctypes.c_int, U64, U32, U64, U64)(("cogni_dequantize_dev", L))
+        if calls is not None:
+            calls.set_library(*(ctypes.cast(f, ctypes.c_void_p).value for f in (L.cogni_matmul_dev, L.cogni_gemv_dev, L.cogni_dequantize_dev)))
         L.mlhip_mem_alloc.argtypes = [ctypes.POINTER(ctypes.c_uint64), ctypes.c_size_t]
         L.mlhip_mem_free.argtypes = [ctypes.c_uint64]
         L.mlhip_memcpy_htod.argtypes = [ctypes.c_uint64, ctypes.c_void_p, ctypes.c_size_t]
@@ -77,6 +87,58 @@ def lib():
         L.mlhip_ctx_create.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_uint32, ctypes.c_int32]
         _lib = L
     return _lib
+
+
+_noting = threading.local()   # .calls, .lib: the list this thread notes its launches in, while it does
+_recording_threads = 0
+_recording_lock = threading.Lock()
+
+
+class _NotingLib:
+    """The library as lib() gives it to a thread that notes its launches: a cogni_*_dev call is made and kept without its stream."""
+
+    def __init__(self, real, calls):
+        self._real, self._calls = real, calls
+
+    def __getattr__(self, name):
+        f = getattr(self._real, name)
+        if not name.endswith("_dev"):
+            return f
+
+        def call(*args):
+            self._calls.append((f, args[:-1]))
+            return f(*args)
+        return call
+
+
+def issue(kept, key, launch, check_status):
+    """launch(), which issues operators on the current stream: the first time with a `key` as it is written, later the same library calls
+    with the same arguments on the stream that is current then, without the Python that chose them (stack of seven projections,
+    48 tokens: 31 us of host time the first way). `kept` holds the calls, at most 32 keys of them; `key` names all that
+    the choice depends on beside what never changes for the owner of `kept`."""
+    calls = kept.get(key)
+    if calls is not None:
+        stream = _current_stream
+        for f, args in calls:
+            code = f(*args, stream)
+            if code != 0:
+                check_status(code)
+        return
+    global _recording_threads
+    calls, outer = [], (getattr(_noting, "calls", None), getattr(_noting, "lib", None))
+    proxy = _NotingLib(lib(), calls)
+    with _recording_lock:
+        _recording_threads += 1
+    _noting.calls, _noting.lib = calls, proxy
+    try:
+        launch()
+    finally:
+        _noting.calls, _noting.lib = outer
+        with _recording_lock:
+            _recording_threads -= 1
+    if len(kept) >= 32:
+        kept.clear()
+    kept[key] = calls
 
 
 _current_stream = None  # module-global, like @@current_stream (driver.cr:55)

@@ -81,6 +81,7 @@ class QwenProjectionStackRunner:
                 if self._one_pass16(t, in_dim) and key not in self._images16:
                     self._images16[key] = self._alloc(quant.gemv_image_bytes(t, in_dim, quant.MAX_GEMV_TOKENS))
             self._prefill_ws = {k: (self._alloc(n), n) for k, n in need.items()}
+        self._issued = {}   # prefill: the library calls of a token count
         self.outputs = {}
         self._runner = hip.ResidentSequenceRunner(
             tokens, self._upload_weights, self._reset_sequence, self._run_token, self._read_outputs,
@@ -257,7 +258,7 @@ class QwenProjectionStackRunner:
 
     def _run_sequence(self, active_tokens):
         if self._prefill_ws and active_tokens > quant.get_gemm_threshold():
-            self._launch_prefill(active_tokens)
+            hip.issue(self._issued, active_tokens, lambda: self._launch_prefill(active_tokens), quant._check)
             return
         for tok0 in range(0, active_tokens, quant.MAX_GEMV_TOKENS):
             self._launch(tok0, min(quant.MAX_GEMV_TOKENS, active_tokens - tok0))

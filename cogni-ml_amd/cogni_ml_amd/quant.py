@@ -595,3 +595,11 @@ def matvec_many(qws, x):
     ptrs = (ctypes.c_void_p * len(qws))(*[o.ctypes.data for o in outs])
     _check(hip.lib().cogni_weight_matvec_many(handles, ctypes.c_int32(len(qws)), ctypes.c_void_p(xa.ctypes.data), ptrs))
     return outs
+
+
+# The calls a program issues one by one, read natively where their arguments are ordinary (csrc/py_calls.cpp; a pass of Q8_0 1024 -> 3584, one
+# token, through matmul_dev: @@). The functions above take what is not, and every call where the module is not built (no Python headers).
+_matmul_dev, _gemv_dev, _dequantize_dev = matmul_dev, gemv_dev, dequantize_dev
+if hip.calls is not None:
+    hip.calls.set_python(_matmul_dev, _gemv_dev, _dequantize_dev, _check, TensorType, ctypes.c_void_p)
+    matmul_dev, gemv_dev, dequantize_dev = hip.calls.matmul_dev, hip.calls.gemv_dev, hip.calls.dequantize_dev
