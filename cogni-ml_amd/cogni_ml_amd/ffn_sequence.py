@@ -174,7 +174,12 @@ class FFNSequenceRunner:
                 x = self._normed.ptr
             quant.gemm_pack_dev(x, TensorType.Q4_K, h, count, self._ws_x.ptr, self._ws_x_bytes, st)
         # silu(gate) * up leaves the GEMM as the down GEMM's packed input (and as fp32 only when `combined` is wanted)
-        pair = quant.gemm_stream_swiglu_pack_dev if quant.gemm_stream_takes(TensorType.Q4_K, h, 2 * f, count) else quant.gemm_packed_swiglu_pack_dev
+        if quant.gemm_stream_takes(TensorType.Q4_K, h, 2 * f, count):
+            pair = quant.gemm_stream_swiglu_pack_dev
+        elif quant.gemm_tall_swiglu_takes(TensorType.Q4_K, h, f, count):
+            pair = quant.gemm_tall_swiglu_pack_dev
+        else:
+            pair = quant.gemm_packed_swiglu_pack_dev
         pair(self._w["gate"].ptr, self._w["up"].ptr, TensorType.Q4_K, self._ws_x.ptr, self._ws_x_bytes,
              self._act.ptr if self.keep_combined else 0, self.down_type, self._ws_act.ptr, self._ws_act_bytes, h, f, count, st)
         res = self._res.ptr if self._res is not None else 0

@@ -247,6 +247,9 @@ class QwenProjectionStackRunner:
                     if quant.gemm_stream_takes(t, in_dim, sum(dims), count):
                         quant.gemm_stream_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, 0, stream)
                         break
+                    if quant.gemm_tall_takes(t, in_dim, dims, count):
+                        quant.gemm_tall_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, stream)
+                        break
                     if len(dims) >= 2 and int(t) in list_types:
                         quant.gemm_packed_many_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, stream)
                         break

@@ -464,6 +464,38 @@ def gemm_packed_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, wor
         ctypes.c_size_t(next_workspace_bytes), ctypes.c_uint32(in_dim), ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
 
 
+def gemm_tall_takes(w_type, in_dim, out_dims, tokens):
+    """Whether the runners take the tiles of 256 tokens for a list of matrices of these row counts."""
+    n = len(out_dims)
+    return bool(hip.lib().cogni_gemm_tall_takes(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(in_dim), (ctypes.c_uint32 * n)(*out_dims),
+                                                ctypes.c_uint32(n), ctypes.c_uint32(tokens)))
+
+
+def gemm_tall_swiglu_takes(w_type, in_dim, out_dim, tokens):
+    """The same for gate | up with SwiGLU, `out_dim` rows each."""
+    return bool(hip.lib().cogni_gemm_tall_swiglu_takes(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(in_dim), ctypes.c_uint32(out_dim),
+                                                       ctypes.c_uint32(tokens)))
+
+
+def gemm_tall_dev(w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, in_dim, tokens, stream=None):
+    """One to six Q4_K matrices of one row length against the same packed activations, in tiles of 256 tokens x 256 rows."""
+    n = len(w_ptrs)
+    if not (n == len(out_ptrs) == len(out_dims)):
+        raise ValueError("w_ptrs, out_ptrs and out_dims must have one entry per matrix")
+    _check(hip.lib().cogni_gemm_tall_dev((ctypes.c_uint64 * n)(*w_ptrs), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(workspace_ptr),
+                                         ctypes.c_size_t(workspace_bytes), (ctypes.c_uint64 * n)(*out_ptrs), (ctypes.c_uint32 * n)(*out_dims),
+                                         ctypes.c_uint32(n), ctypes.c_uint32(in_dim), ctypes.c_uint32(tokens), stream))
+
+
+def gemm_tall_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, workspace_bytes, out_ptr, next_type, next_workspace_ptr,
+                              next_workspace_bytes, in_dim, out_dim, tokens, stream=None):
+    """gemm_packed_swiglu_pack_dev in tiles of 256 tokens x 128 rows of both matrices."""
+    _check(hip.lib().cogni_gemm_tall_swiglu_pack_dev(
+        ctypes.c_uint64(w_gate_ptr), ctypes.c_uint64(w_up_ptr), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(workspace_ptr),
+        ctypes.c_size_t(workspace_bytes), ctypes.c_uint64(out_ptr), ctypes.c_uint32(int(next_type)), ctypes.c_uint64(next_workspace_ptr),
+        ctypes.c_size_t(next_workspace_bytes), ctypes.c_uint32(in_dim), ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
+
+
 def gemm_stream_takes(w_type, in_dim, rows, tokens):
     """Whether the router and the runners take the short-prefill kernels for a launch of `rows` rows in all."""
     return bool(hip.lib().cogni_gemm_stream_takes(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(in_dim), ctypes.c_uint32(rows),

@@ -6,7 +6,7 @@ keep for instructions written inside asm statements:
     destination, a carry-out) must be five wait states ahead of a memory instruction that reads that register as its
     scalar base;
   * a write of M0 must be one wait state ahead of a global load that writes to LDS;
-  * in the kernels whose copies to LDS set M0 inside asm statements (names with "_mt_"), the compiler does not know
+  * in the kernels whose copies to LDS set M0 inside asm statements (names with "_mt_" or "_gemm_tall_"), the compiler does not know
     that M0 changes, so nothing may read a value of M0 that it assumes to have survived: every instruction that reads
     M0 must have a write of M0 within the two instructions in front of it, with no label in between.
 
@@ -42,7 +42,7 @@ def reads_m0(mnemonic, operands):
 
 
 def asm_m0_kernel(name):
-    return "_mt_" in name
+    return "_mt_" in name or "_gemm_tall_" in name
 # vector instructions whose second operand is a scalar destination (carry or scale flag)
 SDST_SECOND = ("v_mad_u64_u32", "v_mad_i64_i32", "v_add_co_u32", "v_sub_co_u32", "v_subrev_co_u32", "v_addc_co_u32",
                "v_subb_co_u32", "v_subbrev_co_u32", "v_div_scale_f32", "v_div_scale_f64")

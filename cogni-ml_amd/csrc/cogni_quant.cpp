@@ -1519,6 +1519,46 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
                 params, stream);
 }
 
+// Launches of many tokens, tiles of 256 tokens x 256 rows (kernels/gemm_q4k_tall.hpp): the same packed activations and precision, each sum
+// added in one order of k (the kernels above add two halves), so not their bits.
+int32_t cogni_gemm_tall_takes(uint32_t w_type, uint32_t in_dim, const uint32_t* out_dims, uint32_t count, uint32_t tokens) {
+  if (!out_dims || count == 0 || count > 6) return 0;
+  return gemm_tall_takes(w_type, in_dim, out_dims, count, tokens);
+}
+int32_t cogni_gemm_tall_swiglu_takes(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens) {
+  return gemm_tall_swiglu_takes(w_type, in_dim, out_dim, tokens);
+}
+int cogni_gemm_tall_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                        const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_tall_dev";
+  if (w_type != COGNI_TYPE_Q4_K)
+    return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the GEMM of 256-token tiles: ") + type_name(w_type));
+  if (!w_raw || !outs || !out_dims || count == 0 || count > 6) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": one to six matrices");
+  GemmManyArgs list{};
+  uint32_t end = 0;
+  for (uint32_t i = 0; i < count; i++) {
+    if (!w_raw[i] || !outs[i]) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+    if (int rc = gemm_check(who, w_type, in_dim, out_dims[i], tokens, workspace, workspace_bytes)) return rc;
+    list.w[i] = w_raw[i];
+    list.out[i] = outs[i];
+    list.out_dim[i] = out_dims[i];
+    list.tile_end[i] = end += (out_dims[i] + 255) / 256;
+  }
+  list.count = count;
+  void* params[] = {&list, &workspace, &in_dim, &tokens};
+  return launch("q4_k_gemm_tall_f16", gemm_tiles_grid((tokens + 255) / 256, end), 256, 0, params, stream);
+}
+int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
+                                    uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
+                                    uint32_t tokens, void* stream) {
+  if (int rc = swiglu_pack_check("cogni_gemm_tall_swiglu_pack_dev", w_gate, w_up, w_type, workspace, workspace_bytes, next_type, next_workspace,
+                                 next_workspace_bytes, in_dim, out_dim, tokens))
+    return rc;
+  void* params[] = {&w_gate, &w_up, &workspace, &out, &next_workspace, &in_dim, &out_dim, &tokens};
+  return launch(next_type == COGNI_TYPE_Q6_K ? "q4_k_gemm_tall_swiglu_pack_q6k_f16" : "q4_k_gemm_tall_swiglu_pack_q4k_f16",
+                gemm_tiles_grid((tokens + 255) / 256, (out_dim + 127) / 128), 256, 0, params, stream);
+}
+
 // Short prefills: the weights streamed through workgroups of four wavefronts (kernels/gemm_stream.hpp). The same packed
 // activations, planes and precision as the tile kernels above.
 // Planes of [tokens][out_dim] that fit behind the packed activations. cogni_gemm_workspace_bytes_split sizes a workspace for the tile

@@ -53,3 +53,4 @@ GEMV_MT_TOP1_LOGITS_ENTRY(q4_k_gemv_mt_top1_logits_partial_f32, MtQ4K)
 GEMV_MT_TOP1_LOGITS_ENTRY(q6_k_gemv_mt_top1_logits_partial_f32, MtQ6K)
 #include "kernels/gemm_terms.hpp"
 #include "kernels/gemm_stream.hpp"
+#include "kernels/gemm_q4k_tall.hpp"

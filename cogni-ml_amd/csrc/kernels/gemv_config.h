@@ -323,6 +323,41 @@ static inline unsigned gemm_list_rows(unsigned type, const unsigned* out_dims, u
   return best;
 }
 
+// The kernels of 256 tokens x 256 rows (gemm_q4k_tall.hpp; Q4_K lists and gate | up, whose tile is 128 rows of both): where their tiles take less
+// time than those of the kernel the rules above pick. A last round that is not full is charged 0.6 + 0.4 fill^2 of a round: the fewer compute units
+// work, the higher the chip's clock. One launch of 64 | 128 | 192 | 256 | 320 | 512 tiles, 4096 columns, us: 192 rows 42.6 | 45.9 | 49.5 | 57.7 | 92.0 |
+// 111.5, 128 rows 31.5 | 34.0 | 36.6 | 42.4 | 67.7 | 78.9, 256 rows 50.7 | 54.8 | 61.4 | 74.5 | 116.7 | 147.5, these 82 | 87.5 | 99.9 | 122.9 | 193 | 242; gate | up
+// with 96 rows 48.4 | 51.4 | 55.5 | 63.8 | 103 | 121, with 128 50.6 | 54.0 | 64.2 | 77.3 | 121 | 154, these 90 | 96 | 112.5 | 135.6 | 217 | 266: a round is 213 in lists
+// and 217 to 232 in gate | up. Weights from memory, what the rules above take | these: lists of 30720 rows x 4096 at 512 tokens 139 to 149 | 116, 1024
+// 270 | 224, 2048 522 | 438, at 256 72 | 82 (not taken); 30720 x 512 | 2048 | 8192 at 512 tokens 40 | 81 | 261 and 31 | 67 | 217; gate | up 4096 -> 12288 at 512 tokens
+// 121 | 110, 2048 431 | 380, 1024 217 | 226 (not taken); 2048 -> 6144 at 1024 75 | 66.
+#define GEMM_TALL_COST 213u
+#define GEMM_TALL_SWIGLU_COST 232u
+static inline unsigned long long gemm_fill_cost(unsigned long long tiles, unsigned cost) {
+  const unsigned long long full = tiles / GEMM_ROUND_TILES, rest = tiles % GEMM_ROUND_TILES;
+  return cost * (256ull * full + (rest ? 154ull + 102ull * rest * rest / 65536ull : 0ull));
+}
+static inline unsigned long long gemm_list_tiles(const unsigned* out_dims, unsigned count, unsigned rows) {
+  unsigned long long n = 0;
+  unsigned i;
+  for (i = 0; i < count; i++) n += ((unsigned long long)out_dims[i] + rows - 1u) / rows;
+  return n;
+}
+static inline int gemm_tall_takes(unsigned type, unsigned in_dim, const unsigned* out_dims, unsigned count, unsigned tokens) {
+  const unsigned long long mt = (tokens + 127ull) / 128ull;
+  if (type != 12u || tokens <= 128u || (in_dim & 255u) != 0 || in_dim == 0) return 0;
+  const unsigned rows = gemm_list_rows(type, out_dims, count, tokens, -1);
+  return gemm_fill_cost((mt + 1u) / 2u * gemm_list_tiles(out_dims, count, 256u), GEMM_TALL_COST) <
+         gemm_fill_cost(mt * gemm_list_tiles(out_dims, count, rows), gemm_tile_cost(type, rows));
+}
+static inline int gemm_tall_swiglu_takes(unsigned type, unsigned in_dim, unsigned out_dim, unsigned tokens) {
+  const unsigned long long mt = (tokens + 127ull) / 128ull;
+  if (type != 12u || tokens <= 128u || (in_dim & 255u) != 0 || in_dim == 0) return 0;
+  const int wide = gemm_swiglu_use_wide(out_dim, tokens, -1);
+  return gemm_fill_cost((mt + 1u) / 2u * gemm_list_tiles(&out_dim, 1u, 128u), GEMM_TALL_SWIGLU_COST) <
+         gemm_fill_cost(mt * gemm_list_tiles(&out_dim, 1u, wide ? 128u : 96u), gemm_tile_cost(12u, wide ? 256u : 192u));
+}
+
 // ---- prefill GEMM: which tile a workgroup takes. Workgroups go to the 8 XCDs round-robin (id % 8), each XCD has its own
 // L2 and 32 compute units, and a GEMM workgroup has a compute unit to itself, so the workgroups id = 8 l + x with the
 // same l / 32 run side by side on XCD x. Every XCD gets an equal share of the tiles (they are numbered in one line and it takes

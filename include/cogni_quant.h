@@ -513,6 +513,18 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
 int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                       uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
                                       uint32_t out_dim, uint32_t tokens, void* stream);
+/* Launches of many tokens in tiles of 256 tokens x 256 rows (Q4_K): one to six matrices of one row length against the packed
+ * activations of cogni_gemm_pack_dev, and gate | up with SwiGLU, whose products leave as cogni_gemm_packed_swiglu_pack_dev writes them. Same
+ * precision as those entry points, each sum in one order of k, so not the same bits. *_takes: whether a launch is the faster one this way
+ * (1 or 0; the resident runners go by it). */
+int32_t cogni_gemm_tall_takes(uint32_t w_type, uint32_t in_dim, const uint32_t* out_dims, uint32_t count, uint32_t tokens);
+int32_t cogni_gemm_tall_swiglu_takes(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens);
+int cogni_gemm_tall_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                        const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
+int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
+                                    uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
+                                    uint32_t tokens, void* stream);
+
 /* The short-prefill forms of the packed GEMMs: the weights streamed through many small workgroups instead of tiles of 128
  * tokens that have a compute unit to themselves. They read the same packed activations, their operands are rounded as the
  * tile kernels round them (fp16, fp32 sums; the order of the sums differs), and cogni_matmul_dev and the resident runners take

@@ -1,0 +1,78 @@
+"""The prefill kernels of 256 tokens x 256 rows: Q4_K lists, gate | up with SwiGLU."""
+import numpy as np
+import pytest
+
+from cogni_ml_amd import quant, synth
+from gpu_common import DevArray, gpu  # noqa: F401
+from helpers import Q4_K, Q6_K
+
+pytestmark = pytest.mark.gpu
+
+
+def sums_bound(oracle, raw, x, out_dim, in_dim):
+    """Two fp32 sums of the same products in different orders differ by at most 2 n 2^-24 of the sum of their magnitudes (n additions)."""
+    w = np.abs(oracle.dequantize(raw, Q4_K, out_dim * in_dim).reshape(out_dim, in_dim))
+    return 2 * in_dim * 2.0**-24 * (np.abs(x) @ w.T) * 1.01   # (1.01: operands rounded to half)
+
+
+# token tiles that are clipped, end at a 128-token tile, are whole; matrices that end inside a tile, inside a wavefront's 64 rows, of no multiple
+# of four rows, of one row; one super-block, an even and an odd number
+@pytest.mark.parametrize("tokens,in_dim,dims", [(129, 256, [300]), (255, 512, [256, 1]), (256, 768, [64, 513, 7]), (257, 256, [1000, 255]),
+                                                (384, 1024, [192, 256]), (513, 512, [321, 64, 100, 5, 256, 257]), (1, 256, [65])])
+def test_lists(gpu, oracle, tokens, in_dim, dims):
+    rng = np.random.default_rng(tokens + in_dim)
+    raws = [synth.make_weights(rng, Q4_K, d, in_dim) for d in dims]
+    x = synth.make_activations(rng, tokens, in_dim)
+    wsb = quant.gemm_workspace_bytes(Q4_K, in_dim, tokens)
+    ws, xd, wd = DevArray(nbytes=wsb), DevArray(x), [DevArray(r) for r in raws]
+    outs = [[DevArray(np.full(tokens * d + 4, np.float32(-3.0))) for d in dims] for _ in range(2)]
+    quant.gemm_pack_dev(xd.ptr, Q4_K, in_dim, tokens, ws.ptr, wsb)
+    for w, o, d in zip(wd, outs[0], dims):
+        quant.gemm_packed_dev(w.ptr, Q4_K, ws.ptr, wsb, o.ptr, in_dim, d, tokens)
+    quant.gemm_tall_dev([w.ptr for w in wd], Q4_K, ws.ptr, wsb, [o.ptr for o in outs[1]], dims, in_dim, tokens)
+    for raw, a, b, d in zip(raws, outs[0], outs[1], dims):
+        want, got = (o.read(np.float32, tokens * d + 4) for o in (a, b))
+        assert np.array_equal(got[tokens * d:], np.full(4, np.float32(-3.0)))
+        diff = np.abs(want[:tokens * d].astype(np.float64) - got[:tokens * d]).reshape(tokens, d)
+        assert (diff <= sums_bound(oracle, raw, x.reshape(tokens, in_dim), d, in_dim)).all(), d
+    for a in [ws, xd] + wd + sum(outs, []):
+        a.close()
+
+
+@pytest.mark.parametrize("next_type", [Q4_K, Q6_K])
+@pytest.mark.parametrize("tokens,out_dim,in_dim,keep", [(129, 256, 256, True), (256, 512, 768, True), (300, 768, 512, False), (513, 256, 1024, True)])
+def test_gate_up_swiglu(gpu, tokens, out_dim, in_dim, next_type, keep):
+    """Products and packed activations (absent tokens zeros) against the 128-token kernels': fp32 to 3e-6 of a token's largest product (sums in another
+    order: 2-norm 6e-7, the two roundings of gemm_tall_silu 1e-7), the packed halves what those products round to."""
+    rng = np.random.default_rng(tokens + next_type)
+    x = synth.make_activations(rng, tokens, in_dim) * np.float32(0.05)
+    wg, wu = (DevArray(synth.make_weights(rng, Q4_K, out_dim, in_dim)) for _ in range(2))
+    wsb, nxb = quant.gemm_workspace_bytes(Q4_K, in_dim, tokens), quant.gemm_workspace_bytes(next_type, out_dim, tokens)
+    xd, ws = DevArray(x), DevArray(nbytes=wsb)
+    o1, o2 = (DevArray(np.full(tokens * out_dim, np.float32(-3.0))) for _ in range(2))
+    p1, p2 = (DevArray(np.full(nxb, 0xFF, np.uint8)) for _ in range(2))
+    quant.gemm_pack_dev(xd.ptr, Q4_K, in_dim, tokens, ws.ptr, wsb)
+    quant.gemm_packed_swiglu_pack_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, o1.ptr, next_type, p1.ptr, nxb, in_dim, out_dim, tokens)
+    quant.gemm_tall_swiglu_pack_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, o2.ptr if keep else 0, next_type, p2.ptr, nxb, in_dim, out_dim, tokens)
+    want, got = (o.read(np.float32, tokens * out_dim).reshape(tokens, out_dim) for o in (o1, o2))
+    if keep:
+        assert np.all(np.abs(want - got) <= 3e-6 * np.abs(want).max(axis=1, keepdims=True))
+        quant.gemm_pack_dev(o2.ptr, next_type, out_dim, tokens, p1.ptr, nxb)
+        assert np.array_equal(p2.read(np.uint8, nxb), p1.read(np.uint8, nxb))
+    else:
+        assert np.array_equal(got, np.full_like(got, -3.0))
+        a, b = (p.read(np.uint8, nxb).view(np.float16).astype(np.float32) for p in (p1, p2))
+        assert np.all(np.abs(a - b) <= 2.0**-10 * np.abs(a) + 3e-6 * np.abs(want).max())
+    for a in (wg, wu, xd, ws, o1, o2, p1, p2):
+        a.close()
+
+
+def test_which_launches_take_these_kernels(gpu):
+    dims = [4096, 1024, 1024, 12288, 12288]
+    assert [quant.gemm_tall_takes(Q4_K, 4096, dims, m) for m in (64, 128, 256, 384, 400, 512, 1024, 2048)] == [False] * 4 + [True] * 4
+    assert not quant.gemm_tall_takes(Q6_K, 4096, dims, 512) and not quant.gemm_tall_takes(Q4_K, 4096, [4096], 512)
+    assert [quant.gemm_tall_swiglu_takes(Q4_K, 4096, 12288, m) for m in (256, 512, 1024, 2048)] == [False, True, False, True]
+    with pytest.raises(quant.QuantError, match="256-token tiles: Q6_K"):
+        quant.gemm_tall_dev([1], Q6_K, 1, 1 << 30, [1], [256], 256, 256)
+    with pytest.raises(quant.QuantError, match="workspace has"):
+        quant.gemm_tall_dev([1], Q4_K, 1, 16, [1], [256], 256, 256)
