@@ -181,6 +181,12 @@ extern "C" {
 const char* cogni_last_error(void) { return g_err.c_str(); }
 int cogni_internal_fail(int code, const char* text) { return fail(code, text); }
 int cogni_internal_hip_fail(int hip_error, const char* what) { return hip_fail((hipError_t)hip_error, what); }
+int cogni_internal_is_kernel(const void* function) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  for (const auto& f : g_rt.fns)
+    if ((const void*)f.second == function) return 1;
+  return 0;
+}
 
 // ---- geometry (reader.cr:51-78, 119-127) -----------------------------------------------------
 int32_t cogni_block_bytes(uint32_t type) {

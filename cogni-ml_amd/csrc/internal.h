@@ -10,6 +10,8 @@ int cogni_internal_hip_fail(int hip_error, const char* what);
 // Resolve, on the current device, the address of the static scratch array behind cogni_gemv_top1_noalloc_dev
 // (top1_noalloc.hip). Called by cogni_quant_init once the device is selected.
 int cogni_internal_noalloc_setup(int device);
+// Whether `function` (a hipFunction_t) is one of the library's kernels that it has looked up.
+int cogni_internal_is_kernel(const void* function);
 #ifdef __cplusplus
 }
 #endif

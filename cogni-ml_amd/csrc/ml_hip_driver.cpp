@@ -2,9 +2,75 @@
 // reference binds from libcuda (src/ml/cuda/driver.cr:20-50). See include/ml_hip_driver.h.
 #include "ml_hip_driver.h"
 
+#include "internal.h"
+
 #include <hip/hip_runtime_api.h>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+// ---- graphs of a few kernels in a row ----------------------------------------------------------------------------------
+// hipGraphLaunch takes 16 us of host time whatever is in the graph, and leaves the device idle for 5 us between one graph and the
+// next; a plain launch takes 2.8 and leaves less than 1 (graphs of empty kernels, one to four of them, back to back: 16.2 to 18.4 us; one
+// kernel of 22.6 us 27.7, two 50.3). A decode step of the runners is two to four kernels one after the other, so a graph that is a chain
+// of up to CHAIN_MOST of this library's kernels and nothing else is launched as those kernels. Anything else - other nodes, branches, other modules'
+// kernels, instantiation flags - goes through hipGraphLaunch.
+namespace {
+constexpr size_t CHAIN_MOST = 5;   // 14 us of launches
+struct Chain {
+  hipGraph_t graph = nullptr;   // a copy of the program's graph: the parameters below are its
+  std::vector<hipKernelNodeParams> kernels;
+  ~Chain() {
+    if (graph) (void)hipGraphDestroy(graph);
+  }
+};
+std::mutex g_chain_mu;
+std::unordered_map<void*, std::shared_ptr<const Chain>> g_chains;   // by executable graph, until that is destroyed
+
+// The chain a graph is, or null.
+std::shared_ptr<const Chain> chain_of(hipGraph_t graph) {
+  auto c = std::make_shared<Chain>();
+  size_t n = 0, edges = 0;
+  if (hipGraphGetNodes(graph, nullptr, &n) != hipSuccess || n == 0 || n > CHAIN_MOST) return nullptr;
+  if (hipGraphClone(&c->graph, graph) != hipSuccess) {
+    c->graph = nullptr;
+    return nullptr;
+  }
+  std::vector<hipGraphNode_t> nodes(n);
+  if (hipGraphGetNodes(c->graph, nodes.data(), &n) != hipSuccess || n != nodes.size()) return nullptr;
+  if (hipGraphGetEdges(c->graph, nullptr, nullptr, &edges) != hipSuccess || edges != n - 1) return nullptr;
+  std::vector<hipGraphNode_t> from(n), to(n);
+  if (edges && (hipGraphGetEdges(c->graph, from.data(), to.data(), &edges) != hipSuccess || edges != n - 1)) return nullptr;
+  from.resize(edges);
+  to.resize(edges);
+  auto count = [](const std::vector<hipGraphNode_t>& v, hipGraphNode_t x) {
+    size_t k = 0;
+    for (hipGraphNode_t y : v) k += y == x;
+    return k;
+  };
+  hipGraphNode_t at = nullptr;
+  for (hipGraphNode_t x : nodes) {
+    if (count(from, x) > 1 || count(to, x) > 1) return nullptr;
+    if (count(to, x) == 0) at = x;   // n - 1 edges, at most one into and out of a node: one start, or a circle beside it
+  }
+  for (size_t k = 0; k < n; k++) {
+    hipGraphNodeType type;
+    hipKernelNodeParams p = {};
+    if (!at || hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel ||
+        hipGraphKernelNodeGetParams(at, &p) != hipSuccess || !p.func || !p.kernelParams || p.extra || !cogni_internal_is_kernel(p.func))
+      return nullptr;
+    c->kernels.push_back(p);
+    hipGraphNode_t next = nullptr;
+    for (size_t e = 0; e < edges; e++)
+      if (from[e] == at) next = to[e];
+    at = next;
+  }
+  return at ? nullptr : c;
+}
+}   // namespace
 
 extern "C" {
 
@@ -100,8 +166,13 @@ int mlhip_stream_end_capture(mlhip_stream stream, mlhip_graph* graph) {
 }
 
 int mlhip_graph_instantiate(mlhip_graph_exec* exec, mlhip_graph graph, uint64_t flags) {
-  return (int)hipGraphInstantiateWithFlags(reinterpret_cast<hipGraphExec_t*>(exec), (hipGraph_t)graph,
-                                           (unsigned long long)flags);
+  const hipError_t e = hipGraphInstantiateWithFlags(reinterpret_cast<hipGraphExec_t*>(exec), (hipGraph_t)graph, (unsigned long long)flags);
+  if (e != hipSuccess) return (int)e;
+  std::shared_ptr<const Chain> c = flags == 0 ? chain_of((hipGraph_t)graph) : nullptr;
+  std::lock_guard<std::mutex> lk(g_chain_mu);
+  if (c) g_chains[*exec] = std::move(c);
+  else g_chains.erase(*exec);
+  return 0;
 }
 
 int mlhip_graph_upload(mlhip_graph_exec exec, mlhip_stream stream) {
@@ -109,12 +180,35 @@ int mlhip_graph_upload(mlhip_graph_exec exec, mlhip_stream stream) {
 }
 
 int mlhip_graph_launch(mlhip_graph_exec exec, mlhip_stream stream) {
+  std::shared_ptr<const Chain> c;
+  {
+    std::lock_guard<std::mutex> lk(g_chain_mu);
+    if (auto it = g_chains.find(exec); it != g_chains.end()) c = it->second;
+  }
+  if (c) {
+    for (const hipKernelNodeParams& k : c->kernels)
+      if (hipError_t e = hipModuleLaunchKernel((hipFunction_t)k.func, k.gridDim.x, k.gridDim.y, k.gridDim.z, k.blockDim.x, k.blockDim.y, k.blockDim.z,
+                                               k.sharedMemBytes, (hipStream_t)stream, k.kernelParams, nullptr);
+          e != hipSuccess)
+        return (int)e;
+    return 0;
+  }
   return (int)hipGraphLaunch((hipGraphExec_t)exec, (hipStream_t)stream);
 }
 
 int mlhip_graph_destroy(mlhip_graph graph) { return (int)hipGraphDestroy((hipGraph_t)graph); }
 
-int mlhip_graph_exec_destroy(mlhip_graph_exec exec) { return (int)hipGraphExecDestroy((hipGraphExec_t)exec); }
+int mlhip_graph_exec_destroy(mlhip_graph_exec exec) {
+  std::shared_ptr<const Chain> c;   // (destroyed outside the lock)
+  {
+    std::lock_guard<std::mutex> lk(g_chain_mu);
+    if (auto it = g_chains.find(exec); it != g_chains.end()) {
+      c = std::move(it->second);
+      g_chains.erase(it);
+    }
+  }
+  return (int)hipGraphExecDestroy((hipGraphExec_t)exec);
+}
 
 int mlhip_mem_alloc(mlhip_deviceptr* dptr, size_t bytesize) {
   void* p = nullptr;
