@@ -197,11 +197,21 @@ class QwenProjectionStackRunner:
         return int(t) in (int(TensorType.Q4_K), int(TensorType.Q5_K), int(TensorType.Q6_K)) and \
             quant.gemv_image_bytes(t, in_dim, quant.MAX_GEMV_TOKENS) > 0
 
+    def _next_input(self, entry):
+        """What a list can write beside this output: ((output name, layout), (type, workspace, bytes)) of a projection that reads it."""
+        for name, src, t, out_dim, in_dim, raw in self.weights.entries:
+            if src == entry[0] and in_dim == entry[3]:
+                ws, nbytes = self._prefill_ws[(src, self._family(t))]
+                return (src, self._family(t)), (t, ws.ptr, nbytes)
+        return None
+
     def _launch_prefill(self, count):
         """All `count` tokens through the GEMMs: one pack per (input, layout), one GEMM per list of projections that share
-        their input, type and row length (or per projection)."""
+        their input, type and row length (or per projection). A list that can leaves its outputs as the packed inputs of the
+        rounds behind it too."""
         stream = hip.current_stream_handle()
         list_types = (int(TensorType.Q4_K), int(TensorType.Q5_K))
+        packed = set()   # the (input, layout) that a list has written
         for groups in self._rounds:
             # the inputs of the round, packed once each, two to a launch
             jobs16, jobs = {}, {}
@@ -210,7 +220,7 @@ class QwenProjectionStackRunner:
                 key = (src, self._family(t))
                 if count <= 16 and self._one_pass16(t, in_dim):
                     jobs16.setdefault(key, (self._act[src].ptr, t, in_dim, self._images16[key].ptr))
-                else:
+                elif key not in packed:
                     jobs.setdefault(key, (self._act[src].ptr, t, in_dim, self._prefill_ws[key][0].ptr, self._prefill_ws[key][1]))
             self._pack_each(list(jobs16.values()), lambda x, t, k, image: quant.gemv_pack16_dev(x, t, k, count, image, stream),
                             lambda *ab: quant.gemv_pack16_two_dev(*ab, count, stream))
@@ -243,8 +253,15 @@ class QwenProjectionStackRunner:
                     quant.gemv_packed16_dev(w, t, self._images16[key].ptr, out, dims, in_dim, count, 0, stream)
                     continue
                 ws, nbytes = self._prefill_ws[key]
+                nexts = [self._next_input(e) for e in grp] if len(grp) >= 2 and int(t) in list_types else []
                 while dims:   # (the prefill counterpart of the qmatvec_many seam)
-                    if quant.gemm_stream_takes(t, in_dim, sum(dims), count):
+                    takes = quant.gemm_stream_takes(t, in_dim, sum(dims), count)
+                    if any(nexts) and (takes or quant.gemm_tall_takes(t, in_dim, dims, count)):
+                        (quant.gemm_stream_pack_dev if takes else quant.gemm_tall_pack_dev)(
+                            w, t, ws.ptr, nbytes, out, dims, [n and n[1] for n in nexts], in_dim, count, stream)
+                        packed.update(n[0] for n in nexts if n)
+                        break
+                    if takes:
                         quant.gemm_stream_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, 0, stream)
                         break
                     if quant.gemm_tall_takes(t, in_dim, dims, count):
@@ -254,7 +271,7 @@ class QwenProjectionStackRunner:
                         quant.gemm_packed_many_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, stream)
                         break
                     quant.gemm_packed_dev(w[0], t, ws.ptr, nbytes, out[0], in_dim, dims[0], count, 0, stream)
-                    w, out, dims = w[1:], out[1:], dims[1:]
+                    w, out, dims, nexts = w[1:], out[1:], dims[1:], nexts[1:]
 
     def _run_token(self, tok):
         self._launch(tok, 1)

@@ -487,6 +487,26 @@ def gemm_tall_dev(w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_
                                          ctypes.c_uint32(n), ctypes.c_uint32(in_dim), ctypes.c_uint32(tokens), stream))
 
 
+def _list_pack(f, w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, nexts, in_dim, tokens, stream):
+    n = len(w_ptrs)
+    if not (n == len(out_ptrs) == len(out_dims) == len(nexts)):
+        raise ValueError("w_ptrs, out_ptrs, out_dims and nexts must have one entry per matrix")
+    t, p, b = zip(*[(int(e[0]), e[1], e[2]) if e else (0, 0, 0) for e in nexts]) if n else ((), (), ())
+    _check(f((ctypes.c_uint64 * n)(*w_ptrs), ctypes.c_uint32(int(w_type)), ctypes.c_uint64(workspace_ptr), ctypes.c_size_t(workspace_bytes),
+             (ctypes.c_uint64 * n)(*out_ptrs), (ctypes.c_uint32 * n)(*out_dims), (ctypes.c_uint32 * n)(*t), (ctypes.c_uint64 * n)(*p),
+             (ctypes.c_size_t * n)(*b), ctypes.c_uint32(n), ctypes.c_uint32(in_dim), ctypes.c_uint32(tokens), stream))
+
+
+def gemm_tall_pack_dev(w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, nexts, in_dim, tokens, stream=None):
+    """gemm_tall_dev that also writes out i as the packed activations of a following GEMM: nexts[i] = (its type, workspace, bytes) | None."""
+    _list_pack(hip.lib().cogni_gemm_tall_pack_dev, w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, nexts, in_dim, tokens, stream)
+
+
+def gemm_stream_pack_dev(w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, nexts, in_dim, tokens, stream=None):
+    """gemm_stream_dev (Q4_K, Q5_K; no residual, no k split) that also writes packed activations, as gemm_tall_pack_dev."""
+    _list_pack(hip.lib().cogni_gemm_stream_pack_dev, w_ptrs, w_type, workspace_ptr, workspace_bytes, out_ptrs, out_dims, nexts, in_dim, tokens, stream)
+
+
 def gemm_tall_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, workspace_bytes, out_ptr, next_type, next_workspace_ptr,
                               next_workspace_bytes, in_dim, out_dim, tokens, stream=None):
     """gemm_packed_swiglu_pack_dev in tiles of 256 tokens x 128 rows of both matrices."""
@@ -630,7 +650,7 @@ def matvec_many(qws, x):
 
 
 # The calls a program issues one by one, read natively where their arguments are ordinary (csrc/py_calls.cpp; a pass of Q8_0 1024 -> 3584, one
-# token, through matmul_dev: @@). The functions above take what is not, and every call where the module is not built (no Python headers).
+# token, through matmul_dev: 4.2 us in Python, 3.65 so). The functions above take what is not, and every call where the module is not built (no Python headers).
 _matmul_dev, _gemv_dev, _dequantize_dev = matmul_dev, gemv_dev, dequantize_dev
 if hip.calls is not None:
     hip.calls.set_python(_matmul_dev, _gemv_dev, _dequantize_dev, _check, TensorType, ctypes.c_void_p)

@@ -1459,6 +1459,10 @@ struct GemmManyArgs {   // the kernels' first parameter (kernels/gemm_q4k.hpp)
   uint32_t tile_end[6];
   uint32_t count;
 };
+struct GemmNextArgs {   // the second one of the kernels that write packed inputs too
+  uint64_t xq[6];
+  uint32_t q6;
+};
 }   // namespace
 int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
                                const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
@@ -1534,12 +1538,24 @@ int32_t cogni_gemm_tall_takes(uint32_t w_type, uint32_t in_dim, const uint32_t* 
 int32_t cogni_gemm_tall_swiglu_takes(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens) {
   return gemm_tall_swiglu_takes(w_type, in_dim, out_dim, tokens);
 }
-int cogni_gemm_tall_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
-                        const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
-  const char* who = "cogni_gemm_tall_dev";
-  if (w_type != COGNI_TYPE_Q4_K)
-    return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the GEMM of 256-token tiles: ") + type_name(w_type));
-  if (!w_raw || !outs || !out_dims || count == 0 || count > 6) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": one to six matrices");
+// The packed inputs a list is to write: next_workspaces[i] (0: none) for a GEMM of type next_types[i] whose rows are out[i]'s values.
+static int gemm_next_of(const char* who, GemmNextArgs* next, const uint32_t* next_types, const uint64_t* next_workspaces, const size_t* next_bytes,
+                        const uint32_t* out_dims, uint32_t count, uint32_t tokens) {
+  if (!next_types || !next_workspaces || !next_bytes) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null array");
+  for (uint32_t i = 0; i < count; i++) {
+    if (!next_workspaces[i]) continue;
+    if (!gemm_type(next_types[i]))
+      return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the prefill GEMM: ") + type_name(next_types[i]));
+    if (out_dims[i] % 256 != 0) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": out_dim must be a multiple of 256");
+    if (next_bytes[i] < cogni_gemm_workspace_bytes(next_types[i], out_dims[i], tokens))
+      return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": next_workspace too small (cogni_gemm_workspace_bytes)");
+    next->xq[i] = next_workspaces[i];
+    next->q6 |= (uint32_t)(next_types[i] == COGNI_TYPE_Q6_K) << i;
+  }
+  return 0;
+}
+static int gemm_tall_launch(const char* who, const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                            const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, const GemmNextArgs* next, void* stream) {
   GemmManyArgs list{};
   uint32_t end = 0;
   for (uint32_t i = 0; i < count; i++) {
@@ -1551,8 +1567,32 @@ int cogni_gemm_tall_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspa
     list.tile_end[i] = end += (out_dims[i] + 255) / 256;
   }
   list.count = count;
+  GemmNextArgs none{};
   void* params[] = {&list, &workspace, &in_dim, &tokens};
-  return launch("q4_k_gemm_tall_f16", gemm_tiles_grid((tokens + 255) / 256, end), 256, 0, params, stream);
+  void* params_next[] = {&list, next ? const_cast<GemmNextArgs*>(next) : &none, &workspace, &in_dim, &tokens};
+  return launch(next ? "q4_k_gemm_tall_pack_f16" : "q4_k_gemm_tall_f16", gemm_tiles_grid((tokens + 255) / 256, end), 256, 0, next ? params_next : params,
+                stream);
+}
+static int gemm_tall_list_check(const char* who, const uint64_t* w_raw, uint32_t w_type, const uint64_t* outs, const uint32_t* out_dims, uint32_t count) {
+  if (w_type != COGNI_TYPE_Q4_K)
+    return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the GEMM of 256-token tiles: ") + type_name(w_type));
+  if (!w_raw || !outs || !out_dims || count == 0 || count > 6) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": one to six matrices");
+  return 0;
+}
+int cogni_gemm_tall_pack_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                             const uint32_t* out_dims, const uint32_t* next_types, const uint64_t* next_workspaces, const size_t* next_bytes,
+                             uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_tall_pack_dev";
+  GemmNextArgs next{};
+  if (int rc = gemm_tall_list_check(who, w_raw, w_type, outs, out_dims, count)) return rc;
+  if (int rc = gemm_next_of(who, &next, next_types, next_workspaces, next_bytes, out_dims, count, tokens)) return rc;
+  return gemm_tall_launch(who, w_raw, w_type, workspace, workspace_bytes, outs, out_dims, count, in_dim, tokens, &next, stream);
+}
+int cogni_gemm_tall_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                        const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_tall_dev";
+  if (int rc = gemm_tall_list_check(who, w_raw, w_type, outs, out_dims, count)) return rc;
+  return gemm_tall_launch(who, w_raw, w_type, workspace, workspace_bytes, outs, out_dims, count, in_dim, tokens, nullptr, stream);
 }
 int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                     uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
@@ -1581,12 +1621,13 @@ static int gemm_stream_sum(uint64_t planes, uint64_t add, uint32_t add_stride, u
 }
 static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t add,
                               uint32_t add_stride, const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim,
-                              uint32_t tokens, void* stream) {
+                              uint32_t tokens, void* stream, GemmNextArgs* next = nullptr) {
   const size_t packed_bytes = cogni_gemm_workspace_bytes(w_type, in_dim, tokens);
   if (packed_bytes > GEMM_STREAM_MAX_PACKED) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": packed activations of 2 GiB or more");
   uint64_t rows = 0;
   for (uint32_t i = 0; i < count; i++) rows += out_dims[i];
-  const uint32_t planes_max = count == 1 ? gemm_stream_planes(packed_bytes, workspace_bytes, tokens, out_dims[0]) : 1u;   // (one matrix only)
+  // (one matrix only, and a plane's sums are not what is packed)
+  const uint32_t planes_max = count == 1 && !next ? gemm_stream_planes(packed_bytes, workspace_bytes, tokens, out_dims[0]) : 1u;
   const GemmStreamPlan p = gemm_stream_plan(w_type, tokens, in_dim, rows, planes_max);
   GemmManyArgs list{};
   uint32_t end = 0;
@@ -1598,6 +1639,11 @@ static int gemm_stream_launch(const char* who, const uint64_t* w_raw, uint32_t w
   }
   list.count = count;
   char name[64];
+  if (next) {
+    std::snprintf(name, sizeof name, "%s_gemm_stream_pack_f16_%ux%u", type_prefix(w_type), p.t, p.rt);
+    void* params[] = {&list, next, &workspace, &in_dim, &tokens};
+    return launch(name, gemm_stream_grid(tokens, p.t, end), 256, 0, params, stream);
+  }
   std::snprintf(name, sizeof name, "%s_gemm_stream_f16_%ux%u", type_prefix(w_type), p.t, p.rt);
   uint64_t kadd = p.splits > 1 ? 0 : add;
   void* params[] = {&list, &workspace, &kadd, &add_stride, &in_dim, &tokens};
@@ -1621,6 +1667,21 @@ int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t works
   }
   return gemm_stream_launch(who, w_raw, w_type, workspace, workspace_bytes, residual, residual ? out_dims[0] : 0, outs, out_dims, count, in_dim,
                             tokens, stream);
+}
+int cogni_gemm_stream_pack_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                               const uint32_t* out_dims, const uint32_t* next_types, const uint64_t* next_workspaces, const size_t* next_bytes,
+                               uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_stream_pack_dev";
+  GemmNextArgs next{};
+  if (w_type != COGNI_TYPE_Q4_K && w_type != COGNI_TYPE_Q5_K)
+    return fail(COGNI_ERR_UNSUPPORTED_TYPE, std::string("Unsupported quant type for the GEMM that packs its outputs: ") + type_name(w_type));
+  if (!w_raw || !outs || !out_dims || count == 0 || count > 6) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": one to six matrices");
+  for (uint32_t i = 0; i < count; i++) {
+    if (!w_raw[i] || !outs[i]) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+    if (int rc = gemm_check(who, w_type, in_dim, out_dims[i], tokens, workspace, workspace_bytes)) return rc;
+  }
+  if (int rc = gemm_next_of(who, &next, next_types, next_workspaces, next_bytes, out_dims, count, tokens)) return rc;
+  return gemm_stream_launch(who, w_raw, w_type, workspace, workspace_bytes, 0, 0, outs, out_dims, count, in_dim, tokens, stream, &next);
 }
 
 // Two matrices with an input each: one launch where both go in tiles of 32 rows (with 64 rows a matrix fills the chip by itself).

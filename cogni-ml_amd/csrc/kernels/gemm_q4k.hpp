@@ -388,6 +388,25 @@ struct GemmManyArgs {
   u32 count;
 };
 
+// Packed inputs that a list writes beside its outputs: xq[i] is the image that pack_x_f16_* would make of out[i] (null: none), of the Q6_K
+// layout where bit i of q6 is set.
+struct GemmNextArgs {
+  uint2* xq[GEMM_MANY_MAX];
+  u32 q6;
+};
+// the cell of a super-block that its values k .. k + 7 fill (pack_x_core)
+__device__ __forceinline__ u32 gemm_next_cell(bool q6, u32 k) {
+  const u32 g6 = k >> 6;
+  return q6 ? 2 * (8 * (k >> 7) + 2 * ((k >> 5) & 3) + ((k >> 3) & 1)) + ((k >> 4) & 1)
+            : 2 * (8 * (g6 >> 1) + 4 * ((k >> 4) & 1) + 2 * ((k >> 5) & 1) + ((k >> 3) & 1)) + (g6 & 1);
+}
+// four neighbouring sums as half a cell; the absent tokens are zeros
+__device__ __forceinline__ uint2 gemm_next_half(float4 v, bool there) {
+  if (!there) v = make_float4(0.f, 0.f, 0.f, 0.f);
+  const __half2 p0 = __floats2half2_rn(v.x, v.z), p1 = __floats2half2_rn(v.y, v.w);   // slot order 0,2,1,3
+  return make_uint2(__builtin_bit_cast(u32, p0), __builtin_bit_cast(u32, p1));
+}
+
 // raw bytes of one group of one super-block of one weight row, as a lane sees them
 template <bool Q5>
 struct GemmRawT {

@@ -3,6 +3,7 @@
 //
 //   q4_k_gemm_tall_f16 (list: GemmManyArgs by value, tile_end in tiles of 256 rows, xp, in_dim:u32, m:u32)
 //                      block 256, grid gemm_tiles_grid(ceil(m/256), tiles) from gemv_config.h, no dynamic LDS (160 KiB static)
+//   q4_k_gemm_tall_pack_f16 (list, next: GemmNextArgs by value, xp, in_dim, m): next.xq[i] gets out[i] as the packed input of a following GEMM
 //   q4_k_gemm_tall_swiglu_pack_q4k|q6k_f16 (w_gate, w_up, xp, out | null, xq, in_dim, out_dim, m): a tile is 128 rows of each matrix;
 //                      grid gemm_tiles_grid(ceil(m/256), ceil(out_dim/128)); products and packed activations as the kernels of gemm_q4k.hpp
 //   xp is the image pack_x_f16_q4k writes.
@@ -179,10 +180,36 @@ __device__ __forceinline__ void gemm_tall_swiglu(const float16_t (&acc)[8][2], f
   else half(std::integral_constant<int, 1>{});
 }
 
-// PACK 0: a list of matrices. 12 | 14: gate | up with SwiGLU, the products packed for a next matrix of that type.
-template <int PACK>
+// The sums as packed inputs of following GEMMs, straight from the registers: the lanes j and 32 + j hold the halves of a cell, two quads of them
+// are exchanged so that each lane has a whole one. (out_dim is whole super-blocks, so all 64 rows exist or none.) 512 tokens x 30720 x 4096, 16384 of the
+// rows packed: 123 us, 129 with a pack launch behind the list; with stores of half cells there was nothing to gain.
+__device__ __forceinline__ void gemm_tall_next(const float16_t (&acc)[8][2], uint4* xq, bool q6, u32 out_dim, u32 m, u32 mt, u32 row0, u32 j, u32 kg) {
+  const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM;
+  if (row0 >= out_dim) return;
+  uint4* const dst = xq + ((size_t)(2 * mt) * (out_dim >> 8) + (row0 >> 8)) * 4096 + j;
+  const size_t tile = (size_t)(out_dim >> 8) * 4096;
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; g4 += 2) {
+      const u32 cell = gemm_next_cell(q6, (row0 & 255u) + 32 * c + 8 * (g4 + kg));
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        if (2 * mt + (r >> 2) >= mtiles) break;
+        const bool there = mt * GEMM_TALL_BM + 32 * r + j < m;
+        const float16_t& t = acc[r][c];
+        const uint2 e = gemm_next_half(make_float4(t[4 * g4], t[4 * g4 + 1], t[4 * g4 + 2], t[4 * g4 + 3]), there);
+        const uint2 o = gemm_next_half(make_float4(t[4 * g4 + 4], t[4 * g4 + 5], t[4 * g4 + 6], t[4 * g4 + 7]), there);
+        const auto x = __builtin_amdgcn_permlane32_swap(e.x, o.x, false, false), y = __builtin_amdgcn_permlane32_swap(e.y, o.y, false, false);
+        dst[(r >> 2) * tile + cell * 128 + 32 * (r & 3)] = make_uint4(x[0], y[0], x[1], y[1]);
+      }
+    }
+}
+
+// PACK 0: a list of matrices, NEXT: their outputs as packed inputs too. 12 | 14: gate | up with SwiGLU, the products packed for a next matrix of that type.
+template <int PACK, bool NEXT = false>
 __device__ __forceinline__ void gemm_tall_core(const uint8_t* w, const uint8_t* w_b, const uint4* xp, float* out, uint2* xq, u32 in_dim, u32 out_dim,
-                                               u32 m, const GemmManyArgs* many) {
+                                               u32 m, const GemmManyArgs* many, const GemmNextArgs* next = nullptr) {
   constexpr u32 BS = 144, TILE_ROWS = PACK ? GEMM_TALL_BN / 2 : GEMM_TALL_BN;   // rows of a matrix a tile covers
   const u32 tid = threadIdx.x, lane = tid & 63;
   const u32 nh = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -192,6 +219,7 @@ __device__ __forceinline__ void gemm_tall_core(const uint8_t* w, const uint8_t* 
   const u32 ntiles = PACK ? (out_dim + TILE_ROWS - 1) / TILE_ROWS : many->tile_end[many->count - 1];
   u32 mt, nt;
   if (!gemm_tile_of(blockIdx.x, mtiles, ntiles, &mt, &nt)) return;
+  [[maybe_unused]] u32 mi = 0;
   if constexpr (PACK == 0) {   // the tile's matrix, uniform over the workgroup
     u32 i = 0, first = 0;
     while (i + 1 < many->count && nt >= many->tile_end[i]) first = many->tile_end[i++];
@@ -199,6 +227,7 @@ __device__ __forceinline__ void gemm_tall_core(const uint8_t* w, const uint8_t* 
     w = many->w[i];
     out = many->out[i];
     out_dim = many->out_dim[i];
+    if constexpr (NEXT) mi = i;
   }
   const size_t row_bytes = (size_t)nkb * BS;
   const u32 sh = 16u * kg;
@@ -415,6 +444,9 @@ __device__ __forceinline__ void gemm_tall_core(const uint8_t* w, const uint8_t* 
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last (unused) copies
   __syncthreads();
+  if constexpr (NEXT) {
+    if (next->xq[mi]) gemm_tall_next(acc, reinterpret_cast<uint4*>(next->xq[mi]), next->q6 >> mi & 1u, out_dim, m, mt, row0, j, kg);
+  }
   if constexpr (PACK != 0) gemm_tall_swiglu<PACK>(acc, out, out_dim, m, mt, nt, nh, j, kg, lane, xq);
   else gemm_tall_store(acc, reinterpret_cast<float4*>(nh == 0 ? gemm_tall_x0 : (nh == 1 ? gemm_tall_x1 : (nh == 2 ? gemm_tall_x2 : gemm_tall_x3))), out, out_dim, m,
                        mt * GEMM_TALL_BM, row0, j, kg, lane);
@@ -423,6 +455,9 @@ __device__ __forceinline__ void gemm_tall_core(const uint8_t* w, const uint8_t* 
 #define GEMM_TALL_KERNEL extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 GEMM_TALL_KERNEL q4_k_gemm_tall_f16(const GemmManyArgs list, const uint4* xp, u32 in_dim, u32 m) {
   gemm_tall_core<0>(nullptr, nullptr, xp, nullptr, nullptr, in_dim, 0, m, &list);
+}
+GEMM_TALL_KERNEL q4_k_gemm_tall_pack_f16(const GemmManyArgs list, const GemmNextArgs next, const uint4* xp, u32 in_dim, u32 m) {
+  gemm_tall_core<0, true>(nullptr, nullptr, xp, nullptr, nullptr, in_dim, 0, m, &list, &next);
 }
 GEMM_TALL_KERNEL q4_k_gemm_tall_swiglu_pack_q4k_f16(const uint8_t* w_gate, const uint8_t* w_up, const uint4* xp, float* out, uint2* xq, u32 in_dim,
                                                     u32 out_dim, u32 m) {

@@ -10,6 +10,9 @@
 //   q4_k_gemm_stream_swiglu_pack_q4k|q6k_f16_<T>x2   (list of the gate matrix (out may be null), w_up, xp, xq, in_dim, m): a gate
 //                                     tile and the up tile of the same 32 rows per wavefront; silu(gate) * up to out and as the packed input
 //                                     of the next GEMM to xq (the absent tokens of a 32-token tile as zeros)
+//   q4_k|q5_k_gemm_stream_pack_f16_<T>x<RT> (list, next, xp, in_dim, m): without splits, and next.xq[i] gets out[i] as the packed input of a
+//                                     following GEMM, rounded from the sums as they are stored. (q | k | v | gate | up of a layer at 48 tokens, packed for o and down: their pack launch
+//                                     of 4 us is gone and the list takes no longer, the layer's projections 62.2 -> 59.2 us.)
 //   <type_a>_and_<type_b>_gemm_stream_f16_<T>x1 (list_a, xp_a, in_dim_a, splits_a, list_b, xp_b, in_dim_b, splits_b, m): two matrices
 //                                     with an input each (o and down of a layer) in one launch, grid = splits x gemm_stream_grid of both
 //
@@ -139,7 +142,7 @@ constexpr u32 gemm_stream_lds() {
 template <class W, int T, int RT, bool SWIGLU = false, int PACK = 0>
 __device__ __forceinline__ void gemm_stream_core(uint4* lds, const GemmManyArgs& list, const uint4* xp, const float* add, u32 add_stride, u32 in_dim,
                                                  u32 m, const uint8_t* w_up = nullptr, uint2* xq = nullptr, u32 bid = blockIdx.x,
-                                                 u32 split = blockIdx.y, u32 nsplits = gridDim.y) {
+                                                 u32 split = blockIdx.y, u32 nsplits = gridDim.y, const GemmNextArgs* next = nullptr) {
   static_assert(!SWIGLU || RT == 2, "a gate tile and the up tile of the same rows");
   constexpr int NM = SWIGLU ? 2 : 1;                             // matrices the workgroup's row tiles come from
   constexpr u32 PIECES = 32 * RT / NM * W::PPR;                  // 16-byte pieces of a matrix's rows per super-block
@@ -324,10 +327,14 @@ __device__ __forceinline__ void gemm_stream_core(uint4* lds, const GemmManyArgs&
   };
   const u32 n4 = n0 + 8 * wave + 4 * kg;
   if constexpr (!SWIGLU) {
+    uint2* const image = PACK ? next->xq[mi] : nullptr;   // (out_dim is whole super-blocks then)
 #pragma unroll
     for (u32 i = 0; i < RT * T; i++) {
       const float4 s = sum(i);
       const u32 n = n4 + 32 * (i / T), token = 32 * (mt * T + i % T) + j;
+      if (PACK && image && n < out_dim && token < 128 * ((m + 127) / 128))
+        image[(((size_t)(token >> 7) * (out_dim >> 8) + (n >> 8)) * 4096 + gemm_next_cell(next->q6 >> mi & 1u, n & 248u) * 128 + (token & 127)) * 2 + kg] =
+            gemm_next_half(s, token < m);
       if (n < out_dim && token < m)
         store(out + (size_t)token * out_dim + n, n, s, add ? add + (size_t)token * add_stride + n : nullptr);
     }
@@ -368,6 +375,20 @@ __device__ __forceinline__ void gemm_stream_core(uint4* lds, const GemmManyArgs&
     __shared__ uint4 lds[gemm_stream_lds<W, T, RT>()];                                                                                \
     gemm_stream_core<W, T, RT>(lds, list, xp, add, add_stride, in_dim, m);                                                            \
   }
+// a list that writes packed inputs too: PACK 1, next->xq[i] of out[i]
+#define GEMM_STREAM_PACK_ENTRY(PREFIX, W, T, RT, OCC)                                                                                     \
+  extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void PREFIX##_gemm_stream_pack_f16_##T##x##RT( \
+      const GemmManyArgs list, const GemmNextArgs next, const uint4* xp, u32 in_dim, u32 m) {                                             \
+    __shared__ uint4 lds[gemm_stream_lds<W, T, RT>()];                                                                                     \
+    gemm_stream_core<W, T, RT, false, 1>(lds, list, xp, nullptr, 0, in_dim, m, nullptr, nullptr, blockIdx.x, 0, 1, &next);                 \
+  }
+#define GEMM_STREAM_PACK_TYPE(PREFIX, W)    \
+  GEMM_STREAM_PACK_ENTRY(PREFIX, W, 1, 1, 3) \
+  GEMM_STREAM_PACK_ENTRY(PREFIX, W, 1, 2, 2) \
+  GEMM_STREAM_PACK_ENTRY(PREFIX, W, 2, 1, 2) \
+  GEMM_STREAM_PACK_ENTRY(PREFIX, W, 2, 2, 2)
+GEMM_STREAM_PACK_TYPE(q4_k, StreamQ4K)
+GEMM_STREAM_PACK_TYPE(q5_k, StreamQ5K)
 #define GEMM_STREAM_TYPE(PREFIX, W)    \
   GEMM_STREAM_ENTRY(PREFIX, W, 1, 1, 3) \
   GEMM_STREAM_ENTRY(PREFIX, W, 1, 2, 2) \

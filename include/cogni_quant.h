@@ -521,6 +521,12 @@ int32_t cogni_gemm_tall_takes(uint32_t w_type, uint32_t in_dim, const uint32_t* 
 int32_t cogni_gemm_tall_swiglu_takes(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens);
 int cogni_gemm_tall_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
                         const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
+/* cogni_gemm_tall_dev that also writes outs[i] as the packed activations of a following GEMM of type next_types[i] to next_workspaces[i]
+ * (0: not), the bytes cogni_gemm_pack_dev would make of it: out_dims[i] a multiple of 256, next_bytes[i] >= cogni_gemm_workspace_bytes(
+ * next_types[i], out_dims[i], tokens), no workspace overlapping another. */
+int cogni_gemm_tall_pack_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                             const uint32_t* out_dims, const uint32_t* next_types, const uint64_t* next_workspaces, const size_t* next_bytes,
+                             uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
 int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                     uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
                                     uint32_t tokens, void* stream);
@@ -540,6 +546,11 @@ int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_t
 int cogni_gemm_stream_takes(uint32_t w_type, uint32_t in_dim, uint32_t rows, uint32_t tokens);
 int cogni_gemm_stream_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t residual,
                           const uint64_t* outs, const uint32_t* out_dims, uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
+/* cogni_gemm_stream_dev (Q4_K, Q5_K) without a residual or a k split that also writes packed activations, as cogni_gemm_tall_pack_dev does; of
+ * the absent tokens only those of the last tile of 32 are written (zeros). */
+int cogni_gemm_stream_pack_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, const uint64_t* outs,
+                               const uint32_t* out_dims, const uint32_t* next_types, const uint64_t* next_workspaces, const size_t* next_bytes,
+                               uint32_t count, uint32_t in_dim, uint32_t tokens, void* stream);
 int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a, size_t bytes_a, uint64_t out_a, uint32_t in_dim_a,
                               uint32_t out_dim_a, uint64_t w_b, uint32_t type_b, uint64_t workspace_b, size_t bytes_b, uint64_t out_b,
                               uint32_t in_dim_b, uint32_t out_dim_b, uint32_t tokens, void* stream);
