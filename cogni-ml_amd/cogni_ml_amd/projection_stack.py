@@ -81,6 +81,10 @@ class QwenProjectionStackRunner:
                 if self._one_pass16(t, in_dim) and key not in self._images16:
                     self._images16[key] = self._alloc(quant.gemv_image_bytes(t, in_dim, quant.MAX_GEMV_TOKENS))
             self._prefill_ws = {k: (self._alloc(n), n) for k, n in need.items()}
+        # planes of two single matrices that share a launch, allocated where some token count may take it
+        self._two_scratch = self._alloc(quant.gemm_wide_two_scratch_bytes()) if self._prefill_ws and any(
+            self._wide_two(g[0], h[0], n) for groups in self._rounds for i, g in enumerate(groups) for h in groups[i + 1:] if len(g) == len(h) == 1
+            for n in [tokens, *range(193, tokens, 64)]) else None
         self._issued = {}   # prefill: the library calls of a token count
         self.outputs = {}
         self._runner = hip.ResidentSequenceRunner(
@@ -189,6 +193,10 @@ class QwenProjectionStackRunner:
         return "q6" if int(t) == int(TensorType.Q6_K) else "q45"
 
     @staticmethod
+    def _wide_two(a, b, count):
+        return quant.gemm_wide_two_takes(a[2], a[4], a[3], b[2], b[4], b[3], count)
+
+    @staticmethod
     def _gemm_capable(entry):
         return int(entry[2]) in (int(TensorType.Q4_K), int(TensorType.Q5_K), int(TensorType.Q6_K)) and entry[4] % 256 == 0
 
@@ -239,7 +247,13 @@ class QwenProjectionStackRunner:
             alone = [g[0] for g in groups if len(g) == 1]
             done = self._pairs([e for e in alone if (e[1], self._family(e[2])) in jobs16],
                                lambda a, b: quant.gemv_packed16_two_dev(*one_image(a), *one_image(b), count, stream))
-            done |= self._pairs([e for e in alone if (e[1], self._family(e[2])) not in jobs16 and
+            if self._two_scratch is not None:
+                for i, a in enumerate(alone):
+                    b = next((e for e in alone[i + 1:] if e[0] not in done and self._wide_two(a, e, count)), None)
+                    if b is not None and a[0] not in done:
+                        quant.gemm_wide_two_dev(*one_packed(a), *one_packed(b), self._two_scratch.ptr, quant.gemm_wide_two_scratch_bytes(), count, stream)
+                        done |= {a[0], b[0]}
+            done |= self._pairs([e for e in alone if (e[1], self._family(e[2])) not in jobs16 and e[0] not in done and
                                  quant.gemm_stream_takes(e[2], e[4], e[3], count)],
                                 lambda a, b: quant.gemm_stream_two_dev(*one_packed(a), *one_packed(b), count, stream))
             for grp in groups:

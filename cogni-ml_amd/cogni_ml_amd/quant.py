@@ -516,6 +516,27 @@ def gemm_tall_swiglu_pack_dev(w_gate_ptr, w_up_ptr, w_type, workspace_ptr, works
         ctypes.c_size_t(next_workspace_bytes), ctypes.c_uint32(in_dim), ctypes.c_uint32(out_dim), ctypes.c_uint32(tokens), stream))
 
 
+def gemm_wide_two_takes(type_a, in_dim_a, out_dim_a, type_b, in_dim_b, out_dim_b, tokens):
+    """Whether two matrices with an input each go into one launch of 128-token x 256-row tiles (gemm_wide_two_dev)."""
+    return bool(hip.lib().cogni_gemm_wide_two_takes(*[ctypes.c_uint32(int(v)) for v in (type_a, in_dim_a, out_dim_a, type_b, in_dim_b, out_dim_b,
+                                                                                        tokens)]))
+
+
+def gemm_wide_two_scratch_bytes():
+    f = hip.lib().cogni_gemm_wide_two_scratch_bytes
+    f.restype = ctypes.c_size_t
+    return f()
+
+
+def gemm_wide_two_dev(w_a, type_a, ws_a, ws_bytes_a, out_a, in_dim_a, out_dim_a, w_b, type_b, ws_b, ws_bytes_b, out_b, in_dim_b, out_dim_b,
+                      scratch_ptr, scratch_bytes, tokens, stream=None):
+    """Both matrices against their packed inputs in one launch, k split where that fills the chip, the planes in `scratch`."""
+    U64, U32, SZ = ctypes.c_uint64, ctypes.c_uint32, ctypes.c_size_t
+    _check(hip.lib().cogni_gemm_wide_two_dev(U64(w_a), U32(int(type_a)), U64(ws_a), SZ(ws_bytes_a), U64(out_a), U32(in_dim_a), U32(out_dim_a),
+                                             U64(w_b), U32(int(type_b)), U64(ws_b), SZ(ws_bytes_b), U64(out_b), U32(in_dim_b), U32(out_dim_b),
+                                             U64(scratch_ptr), SZ(scratch_bytes), U32(tokens), stream))
+
+
 def gemm_stream_takes(w_type, in_dim, rows, tokens):
     """Whether the router and the runners take the short-prefill kernels for a launch of `rows` rows in all."""
     return bool(hip.lib().cogni_gemm_stream_takes(ctypes.c_uint32(int(w_type)), ctypes.c_uint32(in_dim), ctypes.c_uint32(rows),

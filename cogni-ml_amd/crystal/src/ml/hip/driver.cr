@@ -164,6 +164,13 @@ lib LibCogniHIP
   fun cogni_gemm_tall_swiglu_pack_dev(w_gate : UInt64, w_up : UInt64, w_type : UInt32, workspace : UInt64, workspace_bytes : LibC::SizeT,
                                       out_ : UInt64, next_type : UInt32, next_workspace : UInt64, next_workspace_bytes : LibC::SizeT,
                                       in_dim : UInt32, out_dim : UInt32, tokens : UInt32, stream : Void*) : Int32
+  fun cogni_gemm_wide_two_takes(type_a : UInt32, in_dim_a : UInt32, out_dim_a : UInt32, type_b : UInt32, in_dim_b : UInt32, out_dim_b : UInt32,
+                                tokens : UInt32) : Int32
+  fun cogni_gemm_wide_two_scratch_bytes : LibC::SizeT
+  fun cogni_gemm_wide_two_dev(w_a : UInt64, type_a : UInt32, workspace_a : UInt64, bytes_a : LibC::SizeT, out_a : UInt64, in_dim_a : UInt32,
+                              out_dim_a : UInt32, w_b : UInt64, type_b : UInt32, workspace_b : UInt64, bytes_b : LibC::SizeT, out_b : UInt64,
+                              in_dim_b : UInt32, out_dim_b : UInt32, scratch : UInt64, scratch_bytes : LibC::SizeT, tokens : UInt32,
+                              stream : Void*) : Int32
   fun cogni_gemm_stream_takes(w_type : UInt32, in_dim : UInt32, rows : UInt32, tokens : UInt32) : Int32
   fun cogni_gemm_stream_dev(w_raw : UInt64*, w_type : UInt32, workspace : UInt64, workspace_bytes : LibC::SizeT, residual : UInt64,
                             outs : UInt64*, out_dims : UInt32*, count : UInt32, in_dim : UInt32, tokens : UInt32, stream : Void*) : Int32

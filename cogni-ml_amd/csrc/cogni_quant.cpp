@@ -1728,6 +1728,40 @@ int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_
   return gemm_stream_launch(who, &w_b, type_b, workspace_b, bytes_b, 0, 0, &out_b, &out_dim_b, 1, in_dim_b, tokens, stream);
 }
 
+int32_t cogni_gemm_wide_two_takes(uint32_t type_a, uint32_t in_dim_a, uint32_t out_dim_a, uint32_t type_b, uint32_t in_dim_b, uint32_t out_dim_b,
+                                  uint32_t tokens) {
+  unsigned sa, sb;
+  if (type_a == COGNI_TYPE_Q6_K) return gemm_wide_two_plan(type_b, in_dim_b, out_dim_b, type_a, in_dim_a, out_dim_a, tokens, &sa, &sb);
+  return gemm_wide_two_plan(type_a, in_dim_a, out_dim_a, type_b, in_dim_b, out_dim_b, tokens, &sa, &sb);
+}
+size_t cogni_gemm_wide_two_scratch_bytes(void) { return GEMM_WIDE_TWO_SCRATCH; }
+int cogni_gemm_wide_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a, size_t bytes_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a,
+                            uint64_t w_b, uint32_t type_b, uint64_t workspace_b, size_t bytes_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b,
+                            uint64_t scratch, size_t scratch_bytes, uint32_t tokens, void* stream) {
+  const char* who = "cogni_gemm_wide_two_dev";
+  if (type_a == COGNI_TYPE_Q6_K && type_b == COGNI_TYPE_Q4_K)
+    return cogni_gemm_wide_two_dev(w_b, type_b, workspace_b, bytes_b, out_b, in_dim_b, out_dim_b, w_a, type_a, workspace_a, bytes_a, out_a, in_dim_a,
+                                   out_dim_a, scratch, scratch_bytes, tokens, stream);
+  if (!w_a || !w_b || !out_a || !out_b) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
+  if (int rc = gemm_check(who, type_a, in_dim_a, out_dim_a, tokens, workspace_a, bytes_a)) return rc;
+  if (int rc = gemm_check(who, type_b, in_dim_b, out_dim_b, tokens, workspace_b, bytes_b)) return rc;
+  uint32_t sa = 1, sb = 1;
+  if (!gemm_wide_two_plan(type_a, in_dim_a, out_dim_a, type_b, in_dim_b, out_dim_b, tokens, &sa, &sb))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": not a launch for these kernels (cogni_gemm_wide_two_takes)");
+  const size_t planes_a = sa > 1 ? (size_t)sa * tokens * out_dim_a * sizeof(float) : 0, planes_b = sb > 1 ? (size_t)sb * tokens * out_dim_b * sizeof(float) : 0;
+  const size_t at_b = (planes_a + 255) / 256 * 256;
+  if ((planes_a || planes_b) && (!scratch || scratch_bytes < planes_a + planes_b || scratch_bytes < at_b + planes_b))
+    return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": scratch too small (cogni_gemm_wide_two_scratch_bytes)");
+  uint64_t to_a = sa > 1 ? scratch : out_a, to_b = sb > 1 ? scratch + at_b : out_b;
+  const uint32_t mt = (tokens + 127) / 128;
+  void* params[] = {&w_a, &workspace_a, &to_a, &in_dim_a, &out_dim_a, &sa, &w_b, &workspace_b, &to_b, &in_dim_b, &out_dim_b, &sb, &tokens};
+  const uint32_t grid = sa * gemm_tiles_grid(mt, (out_dim_a + 255) / 256) + sb * gemm_tiles_grid(mt, (out_dim_b + 255) / 256);
+  if (int rc = launch(type_b == COGNI_TYPE_Q6_K ? "q4_k_and_q6_k_gemm_wide_f16" : "q4_k_and_q4_k_gemm_wide_f16", grid, 512, 0, params, stream)) return rc;
+  if (sa > 1)
+    if (int rc = gemm_stream_sum(scratch, 0, 0, out_a, out_dim_a, tokens, sa, stream)) return rc;
+  return sb > 1 ? gemm_stream_sum(scratch + at_b, 0, 0, out_b, out_dim_b, tokens, sb, stream) : 0;
+}
+
 int cogni_gemm_stream_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type, uint64_t workspace, size_t workspace_bytes, uint64_t out,
                                       uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim,
                                       uint32_t out_dim, uint32_t tokens, void* stream) {

@@ -21,9 +21,13 @@ __shared__ uint4 gemm_q6w_x0[2048];        // [kh][k-step 0..3][k-group][128 tok
 __shared__ uint4 gemm_q6w_x1[2048];        // the same of k-steps 4..7
 __shared__ uint4 gemm_q6w_wbuf[8 * 384];   // [wavefront][64 rows][ql 4 pieces, qh 2 pieces]
 
-extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void q6_k_gemm_wide_f16(
-    const uint8_t* w, const uint4* xp, const float* bias, float* out, u32 in_dim, u32 out_dim, u32 m, u32 bias_stride) {
-  constexpr u32 BS = 210;
+// Q4: raw Q4_K weights (codes 64 kh of a row's super-block, four copies into the same region; headers from global memory) in the same loop. The
+// super-blocks [kb0, kb1) of the rows, by workgroup bid of the matrix's.
+template <bool Q4>
+__device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4* xp, const float* bias, float* out, u32 in_dim, u32 out_dim, u32 m,
+                                                   u32 bias_stride, u32 bid, u32 kb0, u32 kb1) {
+  constexpr u32 BS = Q4 ? 144 : 210;
+  constexpr int NW = Q4 ? 4 : 6;   // copies of a wavefront's weights per super-block
   const u32 tid = threadIdx.x, lane = tid & 63;
   const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const u32 nh = wave & 3, kh = wave >> 2;
@@ -31,7 +35,7 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   const u32 nkb = in_dim >> 8;
   const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM, ntiles = (out_dim + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN;
   u32 mt, nt;
-  if (!gemm_tile_of(blockIdx.x, mtiles, ntiles, &mt, &nt)) return;
+  if (!gemm_tile_of(bid, mtiles, ntiles, &mt, &nt)) return;
   const size_t row_bytes = (size_t)nkb * BS;
   // constants of the code assembly, kept in registers (as literals each (a & mask) | b would be two instructions): the masks
   // in scalar ones, of which an instruction takes one
@@ -44,17 +48,20 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   // loads through a buffer descriptor: scalar base, scalar offset of the super-block, a 32-bit offset per lane
   const __amdgpu_buffer_rsrc_t wrsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w + (size_t)base_row * row_bytes), 0, 0xFFFFFFFFu, 0x00027000);
-  // copy i of this wavefront: piece p = 64 i + lane is piece p % 6 of wave-local row p / 6
-  u32 woff[6];
+  // copy i of this wavefront: piece p = 64 i + lane is piece p % 6 of wave-local row p / 6 (Q4_K: of row p / 4 the piece that belongs in slot p % 4,
+  // as in gemm_q4k_wide.hpp)
+  u32 woff[NW];
 #pragma unroll
-  for (int i = 0; i < 6; i++) {
-    const u32 p = 64u * i + lane, r = p / 6u, part = p - 6u * r;
-    woff[i] = (min(row0 + r, out_dim - 1) - base_row) * (u32)row_bytes + (part < 4u ? 64u * kh + 16u * part : 128u + 32u * kh + 16u * (part - 4u));
+  for (int i = 0; i < NW; i++) {
+    const u32 p = 64u * i + lane, r = p / (u32)NW, part = p - NW * r;
+    const u32 at = Q4 ? 16u + 64u * kh + 16u * (part ^ ((r >> 2) & 3u)) : part < 4u ? 64u * kh + 16u * part : 128u + 32u * kh + 16u * (part - 4u);
+    woff[i] = (min(row0 + r, out_dim - 1) - base_row) * (u32)row_bytes + at;
   }
-  u32 soff[2];   // scales of the half, row c of this lane (d is 16 - 8 kh bytes further)
+  u32 soff[2];   // scales of the half, row c of this lane (d is 16 - 8 kh bytes further); Q4_K: the header
 #pragma unroll
-  for (int c = 0; c < 2; c++) soff[c] = (min(row0 + 32 * c + j, out_dim - 1) - base_row) * (u32)row_bytes + 192u + 8u * kh;
+  for (int c = 0; c < 2; c++) soff[c] = (min(row0 + 32 * c + j, out_dim - 1) - base_row) * (u32)row_bytes + (Q4 ? 0u : 192u + 8u * kh);
   const u32 wrow = wave * 384 + j * 6 + kg;   // the lane's first ql piece of its row c = 0 (c = 1: 192 further)
+  const u32 wrow4 = wave * 384 + j * 4, slot4 = (2u * kg) ^ ((j >> 2) & 3u);   // its two pieces 2 kg, 2 kg + 1: slots slot4, slot4 ^ 1 (c = 1: 128 further)
   const __amdgpu_buffer_rsrc_t xrsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(xp + (size_t)mt * nkb * 4096), 0, 0xFFFFFFFFu, 0x00027000);
 
@@ -71,7 +78,12 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   };
   uint2 nsc[2];
   u32 nd[2];
+  uint4 nh4[2];
   auto load_sc = [&](u32 kb, int c) {
+    if constexpr (Q4) {
+      nh4[c] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wrsrc, soff[c], kb * BS, 0));
+      return;
+    }
     nsc[c] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(wrsrc, soff[c], kb * BS, 0));
     nd[c] = (u32)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(wrsrc, soff[c], kb * BS + (16u - 8u * kh), 0);
   };
@@ -89,6 +101,11 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   auto take_raw = [&]() {
 #pragma unroll
     for (int c = 0; c < 2; c++) {
+      if constexpr (Q4) {
+        cur[c].qa = gemm_q6w_wbuf[wrow4 + 128 * c + slot4];
+        cur[c].qb = gemm_q6w_wbuf[wrow4 + 128 * c + (slot4 ^ 1u)];
+        continue;
+      }
       cur[c].qa = gemm_q6w_wbuf[wrow + 192 * c];
       cur[c].qb = gemm_q6w_wbuf[wrow + 192 * c + 2];
       cur[c].qh = gemm_q6w_wbuf[wrow + 192 * c + 4];
@@ -98,6 +115,17 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   auto decode_scales = [&]() {
 #pragma unroll
     for (int c = 0; c < 2; c++) {
+      if constexpr (Q4) {
+        const float d4 = h2f(nh4[c].x), dm = h2f(nh4[c].x >> 16);
+        const u32 a0 = nh4[c].y >> (16 * kg), a1 = nh4[c].z >> (16 * kg), a2 = nh4[c].w >> (16 * kg);
+        const u32 scp = kh ? (a2 & 0x0F0Fu) | ((a0 >> 2) & 0x3030u) : a0 & 0x3F3Fu;
+        const u32 mp = kh ? ((a2 >> 4) & 0x0F0Fu) | ((a1 >> 2) & 0x3030u) : a1 & 0x3F3Fu;
+        S[c][0] = h2_dup(d4 * ubyte_f<0>(scp));
+        S[c][1] = h2_dup(-(dm * ubyte_f<0>(mp)));
+        S[c][2] = h2_dup(d4 * ubyte_f<1>(scp));
+        S[c][3] = h2_dup(-(dm * ubyte_f<1>(mp)));
+        continue;
+      }
       const float d = h2f(nd[c]);
       const u32 lo = nsc[c].x >> (8 * kg), hi = nsc[c].y >> (8 * kg);
       S[c][0] = h2_dup(d * (float)(int)(signed char)(lo & 0xFFu));
@@ -110,6 +138,19 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     const int qd = t >> 1, h8 = t & 1, hi = qd >> 1;
 #pragma unroll
     for (int c = 0; c < 2; c++) {
+      if constexpr (Q4) {   // as in gemm_wide_core
+        const int op = t & 3, up = op >> 1;
+        const uint4 P = (t >> 2) ? cur[c].qb : cur[c].qa;
+        const u32 q0 = (op & 1) ? P.z : P.x, q1 = (op & 1) ? P.w : P.y;
+        const u32 msk = up ? mask_hi : mask_lo, mag = up ? magic_hi : magic_lo, of = up ? 0xD400D400u : 0xE400E400u;
+        uint4 b4;
+        b4.x = h2_fma_off((q0 & msk) | mag, of, S[c][2 * up], S[c][2 * up + 1]);
+        b4.y = h2_fma_off(((q0 >> 8) & msk) | mag, of, S[c][2 * up], S[c][2 * up + 1]);
+        b4.z = h2_fma_off((q1 & msk) | mag, of, S[c][2 * up], S[c][2 * up + 1]);
+        b4.w = h2_fma_off(((q1 >> 8) & msk) | mag, of, S[c][2 * up], S[c][2 * up + 1]);
+        Bd[c] = *reinterpret_cast<const half8_t*>(&b4);
+        continue;
+      }
       const uint4 Q = (qd & 1) ? cur[c].qb : cur[c].qa;
       const u32 qa = h8 ? Q.z : Q.x, qb = h8 ? Q.w : Q.y;
       const u32 ha = h8 ? cur[c].qh.z : cur[c].qh.x, hb = h8 ? cur[c].qh.w : cur[c].qh.y;
@@ -135,13 +176,13 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   };
 
 #pragma unroll
-  for (int i = 0; i < 6; i++) copy_w(0, i);
+  for (int i = 0; i < NW; i++) copy_w(kb0, i);
 #pragma unroll
-  for (int c = 0; c < 2; c++) load_sc(0, c);
+  for (int c = 0; c < 2; c++) load_sc(kb0, c);
 #pragma unroll
-  for (int i = 0; i < 4; i++) copy_x(0, 0, i);
+  for (int i = 0; i < 4; i++) copy_x(kb0, 0, i);
 #pragma unroll
-  for (int i = 0; i < 4; i++) copy_x(0, 1, i);
+  for (int i = 0; i < 4; i++) copy_x(kb0, 1, i);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   take_raw();
@@ -150,8 +191,8 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   build_b(B[0], 0);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 
-  for (u32 kb = 0; kb < nkb; kb++) {
-    const u32 kn = min(kb + 1, nkb - 1);   // the last iteration copies its own tile again; it is not used
+  for (u32 kb = kb0; kb < kb1; kb++) {
+    const u32 kn = min(kb + 1, kb1 - 1);   // the last iteration copies its own tile again; it is not used
 #pragma unroll
     for (int t = 0; t < 8; t++) {
       const int p = t & 1;
@@ -160,7 +201,7 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
       // other, in front of which the compiler waits for every load in flight.
       if (t == 0) {
 #pragma unroll
-        for (int i = 0; i < 6; i++) copy_w(kn, i);
+        for (int i = 0; i < NW; i++) copy_w(kn, i);
       }
       if (t == 3) {
         read_a(A[p ^ 1], t + 1);
@@ -210,9 +251,9 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
       }
       __builtin_amdgcn_sched_barrier(0);
       if (t == 2) {
-        // half 1 of this super-block (copies of the last k-step before; the six weight copies of k-step 0 are younger) is there
+        // half 1 of this super-block (copies of the last k-step before; the NW weight copies of k-step 0 are younger) is there
         // and half 0 has been read, for every wavefront
-        asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(NW) : "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -234,3 +275,33 @@ extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   if (kh == 0) gemm_wide_epilogue_half<0, 2>(acc, h0, h1, bias, out, out_dim, m, mt, nt, nh, j, kg, lane, bias_stride);
   else gemm_wide_epilogue_half<1, 2>(acc, h1, h0, bias, out, out_dim, m, mt, nt, nh, j, kg, lane, bias_stride);
 }
+
+extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void q6_k_gemm_wide_f16(
+    const uint8_t* w, const uint4* xp, const float* bias, float* out, u32 in_dim, u32 out_dim, u32 m, u32 bias_stride) {
+  gemm_q6k_wide_core<false>(w, xp, bias, out, in_dim, out_dim, m, bias_stride, blockIdx.x, 0, in_dim >> 8);
+}
+
+// Two matrices with an input each (Q4_K, and Q4_K or Q6_K: o and down of a layer), each over all its super-blocks or split in planes out + split m out_dim:
+//   q4_k_and_q6_k|q4_k_gemm_wide_f16 (w_a, xp_a, out_a, in_dim_a, out_dim_a, splits_a, w_b, xp_b, out_b, in_dim_b, out_dim_b, splits_b, m)
+//                      grid = splits x gemm_tiles_grid of both, b's first: the rows of down are the longer ones
+// 512 tokens of 4096 -> 4096 beside Q6_K 12288 -> 4096, plane sums included: 90 us; 110 as launches of their own, of which o's fills half the chip and down's
+// 128-row tiles reach 0.7 PFLOP/s. Splits by gemm_wide_two_plan (gemv_config.h). Q4_K in this loop instead of gemm_wide_core's because both have to share LDS.
+#define GEMM_WIDE_TWO_ENTRY(PREFIX_A, A4, PREFIX_B, B4)                                                                                           \
+  extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void PREFIX_A##_and_##PREFIX_B##_gemm_wide_f16(         \
+      const uint8_t* w_a, const uint4* xp_a, float* out_a, u32 in_dim_a, u32 out_dim_a, u32 splits_a, const uint8_t* w_b, const uint4* xp_b,      \
+      float* out_b, u32 in_dim_b, u32 out_dim_b, u32 splits_b, u32 m) {                                                                           \
+    const u32 mt = (m + GEMM_BM - 1) / GEMM_BM;                                                                                                   \
+    const u32 wgs_a = gemm_tiles_grid(mt, (out_dim_a + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN);                                                         \
+    const u32 wgs_b = gemm_tiles_grid(mt, (out_dim_b + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN), first_a = wgs_b * splits_b;                             \
+    if (blockIdx.x < first_a) {                                                                                                                   \
+      const u32 s = blockIdx.x / wgs_b, n = in_dim_b >> 8;                                                                                        \
+      gemm_q6k_wide_core<B4>(w_b, xp_b, nullptr, out_b + (size_t)s * m * out_dim_b, in_dim_b, out_dim_b, m, 0, blockIdx.x % wgs_b,                \
+                             s * n / splits_b, (s + 1) * n / splits_b);                                                                           \
+    } else {                                                                                                                                      \
+      const u32 id = blockIdx.x - first_a, s = id / wgs_a, n = in_dim_a >> 8;                                                                     \
+      gemm_q6k_wide_core<A4>(w_a, xp_a, nullptr, out_a + (size_t)s * m * out_dim_a, in_dim_a, out_dim_a, m, 0, id % wgs_a, s * n / splits_a,      \
+                             (s + 1) * n / splits_a);                                                                                             \
+    }                                                                                                                                             \
+  }
+GEMM_WIDE_TWO_ENTRY(q4_k, true, q6_k, false)
+GEMM_WIDE_TWO_ENTRY(q4_k, true, q4_k, true)

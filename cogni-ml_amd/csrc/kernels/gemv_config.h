@@ -358,6 +358,35 @@ static inline int gemm_tall_swiglu_takes(unsigned type, unsigned in_dim, unsigne
          gemm_fill_cost(mt * gemm_list_tiles(&out_dim, 1u, wide ? 128u : 96u), gemm_tile_cost(12u, wide ? 256u : 192u));
 }
 
+// Two matrices with an input each in one launch of 128-token x 256-row tiles, each with its own k splits (gemm_q6k_wide.hpp; a: Q4_K, b: Q4_K
+// or Q6_K: o and down of a layer): the two share the chip where one alone would leave half of it idle, and the splits even their chains out. The plan is the
+// cheapest of those whose tiles fit one round of the chip: start and end 11 us, the longer chain at 3.7 (Q4_K) or 4.2 us (Q6_K) a super-block, a split
+// matrix's planes at 5 TB/s and a launch (within a tenth of what 36 shapes measured). Taken from 1300 tile super-blocks in all, below which the
+// launches of their own do better, and where the plan's time is less than what those reach at their best, 19.5 ns a tile super-block and
+// 36 us of starts, ends and sums. Weights from memory, us, launches of their own | this: o 4096 -> 4096 and Q6_K down 12288 -> 4096 at 256 | 384 | 512 | 640 tokens 59.9 |
+// 94 | 110 | 159 and 59.0 | 73.5 | 90 | 115 (1024: 162 | 180, not taken: chains of 48), Q4_K down at 512 90.5 | 83.6; 2560 -> 2560 and 9728 -> 2560 at 300 | 700
+// tokens 78.5 | 130 and 50 | 72.5; 2048 and 11008 at 700 85.6 | 64; 1536 and 8448 at 546 (1170 super-blocks) 36.5 | 40.6, 2048 and 10240 at 290 (1152) 35.4 | 39.7: not taken.
+#define GEMM_WIDE_TWO_SCRATCH (256ull * 128ull * 256ull * 4ull)   // the planes of a launch of one round at most
+static inline int gemm_wide_two_plan(unsigned type_a, unsigned in_a, unsigned out_a, unsigned type_b, unsigned in_b, unsigned out_b, unsigned tokens,
+                                     unsigned* splits_a, unsigned* splits_b) {
+  const unsigned long long mt = (tokens + 127ull) / 128ull, ta = mt * ((out_a + 255ull) / 256ull), tb = mt * ((out_b + 255ull) / 256ull);
+  const unsigned na = in_a >> 8, nb = in_b >> 8;
+  const unsigned long long work = ta * na + tb * nb;
+  unsigned long long least = ~0ull;   // ns
+  unsigned sa, sb;
+  if (type_a != 12u || (type_b != 12u && type_b != 14u) || ((in_a | in_b) & 255u) != 0 || tokens <= 192u || ta + tb > 256u || work < 1300u) return 0;
+  for (sa = 1; sa == 1u || (sa <= 4u && 2u * sa <= na); sa++)
+    for (sb = 1; sb == 1u || (sb <= 8u && 2u * sb <= nb); sb++) {
+      const unsigned long long ca = ((na + sa - 1u) / sa) * 3700ull, cb = ((nb + sb - 1u) / sb) * (type_b == 14u ? 4200ull : 3700ull);
+      unsigned long long c = 11000ull + (ca > cb ? ca : cb);
+      if (ta * sa + tb * sb > 256u) break;
+      if (sa > 1u) c += 2000ull + (sa + 1ull) * tokens * out_a / 1250ull;
+      if (sb > 1u) c += 2000ull + (sb + 1ull) * tokens * out_b / 1250ull;
+      if (c < least) least = c, *splits_a = sa, *splits_b = sb;
+    }
+  return least < work * 195ull / 10ull + 36000ull;
+}
+
 // ---- prefill GEMM: which tile a workgroup takes. Workgroups go to the 8 XCDs round-robin (id % 8), each XCD has its own
 // L2 and 32 compute units, and a GEMM workgroup has a compute unit to itself, so the workgroups id = 8 l + x with the
 // same l / 32 run side by side on XCD x. Every XCD gets an equal share of the tiles (they are numbered in one line and it takes

@@ -531,6 +531,17 @@ int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_t
                                     uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
                                     uint32_t tokens, void* stream);
 
+/* Two matrices with an input each (o and down of a layer; Q4_K and a Q4_K or Q6_K one, in either order) in one launch of 128-token x 256-row tiles, the
+ * k range of each split as that fills the chip: the precision of cogni_gemm_packed_dev, sums in another order. Only what cogni_gemm_wide_two_takes says
+ * (1 or 0) is launched this way; scratch: cogni_gemm_wide_two_scratch_bytes() (32 MiB) are enough for any such launch. Nothing may overlap but the two
+ * workspaces, which are only read. */
+int32_t cogni_gemm_wide_two_takes(uint32_t type_a, uint32_t in_dim_a, uint32_t out_dim_a, uint32_t type_b, uint32_t in_dim_b, uint32_t out_dim_b,
+                                  uint32_t tokens);
+size_t cogni_gemm_wide_two_scratch_bytes(void);
+int cogni_gemm_wide_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a, size_t bytes_a, uint64_t out_a, uint32_t in_dim_a, uint32_t out_dim_a,
+                            uint64_t w_b, uint32_t type_b, uint64_t workspace_b, size_t bytes_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b,
+                            uint64_t scratch, size_t scratch_bytes, uint32_t tokens, void* stream);
+
 /* The short-prefill forms of the packed GEMMs: the weights streamed through many small workgroups instead of tiles of 128
  * tokens that have a compute unit to themselves. They read the same packed activations, their operands are rounded as the
  * tile kernels round them (fp16, fp32 sums; the order of the sums differs), and cogni_matmul_dev and the resident runners take

@@ -1,0 +1,92 @@
+"""Two prefill matrices with an input each in one launch, both with k splits of their own (o and down of a layer)."""
+import numpy as np
+import pytest
+
+from cogni_ml_amd import quant, synth
+from cogni_ml_amd.projection_stack import QwenProjectionStackRunner, Weights
+from gpu_common import DevArray, gpu  # noqa: F401
+from helpers import Q4_K, Q5_K, Q6_K
+
+pytestmark = pytest.mark.gpu
+
+
+def sums_bound(oracle, raw, t, x, out_dim, in_dim):
+    """Two fp32 sums of the same products in different orders differ by at most 2 n 2^-24 of the sum of their magnitudes (n additions)."""
+    w = np.abs(oracle.dequantize(raw, t, out_dim * in_dim).reshape(out_dim, in_dim))
+    return 2 * in_dim * 2.0**-24 * (np.abs(x) @ w.T) * 1.01   # (1.01: operands rounded to half)
+
+
+# tokens and rows that end inside a tile, inside a wavefront's rows, at them, of no multiple of four rows; no split, one matrix split, both;
+# splits that do not divide the super-blocks; the fewest tokens; either order; up to the 256 tiles of a round
+@pytest.mark.parametrize("tokens,a,b", [(897, (Q4_K, 512, 300), (Q6_K, 8448, 1283)), (193, (Q4_K, 2560, 2560), (Q4_K, 12288, 3072)),
+                                        (1024, (Q4_K, 2048, 1024), (Q4_K, 4096, 2560)), (320, (Q6_K, 9728, 2305), (Q4_K, 2304, 2304)),
+                                        (2049, (Q4_K, 256, 1), (Q6_K, 2048, 2560)), (640, (Q4_K, 2048, 1030), (Q6_K, 11008, 1536))])
+def test_two_matrices(gpu, oracle, tokens, a, b):
+    rng = np.random.default_rng(tokens)
+    assert quant.gemm_wide_two_takes(*a, *b, tokens)
+    mats, args = [], []
+    for t, in_dim, out_dim in (a, b):
+        raw, x = synth.make_weights(rng, t, out_dim, in_dim), synth.make_activations(rng, tokens, in_dim)
+        n = quant.gemm_workspace_bytes(t, in_dim, tokens)
+        w, xd, ws = DevArray(raw), DevArray(x), DevArray(nbytes=n)
+        one, two = (DevArray(np.full(tokens * out_dim + 4, np.float32(-3.0))) for _ in range(2))
+        quant.gemm_pack_dev(xd.ptr, t, in_dim, tokens, ws.ptr, n)
+        quant.gemm_packed_dev(w.ptr, t, ws.ptr, n, one.ptr, in_dim, out_dim, tokens)
+        mats.append((raw, t, x, in_dim, out_dim, w, xd, ws, one, two))
+        args += [w.ptr, t, ws.ptr, n, two.ptr, in_dim, out_dim]
+    size = quant.gemm_wide_two_scratch_bytes()
+    scratch = DevArray(np.full(size + 64, 0xFF, np.uint8))   # (NaN in every plane that nothing writes)
+    quant.gemm_wide_two_dev(*args, scratch.ptr, size, tokens)
+    assert np.all(scratch.read(np.uint8, size + 64)[size:] == 0xFF)
+    for raw, t, x, in_dim, out_dim, w, xd, ws, one, two in mats:
+        want, got = (o.read(np.float32, tokens * out_dim + 4) for o in (one, two))
+        assert np.array_equal(got[tokens * out_dim:], np.full(4, np.float32(-3.0)))
+        diff = np.abs(want[:-4].astype(np.float64) - got[:-4]).reshape(tokens, out_dim)
+        assert (diff <= sums_bound(oracle, raw, t, x.reshape(tokens, in_dim), out_dim, in_dim)).all(), (t, out_dim)
+        for v in (w, xd, ws, one, two):
+            v.close()
+    scratch.close()
+
+
+@pytest.mark.parametrize("down", [Q4_K, Q6_K])
+def test_runner_of_the_two(gpu, down, monkeypatch):
+    """The runner with and without this launch, a token count that it takes and one that it does not: the sums in another order, so fp32 to 2e-5 of a
+    token's largest (11008 terms: 2-norm 4e-7)."""
+    rng = np.random.default_rng(int(down))
+    weights = Weights.synthetic(rng, [("q", "x", Q4_K, 2048, 2048), ("gate", "x", Q4_K, 256, 2048), ("up", "x", Q4_K, 11008, 2048),
+                                      ("o", "q", Q4_K, 2048, 2048), ("down", "up", down, 2048, 11008)])
+    xs = synth.make_activations(rng, 500, 2048).reshape(-1) * np.float32(0.1)
+    seen, results = [], []
+    f = quant.gemm_wide_two_dev
+    monkeypatch.setattr(quant, "gemm_wide_two_dev", lambda *a: (seen.append(a[-2]), f(*a))[1])
+    for without in (False, True):
+        if without:
+            monkeypatch.setattr(quant, "gemm_wide_two_takes", lambda *a: False)
+        r = QwenProjectionStackRunner.from_weights(weights, 500, xs)
+        r.upload_weights()
+        r.reset_sequence()
+        for count in (100, 500):
+            r.active_tokens = count
+            r.run_sequence()
+        r.read_outputs()
+        results.append({k: v.reshape(500, -1).copy() for k, v in r.outputs.items()})
+        r.close()
+    assert seen == [500]
+    for k in results[0]:
+        a, b = results[0][k], results[1][k]
+        assert np.all(np.abs(a - b) <= 2e-5 * np.abs(b).max(axis=1, keepdims=True)), k
+
+
+def test_what_is_not_taken(gpu):
+    takes = quant.gemm_wide_two_takes
+    o, down = (Q4_K, 4096, 4096), (Q6_K, 12288, 4096)
+    assert [takes(*o, *down, m) for m in (64, 192, 256, 512, 640, 1024)] == [False, False, True, True, True, False]
+    assert takes(*down, *o, 512) and not takes(*down, *down, 512) and not takes(Q5_K, 4096, 4096, *down, 512)
+    assert not takes(Q4_K, 1792, 1792, Q6_K, 2560, 1792, 289) and not takes(Q4_K, 4096, 4096, Q6_K, 12200, 4096, 512)
+    args = [64, *o[:1], 64, 1 << 30, 64, *o[1:], 64, *down[:1], 64, 1 << 30, 64, *down[1:]]
+    with pytest.raises(quant.QuantError, match="not a launch for these kernels"):
+        quant.gemm_wide_two_dev(*args, 64, 1 << 30, 1024)
+    with pytest.raises(quant.QuantError, match="scratch too small"):
+        quant.gemm_wide_two_dev(*args, 64, 1 << 20, 512)
+    with pytest.raises(quant.QuantError, match="workspace has"):
+        quant.gemm_wide_two_dev(*(args[:3] + [16] + args[4:]), 64, 1 << 30, 512)
