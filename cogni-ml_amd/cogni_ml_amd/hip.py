@@ -112,17 +112,24 @@ class _NotingLib:
 
 
 def issue(kept, key, launch, check_status):
-    """launch(), which issues operators on the current stream: the first time with a `key` as it is written, later the same library calls
-    with the same arguments on the stream that is current then, without the Python that chose them (stack of seven projections,
-    48 tokens: 31 us of host time the first way). `kept` holds the calls, at most 32 keys of them; `key` names all that
-    the choice depends on beside what never changes for the owner of `kept`."""
+    """launch(), which issues operators on the current stream: the second time with a `key` the library calls that it makes are noted, and from the
+    third those are made again, with the same arguments on the stream that is current then, without the Python that chose them (stack of seven
+    projections, 48 tokens: 31 us of host time by launch()). Not the first time: noting takes 5 to 9 us, which one that is run only once would pay for
+    nothing. `kept` holds the calls, at most 32 keys of them; `key` names all that the choice depends on beside what never changes for the
+    owner of `kept`."""
     calls = kept.get(key)
-    if calls is not None:
+    if calls:
         stream = _current_stream
         for f, args in calls:
             code = f(*args, stream)
             if code != 0:
                 check_status(code)
+        return
+    if calls is None:
+        launch()
+        if len(kept) >= 32:
+            kept.clear()
+        kept[key] = ()
         return
     global _recording_threads
     calls, outer = [], (getattr(_noting, "calls", None), getattr(_noting, "lib", None))
@@ -136,8 +143,6 @@ def issue(kept, key, launch, check_status):
         _noting.calls, _noting.lib = outer
         with _recording_lock:
             _recording_threads -= 1
-    if len(kept) >= 32:
-        kept.clear()
     kept[key] = calls
 
 

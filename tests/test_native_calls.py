@@ -131,9 +131,10 @@ def test_a_sequence_is_issued_again_with_the_same_calls(monkeypatch):
         hip.lib().cogni_b_dev(2, hip.current_stream_handle())
 
     kept = {}
-    hip.issue(kept, 3, launch, raised.append)
-    assert fake.log == [("rule", 5), ("a", 1, 7, None), ("b", 99, None), ("b", 2, None)] and hip.lib() is fake
-    fake.log.clear()
+    for _ in range(2):   # as it is written; the same, noted
+        hip.issue(kept, 3, launch, raised.append)
+        assert fake.log == [("rule", 5), ("a", 1, 7, None), ("b", 99, None), ("b", 2, None)] and hip.lib() is fake
+        fake.log.clear()
     with hip.with_stream(stream):
         hip.issue(kept, 3, launch, raised.append)
     assert fake.log == [("a", 1, 7, "s1"), ("b", 2, "s1")] and raised == []
@@ -147,9 +148,14 @@ def test_a_sequence_is_issued_again_with_the_same_calls(monkeypatch):
     def fails():
         hip.lib().cogni_a_dev(1, None)
         raise KeyError("no")
+    fake.status = 0
     with pytest.raises(KeyError):
         hip.issue(kept, 5, fails, raised.append)
-    assert 5 not in kept and hip.lib() is fake
-    for k in range(100):
-        hip.issue(kept, 100 + k, launch, raised.append)
+    assert 5 not in kept
+    hip.issue(kept, 5, launch, raised.append)
+    with pytest.raises(KeyError):
+        hip.issue(kept, 5, fails, raised.append)
+    assert not kept[5] and hip.lib() is fake
+    for k in range(200):
+        hip.issue(kept, 100 + k // 2, launch, raised.append)
     assert len(kept) <= 32
