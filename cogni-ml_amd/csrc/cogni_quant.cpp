@@ -1493,7 +1493,7 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
       {{"q4_k_gemm_many_f16", "q4_k_gemm_many_n128_f16"}, {"q4_k_gemm_many_m64_f16", "q4_k_gemm_many_m64_n128_f16"}},
       {{"q5_k_gemm_many_f16", "q5_k_gemm_many_n128_f16"}, {"q5_k_gemm_many_m64_f16", "q5_k_gemm_many_m64_n128_f16"}}};
   void* params[] = {&list, &workspace, &in_dim, &tokens};
-  if (bn == 256) return launch("q4_k_gemm_many_wide_f16", gemm_tiles_grid((uint32_t)mtiles, end), 512, 0, params, stream);
+  if (bn == 256) return launch(w_type == COGNI_TYPE_Q5_K ? "q5_k_gemm_many_wide_f16" : "q4_k_gemm_many_wide_f16", gemm_tiles_grid((uint32_t)mtiles, end), 512, 0, params, stream);
   return launch(names[w_type == COGNI_TYPE_Q5_K][m64][bn == 128], gemm_tiles_grid((uint32_t)mtiles, end), 256, 0, params, stream);
 }
 
@@ -1728,10 +1728,11 @@ int cogni_gemm_stream_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_
   return gemm_stream_launch(who, &w_b, type_b, workspace_b, bytes_b, 0, 0, &out_b, &out_dim_b, 1, in_dim_b, tokens, stream);
 }
 
+static bool wide_two_swaps(uint32_t type_a, uint32_t type_b) { return type_a != type_b && (type_a == COGNI_TYPE_Q6_K || type_b == COGNI_TYPE_Q5_K); }
 int32_t cogni_gemm_wide_two_takes(uint32_t type_a, uint32_t in_dim_a, uint32_t out_dim_a, uint32_t type_b, uint32_t in_dim_b, uint32_t out_dim_b,
                                   uint32_t tokens) {
   unsigned sa, sb;
-  if (type_a == COGNI_TYPE_Q6_K) return gemm_wide_two_plan(type_b, in_dim_b, out_dim_b, type_a, in_dim_a, out_dim_a, tokens, &sa, &sb);
+  if (wide_two_swaps(type_a, type_b)) return gemm_wide_two_plan(type_b, in_dim_b, out_dim_b, type_a, in_dim_a, out_dim_a, tokens, &sa, &sb);
   return gemm_wide_two_plan(type_a, in_dim_a, out_dim_a, type_b, in_dim_b, out_dim_b, tokens, &sa, &sb);
 }
 size_t cogni_gemm_wide_two_scratch_bytes(void) { return GEMM_WIDE_TWO_SCRATCH; }
@@ -1739,7 +1740,7 @@ int cogni_gemm_wide_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a,
                             uint64_t w_b, uint32_t type_b, uint64_t workspace_b, size_t bytes_b, uint64_t out_b, uint32_t in_dim_b, uint32_t out_dim_b,
                             uint64_t scratch, size_t scratch_bytes, uint32_t tokens, void* stream) {
   const char* who = "cogni_gemm_wide_two_dev";
-  if (type_a == COGNI_TYPE_Q6_K && type_b == COGNI_TYPE_Q4_K)
+  if (wide_two_swaps(type_a, type_b) && !wide_two_swaps(type_b, type_a))
     return cogni_gemm_wide_two_dev(w_b, type_b, workspace_b, bytes_b, out_b, in_dim_b, out_dim_b, w_a, type_a, workspace_a, bytes_a, out_a, in_dim_a,
                                    out_dim_a, scratch, scratch_bytes, tokens, stream);
   if (!w_a || !w_b || !out_a || !out_b) return fail(COGNI_ERR_INVALID_ARGUMENT, std::string(who) + ": null device pointer");
@@ -1756,7 +1757,9 @@ int cogni_gemm_wide_two_dev(uint64_t w_a, uint32_t type_a, uint64_t workspace_a,
   const uint32_t mt = (tokens + 127) / 128;
   void* params[] = {&w_a, &workspace_a, &to_a, &in_dim_a, &out_dim_a, &sa, &w_b, &workspace_b, &to_b, &in_dim_b, &out_dim_b, &sb, &tokens};
   const uint32_t grid = sa * gemm_tiles_grid(mt, (out_dim_a + 255) / 256) + sb * gemm_tiles_grid(mt, (out_dim_b + 255) / 256);
-  if (int rc = launch(type_b == COGNI_TYPE_Q6_K ? "q4_k_and_q6_k_gemm_wide_f16" : "q4_k_and_q4_k_gemm_wide_f16", grid, 512, 0, params, stream)) return rc;
+  char name[64];
+  std::snprintf(name, sizeof name, "%s_and_%s_gemm_wide_f16", type_prefix(type_a), type_prefix(type_b));
+  if (int rc = launch(name, grid, 512, 0, params, stream)) return rc;
   if (sa > 1)
     if (int rc = gemm_stream_sum(scratch, 0, 0, out_a, out_dim_a, tokens, sa, stream)) return rc;
   return sb > 1 ? gemm_stream_sum(scratch + at_b, 0, 0, out_b, out_dim_b, tokens, sb, stream) : 0;

@@ -21,21 +21,20 @@ __shared__ uint4 gemm_q6w_x0[2048];        // [kh][k-step 0..3][k-group][128 tok
 __shared__ uint4 gemm_q6w_x1[2048];        // the same of k-steps 4..7
 __shared__ uint4 gemm_q6w_wbuf[8 * 384];   // [wavefront][64 rows][ql 4 pieces, qh 2 pieces]
 
-// Q4: raw Q4_K weights (codes 64 kh of a row's super-block, four copies into the same region; headers from global memory) in the same loop. The
-// super-blocks [kb0, kb1) of the rows, by workgroup bid of the matrix's.
-template <bool Q4>
+// T4: raw Q4_K weights (codes 64 kh of a row's super-block, four copies into the same region; headers from global memory) in the same loop, T5: Q5_K
+// (the 32 bytes of fifth bits behind the codes, six copies as here). Tile (mt, nt) of the matrix, super-blocks [kb0, kb1) of its rows.
+enum GemmWideType { T6, T4, T5 };
+template <GemmWideType W>
 __device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4* xp, const float* bias, float* out, u32 in_dim, u32 out_dim, u32 m,
-                                                   u32 bias_stride, u32 bid, u32 kb0, u32 kb1) {
-  constexpr u32 BS = Q4 ? 144 : 210;
-  constexpr int NW = Q4 ? 4 : 6;   // copies of a wavefront's weights per super-block
+                                                   u32 bias_stride, u32 mt, u32 nt, u32 kb0, u32 kb1) {
+  constexpr bool Q4 = W != T6, Q5 = W == T5;
+  constexpr u32 BS = Q5 ? 176 : (Q4 ? 144 : 210);
+  constexpr int NW = W == T4 ? 4 : 6;   // copies of a wavefront's weights per super-block
   const u32 tid = threadIdx.x, lane = tid & 63;
   const u32 wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const u32 nh = wave & 3, kh = wave >> 2;
   const u32 j = lane & 31, kg = lane >> 5;
   const u32 nkb = in_dim >> 8;
-  const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM, ntiles = (out_dim + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN;
-  u32 mt, nt;
-  if (!gemm_tile_of(bid, mtiles, ntiles, &mt, &nt)) return;
   const size_t row_bytes = (size_t)nkb * BS;
   // constants of the code assembly, kept in registers (as literals each (a & mask) | b would be two instructions): the masks
   // in scalar ones, of which an instruction takes one
@@ -54,7 +53,7 @@ __device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4
 #pragma unroll
   for (int i = 0; i < NW; i++) {
     const u32 p = 64u * i + lane, r = p / (u32)NW, part = p - NW * r;
-    const u32 at = Q4 ? 16u + 64u * kh + 16u * (part ^ ((r >> 2) & 3u)) : part < 4u ? 64u * kh + 16u * part : 128u + 32u * kh + 16u * (part - 4u);
+    const u32 at = Q5 ? (part < 4u ? 48u + 64u * kh + 16u * part : 16u * (part - 3u)) : Q4 ? 16u + 64u * kh + 16u * (part ^ ((r >> 2) & 3u)) : part < 4u ? 64u * kh + 16u * part : 128u + 32u * kh + 16u * (part - 4u);
     woff[i] = (min(row0 + r, out_dim - 1) - base_row) * (u32)row_bytes + at;
   }
   u32 soff[2];   // scales of the half, row c of this lane (d is 16 - 8 kh bytes further); Q4_K: the header
@@ -95,12 +94,20 @@ __device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4
   };
 
   GemmRaw6 cur[2];
+  uint4 cur5[2];   // Q5_K: the fifth bits of values 16 .. 31 of a run of 32 (cur.qh: 0 .. 15)
   u32 S[2][4];
   uint4 A[2][4];
   half8_t B[2][2];
   auto take_raw = [&]() {
 #pragma unroll
     for (int c = 0; c < 2; c++) {
+      if constexpr (Q5) {
+        cur[c].qa = gemm_q6w_wbuf[wrow + kg + 192 * c];
+        cur[c].qb = gemm_q6w_wbuf[wrow + kg + 192 * c + 1];
+        cur[c].qh = gemm_q6w_wbuf[wrow - kg + 192 * c + 4];
+        cur5[c] = gemm_q6w_wbuf[wrow - kg + 192 * c + 5];
+        continue;
+      }
       if constexpr (Q4) {
         cur[c].qa = gemm_q6w_wbuf[wrow4 + 128 * c + slot4];
         cur[c].qb = gemm_q6w_wbuf[wrow4 + 128 * c + (slot4 ^ 1u)];
@@ -143,6 +150,20 @@ __device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4
         const uint4 P = (t >> 2) ? cur[c].qb : cur[c].qa;
         const u32 q0 = (op & 1) ? P.z : P.x, q1 = (op & 1) ? P.w : P.y;
         const u32 msk = up ? mask_hi : mask_lo, mag = up ? magic_hi : magic_lo, of = up ? 0xD400D400u : 0xE400E400u;
+        if constexpr (Q5) {   // the fifth bit beside the nibble, as in gemm_k45_core
+          const uint4 H = (t >> 2) ? cur5[c] : cur[c].qh;
+          const u32 s5 = 2 * (2 * kh + kg) + up;
+          const u32 h0 = ((op & 1) ? H.z : H.x) >> s5, h1 = ((op & 1) ? H.w : H.y) >> s5;
+          constexpr u32 one = 0x00010001u;
+          const int at = up ? 8 : 4;
+          uint4 b5;
+          b5.x = h2_fma_off((q0 & msk) | mag | ((h0 & one) << at), of, S[c][2 * up], S[c][2 * up + 1]);
+          b5.y = h2_fma_off(((q0 >> 8) & msk) | mag | (((h0 >> 8) & one) << at), of, S[c][2 * up], S[c][2 * up + 1]);
+          b5.z = h2_fma_off((q1 & msk) | mag | ((h1 & one) << at), of, S[c][2 * up], S[c][2 * up + 1]);
+          b5.w = h2_fma_off(((q1 >> 8) & msk) | mag | (((h1 >> 8) & one) << at), of, S[c][2 * up], S[c][2 * up + 1]);
+          Bd[c] = *reinterpret_cast<const half8_t*>(&b5);
+          continue;
+        }
         uint4 b4;
         b4.x = h2_fma_off((q0 & msk) | mag, of, S[c][2 * up], S[c][2 * up + 1]);
         b4.y = h2_fma_off(((q0 >> 8) & msk) | mag, of, S[c][2 * up], S[c][2 * up + 1]);
@@ -278,30 +299,47 @@ __device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4
 
 extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void q6_k_gemm_wide_f16(
     const uint8_t* w, const uint4* xp, const float* bias, float* out, u32 in_dim, u32 out_dim, u32 m, u32 bias_stride) {
-  gemm_q6k_wide_core<false>(w, xp, bias, out, in_dim, out_dim, m, bias_stride, blockIdx.x, 0, in_dim >> 8);
+  u32 mt, nt;
+  if (!gemm_tile_of(blockIdx.x, (m + GEMM_BM - 1) / GEMM_BM, (out_dim + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN, &mt, &nt)) return;
+  gemm_q6k_wide_core<T6>(w, xp, bias, out, in_dim, out_dim, m, bias_stride, mt, nt, 0, in_dim >> 8);
 }
 
-// Two matrices with an input each (Q4_K, and Q4_K or Q6_K: o and down of a layer), each over all its super-blocks or split in planes out + split m out_dim:
-//   q4_k_and_q6_k|q4_k_gemm_wide_f16 (w_a, xp_a, out_a, in_dim_a, out_dim_a, splits_a, w_b, xp_b, out_b, in_dim_b, out_dim_b, splits_b, m)
+// A list of Q5_K matrices (list, xp, in_dim, m; tile_end in tiles of 256 rows; grid gemm_tiles_grid): the values of q5_k_gemm_many_f16, bit for bit.
+// 30720 rows x 4096 at 256 | 512 | 1024 tokens: 77 | 151 | 298 us, 88 | 169 | 334 on the better of the four-wavefront tiles (gemm_list_rows).
+extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void q5_k_gemm_many_wide_f16(const GemmManyArgs list, const uint4* xp,
+                                                                                                                  u32 in_dim, u32 m) {
+  u32 mt, nt, i = 0, first = 0;
+  if (!gemm_tile_of(blockIdx.x, (m + GEMM_BM - 1) / GEMM_BM, list.tile_end[list.count - 1], &mt, &nt)) return;
+  while (i + 1 < list.count && nt >= list.tile_end[i]) first = list.tile_end[i++];
+  gemm_q6k_wide_core<T5>(list.w[i], xp, nullptr, list.out[i], in_dim, list.out_dim[i], m, 0, mt, nt - first, 0, in_dim >> 8);
+}
+
+// Two matrices with an input each (Q4_K or Q5_K, and Q4_K or Q6_K: o and down of a layer), each over all its super-blocks or split in planes out + split m out_dim:
+//   q4_k|q5_k_and_q6_k|q4_k_gemm_wide_f16 (w_a, xp_a, out_a, in_dim_a, out_dim_a, splits_a, w_b, xp_b, out_b, in_dim_b, out_dim_b, splits_b, m)
 //                      grid = splits x gemm_tiles_grid of both, b's first: the rows of down are the longer ones
 // 512 tokens of 4096 -> 4096 beside Q6_K 12288 -> 4096, plane sums included: 90 us; 110 as launches of their own, of which o's fills half the chip and down's
 // 128-row tiles reach 0.7 PFLOP/s. Splits by gemm_wide_two_plan (gemv_config.h). Q4_K in this loop instead of gemm_wide_core's because both have to share LDS.
-#define GEMM_WIDE_TWO_ENTRY(PREFIX_A, A4, PREFIX_B, B4)                                                                                           \
+#define GEMM_WIDE_TWO_ENTRY(PREFIX_A, WA, PREFIX_B, WB)                                                                                           \
   extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void PREFIX_A##_and_##PREFIX_B##_gemm_wide_f16(         \
       const uint8_t* w_a, const uint4* xp_a, float* out_a, u32 in_dim_a, u32 out_dim_a, u32 splits_a, const uint8_t* w_b, const uint4* xp_b,      \
       float* out_b, u32 in_dim_b, u32 out_dim_b, u32 splits_b, u32 m) {                                                                           \
-    const u32 mt = (m + GEMM_BM - 1) / GEMM_BM;                                                                                                   \
-    const u32 wgs_a = gemm_tiles_grid(mt, (out_dim_a + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN);                                                         \
-    const u32 wgs_b = gemm_tiles_grid(mt, (out_dim_b + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN), first_a = wgs_b * splits_b;                             \
+    const u32 mtiles = (m + GEMM_BM - 1) / GEMM_BM, nt_a = (out_dim_a + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN;                                        \
+    const u32 nt_b = (out_dim_b + GEMM_WIDE_BN - 1) / GEMM_WIDE_BN, wgs_a = gemm_tiles_grid(mtiles, nt_a), wgs_b = gemm_tiles_grid(mtiles, nt_b); \
+    const u32 first_a = wgs_b * splits_b;                                                                                                         \
+    u32 mt, nt;                                                                                                                                   \
     if (blockIdx.x < first_a) {                                                                                                                   \
       const u32 s = blockIdx.x / wgs_b, n = in_dim_b >> 8;                                                                                        \
-      gemm_q6k_wide_core<B4>(w_b, xp_b, nullptr, out_b + (size_t)s * m * out_dim_b, in_dim_b, out_dim_b, m, 0, blockIdx.x % wgs_b,                \
-                             s * n / splits_b, (s + 1) * n / splits_b);                                                                           \
+      if (!gemm_tile_of(blockIdx.x % wgs_b, mtiles, nt_b, &mt, &nt)) return;                                                                      \
+      gemm_q6k_wide_core<WB>(w_b, xp_b, nullptr, out_b + (size_t)s * m * out_dim_b, in_dim_b, out_dim_b, m, 0, mt, nt, s * n / splits_b,          \
+                             (s + 1) * n / splits_b);                                                                                             \
     } else {                                                                                                                                      \
       const u32 id = blockIdx.x - first_a, s = id / wgs_a, n = in_dim_a >> 8;                                                                     \
-      gemm_q6k_wide_core<A4>(w_a, xp_a, nullptr, out_a + (size_t)s * m * out_dim_a, in_dim_a, out_dim_a, m, 0, id % wgs_a, s * n / splits_a,      \
+      if (!gemm_tile_of(id % wgs_a, mtiles, nt_a, &mt, &nt)) return;                                                                              \
+      gemm_q6k_wide_core<WA>(w_a, xp_a, nullptr, out_a + (size_t)s * m * out_dim_a, in_dim_a, out_dim_a, m, 0, mt, nt, s * n / splits_a,          \
                              (s + 1) * n / splits_a);                                                                                             \
     }                                                                                                                                             \
   }
-GEMM_WIDE_TWO_ENTRY(q4_k, true, q6_k, false)
-GEMM_WIDE_TWO_ENTRY(q4_k, true, q4_k, true)
+GEMM_WIDE_TWO_ENTRY(q4_k, T4, q6_k, T6)
+GEMM_WIDE_TWO_ENTRY(q4_k, T4, q4_k, T4)
+GEMM_WIDE_TWO_ENTRY(q5_k, T5, q6_k, T6)
+GEMM_WIDE_TWO_ENTRY(q5_k, T5, q4_k, T4)

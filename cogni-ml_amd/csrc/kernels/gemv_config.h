@@ -298,7 +298,7 @@ static inline int gemm_q4k_use_wide(unsigned out_dim, unsigned tokens) {
   const unsigned rn = (narrow + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES, rw = (wide + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
   return wide >= GEMM_ROUND_TILES && rw * GEMM_Q4K_WIDE_COST < rn * 100u;
 }
-static inline unsigned gemm_tile_cost(unsigned type, unsigned rows) { return rows == 192u ? 100u : (rows == 128u ? 75u : (type == 14u ? 107u : 131u)); }
+static inline unsigned gemm_tile_cost(unsigned type, unsigned rows) { return rows == 192u ? 100u : (rows == 128u ? 75u : (type == 14u ? 107u : (type == 13u ? 117u : 131u))); }
 // knob: COGNI_GEMM_WIDE, 0 | 1 where it is set (no 256-row tiles | those wherever there is a kernel for them), else -1.
 // gate | up with SwiGLU: tiles of 96 rows of both matrices (four wavefronts) or of 128 (eight). 4096 -> 12288, us: 441 | 410 at 2048
 // tokens, 225 | 208 at 1024, 114 | 123 at 512, 58 | 59 at 256; 2048 -> 4096 at 1024 61.6 | 41.3; 3072 -> 8192 at 300 76.7 | 45.5.
@@ -308,13 +308,15 @@ static inline int gemm_swiglu_use_wide(unsigned out_dim, unsigned tokens, int kn
   const unsigned long long rw = (mtiles * ((out_dim + 127u) / 128u) + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
   return knob >= 0 ? knob : tokens > 64u && rw * gemm_tile_cost(12u, 256u) < rn * gemm_tile_cost(12u, 192u);
 }
-// A list of Q4_K or Q5_K matrices as one launch: rows of its tiles. The 256-row ones: Q4_K, more tokens than the 64-token kernels take.
+// A list of Q4_K or Q5_K matrices as one launch: rows of its tiles. The 256-row ones: more tokens than the 64-token kernels take. (Q5_K, 4096 columns, weights
+// from memory, us, 192 | 128 | 256 rows: 30720 rows at 256 tokens 107.8 | 87.7 | 77.3, 384 120.9 | 128.3 | 135.8, 512 169 | 170 | 151, 1024 341 | 334 | 298; 65536 rows at 128
+// 126.5 | 105.3 | 89.0, 81920 129.9 | 142.4 | 150; 19456 x 2048 at 300 61.4 | 49.7 | 44.2, at 512 66.4 | 73.2 | 77.5: the costs pick the fastest of each.)
 static inline unsigned gemm_list_rows(unsigned type, const unsigned* out_dims, unsigned count, unsigned tokens, int knob) {
   const unsigned of[3] = {192u, 128u, 256u};
   unsigned long long least = ~0ull;
   unsigned best = 192u, k, i;
   if (type == 12u && knob == 1) return 256u;
-  for (k = 0; k < (type == 12u && tokens > 64u && knob != 0 ? 3u : 2u); k++) {
+  for (k = 0; k < (tokens > 64u && knob != 0 ? 3u : 2u); k++) {
     unsigned long long tiles = 0, cost;
     for (i = 0; i < count; i++) tiles += ((unsigned long long)out_dims[i] + of[k] - 1u) / of[k];
     cost = ((tokens + 127u) / 128u * tiles + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES * gemm_tile_cost(type, of[k]);
@@ -358,14 +360,15 @@ static inline int gemm_tall_swiglu_takes(unsigned type, unsigned in_dim, unsigne
          gemm_fill_cost(mt * gemm_list_tiles(&out_dim, 1u, wide ? 128u : 96u), gemm_tile_cost(12u, wide ? 256u : 192u));
 }
 
-// Two matrices with an input each in one launch of 128-token x 256-row tiles, each with its own k splits (gemm_q6k_wide.hpp; a: Q4_K, b: Q4_K
-// or Q6_K: o and down of a layer): the two share the chip where one alone would leave half of it idle, and the splits even their chains out. The plan is the
-// cheapest of those whose tiles fit one round of the chip: start and end 11 us, the longer chain at 3.7 (Q4_K) or 4.2 us (Q6_K) a super-block, a split
+// Two matrices with an input each in one launch of 128-token x 256-row tiles, each with its own k splits (gemm_q6k_wide.hpp; a: Q4_K or Q5_K, b:
+// Q4_K or Q6_K: o and down of a layer): the two share the chip where one alone would leave half of it idle, and the splits even their chains out. The plan is the
+// cheapest of those whose tiles fit one round of the chip: start and end 11 us, the longer chain at 3.7 (Q4_K) or 4.2 us (Q5_K, Q6_K) a super-block, a split
 // matrix's planes at 5 TB/s and a launch (within a tenth of what 36 shapes measured). Taken from 1300 tile super-blocks in all, below which the
 // launches of their own do better, and where the plan's time is less than what those reach at their best, 19.5 ns a tile super-block and
 // 36 us of starts, ends and sums. Weights from memory, us, launches of their own | this: o 4096 -> 4096 and Q6_K down 12288 -> 4096 at 256 | 384 | 512 | 640 tokens 59.9 |
 // 94 | 110 | 159 and 59.0 | 73.5 | 90 | 115 (1024: 162 | 180, not taken: chains of 48), Q4_K down at 512 90.5 | 83.6; 2560 -> 2560 and 9728 -> 2560 at 300 | 700
-// tokens 78.5 | 130 and 50 | 72.5; 2048 and 11008 at 700 85.6 | 64; 1536 and 8448 at 546 (1170 super-blocks) 36.5 | 40.6, 2048 and 10240 at 290 (1152) 35.4 | 39.7: not taken.
+// tokens 78.5 | 130 and 50 | 72.5; 2048 and 11008 at 700 85.6 | 64; 1536 and 8448 at 546 (1170 super-blocks) 36.5 | 40.6, 2048 and 10240 at 290 (1152) 35.4 | 39.7: not taken. Q5_K o: 4096 and Q6_K
+// 12288 -> 4096 at 256 | 512 63.6 | 117 and 58.8 | 91.4, Q4_K down at 640 118 | 99.5; 2560 and 9728 at 300 78.3 | 49.
 #define GEMM_WIDE_TWO_SCRATCH (256ull * 128ull * 256ull * 4ull)   // the planes of a launch of one round at most
 static inline int gemm_wide_two_plan(unsigned type_a, unsigned in_a, unsigned out_a, unsigned type_b, unsigned in_b, unsigned out_b, unsigned tokens,
                                      unsigned* splits_a, unsigned* splits_b) {
@@ -374,10 +377,10 @@ static inline int gemm_wide_two_plan(unsigned type_a, unsigned in_a, unsigned ou
   const unsigned long long work = ta * na + tb * nb;
   unsigned long long least = ~0ull;   // ns
   unsigned sa, sb;
-  if (type_a != 12u || (type_b != 12u && type_b != 14u) || ((in_a | in_b) & 255u) != 0 || tokens <= 192u || ta + tb > 256u || work < 1300u) return 0;
+  if ((type_a != 12u && type_a != 13u) || (type_b != 12u && type_b != 14u) || ((in_a | in_b) & 255u) != 0 || tokens <= 192u || ta + tb > 256u || work < 1300u) return 0;
   for (sa = 1; sa == 1u || (sa <= 4u && 2u * sa <= na); sa++)
     for (sb = 1; sb == 1u || (sb <= 8u && 2u * sb <= nb); sb++) {
-      const unsigned long long ca = ((na + sa - 1u) / sa) * 3700ull, cb = ((nb + sb - 1u) / sb) * (type_b == 14u ? 4200ull : 3700ull);
+      const unsigned long long ca = ((na + sa - 1u) / sa) * (type_a == 13u ? 4200ull : 3700ull), cb = ((nb + sb - 1u) / sb) * (type_b == 14u ? 4200ull : 3700ull);
       unsigned long long c = 11000ull + (ca > cb ? ca : cb);
       if (ta * sa + tb * sb > 256u) break;
       if (sa > 1u) c += 2000ull + (sa + 1ull) * tokens * out_a / 1250ull;

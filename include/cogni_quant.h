@@ -531,7 +531,7 @@ int cogni_gemm_tall_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_t
                                     uint32_t next_type, uint64_t next_workspace, size_t next_workspace_bytes, uint32_t in_dim, uint32_t out_dim,
                                     uint32_t tokens, void* stream);
 
-/* Two matrices with an input each (o and down of a layer; Q4_K and a Q4_K or Q6_K one, in either order) in one launch of 128-token x 256-row tiles, the
+/* Two matrices with an input each (o and down of a layer; Q4_K or Q5_K and a Q4_K or Q6_K one, in either order) in one launch of 128-token x 256-row tiles, the
  * k range of each split as that fills the chip: the precision of cogni_gemm_packed_dev, sums in another order. Only what cogni_gemm_wide_two_takes says
  * (1 or 0) is launched this way; scratch: cogni_gemm_wide_two_scratch_bytes() (32 MiB) are enough for any such launch. Nothing may overlap but the two
  * workspaces, which are only read. */

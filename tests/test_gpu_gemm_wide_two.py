@@ -20,7 +20,8 @@ def sums_bound(oracle, raw, t, x, out_dim, in_dim):
 # splits that do not divide the super-blocks; the fewest tokens; either order; up to the 256 tiles of a round
 @pytest.mark.parametrize("tokens,a,b", [(897, (Q4_K, 512, 300), (Q6_K, 8448, 1283)), (193, (Q4_K, 2560, 2560), (Q4_K, 12288, 3072)),
                                         (1024, (Q4_K, 2048, 1024), (Q4_K, 4096, 2560)), (320, (Q6_K, 9728, 2305), (Q4_K, 2304, 2304)),
-                                        (2049, (Q4_K, 256, 1), (Q6_K, 2048, 2560)), (640, (Q4_K, 2048, 1030), (Q6_K, 11008, 1536))])
+                                        (2049, (Q4_K, 256, 1), (Q6_K, 2048, 2560)), (640, (Q4_K, 2048, 1030), (Q6_K, 11008, 1536)),
+                                        (300, (Q5_K, 3072, 2001), (Q6_K, 9728, 2304)), (257, (Q4_K, 10240, 2304), (Q5_K, 2304, 2304))])
 def test_two_matrices(gpu, oracle, tokens, a, b):
     rng = np.random.default_rng(tokens)
     assert quant.gemm_wide_two_takes(*a, *b, tokens)
@@ -77,11 +78,30 @@ def test_runner_of_the_two(gpu, down, monkeypatch):
         assert np.all(np.abs(a - b) <= 2e-5 * np.abs(b).max(axis=1, keepdims=True)), k
 
 
+@pytest.mark.parametrize("tokens,in_dim,dims", [(200, 256, [16384, 8199, 5, 4100]), (65, 512, [40960, 1, 16384]), (385, 768, [7936, 8190])])
+def test_q5_k_lists_of_256_row_tiles(gpu, tokens, in_dim, dims):
+    """Lists that this tile takes fewer rounds for: the bits of each matrix on its own (four wavefronts, no k split)."""
+    rng = np.random.default_rng(tokens)
+    n = quant.gemm_workspace_bytes(Q5_K, in_dim, tokens)
+    x, ws = DevArray(synth.make_activations(rng, tokens, in_dim)), DevArray(nbytes=n)
+    quant.gemm_pack_dev(x.ptr, Q5_K, in_dim, tokens, ws.ptr, n)
+    w = [DevArray(synth.make_weights(rng, Q5_K, d, in_dim)) for d in dims]
+    one, many = ([DevArray(np.full(tokens * d + 4, np.float32(-3.0))) for d in dims] for _ in range(2))
+    for a, o, d in zip(w, one, dims):
+        quant.gemm_packed_dev(a.ptr, Q5_K, ws.ptr, n, o.ptr, in_dim, d, tokens)
+    quant.gemm_packed_many_dev([a.ptr for a in w], Q5_K, ws.ptr, n, [o.ptr for o in many], dims, in_dim, tokens)
+    for a, b, d in zip(one, many, dims):
+        assert np.array_equal(a.read(np.uint32, tokens * d + 4), b.read(np.uint32, tokens * d + 4)), d
+    for a in [x, ws] + w + one + many:
+        a.close()
+
+
 def test_what_is_not_taken(gpu):
     takes = quant.gemm_wide_two_takes
     o, down = (Q4_K, 4096, 4096), (Q6_K, 12288, 4096)
     assert [takes(*o, *down, m) for m in (64, 192, 256, 512, 640, 1024)] == [False, False, True, True, True, False]
-    assert takes(*down, *o, 512) and not takes(*down, *down, 512) and not takes(Q5_K, 4096, 4096, *down, 512)
+    assert takes(*down, *o, 512) and not takes(*down, *down, 512) and takes(Q5_K, 4096, 4096, *down, 512)
+    assert not takes(Q5_K, 4096, 4096, Q5_K, 12288, 4096, 512) and not takes(Q6_K, 4096, 4096, *down, 512)
     assert not takes(Q4_K, 1792, 1792, Q6_K, 2560, 1792, 289) and not takes(Q4_K, 4096, 4096, Q6_K, 12200, 4096, 512)
     args = [64, *o[:1], 64, 1 << 30, 64, *o[1:], 64, *down[:1], 64, 1 << 30, 64, *down[1:]]
     with pytest.raises(quant.QuantError, match="not a launch for these kernels"):
