@@ -645,7 +645,7 @@ def main():
     cases["cfg4 ffn block prefill M=512 (add+rmsnorm, gate|up|swiglu gemm, q6_k down gemm + residual)"] = {
         "us": round(r["us"], 2), "tflops": round(fflops / r["us"] / 1e6, 1),
         "frac_mfma_f16": round(fflops / r["us"] / 1e6 / MFMA_F16_PEAK_TFLOPS, 4), "flops": fflops,
-        "launches": "add_rmsnorm, pack, q4_k_gemm_swiglu_pack_q6k_f16, q6_k_gemm_n128_f16 (k split) + plane sum with the residual"}
+        "launches": "add_rmsnorm_gemm_pack, q4_k_gemm_tall_swiglu_pack_q6k_f16, q6_k_gemm_n128_f16 (k split) + plane sum with the residual"}
     log("case=ffn block prefill M=512\nhip_us=%.2f\ntflops=%.1f\nfrac_mfma_f16_peak=%.4f\n" % (
         r["us"], fflops / r["us"] / 1e6, fflops / r["us"] / 1e6 / MFMA_F16_PEAK_TFLOPS))
     for fr in ffns:
@@ -754,7 +754,7 @@ def main():
             "us": round(r["us"], 2), "tflops": round(pflops / r["us"] / 1e6, 1),
             "frac_mfma_f16": round(pflops / r["us"] / 1e6 / MFMA_F16_PEAK_TFLOPS, 4), "flops": pflops, "steps": steps,
             "launches": ("images of x, q and gate for sixteen single-term tokens; q|k|v, gate|up, o, down on the one-pass decode kernels" if tokens <= 16 else
-                         "pack x, list GEMM q|k|v|gate|up, pack q, o GEMM, pack gate, Q6_K down GEMM (+ plane sums where the k range is split)")}
+                         "pack x, list GEMM q|k|v|gate|up that packs the inputs of o and down, o and Q6_K down in one launch (+ plane sums)")}
         log("case=projection stack prefill\ntokens=%d\nhip_us=%.2f\ntflops=%.1f\nfrac_mfma_f16_peak=%.4f\n" % (
             tokens, r["us"], pflops / r["us"] / 1e6, pflops / r["us"] / 1e6 / MFMA_F16_PEAK_TFLOPS))
         for r_ in runners:
