@@ -1804,6 +1804,16 @@ int32_t cogni_get_gemm_threshold(void) {
   return g_gemm_threshold;
 }
 
+// One Q4_K matrix of many tokens: the 256-token tiles where they cost a twentieth less than the tiles of a list, which is how near the costs are to the times
+// of single matrices (pack included, us, cogni_gemm_dev | these: 4096 -> 12288 at 700 | 1024 tokens 92.8 | 130.7 and 85.4 | 108.3, 4608 -> 8213 at 932 130.6 and 107.7,
+// 512 -> 11102 at 998 58.1 and 38.3, 8448 -> 11372 at 721 174.4 and 171.7; not taken: 1280 -> 10773 at 643, costs level, 50.2 and 50.5, 4096 -> 8192 at 1024 77.3 and 89.8).
+static bool matmul_takes_tall(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens) {
+  if (!gemm_tall_takes(w_type, in_dim, &out_dim, 1, tokens)) return false;
+  const unsigned long long mt = (tokens + 127ull) / 128ull;
+  const unsigned rows = gemm_list_rows(w_type, &out_dim, 1, tokens, -1);
+  return 20 * gemm_fill_cost((mt + 1) / 2 * gemm_list_tiles(&out_dim, 1, 256), GEMM_TALL_COST) <
+         19 * gemm_fill_cost(mt * gemm_list_tiles(&out_dim, 1, rows), gemm_tile_cost(w_type, rows));
+}
 int cogni_matmul_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias, uint64_t out, uint32_t in_dim,
                      uint32_t out_dim, uint32_t tokens, uint64_t workspace, size_t workspace_bytes, void* stream) {
   if (gemm_type(w_type) && tokens > (uint32_t)cogni_get_gemm_threshold()) {
@@ -1827,6 +1837,13 @@ int cogni_matmul_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t bias,
       if (int rc = gemm_check("cogni_matmul_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;
       if (int rc = cogni_gemm_pack_dev(x, w_type, in_dim, tokens, workspace, workspace_bytes, stream)) return rc;
       return gemm_stream_launch("cogni_matmul_dev", &w_raw, w_type, workspace, workspace_bytes, bias, 0, &out, &out_dim, 1, in_dim, tokens, stream);
+    }
+    // (the 256-token tiles have no bias)
+    if (!bias && matmul_takes_tall(w_type, in_dim, out_dim, tokens)) {
+      if (!w_raw || !x || !out) return fail(COGNI_ERR_INVALID_ARGUMENT, "cogni_matmul_dev: null device pointer");
+      if (int rc = gemm_check("cogni_matmul_dev", w_type, in_dim, out_dim, tokens, workspace, workspace_bytes)) return rc;
+      if (int rc = cogni_gemm_pack_dev(x, w_type, in_dim, tokens, workspace, workspace_bytes, stream)) return rc;
+      return gemm_tall_launch("cogni_matmul_dev", &w_raw, w_type, workspace, workspace_bytes, &out, &out_dim, 1, in_dim, tokens, nullptr, stream);
     }
     return cogni_gemm_dev(w_raw, w_type, x, bias, out, in_dim, out_dim, tokens, workspace, workspace_bytes, stream);
   }

@@ -577,7 +577,7 @@ int cogni_gemm_plan(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t
                     uint32_t* grid_x, uint32_t* grid_y, uint32_t* block_x);
 
 /* The router of the reference's GPU arm (Qwen35Metal.matmul, src/ml/gguf/qwen35_metal.cr:11404-11449):
- * tokens > threshold and a type with a GEMM kernel -> cogni_gemm_dev, else cogni_gemv_dev. The threshold
+ * tokens > threshold and a type with a GEMM kernel -> cogni_gemm_dev (or, faster, a kernel of its precision class), else cogni_gemv_dev. The threshold
  * defaults to 8 (GEMM_BATCH_THRESHOLD, qwen35_metal.cr:70-75) and can be changed with
  * cogni_set_gemm_threshold or the QWEN35_GEMM_BATCH_THRESHOLD environment variable the reference reads.
  * `bias` ([out_dim], may be 0) is only accepted with tokens == 1 or on the GEMM path. `workspace` may be 0

@@ -67,6 +67,32 @@ def test_gate_up_swiglu(gpu, tokens, out_dim, in_dim, next_type, keep):
         a.close()
 
 
+@pytest.mark.parametrize("tokens,in_dim,out_dim,taken", [(998, 512, 11102, True), (1024, 512, 12287, True), (1024, 1024, 8192, False), (300, 3840, 5000, False), (643, 1280, 10773, False)])
+def test_router_takes_them(gpu, tokens, in_dim, out_dim, taken):
+    """cogni_matmul_dev: the bits of a pack and these tiles where the rule says so and there is no bias, else of cogni_gemm_dev."""
+    rng = np.random.default_rng(tokens + out_dim)
+    n, wsb = tokens * out_dim, quant.gemm_workspace_bytes(Q4_K, in_dim, tokens)
+    w, x = DevArray(synth.make_weights(rng, Q4_K, out_dim, in_dim)), DevArray(synth.make_activations(rng, tokens, in_dim))
+    bias, ws = DevArray(synth.make_activations(rng, 1, out_dim)), DevArray(nbytes=wsb)
+    a, b, c, d = (DevArray(np.full(n, np.float32(-3.0))) for _ in range(4))
+    quant.matmul_dev(w.ptr, Q4_K, x.ptr, a.ptr, in_dim, out_dim, tokens, ws.ptr, wsb)
+    if taken:
+        quant.gemm_tall_dev([w.ptr], Q4_K, ws.ptr, wsb, [b.ptr], [out_dim], in_dim, tokens)
+    else:
+        quant.gemm_dev(w.ptr, Q4_K, x.ptr, b.ptr, in_dim, out_dim, tokens, ws.ptr, wsb)
+    quant.matmul_dev(w.ptr, Q4_K, x.ptr, c.ptr, in_dim, out_dim, tokens, ws.ptr, wsb, bias.ptr)
+    quant.gemm_dev(w.ptr, Q4_K, x.ptr, d.ptr, in_dim, out_dim, tokens, ws.ptr, wsb, bias.ptr)
+    for p, q in ((a, b), (c, d)):
+        assert np.array_equal(p.read(np.uint32, n), q.read(np.uint32, n))
+    if taken:
+        with pytest.raises(quant.QuantError, match="workspace has"):
+            quant.matmul_dev(w.ptr, Q4_K, x.ptr, a.ptr, in_dim, out_dim, tokens, ws.ptr, wsb - 256)
+        with pytest.raises(quant.QuantError, match="null device pointer"):
+            quant.matmul_dev(w.ptr, Q4_K, 0, a.ptr, in_dim, out_dim, tokens, ws.ptr, wsb)
+    for v in (w, x, bias, ws, a, b, c, d):
+        v.close()
+
+
 def test_which_launches_take_these_kernels(gpu):
     dims = [4096, 1024, 1024, 12288, 12288]
     assert [quant.gemm_tall_takes(Q4_K, 4096, dims, m) for m in (64, 128, 256, 384, 400, 512, 1024, 2048)] == [False] * 4 + [True] * 4
