@@ -1286,9 +1286,9 @@ static GemmShape gemm_shape(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, 
   }
   GemmShape best = n128 ? GemmShape{128, s128} : GemmShape{192, s192};
   // the eight-wavefront kernels, for more tokens than the 64-token tiles have and launches that are not split: Q4_K by
-  // gemm_q4k_use_wide; Q6_K where the 192-row tiles are not the better of the two others (and the activations of a token tile stay
-  // below 4 GiB, which its 32-bit offsets reach)
-  if (best.splits == 1 && (w_type == COGNI_TYPE_Q4_K || (w_type == COGNI_TYPE_Q6_K && nkb < 65536u))) {
+  // gemm_q4k_use_wide; Q6_K where the 192-row tiles are not the better of the two others (and the row is one that its 32-bit
+  // offsets reach)
+  if (best.splits == 1 && (w_type == COGNI_TYPE_Q4_K || (w_type == COGNI_TYPE_Q6_K && nkb <= GEMM_Q6W_MAX_KB))) {
     (void)eval(256, w_type == COGNI_TYPE_Q4_K ? GEMM_Q4K_WIDE_COST : gemm_tile_cost(w_type, 256), &cost256);
     bool wide = tokens > 64 && (w_type == COGNI_TYPE_Q4_K ? gemm_q4k_use_wide(out_dim, tokens) != 0 : n128) && cost256 < (n128 ? cost128 : cost192);
     if (const int knob = gemm_wide_knob(); knob >= 0) wide = knob != 0;
@@ -1479,7 +1479,7 @@ int cogni_gemm_packed_many_dev(const uint64_t* w_raw, uint32_t w_type, uint64_t 
                               out_dims[0], tokens, stream);
   const uint64_t mtiles = (tokens + 127) / 128;
   const bool m64 = tokens <= 64;
-  const uint32_t bn = gemm_list_rows(w_type, out_dims, count, tokens, gemm_wide_knob());
+  const uint32_t bn = gemm_list_rows(w_type, in_dim, out_dims, count, tokens, gemm_wide_knob());
   GemmManyArgs list{};
   uint32_t end = 0;
   for (uint32_t i = 0; i < count; i++) {
@@ -1810,7 +1810,7 @@ int32_t cogni_get_gemm_threshold(void) {
 static bool matmul_takes_tall(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens) {
   if (!gemm_tall_takes(w_type, in_dim, &out_dim, 1, tokens)) return false;
   const unsigned long long mt = (tokens + 127ull) / 128ull;
-  const unsigned rows = gemm_list_rows(w_type, &out_dim, 1, tokens, -1);
+  const unsigned rows = gemm_list_rows(w_type, in_dim, &out_dim, 1, tokens, -1);
   return 20 * gemm_fill_cost((mt + 1) / 2 * gemm_list_tiles(&out_dim, 1, 256), GEMM_TALL_COST) <
          19 * gemm_fill_cost(mt * gemm_list_tiles(&out_dim, 1, rows), gemm_tile_cost(w_type, rows));
 }

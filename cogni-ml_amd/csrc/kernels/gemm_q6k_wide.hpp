@@ -89,7 +89,7 @@ __device__ __forceinline__ void gemm_q6k_wide_core(const uint8_t* w, const uint4
   // copy i of half `hs` of a super-block's x: KiB 8 i + wave of the buffer, 16 of each kh
   const u32 xw = (wave & 7u) * 64;
   auto copy_x = [&](u32 kb, int hs, int i) {
-    const u32 src = kb * 65536u + ((i >> 1) * 2048 + hs * 1024 + (i & 1) * 512 + xw) * 16u;   // uniform
+    const u32 src = kb * 65536u + ((i >> 1) * 2048 + hs * 1024 + (i & 1) * 512 + xw) * 16u;   // uniform; 32 bits: GEMM_Q6W_MAX_KB
     __builtin_amdgcn_raw_ptr_buffer_load_lds(xrsrc, (lds_void*)((hs ? gemm_q6w_x1 : gemm_q6w_x0) + i * 512 + xw), 16, lane * 16, src, 0, 0);
   };
 

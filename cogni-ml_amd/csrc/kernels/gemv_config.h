@@ -308,15 +308,19 @@ static inline int gemm_swiglu_use_wide(unsigned out_dim, unsigned tokens, int kn
   const unsigned long long rw = (mtiles * ((out_dim + 127u) / 128u) + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES;
   return knob >= 0 ? knob : tokens > 64u && rw * gemm_tile_cost(12u, 256u) < rn * gemm_tile_cost(12u, 192u);
 }
+// Super-blocks of a row that the loop of gemm_q6k_wide.hpp takes: its offset into the activations of a token tile, 64 KiB a super-block, has 32 bits, and its
+// buffers end a byte short of 4 GiB. It runs Q6_K and Q5_K tiles of 256 rows and both matrices of gemm_wide_two_plan; longer rows go to the other
+// tiles, which have 64-bit addresses.
+#define GEMM_Q6W_MAX_KB 65535u
 // A list of Q4_K or Q5_K matrices as one launch: rows of its tiles. The 256-row ones: more tokens than the 64-token kernels take. (Q5_K, 4096 columns, weights
 // from memory, us, 192 | 128 | 256 rows: 30720 rows at 256 tokens 107.8 | 87.7 | 77.3, 384 120.9 | 128.3 | 135.8, 512 169 | 170 | 151, 1024 341 | 334 | 298; 65536 rows at 128
 // 126.5 | 105.3 | 89.0, 81920 129.9 | 142.4 | 150; 19456 x 2048 at 300 61.4 | 49.7 | 44.2, at 512 66.4 | 73.2 | 77.5: the costs pick the fastest of each.)
-static inline unsigned gemm_list_rows(unsigned type, const unsigned* out_dims, unsigned count, unsigned tokens, int knob) {
+static inline unsigned gemm_list_rows(unsigned type, unsigned in_dim, const unsigned* out_dims, unsigned count, unsigned tokens, int knob) {
   const unsigned of[3] = {192u, 128u, 256u};
   unsigned long long least = ~0ull;
   unsigned best = 192u, k, i;
   if (type == 12u && knob == 1) return 256u;
-  for (k = 0; k < (tokens > 64u && knob != 0 ? 3u : 2u); k++) {
+  for (k = 0; k < (tokens > 64u && knob != 0 && (type == 12u || in_dim / 256u <= GEMM_Q6W_MAX_KB) ? 3u : 2u); k++) {
     unsigned long long tiles = 0, cost;
     for (i = 0; i < count; i++) tiles += ((unsigned long long)out_dims[i] + of[k] - 1u) / of[k];
     cost = ((tokens + 127u) / 128u * tiles + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES * gemm_tile_cost(type, of[k]);
@@ -348,7 +352,7 @@ static inline unsigned long long gemm_list_tiles(const unsigned* out_dims, unsig
 static inline int gemm_tall_takes(unsigned type, unsigned in_dim, const unsigned* out_dims, unsigned count, unsigned tokens) {
   const unsigned long long mt = (tokens + 127ull) / 128ull;
   if (type != 12u || tokens <= 128u || (in_dim & 255u) != 0 || in_dim == 0) return 0;
-  const unsigned rows = gemm_list_rows(type, out_dims, count, tokens, -1);
+  const unsigned rows = gemm_list_rows(type, in_dim, out_dims, count, tokens, -1);
   return gemm_fill_cost((mt + 1u) / 2u * gemm_list_tiles(out_dims, count, 256u), GEMM_TALL_COST) <
          gemm_fill_cost(mt * gemm_list_tiles(out_dims, count, rows), gemm_tile_cost(type, rows));
 }
@@ -377,7 +381,9 @@ static inline int gemm_wide_two_plan(unsigned type_a, unsigned in_a, unsigned ou
   const unsigned long long work = ta * na + tb * nb;
   unsigned long long least = ~0ull;   // ns
   unsigned sa, sb;
-  if ((type_a != 12u && type_a != 13u) || (type_b != 12u && type_b != 14u) || ((in_a | in_b) & 255u) != 0 || tokens <= 192u || ta + tb > 256u || work < 1300u) return 0;
+  if ((type_a != 12u && type_a != 13u) || (type_b != 12u && type_b != 14u) || ((in_a | in_b) & 255u) != 0 || na > GEMM_Q6W_MAX_KB || nb > GEMM_Q6W_MAX_KB || tokens <= 192u ||
+      ta + tb > 256u || work < 1300u)
+    return 0;
   for (sa = 1; sa == 1u || (sa <= 4u && 2u * sa <= na); sa++)
     for (sb = 1; sb == 1u || (sb <= 8u && 2u * sb <= nb); sb++) {
       const unsigned long long ca = ((na + sa - 1u) / sa) * (type_a == 13u ? 4200ull : 3700ull), cb = ((nb + sb - 1u) / sb) * (type_b == 14u ? 4200ull : 3700ull);

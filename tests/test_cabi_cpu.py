@@ -479,3 +479,37 @@ int main() {
                         os.path.join(d, "t.cpp")], check=True)
         r = subprocess.run([os.path.join(d, "t")], capture_output=True, text=True)
         assert r.returncode == 0 and "bad=0" in r.stdout, r.stdout + r.stderr
+
+
+def test_rows_that_the_wide_loop_does_not_reach_go_to_other_tiles():
+    """The loop of gemm_q6k_wide.hpp has a 32-bit offset into the activations: 65535 super-blocks of a row and no more, in each rule that sends a launch there
+    (single matrices, lists, two matrices of one launch)."""
+    import subprocess
+    import tempfile
+    src = r'''
+#include <cstdio>
+#include "gemv_config.h"
+int main() {
+  unsigned t, k, n, m, rows[6];
+  while (std::scanf("%u %u %u %u", &t, &k, &n, &m) == 4) {
+    for (unsigned i = 0; i < n; i++) if (std::scanf("%u", &rows[i]) != 1) return 1;
+    std::printf("%u\n", gemm_list_rows(t, k, rows, n, m, -1));
+  }
+}
+'''
+    at, over = 65535 * 256, 65536 * 256
+    asked = [(13, k, 2, 1344, 2304, 2304) for k in (4096, at, over, over + 256, 1 << 31)] + [(12, over, 2, 1024, 8192, 8192)]
+    with tempfile.TemporaryDirectory() as d:
+        open(os.path.join(d, "t.cpp"), "w").write(src)
+        subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "cogni-ml_amd", "csrc", "kernels"), "-o", os.path.join(d, "t"),
+                        os.path.join(d, "t.cpp")], check=True)
+        got = subprocess.run([os.path.join(d, "t")], input="\n".join(" ".join(map(str, a)) for a in asked), capture_output=True, text=True, check=True)
+    got = [int(v) for v in got.stdout.split()]
+    assert got[:2] == [256, 256] and all(v in (128, 192) for v in got[2:5]) and got[5] == 256, got   # (Q4_K lists: a loop with 64-bit addresses)
+    two = quant.gemm_wide_two_takes
+    for a, b in (((12, 4096), (14, at)), ((13, 4096), (12, at)), ((12, at), (14, at)), ((12, 12288), (12, at))):
+        assert two(*a, 4096, *b, 4096, 256), (a, b)
+    for a, b in (((12, 4096), (14, over)), ((13, 4096), (12, over + 256)), ((12, over), (14, at)), ((12, over), (14, over)), ((12, 12288), (12, 1 << 31))):
+        assert not two(*a, 4096, *b, 4096, 256) and not two(*b, 4096, *a, 4096, 256), (a, b)
+    for k, wide in ((at, True), (over, False)):
+        assert quant.gemm_plan(14, k, 65536, 256, 1 << 40)[0].endswith("wide_f16") == wide
