@@ -512,4 +512,4 @@ int main() {
     for a, b in (((12, 4096), (14, over)), ((13, 4096), (12, over + 256)), ((12, over), (14, at)), ((12, over), (14, over)), ((12, 12288), (12, 1 << 31))):
         assert not two(*a, 4096, *b, 4096, 256) and not two(*b, 4096, *a, 4096, 256), (a, b)
     for k, wide in ((at, True), (over, False)):
-        assert quant.gemm_plan(14, k, 65536, 256, 1 << 40)[0].endswith("wide_f16") == wide
+        assert quant.gemm_plan(14, k, 4096, 2048, 1 << 40)[0].endswith("wide_f16") == wide
