@@ -9,6 +9,10 @@ from helpers import Q4_K, Q6_K
 pytestmark = pytest.mark.gpu
 
 
+def _dequantized(raw, out_dim, in_dim):
+    return quant.dequantize(raw, Q4_K, out_dim * in_dim).reshape(out_dim, in_dim)
+
+
 def sums_bound(oracle, raw, x, out_dim, in_dim):
     """Two fp32 sums of the same products in different orders differ by at most 2 n 2^-24 of the sum of their magnitudes (n additions)."""
     w = np.abs(oracle.dequantize(raw, Q4_K, out_dim * in_dim).reshape(out_dim, in_dim))
@@ -65,6 +69,40 @@ def test_gate_up_swiglu(gpu, tokens, out_dim, in_dim, next_type, keep):
         assert np.all(np.abs(a - b) <= 2.0**-10 * np.abs(a) + 3e-6 * np.abs(want).max())
     for a in (wg, wu, xd, ws, o1, o2, p1, p2):
         a.close()
+
+
+@pytest.mark.parametrize("scale", [1.0, 45.0])
+def test_gate_up_products_are_those_of_swiglu(gpu, scale):
+    """silu(gate) * up in the epilogue against swiglu_f32 of the same sums (gemm_tall_dev adds them in the same order): one function computed two ways, each within
+    an ulp of the same value at every step, so at most two ulps apart (the same bits on the MI355X); with scale 45 gates of +-200, the ones below -87.3 among
+    them where 1 / (1 + e^-g) is subnormal, and gates of either infinity and NaN: the same infinities and NaNs."""
+    tokens, in_dim, out_dim = 257, 512, 512
+    rng = np.random.default_rng(7)
+    x = synth.make_activations(rng, tokens, in_dim).reshape(tokens, in_dim)
+    rg, ru = (synth.make_weights(rng, Q4_K, out_dim, in_dim) for _ in range(2))
+    gates = x[:64] @ _dequantized(rg, out_dim, in_dim).T
+    x *= np.float32(scale / gates.std())
+    x[0], x[1], x[2, 3] = 1.0, -1.0, np.nan
+    blocks = rg.reshape(out_dim, in_dim // 256, 144)
+    blocks[5, :, :2], blocks[5, :, 2:4] = (0x00, 0x7C), 0   # row 5 of gate: d infinite, every scale and every code one, no minimum
+    blocks[5, :, 4:8], blocks[5, :, 8:12], blocks[5, :, 12:16], blocks[5, :, 16:] = 1, 0, 1, 0x11
+    n, wsb, nxb = tokens * out_dim, quant.gemm_workspace_bytes(Q4_K, in_dim, tokens), quant.gemm_workspace_bytes(Q6_K, out_dim, tokens)
+    xd, ws, nx, wg, wu = DevArray(x.reshape(-1)), DevArray(nbytes=wsb), DevArray(nbytes=nxb), DevArray(rg), DevArray(ru)
+    g, u, a, b = (DevArray(np.full(n, np.float32(-3.0))) for _ in range(4))
+    quant.gemm_pack_dev(xd.ptr, Q4_K, in_dim, tokens, ws.ptr, wsb)
+    quant.gemm_tall_swiglu_pack_dev(wg.ptr, wu.ptr, Q4_K, ws.ptr, wsb, a.ptr, Q6_K, nx.ptr, nxb, in_dim, out_dim, tokens)
+    quant.gemm_tall_dev([wg.ptr, wu.ptr], Q4_K, ws.ptr, wsb, [g.ptr, u.ptr], [out_dim, out_dim], in_dim, tokens)
+    quant.swiglu_dev(g.ptr, u.ptr, b.ptr, n)
+    gate, got, want = (v.read(np.float32, n) for v in (g, a, b))
+    assert gate[5] == np.inf and gate[out_dim + 5] == -np.inf and np.isnan(gate[2 * out_dim:3 * out_dim]).all()
+    if scale > 1:
+        assert (gate > 150).any() and (gate < -150).any() and ((gate > -88.7) & (gate < -87.4)).sum() > 20
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    finite = np.isfinite(want)
+    assert np.array_equal(np.signbit(got[finite]), np.signbit(want[finite]))
+    assert np.abs(got[finite].view(np.int32).astype(np.int64) - want[finite].view(np.int32)).max() <= 2
+    for v in (xd, ws, nx, wg, wu, g, u, a, b):
+        v.close()
 
 
 @pytest.mark.parametrize("tokens,in_dim,out_dim,taken", [(998, 512, 11102, True), (1024, 512, 12287, True), (1024, 1024, 8192, False), (300, 3840, 5000, False), (643, 1280, 10773, False)])
