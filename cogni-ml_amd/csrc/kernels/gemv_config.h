@@ -219,18 +219,20 @@ static inline unsigned gemv_mt_from(unsigned type, unsigned in_dim, unsigned out
   return type == 14 ? 3u : (in_dim >= 4096u ? 4u : 5u);
 }
 // The resident output head (a norm that writes the image in front, top-1 inside, with or without the logits): tokens of a group that go
-// through one pass. Beside the counts above, two and more tokens of at least GEMV_MT_HEAD_ROWS rows (the fewest timed), whatever the row
-// length: the other kernels take two tokens a pass there, or walk the weights once for the logits and once for the top-1. Q6_K, rows of 1024 | 1280 |
-// 2304 | 2816 values, 151936 rows, us a step, before -> one pass: 2 tokens 137 -> 62 | 138 -> 63 | 148 -> 109 | 152 -> 115, 3 tokens
-// with logits 132 -> 64 | 191 -> 65 | 336 -> 110 | 381 -> 117; 32000 rows, 2 tokens 42 -> 28 | 42 -> 28 | 43 -> 38 | 43 -> 38. Q4_K 109 -> 48 | 108 -> 48 |
-// 112 -> 70 | 112 -> 71 (32000 rows of 1024 35 -> 24, of 4096 39 -> 32); 3 tokens with logits 68 -> 48 | 105 -> 49 | 153 -> 74 | 168 -> 74. Not Q4_K rows of 1024 values,
-// three or four tokens, top-1 alone: the matrix-core kernel fills its k-slices there (151936 rows 43 | 48, 50000 27 | 30, 32000 24 | 25).
+// through one pass. Beside the counts above, three and four tokens of at least GEMV_MT_HEAD_ROWS rows, whatever the row length: the other kernels walk the
+// weights once for the logits and once for the top-1. Two tokens never: their other kernel has activations of 32 bits, the image 22 (2-norm of the
+// logits' error against 64 bits, Q4_K 1.2e-7 | 1.0e-6, Q6_K 1.9e-7 | 3.8e-7), where that of three and four has 22 as well (Q4_K 0.79e-6 to 1.46e-6 | 0.79e-6 to 1.49e-6, Q6_K 3.67e-7 to
+// 4.09e-7 | 3.79e-7 to 4.09e-7). Us a step, before | one pass. Q6_K, 151936 rows of 1024 | 1280 | 2304 | 2816 values, 3 tokens with logits 132 | 64, 191 | 65, 336 | 110, 381 | 117; 32000
+// rows, 3 tokens, top-1 alone 25.5 | 21.7, 34.5 | 22.2, 47.1 | 31.5, 52.6 | 32.0. Q4_K, 151936 rows with logits 68 | 48, 105 | 49, 153 | 74, 168 | 74. Not Q4_K, top-1 alone, rows of 1024 values,
+// whose k-slices the matrix-core kernel fills (151936 rows 38.3 | 41.9, 32000 16.6 | 18.0), and four tokens below GEMV_MT_TALL_ROWS (2304 values, 32000 | 36000 | 40000 | 50000 rows
+// 24.6 | 25.5 | 30.4 | 35.4 and 25.0 | 27.7 | 29.0 | 34.7). The line is where vocabularies start, not where the ways cross: with logits the one pass is ahead from 4096 rows on (Q6_K 1024 values,
+// 3 tokens, 4096 | 16384 rows 18.1 | 23.0 and 12.2 | 17.5), with the top-1 alone from 8192 to 32000 (at 24576 Q6_K 17.2 | 19.5, 2304 values 34.8 | 26.1).
 #define GEMV_MT_HEAD_ROWS 32000u
 static inline int gemv_mt_head_takes(unsigned type, unsigned tokens, unsigned in_dim, unsigned out_dim, int logits) {
   if ((type != 12 && type != 14) || in_dim > 4096u || tokens > (unsigned)GEMV_MT_MAX_TOKENS || !gemv_mt_supported(type, 2, in_dim)) return 0;
   if (tokens >= gemv_mt_from(type, in_dim, out_dim)) return 1;
-  if (tokens < 2u || out_dim < GEMV_MT_HEAD_ROWS) return 0;
-  return !(type == 12 && in_dim <= 1024u && tokens >= 3u && !logits);
+  if (tokens < 3u || out_dim < GEMV_MT_HEAD_ROWS) return 0;
+  return logits || type != 12 || (in_dim > 1024u && (tokens == 3u || out_dim >= GEMV_MT_TALL_ROWS));
 }
 // The same for a pair, a list of matrices or the fused gate | up | SwiGLU: from two tokens (one pack serves all of them and
 // the weights are read once), from five on rows that fill less than three quarters of their k-slices.

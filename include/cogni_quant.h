@@ -179,7 +179,7 @@ uint32_t cogni_gemv_one_pass_from(uint32_t w_type, uint32_t in_dim, uint32_t out
  * than that. No GPU needed. */
 uint32_t cogni_gemv_one_pass_multi_from(uint32_t w_type, uint32_t in_dim);
 /* Whether an output head whose norm writes the image (cogni_rmsnorm_pack_dev, then cogni_gemv_packed_top1[_logits]_dev) is the faster way for
- * `tokens` tokens: 1 or 0. Earlier than cogni_gemv_one_pass_from for vocabularies. */
+ * `tokens` tokens without less precision: 1 or 0. Three and four tokens of vocabularies earlier than cogni_gemv_one_pass_from, two never. */
 int32_t cogni_gemv_top1_one_pass(uint32_t w_type, uint32_t tokens, uint32_t in_dim, uint32_t out_dim, int32_t logits);
 /* Gives back the image the library keeps for `stream` (waits for the stream's work first; nothing to do and no error if it
  * has none). Call it before destroying a stream that ran multi-token GEMVs: the eight slots are otherwise used up by the

@@ -198,11 +198,12 @@ def test_output_head_runner(gpu, oracle, hidden, vocab, tokens):
 
 
 @pytest.mark.parametrize("t,hidden,vocab,tokens,logits,packed", [
-    (Q6_K, 1024, 32003, 2, True, True), (Q6_K, 2304, 32000, 3, False, True), (Q6_K, 1280, 31999, 4, True, False),
-    (Q4_K, 2816, 32001, 2, False, True), (Q4_K, 1024, 32000, 4, True, True), (Q4_K, 1024, 32000, 3, False, False)])
+    (Q6_K, 1024, 32003, 2, True, False), (Q6_K, 2304, 32000, 3, False, True), (Q6_K, 1280, 31999, 4, True, False),
+    (Q4_K, 2816, 32001, 2, False, False), (Q4_K, 1024, 32000, 4, True, True), (Q4_K, 1024, 32000, 3, False, False),
+    (Q4_K, 1280, 32000, 3, False, True), (Q4_K, 1280, 40959, 4, False, False), (Q4_K, 1280, 40960, 4, False, True)])
 def test_output_head_runner_of_few_tokens(gpu, oracle, t, hidden, vocab, tokens, logits, packed):
-    """Two to four tokens of a vocabulary whose rows do not fill the k-slices: the norm writes the image and the one-pass kernel takes
-    them from GEMV_MT_HEAD_ROWS rows on. Top-1 and logits within the GEMV bar of the oracle, and the top-1 that of the logits."""
+    """Two to four tokens of a vocabulary whose rows do not fill the k-slices: three and four go through a norm that writes the image and the
+    one-pass kernel from GEMV_MT_HEAD_ROWS rows on, by gemv_mt_head_takes; two, whose other kernel has activations of more bits, do not. Top-1 and logits within the GEMV bar of the oracle, and the top-1 that of the logits."""
     rng = np.random.default_rng(hidden + vocab + tokens)
     w = Weights((1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32), synth.make_weights(rng, t, vocab, hidden), t, hidden, vocab)
     xs = (rng.standard_normal(tokens * hidden) * 3).astype(np.float32)
@@ -224,6 +225,34 @@ def test_output_head_runner_of_few_tokens(gpu, oracle, t, hidden, vocab, tokens,
                 assert runner.top1_ids[tok] == first_max(dev) and runner.top1_values[tok] == dev.max()
     finally:
         runner.close()
+
+
+@pytest.mark.parametrize("t,hidden,vocab,logits", [(Q6_K, 1024, 32003, True), (Q4_K, 2304, 32000, True), (Q6_K, 2816, 33000, False), (Q4_K, 4096, 32000, True), (Q4_K, 1280, 50000, False)])
+def test_two_tokens_of_a_head_keep_32_bit_activations(gpu, t, hidden, vocab, logits):
+    """The bits of the norm and of the head's operator, one after the other."""
+    rng = np.random.default_rng(hidden)
+    w = Weights((1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32), synth.make_weights(rng, t, vocab, hidden), t, hidden, vocab)
+    xs = (rng.standard_normal(2 * hidden) * 3).astype(np.float32)
+    runner = QwenOutputHeadRunner.from_weights(w, 2, xs, 1e-6, read_logits=logits)
+    stride = quant.gemv_top1_partials(t, vocab)
+    x, norm, raw, normed = DevArray(xs), DevArray(w.norm), DevArray(w.output_raw), DevArray(nbytes=8 * hidden)
+    pi, pv, oi, ov, lo = (DevArray(nbytes=n) for n in (8 * stride, 8 * stride, 8, 8, 8 * vocab))
+    try:
+        runner.upload_weights()
+        runner.reset_sequence()
+        runner.run_sequence()
+        runner.read_outputs()
+        quant.rmsnorm_dev(x.ptr, norm.ptr, normed.ptr, hidden, 2, 1e-6)
+        if logits:
+            quant.gemv_top1_logits_dev(raw.ptr, t, normed.ptr, pi.ptr, pv.ptr, oi.ptr, ov.ptr, lo.ptr, hidden, vocab, 2)
+            assert np.array_equal(runner.logits.view(np.uint32), lo.read(np.uint32, 2 * vocab))
+        else:
+            quant.gemv_top1_dev(raw.ptr, t, normed.ptr, pi.ptr, pv.ptr, oi.ptr, ov.ptr, hidden, vocab, 2)
+        assert np.array_equal(runner.top1_values.view(np.uint32), ov.read(np.uint32, 2)) and np.array_equal(runner.top1_ids, oi.read(np.int32, 2))
+    finally:
+        runner.close()
+        for a in (x, norm, raw, normed, pi, pv, oi, ov, lo):
+            a.close()
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K])
