@@ -680,7 +680,7 @@ int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residua
       uint32_t tm, tn;
       const uint32_t grid = gemm_terms_plan(m, out_dim, &tm, &tn);
       char name[48];
-      std::snprintf(name, sizeof name, "%s_gemm_terms_f32_%ux%u", type_prefix(w_type), tm, tn);
+      std::snprintf(name, sizeof name, "%s_gemm_terms_f32_%ux%u%s", type_prefix(w_type), tm, tn, gemm_terms_interleaved(w_type, tm, tn, in_dim) ? "_i" : "");
       uint64_t xm = x + (uint64_t)t0 * in_dim * 4, om = out + (uint64_t)t0 * out_dim * 4;
       uint64_t rm = residual ? residual + (uint64_t)t0 * out_dim * 4 : 0;
       void* params[] = {&w_raw, &xm, &rm, &om, &in_dim, &out_dim, &m};

@@ -22,9 +22,10 @@
 // wavefront uses: no barrier in the loop.
 // What bounds it: small calls the chain load - LDS - sums (4 us), large ones the issue slots of a SIMD: Q8_0 4096 -> 4096, 256 tokens, 13300
 // instructions per SIMD, 82 % of its cycles, where a kernel without any load still takes 36 of the 42 us and one without the splitting of
-// x 39. A matrix instruction takes 7 to 8 clocks of issue, but its sum is there only 16 clocks later: the products of a token tile go out row tile by
+// x 39. A matrix instruction takes 7 to 8 clocks of issue, but its sum is there only 16 clocks later. Interleaved, the products of a token tile go out row tile by
 // row tile (TN independent sums), with the next tile's terms and the last one's sums in between, instead of one sum after the other: Q8_0 1024 ->
-// 3584, 200 tokens 15.1 -> 14.6 us, 4096 -> 4096, 256 tokens 43.5 -> 42.3; F16 2048 -> 2048, 33 tokens 8.65 -> 8.45; F32 4096 -> 4096, 256 tokens 79 -> 72.
+// 3584, 200 tokens 15.1 -> 14.6 us, 4096 -> 4096, 256 tokens 43.5 -> 42.3; F16 2048 -> 2048, 33 tokens 8.65 -> 8.45; F32 4096 -> 4096, 256 tokens 79 -> 72. Smaller
+// tiles have less to put between the products and lose by it on short rows: which take it is measured (gemm_terms_interleaved, gemv_config.h).
 // Splitting by v_cvt_pk_bf16_f32 and v_dot2_f32_bf16, half the instructions, gained nothing: the second takes twice as long.
 // Measured, weights from memory, row kernels (Q8_0: one-pass launches of eight tokens) -> these: Q8_0 1024 -> 3584, 9 / 48 / 200
 // tokens 9.6 / 35 / 143 -> 5.0 / 7.8 / 15.4 us; F16 2048 -> 2048, 33 tokens 41.8 -> 9.1; F32 4096 -> 4096, 33 tokens 174 -> 26; IQ4_NL
@@ -266,8 +267,9 @@ __device__ __forceinline__ void terms_plain_sums(const uint8_t* row, const float
   for (int v = 0; v < 4; v++) s[v] = wave_sum(s[v]);
 }
 
-// D: steps whose loads are in flight while one is computed (a ring of registers).
-template <class W, int TM, int TN, int D>
+// D: steps whose loads are in flight while one is computed (a ring of registers). INTERLEAVED: the order of a step's instructions
+// (gemm_terms_interleaved in gemv_config.h).
+template <class W, int TM, int TN, int D, bool INTERLEAVED>
 __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, const float* __restrict__ x, const float* residual,
                                                 float* out, u32 in_dim, u32 out_dim, u32 tokens) {
   constexpr u32 XD = 16 * TERMS_F32_STRIDE;                      // dwords of 16 rows of x
@@ -317,63 +319,93 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
     for (int t = 0; t < TM; t++) r.x[t].put(mine + t * XD, lane);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the lanes read what other lanes of the wavefront wrote
   };
-  // One step. Token tile t's matrix instructions go out term product by term product across the TN row tiles (TN independent sums: one
-  // after the other the three to eight of a sum wait for each other), with tile t + 1's terms and tile t - 1's sums made in between.
+  // One step. INTERLEAVED: token tile t's matrix instructions go out term product by term product across the TN row tiles (TN independent
+  // sums), with tile t + 1's terms and tile t - 1's sums made in between; else row tile by row tile, the three to eight products of a sum one after the
+  // other. The same sums, bit for bit.
   auto compute = [&]() {
-    constexpr bool AHEAD = W::TERMS == 1 || TM < 4;   // room for two sets of terms of x
-    constexpr int XB = AHEAD ? 2 : 1;
-    bf16x8_t B[TN][W::TERMS], X[XB][3];
-    float d[TN];
-    terms_f4 p[2][TN];
-    float v[8];
-    TermsF32Tile::get(mine, lane, v);
-    if constexpr (TM * TN == 1) terms_split<3>(v, X[0]);
+    if constexpr (INTERLEAVED) {
+      constexpr bool AHEAD = W::TERMS == 1 || TM < 4;   // room for two sets of terms of x
+      constexpr int XB = AHEAD ? 2 : 1;
+      bf16x8_t B[TN][W::TERMS], X[XB][3];
+      float d[TN];
+      terms_f4 p[2][TN];
+      float v[8];
+      TermsF32Tile::get(mine, lane, v);
 #pragma unroll
-    for (int c = 0; c < TN; c++) {
-      const u32* wl = mine + TM * XD + c * W::LDS_DWORDS;
-      W::terms(wl, lane, B[c]);
-      d[c] = W::scale(wl, lane);
-    }
-    if constexpr (TM * TN > 1) terms_split<3>(v, X[0]);
-    auto fold = [&](int t) {   // the sum over the step's 32 values joins the running sum in one rounding
+      for (int c = 0; c < TN; c++) {
+        const u32* wl = mine + TM * XD + c * W::LDS_DWORDS;
+        W::terms(wl, lane, B[c]);
+        d[c] = W::scale(wl, lane);
+      }
+      terms_split<3>(v, X[0]);
+      auto fold = [&](int t) {   // the sum over the step's 32 values joins the running sum in one rounding
 #pragma unroll
-      for (int c = 0; c < TN; c++)
+        for (int c = 0; c < TN; c++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[t][c][e] = W::SCALED ? fmaf(d[c], p[t & 1][c][e], acc[t][c][e]) : acc[t][c][e] + p[t & 1][c][e];
-    };
+          for (int e = 0; e < 4; e++) acc[t][c][e] = W::SCALED ? fmaf(d[c], p[t & 1][c][e], acc[t][c][e]) : acc[t][c][e] + p[t & 1][c][e];
+      };
 #pragma unroll
-    for (int t = 0; t < TM; t++) {
+      for (int t = 0; t < TM; t++) {
+        if (TM > 1) __builtin_amdgcn_sched_barrier(0);
+        if (AHEAD && t + 1 < TM) TermsF32Tile::get(mine + (t + 1) * XD, lane, v);
+        if (!AHEAD && t > 0) {
+          TermsF32Tile::get(mine + t * XD, lane, v);
+          terms_split<3>(v, X[0]);
+        }
+#pragma unroll
+        for (int c = 0; c < TN; c++) p[t & 1][c] = terms_f4{0.f, 0.f, 0.f, 0.f};
+        // term i of x against term j of w, i + j <= 3, smallest first
+#pragma unroll
+        for (int ij = 3; ij >= 0; ij--)
+#pragma unroll
+          for (int j = 0; j < W::TERMS; j++)
+            if (ij - j >= 0 && ij - j < 3) {
+#pragma unroll
+              for (int c = 0; c < TN; c++) p[t & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t % XB][ij - j], B[c][j], p[t & 1][c], 0, 0, 0);
+            }
+        if (AHEAD && t + 1 < TM) terms_split<3>(v, X[(t + 1) % XB]);
+        if (t > 0) fold(t - 1);
+        if (AHEAD && TM > 1) {
+          constexpr int MFMAS = TN * (W::TERMS == 1 ? 3 : (W::TERMS == 2 ? 6 : 8)), VALU = (72 + 4 * TN + MFMAS - 1) / MFMAS;
+          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+#pragma unroll
+          for (int i = 0; i < MFMAS; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+          }
+        }
+      }
       if (TM > 1) __builtin_amdgcn_sched_barrier(0);
-      if (AHEAD && t + 1 < TM) TermsF32Tile::get(mine + (t + 1) * XD, lane, v);
-      if (!AHEAD && t > 0) {
+      fold(TM - 1);
+    } else {
+      bf16x8_t X[TM][3];
+#pragma unroll
+      for (int t = 0; t < TM; t++) {
+        float v[8];
         TermsF32Tile::get(mine + t * XD, lane, v);
-        terms_split<3>(v, X[0]);
+        terms_split<3>(v, X[t]);
       }
 #pragma unroll
-      for (int c = 0; c < TN; c++) p[t & 1][c] = terms_f4{0.f, 0.f, 0.f, 0.f};
-      // term i of x against term j of w, i + j <= 3, smallest first
+      for (int c = 0; c < TN; c++) {
+        const u32* wl = mine + TM * XD + c * W::LDS_DWORDS;
+        bf16x8_t B[W::TERMS];
+        W::terms(wl, lane, B);
+        const float d = W::scale(wl, lane);
 #pragma unroll
-      for (int ij = 3; ij >= 0; ij--)
+        for (int t = 0; t < TM; t++) {
+          // term i of x against term j of w, i + j <= 3, smallest first; the sum over the step's 32 values joins the running sum
+          // in one rounding
+          terms_f4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < W::TERMS; j++)
-          if (ij - j >= 0 && ij - j < 3) {
+          for (int ij = 3; ij >= 0; ij--)
 #pragma unroll
-            for (int c = 0; c < TN; c++) p[t & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t % XB][ij - j], B[c][j], p[t & 1][c], 0, 0, 0);
-          }
-      if (AHEAD && t + 1 < TM) terms_split<3>(v, X[(t + 1) % XB]);
-      if (t > 0) fold(t - 1);
-      if (AHEAD && TM > 1) {
-        constexpr int MFMAS = TN * (W::TERMS == 1 ? 3 : (W::TERMS == 2 ? 6 : 8)), VALU = (72 + 4 * TN + MFMAS - 1) / MFMAS;
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            for (int j = 0; j < W::TERMS; j++)
+              if (ij - j >= 0 && ij - j < 3) p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(X[t][ij - j], B[j], p, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < MFMAS; i++) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, VALU, 0);
+          for (int v = 0; v < 4; v++) acc[t][c][v] = W::SCALED ? fmaf(d, p[v], acc[t][c][v]) : acc[t][c][v] + p[v];
         }
       }
     }
-    if (TM > 1) __builtin_amdgcn_sched_barrier(0);
-    fold(TM - 1);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   };
   // whole steps: contiguous runs of them per wavefront; a last step that the row ends inside is added by the last wavefront
@@ -474,18 +506,23 @@ __device__ __forceinline__ void gemm_terms_core(const uint8_t* __restrict__ w, c
   }
 }
 
-#define GEMM_TERMS_ENTRY(NAME, W, TM, TN, D)                                                                                    \
+#define GEMM_TERMS_ENTRY(NAME, W, TM, TN, D, INTERLEAVED)                                                                       \
   extern "C" __global__ __launch_bounds__(64 * GEMM_TERMS_WAVES) void NAME(const uint8_t* w, const float* x, const float* residual, \
                                                                            float* out, u32 in_dim, u32 out_dim, u32 tokens) {  \
-    gemm_terms_core<W, TM, TN, D>(w, x, residual, out, in_dim, out_dim, tokens);                                               \
+    gemm_terms_core<W, TM, TN, D, INTERLEAVED>(w, x, residual, out, in_dim, out_dim, tokens);                                  \
   }
-#define GEMM_TERMS_TYPE(PREFIX, W, D4)                      \
-  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_1x1, W, 1, 1, 2) \
-  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_1x2, W, 1, 2, 2) \
-  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_2x2, W, 2, 2, 2) \
-  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_2x4, W, 2, 4, 1) \
-  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_4x4, W, 4, 4, D4)
-GEMM_TERMS_TYPE(f32, TermsF32, 1)
-GEMM_TERMS_TYPE(f16, TermsF16, 1)
-GEMM_TERMS_TYPE(iq4_nl, TermsIq4nl, 1)
-GEMM_TERMS_TYPE(q8_0, TermsQ80, 1)
+// The tiles that are interleaved at every row length or at none have one kernel, the others a second one of the name with "_i".
+#define GEMM_TERMS_TYPE(PREFIX, W, SHORT)                            \
+  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_1x1, W, 1, 1, 2, false)   \
+  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_1x2, W, 1, 2, 2, SHORT)   \
+  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_2x2, W, 2, 2, 2, false)   \
+  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_2x2_i, W, 2, 2, 2, true)  \
+  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_2x4, W, 2, 4, 1, false)   \
+  GEMM_TERMS_ENTRY(PREFIX##_gemm_terms_f32_4x4, W, 4, 4, 1, true)
+GEMM_TERMS_TYPE(f32, TermsF32, true)
+GEMM_TERMS_TYPE(f16, TermsF16, true)
+GEMM_TERMS_TYPE(iq4_nl, TermsIq4nl, false)
+GEMM_TERMS_TYPE(q8_0, TermsQ80, false)
+GEMM_TERMS_ENTRY(f16_gemm_terms_f32_2x4_i, TermsF16, 2, 4, 1, true)
+GEMM_TERMS_ENTRY(iq4_nl_gemm_terms_f32_2x4_i, TermsIq4nl, 2, 4, 1, true)
+GEMM_TERMS_ENTRY(q8_0_gemm_terms_f32_2x4_i, TermsQ80, 2, 4, 1, true)

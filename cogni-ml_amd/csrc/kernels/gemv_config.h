@@ -485,6 +485,19 @@ static inline unsigned gemm_terms_plan(unsigned tokens, unsigned out_dim, unsign
   return mt * ((nt + GEMM_XCD_COUNT - 1u) / GEMM_XCD_COUNT) * GEMM_XCD_COUNT;
 }
 
+// Whether a tile's kernel for rows of in_dim values is a second one whose steps are interleaved (gemm_terms.hpp), "<name>_i"; the sums are the same bits. The
+// kernels alone, weights from memory, one round of 160 to 240 workgroups, us, row tile by row tile | interleaved. 2 x 2 at 1024, 1184, 1408, 2048 and 3072 columns: Q8_0 7.67 | 7.78,
+// 9.40 | 9.15, 9.57 | 9.45, 12.8 | 12.7, 16.2 | 16.2; F32 10.77 | 10.82, 11.98 | 11.96, 12.85 | 12.82, 16.2 | 15.7, 21.6 | 21.4; IQ4_NL 7.54 | 7.86, 8.42 | 8.71, 9.71 | 9.60, 12.2 | 12.3, 17.0 | 16.6;
+// F16 8.79 | 9.05, 10.3 | 10.4, 10.7 | 10.8, 13.2 | 13.0, 17.7 | 17.5. 2 x 4 at 1184, 1536, 2592 and 3488: Q8_0 11.8 | 12.0, 13.9 | 13.8 (calls of 1632 11.7 | 12.0), 20.6 | 19.5, 28.9 | 26.1; F16 13.4 | 13.6, 16.7 | 16.1, 22.2 | 22.3,
+// 30.2 | 30.1 (4096 32.7 | 31.5); IQ4_NL 11.5 | 12.0, 13.9 | 14.3, level at 2592, 26.8 | 25.8. One order is the better one at (nearly) every length, and has the name, for 1 x 1 (no other sum to
+// go to); 1 x 2 of F32 (interleaved, 8.35 | 8.17, 18.7 | 18.1), F16 (level), Q8_0 and IQ4_NL (not, 768 columns 5.18 | 5.31, 5.73 | 5.77, long rows level); 2 x 4 of F32 (not, 12.5 | 13.4,
+// 39.3 | 40.4); 4 x 4 (interleaved, 1024 and 4096 columns, Q8_0 15.2 | 14.7, 40.0 | 38.3, the others alike).
+static inline int gemm_terms_interleaved(unsigned type, unsigned tm, unsigned tn, unsigned in_dim) {
+  if (tm != 2u) return 0;
+  if (tn == 2u) return in_dim >= (type == 1u ? 1536u : (type == 20u ? 1408u : 1152u));
+  return type != 0u && in_dim >= (type == 1u ? 1536u : (type == 20u ? 2560u : 1696u));
+}
+
 // ---- short prefills of Q4_K, Q5_K and Q6_K (gemm_stream.hpp): a workgroup takes 32 t tokens x 32 rt rows
 #define GEMM_STREAM_MAX_SPLITS 8u
 #define GEMM_STREAM_MAX_PACKED 0x7FFFFFFFu   // bytes of packed activations the kernels can address

@@ -127,7 +127,7 @@ int cogni_dequantize_dev(uint64_t w_raw, uint32_t w_type, uint64_t n_elements, u
  * tokens of F32 and F16, IQ4_NL at any token count, and Q8_0 with more than eight tokens (or with rows that are no multiple of
  * 256 from three) take the matrix cores in one launch (of fewer than 2^32 threads: from 2^24 tokens of up to 128 rows, or as many outputs
  * of taller matrices, in several) to the same precision, operands as exact bfloat16 terms:
- * "<type>_gemm_terms_f32_<TM>x<TN>". The code object also holds "iq4_nl_gemv_plain_f32", a row kernel of the same parameters that
+ * "<type>_gemm_terms_f32_<TM>x<TN>", and for long rows of some tiles the same sums in another order of instructions, "..._i". The code object also holds "iq4_nl_gemv_plain_f32", a row kernel of the same parameters that
  * only hosts launching by name reach. Every other ggml type is refused with COGNI_ERR_UNSUPPORTED_TYPE and the reference's
  * message. */
 int cogni_gemv_dev(uint64_t w_raw, uint32_t w_type, uint64_t x, uint64_t residual, uint64_t out,

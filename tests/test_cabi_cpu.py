@@ -513,3 +513,32 @@ int main() {
         assert not two(*a, 4096, *b, 4096, 256) and not two(*b, 4096, *a, 4096, 256), (a, b)
     for k, wide in ((at, True), (over, False)):
         assert quant.gemm_plan(14, k, 4096, 2048, 1 << 40)[0].endswith("wide_f16") == wide
+
+
+def test_interleaved_term_kernels_are_taken_where_they_are_faster():
+    """gemm_terms_interleaved (gemv_config.h) against times of the kernels alone, step by step | interleaved, at a row length (MI355X, us, one round of workgroups,
+    weights from memory): the pick is never more than 2 % behind the other; the tiles with one kernel have one order at every length."""
+    import subprocess
+    import tempfile
+    timed = [
+        (0, 2, 2, (768, 9.81, 9.96), (1024, 10.77, 10.82), (1184, 11.98, 11.96), (1408, 12.85, 12.82), (1536, 14.13, 13.94), (1696, 14.62, 14.34), (1856, 17.53, 17.21), (2048, 16.15, 15.73), (2304, 17.41, 16.97), (2592, 19.61, 19.35), (2816, 19.66, 19.36), (3072, 21.62, 21.43), (3488, 25.16, 24.65), (3680, 24.39, 23.91), (4096, 25.30, 24.75)),
+        (1, 2, 2, (768, 8.24, 8.59), (1024, 8.79, 9.05), (1184, 10.29, 10.40), (1408, 10.68, 10.79), (1536, 11.57, 11.55), (1696, 12.30, 12.20), (1856, 13.88, 13.84), (2048, 13.15, 12.96), (2304, 14.59, 14.31), (2592, 16.48, 16.32), (2816, 16.53, 16.30), (3072, 17.66, 17.50), (3488, 20.88, 20.69), (3680, 20.48, 20.04), (4096, 20.93, 20.58)),
+        (1, 2, 4, (768, 9.30, 9.72), (1024, 11.37, 11.15), (1184, 13.35, 13.55), (1408, 14.59, 14.83), (1536, 16.71, 16.09), (1696, 17.24, 17.09), (1856, 19.39, 19.08), (2048, 18.08, 17.95), (2304, 21.06, 21.02), (2592, 22.16, 22.32), (2816, 23.78, 23.32), (3072, 24.97, 24.44), (3488, 30.22, 30.07), (3680, 29.49, 29.02), (4096, 32.71, 31.52)),
+        (20, 2, 2, (768, 7.00, 7.20), (1024, 7.54, 7.86), (1184, 8.42, 8.71), (1408, 9.71, 9.60), (1536, 9.94, 9.76), (1696, 10.48, 10.39), (1856, 12.09, 12.03), (2048, 12.23, 12.27), (2304, 13.22, 12.80), (2592, 15.30, 14.87), (2816, 15.25, 14.88), (3072, 16.95, 16.56), (3488, 18.74, 18.42), (3680, 18.97, 18.64), (4096, 20.72, 20.13)),
+        (20, 2, 4, (768, 8.27, 8.88), (1024, 9.51, 10.01), (1184, 11.54, 12.01), (1408, 12.27, 12.71), (1536, 13.92, 14.33), (1696, 14.94, 15.22), (1856, 16.23, 16.23), (2048, 16.49, 17.19), (2304, 18.28, 18.28), (2592, 19.90, 19.87), (2816, 21.40, 20.97), (3072, 22.19, 22.03), (3488, 26.81, 25.84), (3680, 26.17, 25.53), (4096, 29.37, 29.76)),
+        (8, 2, 2, (768, 6.89, 7.08), (1024, 7.67, 7.78), (1184, 9.40, 9.15), (1408, 9.57, 9.45), (1536, 10.63, 10.48), (1696, 10.90, 10.87), (1856, 12.84, 12.62), (2048, 12.82, 12.73), (2304, 13.65, 13.30), (2592, 16.13, 15.81), (2816, 15.69, 15.63), (3072, 16.20, 16.24), (3488, 18.66, 18.48), (3680, 18.95, 18.97), (4096, 19.64, 19.41)),
+        (8, 2, 4, (768, 7.69, 8.15), (1024, 9.24, 9.69), (1184, 11.82, 12.00), (1408, 12.69, 12.66), (1536, 13.88, 13.76), (1696, 15.59, 15.12), (1856, 17.09, 16.43), (2048, 16.03, 16.02), (2304, 18.51, 17.79), (2592, 20.61, 19.47), (2816, 22.17, 20.84), (3072, 21.86, 21.24), (3488, 28.93, 26.13), (3680, 28.06, 25.58), (4096, 27.52, 26.98))]
+    src = '#include <cstdio>\n#include "gemv_config.h"\nint main() { unsigned t, m, n, k; while (std::scanf("%u %u %u %u", &t, &m, &n, &k) == 4) ' \
+          'std::printf("%d\\n", gemm_terms_interleaved(t, m, n, k)); }'
+    both = {c[:3] for c in timed}
+    asked = [c[:3] + v[:1] for c in timed for v in c[3:]]
+    alone = [(t, m, n, k) for t in (0, 1, 8, 20) for m, n in ((1, 1), (1, 2), (2, 2), (2, 4), (4, 4)) if (t, m, n) not in both for k in (32, 2048, 4096, 1 << 20)]
+    with tempfile.TemporaryDirectory() as d:
+        open(os.path.join(d, "t.cpp"), "w").write(src)
+        subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "cogni-ml_amd", "csrc", "kernels"), "-o", os.path.join(d, "t"),
+                        os.path.join(d, "t.cpp")], check=True)
+        got = subprocess.run([os.path.join(d, "t")], input="\n".join("%d %d %d %d" % a for a in asked + alone), capture_output=True, text=True, check=True)
+    picks = [int(v) for v in got.stdout.split()]
+    for (t, m, n, k), us, pick in zip(asked, [v[1:] for c in timed for v in c[3:]], picks):
+        assert us[pick] <= 1.02 * min(us), (t, m, n, k, us, pick)
+    assert not any(picks[len(asked):])

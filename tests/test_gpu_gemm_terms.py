@@ -253,6 +253,38 @@ def test_more_tokens_than_a_launch_has_threads_for(gpu, t):
             a.close()
 
 
+@pytest.mark.parametrize("t,prefix,tm,tn,name", [(IQ4_NL, "iq4_nl", 2, 4, "2x4"), (F32, "f32", 2, 2, "2x2"), (F16, "f16", 2, 2, "2x2"), (IQ4_NL, "iq4_nl", 2, 2, "2x2"),
+                                                 (Q8_0, "q8_0", 2, 2, "2x2"), (F16, "f16", 2, 4, "2x4"), (Q8_0, "q8_0", 2, 4, "2x4")])
+@pytest.mark.parametrize("in_dim", [32, 70, 300, 544, 4096])
+def test_both_orders_of_a_step_give_the_same_bits(gpu, t, prefix, tm, tn, name, in_dim):
+    """The interleaved kernel of a tile and the other, launched by name: one step, fewer than wavefronts, a row that ends inside one, many; tiles that end
+    behind the last row and token, one row of tiles for each XCD."""
+    out_dim, tokens = 16 * tn * 8 - 3, 16 * tm * 3 - 5
+    rng = np.random.default_rng(t + in_dim)
+    w, x = DevArray(synth.make_weights(rng, t, out_dim, in_dim)), DevArray(synth.make_activations(rng, tokens, in_dim))
+    res = DevArray(synth.make_activations(rng, tokens, out_dim))
+    outs = [DevArray(np.full(tokens * out_dim + 4, np.float32(-3.0))) for _ in range(2)]
+    module = hip.HIPModule.load_builtin()
+    try:
+        for o, suffix in zip(outs, ("", "_i")):
+            kernel = "%s_gemm_terms_f32_%s%s" % (prefix, name, suffix)
+            params = hip.KernelParams(*[ctypes.c_uint64(v) for v in (w.ptr, x.ptr, res.ptr, o.ptr)], *[ctypes.c_uint32(v) for v in (in_dim, out_dim, tokens)])
+            hip.launch(module.function(kernel), 3 * 8, 1, 1, 512, 1, 1, params, kernel)
+        a, b = (o.read(np.uint32, tokens * out_dim + 4) for o in outs)
+        assert np.array_equal(a, b) and np.all(a[tokens * out_dim:].view(np.float32) == -3.0)
+    finally:
+        module.close()
+        for v in [w, x, res] + outs:
+            v.close()
+
+
+@pytest.mark.parametrize("t,out_dim,tokens,in_dim", [(F32, 3584, 47, 1184), (F16, 2049, 60, 1540), (IQ4_NL, 3001, 35, 1408), (Q8_0, 924, 227, 1152),
+                                                     (F16, 1796, 189, 1536), (IQ4_NL, 1605, 173, 2560), (Q8_0, 1605, 173, 1696)])
+def test_rows_long_enough_for_the_interleaved_kernels(gpu, oracle, t, out_dim, tokens, in_dim):
+    """gemv_dev where it takes them, to the bound of test_terms_kernels_match_the_oracle."""
+    test_terms_kernels_match_the_oracle(gpu, oracle, t, in_dim, out_dim, tokens)
+
+
 def test_token_limit_of_a_launch(gpu):
     """The launches of one call, by the number of rows; matrices of 2^27 rows keep the kernels that walk them."""
     for out_dim in (1, 129, 3584, 151936, 1 << 26):
