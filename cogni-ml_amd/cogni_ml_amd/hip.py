@@ -10,6 +10,7 @@ import contextlib
 import ctypes
 import enum
 import os
+import re
 import threading
 
 try:
@@ -33,8 +34,8 @@ class HIPError(RuntimeError):
 def lib():
     """Load libcogni_hip.so. There is no fallback: a missing library is an error."""
     global _lib
-    if _recording_threads and getattr(_noting, "calls", None) is not None:
-        return _noting.lib
+    if _recording_threads and getattr(_noting, "on", False):
+        return _noting.proxy
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError("%s is missing: build it with `make -C cogni-ml_amd/csrc` "
@@ -89,61 +90,93 @@ def lib():
     return _lib
 
 
-_noting = threading.local()   # .calls, .lib: the list this thread notes its launches in, while it does
+_noting = threading.local()   # .on, .proxy: whether this thread notes its launches, and the library as lib() then gives it
 _recording_threads = 0
 _recording_lock = threading.Lock()
+# what cannot be noted: entry points that change or move something without being operators, and everything of the driver layer
+_NOT_AN_OPERATOR = re.compile(r"(?!cogni_)(?!typed_)|cogni_(quant_|weight_|matmul_add$|dequantize$|gemv_release_stream$|set_)")
 
 
 class _NotingLib:
-    """The library as lib() gives it to a thread that notes its launches: a cogni_*_dev call is made and kept without its stream."""
+    """The library as lib() gives it to a thread that notes its launches: an operator (*_dev) on the current stream is made and kept without its stream,
+    a question is asked, and anything else leaves the notes incomplete."""
 
-    def __init__(self, real, calls):
-        self._real, self._calls = real, calls
+    def __init__(self, real):
+        self._real = real
+        self.begin()
+
+    def begin(self):
+        self._calls, self._complete = [], True
+
+    def notes(self):
+        """The calls noted since begin(), or False where they are not all that was done."""
+        return self._complete and self._calls or False
 
     def __getattr__(self, name):
         f = getattr(self._real, name)
-        if not name.endswith("_dev"):
+        if _NOT_AN_OPERATOR.match(name):
+            self._complete = False
             return f
+        if name.endswith("_dev"):
+            real = f
 
-        def call(*args):
-            self._calls.append((f, args[:-1]))
-            return f(*args)
-        return call
+            def f(*args):
+                if args and args[-1] is _current_stream:
+                    self._calls.append((real, args[:-1]))
+                else:
+                    self._complete = False
+                return real(*args)
+        self.__dict__[name] = f   # (found without this function from now on)
+        return f
 
 
 def issue(kept, key, launch, check_status):
     """launch(), which issues operators on the current stream: the second time with a `key` the library calls that it makes are noted, and from the
     third those are made again, with the same arguments on the stream that is current then, without the Python that chose them (stack of seven
-    projections, 48 tokens: 31 us of host time by launch()). Not the first time: noting takes 5 to 9 us, which one that is run only once would pay for
-    nothing. `kept` holds the calls, at most 32 keys of them; `key` names all that the choice depends on beside what never changes for the
-    owner of `kept`."""
-    calls = kept.get(key)
-    if calls:
+    projections, 48 tokens: 31 us of host time by launch(), 11 from the notes). Not the first time: noting takes some microseconds, which one that is run
+    only once would pay for nothing. A launch() that does more than call operators on the current stream (copies, other streams, the driver layer) is
+    never noted, and within another issue() it is part of what that notes. Who counts or traces calls of this package's Python functions sees the first
+    two passes; the library's own entry points are called every time. `kept` holds the calls, of 32 keys at most; `key` names all that
+    the choice depends on beside what never changes for the owner of `kept`."""
+    if _recording_threads and getattr(_noting, "on", False):
+        launch()
+        return
+    noted = kept.get(key)
+    if noted:
         stream = _current_stream
-        for f, args in calls:
+        for f, args in noted:
             code = f(*args, stream)
             if code != 0:
                 check_status(code)
         return
-    if calls is None:
+    if noted is None or noted is False:
         launch()
-        if len(kept) >= 32:
-            kept.clear()
-        kept[key] = ()
+        if noted is None:
+            with _recording_lock:
+                if len(kept) >= 32:
+                    kept.clear()
+                kept[key] = ()
         return
-    global _recording_threads
-    calls, outer = [], (getattr(_noting, "calls", None), getattr(_noting, "lib", None))
-    proxy = _NotingLib(lib(), calls)
-    with _recording_lock:
-        _recording_threads += 1
-    _noting.calls, _noting.lib = calls, proxy
+    proxy, real = getattr(_noting, "proxy", None), lib()
+    if proxy is None or proxy._real is not real:
+        proxy = _noting.proxy = _NotingLib(real)
+    proxy.begin()
+    _count_noting(1)
+    _noting.on = True
     try:
         launch()
     finally:
-        _noting.calls, _noting.lib = outer
-        with _recording_lock:
-            _recording_threads -= 1
-    kept[key] = calls
+        _noting.on = False
+        _count_noting(-1)
+    kept[key] = proxy.notes()
+
+
+def _count_noting(by):
+    global _recording_threads
+    with _recording_lock:
+        _recording_threads += by
+        if calls is not None:
+            calls.set_noting(_recording_threads)   # (the native calls then go through the Python functions, and so through lib())
 
 
 _current_stream = None  # module-global, like @@current_stream (driver.cr:55)

@@ -6,9 +6,9 @@
 // short GEMM 10.65 -> 9.88.
 //
 // A call with ordinary arguments (plain integers, a TensorType, a stream that is None, an integer or a ctypes.c_void_p) goes straight to
-// the library. Everything else - other types, values out of range, missing or repeated arguments, a library that is not loaded yet, a
-// status other than 0 - is handed to the Python function of the same name, so what is refused, converted or raised there stays
-// exactly that.
+// the library, a status other than 0 to the check that raises. Everything else - other types, values out of range, missing or repeated
+// arguments, a library that is not loaded yet, a sequence that is being noted (hip.issue) - is handed to the Python function of the same name, so what is refused,
+// converted or raised there stays exactly that.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -26,6 +26,8 @@ PyObject *slow_matmul, *slow_gemv, *slow_dequantize, *check, *tensor_type, *void
 matmul_fn f_matmul;
 gemv_fn f_gemv;
 dequantize_fn f_dequantize;
+// threads that note the calls of a sequence: they see those that go through hip.lib()
+int noting;
 
 // The parameters of a function in order; arguments by position, by keyword or left out are put in their places. False: not a call
 // this module takes.
@@ -116,7 +118,7 @@ PyObject* matmul_dev(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObjec
   uint64_t w = 0, x = 0, out = 0, ws = 0, ws_bytes = 0, bias = 0;
   uint32_t type = 0, in_dim = 0, out_dim = 0, tokens = 0;
   void* stream;
-  if (!f_matmul || !place(n_matmul, args, nargs, kw, 7, a) || !as_u64(a[0], &w) || !as_type(a[1], &type) || !as_u64(a[2], &x) ||
+  if (noting || !f_matmul || !place(n_matmul, args, nargs, kw, 7, a) || !as_u64(a[0], &w) || !as_type(a[1], &type) || !as_u64(a[2], &x) ||
       !as_u64(a[3], &out) || !as_u32(a[4], &in_dim) || !as_u32(a[5], &out_dim) || !as_u32(a[6], &tokens) || !as_u64(a[7], &ws) ||
       !as_u64(a[8], &ws_bytes) || !as_u64(a[9], &bias) || !as_stream(a[10], &stream))
     return hand_on(slow_matmul, args, nargs, kw);
@@ -132,7 +134,7 @@ PyObject* gemv_dev(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject*
   uint64_t w = 0, x = 0, out = 0, residual = 0;
   uint32_t type = 0, in_dim = 0, out_dim = 0, tokens = 1;
   void* stream;
-  if (!f_gemv || !place(n_gemv, args, nargs, kw, 6, a) || !as_u64(a[0], &w) || !as_type(a[1], &type) || !as_u64(a[2], &x) ||
+  if (noting || !f_gemv || !place(n_gemv, args, nargs, kw, 6, a) || !as_u64(a[0], &w) || !as_type(a[1], &type) || !as_u64(a[2], &x) ||
       !as_u64(a[3], &out) || !as_u32(a[4], &in_dim) || !as_u32(a[5], &out_dim) || !as_u32(a[6], &tokens) || !as_u64(a[7], &residual) ||
       !as_stream(a[8], &stream))
     return hand_on(slow_gemv, args, nargs, kw);
@@ -148,7 +150,7 @@ PyObject* dequantize_dev(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyO
   uint64_t w = 0, n = 0, out = 0;
   uint32_t type = 0;
   void* stream;
-  if (!f_dequantize || !place(n_dequantize, args, nargs, kw, 4, a) || !as_u64(a[0], &w) || !as_type(a[1], &type) || !as_u64(a[2], &n) ||
+  if (noting || !f_dequantize || !place(n_dequantize, args, nargs, kw, 4, a) || !as_u64(a[0], &w) || !as_type(a[1], &type) || !as_u64(a[2], &n) ||
       !as_u64(a[3], &out) || !as_stream(a[4], &stream))
     return hand_on(slow_dequantize, args, nargs, kw);
   int status;
@@ -179,6 +181,12 @@ PyObject* set_library(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
+// set_noting(number of threads)
+PyObject* set_noting(PyObject*, PyObject* args) {
+  if (!PyArg_ParseTuple(args, "i", &noting)) return nullptr;
+  Py_RETURN_NONE;
+}
+
 PyMethodDef methods[] = {
     {"matmul_dev", (PyCFunction)(void (*)(void))matmul_dev, METH_FASTCALL | METH_KEYWORDS,
      "matmul_dev($module, /, w_ptr, w_type, x_ptr, out_ptr, in_dim, out_dim, tokens, workspace_ptr=0, workspace_bytes=0, bias_ptr=0, stream=None)\n"
@@ -189,6 +197,7 @@ PyMethodDef methods[] = {
      "dequantize_dev($module, /, w_ptr, w_type, n_elements, out_ptr, stream=None)\n--\n\n"},
     {"set_python", set_python, METH_VARARGS, nullptr},
     {"set_library", set_library, METH_VARARGS, nullptr},
+    {"set_noting", set_noting, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "cogni_ml_amd._calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
