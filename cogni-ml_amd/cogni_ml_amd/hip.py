@@ -136,7 +136,7 @@ def issue(kept, key, launch, check_status):
     projections, 48 tokens: 31 us of host time by launch(), 11 from the notes). Not the first time: noting takes some microseconds, which one that is run
     only once would pay for nothing. A launch() that does more than call operators on the current stream (copies, other streams, the driver layer) is
     never noted, and within another issue() it is part of what that notes. Who counts or traces calls of this package's Python functions sees the first
-    two passes; the library's own entry points are called every time. `kept` holds the calls, of 32 keys at most; `key` names all that
+    two passes; the library's own entry points are called every time. `kept` holds the calls, of 32 keys at most, the oldest going first; `key` names all that
     the choice depends on beside what never changes for the owner of `kept`."""
     if _recording_threads and getattr(_noting, "on", False):
         launch()
@@ -153,8 +153,8 @@ def issue(kept, key, launch, check_status):
         launch()
         if noted is None:
             with _recording_lock:
-                if len(kept) >= 32:
-                    kept.clear()
+                while len(kept) >= 32:
+                    del kept[next(iter(kept))]
                 kept[key] = ()
         return
     proxy, real = getattr(_noting, "proxy", None), lib()

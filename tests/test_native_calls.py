@@ -246,6 +246,19 @@ def test_a_sequence_within_a_sequence(other):
     assert len(outer[1]) == 2
 
 
+def test_the_oldest_notes_go_first(other):
+    kept = {}
+
+    def launch():
+        hip.lib().cogni_gemm_tall_takes(1)
+        hip.lib().cogni_a_dev(2, hip.current_stream_handle())
+
+    for key in range(40):
+        passes(other, kept, key, launch, 2)
+    assert sorted(kept) == list(range(8, 40)) and all(len(kept[k]) == 1 for k in kept)
+    assert passes(other, kept, 8, launch, 1) == [[("a", 2, None)]]
+
+
 def test_threads_note_their_own_calls(other):
     import threading
     kept, go = [{} for _ in range(4)], threading.Barrier(4)
