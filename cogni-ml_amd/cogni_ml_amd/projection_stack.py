@@ -13,6 +13,8 @@ in the reference's router) goes through the prefill GEMMs instead, all tokens at
 once (q | k | v and gate | up share x) and each projection is one GEMM against it - the reference's
 `qmatmul_nobias(qw, x, batch)` calls of a prefill layer (src/ml/gguf/qwen35_cpu.cr:1478-1490).
 """
+import collections
+
 import numpy as np
 
 from . import hip, quant
@@ -47,6 +49,10 @@ class Weights:
     @property
     def raw_bytes(self):
         return sum(e[5].size for e in self.entries)
+
+
+# a group of projections as a prefill launches it (the first field is the name of its first projection, as in Weights.entries)
+PrefillGroup = collections.namedtuple("PrefillGroup", "name key type in_dim x ws nbytes image16 lists w out dims nexts entry")
 
 
 class QwenProjectionStackRunner:
@@ -85,6 +91,7 @@ class QwenProjectionStackRunner:
         self._two_scratch = self._alloc(quant.gemm_wide_two_scratch_bytes()) if self._prefill_ws and any(
             self._wide_two(g[0], h[0], n) for groups in self._rounds for i, g in enumerate(groups) for h in groups[i + 1:] if len(g) == len(h) == 1
             for n in [tokens, *range(193, tokens, 64)]) else None
+        self._prefill_groups = [[self._prefill_group(g) for g in groups] for groups in self._rounds] if self._prefill_ws else []
         self._issued = {}   # prefill: the library calls of a token count
         self.outputs = {}
         self._runner = hip.ResidentSequenceRunner(
@@ -213,78 +220,84 @@ class QwenProjectionStackRunner:
                 return (src, self._family(t)), (t, ws.ptr, nbytes)
         return None
 
+    def _prefill_group(self, grp):
+        """What a prefill of any token count has to know of a group of a round."""
+        name, src, t, out_dim, in_dim, raw = grp[0]
+        key = (src, self._family(t))
+        ws, nbytes = self._prefill_ws[key]
+        lists = int(t) in (int(TensorType.Q4_K), int(TensorType.Q5_K))
+        nexts = [self._next_input(e) for e in grp] if len(grp) >= 2 and lists else []
+        return PrefillGroup(name=name, key=key, type=t, in_dim=in_dim, x=self._act[src].ptr, ws=ws.ptr, nbytes=nbytes,
+                            image16=self._images16[key].ptr if self._one_pass16(t, in_dim) else None, lists=lists,
+                            w=[self._w[e[0]].ptr for e in grp], out=[self._act[e[0]].ptr for e in grp], dims=[e[3] for e in grp],
+                            nexts=nexts if any(nexts) else [], entry=grp[0])
+
     def _launch_prefill(self, count):
         """All `count` tokens through the GEMMs: one pack per (input, layout), one GEMM per list of projections that share
         their input, type and row length (or per projection). A list that can leaves its outputs as the packed inputs of the
         rounds behind it too."""
         stream = hip.current_stream_handle()
-        list_types = (int(TensorType.Q4_K), int(TensorType.Q5_K))
         packed = set()   # the (input, layout) that a list has written
-        for groups in self._rounds:
+
+        # single matrices of up to sixteen tokens, or of short prefills, or two that share the chip: two to a launch (o and down)
+        def one_image(g):
+            return g.w[0], g.type, g.image16, g.out[0], g.in_dim, g.dims[0]
+
+        def one_packed(g):
+            return g.w[0], g.type, g.ws, g.nbytes, g.out[0], g.in_dim, g.dims[0]
+
+        for groups in self._prefill_groups:
             # the inputs of the round, packed once each, two to a launch
             jobs16, jobs = {}, {}
-            for grp in groups:
-                name, src, t, out_dim, in_dim, raw = grp[0]
-                key = (src, self._family(t))
-                if count <= 16 and self._one_pass16(t, in_dim):
-                    jobs16.setdefault(key, (self._act[src].ptr, t, in_dim, self._images16[key].ptr))
-                elif key not in packed:
-                    jobs.setdefault(key, (self._act[src].ptr, t, in_dim, self._prefill_ws[key][0].ptr, self._prefill_ws[key][1]))
+            for g in groups:
+                if count <= 16 and g.image16:
+                    jobs16.setdefault(g.key, (g.x, g.type, g.in_dim, g.image16))
+                elif g.key not in packed:
+                    jobs.setdefault(g.key, (g.x, g.type, g.in_dim, g.ws, g.nbytes))
             self._pack_each(list(jobs16.values()), lambda x, t, k, image: quant.gemv_pack16_dev(x, t, k, count, image, stream),
                             lambda *ab: quant.gemv_pack16_two_dev(*ab, count, stream))
             self._pack_each(list(jobs.values()), lambda x, t, k, ws, nbytes: quant.gemm_pack_dev(x, t, k, count, ws, nbytes, stream),
                             lambda *ab: quant.gemm_pack_two_dev(*ab, count, stream))
-            # single matrices of up to sixteen tokens, or of short prefills: two to a launch (o and down)
-            def one_image(e):
-                name, src, t, out_dim, in_dim, raw = e
-                return self._w[name].ptr, t, self._images16[(src, self._family(t))].ptr, self._act[name].ptr, in_dim, out_dim
-
-            def one_packed(e):
-                name, src, t, out_dim, in_dim, raw = e
-                ws, nbytes = self._prefill_ws[(src, self._family(t))]
-                return self._w[name].ptr, t, ws.ptr, nbytes, self._act[name].ptr, in_dim, out_dim
-
-            alone = [g[0] for g in groups if len(g) == 1]
-            done = self._pairs([e for e in alone if (e[1], self._family(e[2])) in jobs16],
-                               lambda a, b: quant.gemv_packed16_two_dev(*one_image(a), *one_image(b), count, stream))
-            if self._two_scratch is not None:
-                for i, a in enumerate(alone):
-                    b = next((e for e in alone[i + 1:] if e[0] not in done and self._wide_two(a, e, count)), None)
-                    if b is not None and a[0] not in done:
-                        quant.gemm_wide_two_dev(*one_packed(a), *one_packed(b), self._two_scratch.ptr, quant.gemm_wide_two_scratch_bytes(), count, stream)
-                        done |= {a[0], b[0]}
-            done |= self._pairs([e for e in alone if (e[1], self._family(e[2])) not in jobs16 and e[0] not in done and
-                                 quant.gemm_stream_takes(e[2], e[4], e[3], count)],
-                                lambda a, b: quant.gemm_stream_two_dev(*one_packed(a), *one_packed(b), count, stream))
-            for grp in groups:
-                if grp[0][0] in done:
+            alone = [g for g in groups if len(g.w) == 1]
+            done = set()
+            if len(alone) >= 2:
+                done = self._pairs([g for g in alone if g.key in jobs16],
+                                   lambda a, b: quant.gemv_packed16_two_dev(*one_image(a), *one_image(b), count, stream))
+                if self._two_scratch is not None and count > 128:   # (tiles of 128 tokens)
+                    for i, a in enumerate(alone):
+                        b = next((g for g in alone[i + 1:] if g.name not in done and self._wide_two(a.entry, g.entry, count)), None)
+                        if b is not None and a.name not in done:
+                            quant.gemm_wide_two_dev(*one_packed(a), *one_packed(b), self._two_scratch.ptr, quant.gemm_wide_two_scratch_bytes(), count, stream)
+                            done |= {a.name, b.name}
+                done |= self._pairs([g for g in alone if g.key not in jobs16 and g.name not in done and
+                                     quant.gemm_stream_takes(g.type, g.in_dim, g.dims[0], count)],
+                                    lambda a, b: quant.gemm_stream_two_dev(*one_packed(a), *one_packed(b), count, stream))
+            for g in groups:
+                if g.name in done:
                     continue
-                name, src, t, out_dim, in_dim, raw = grp[0]
-                key = (src, self._family(t))
-                w, out, dims = [self._w[e[0]].ptr for e in grp], [self._act[e[0]].ptr for e in grp], [e[3] for e in grp]
-                if key in jobs16:
+                t, in_dim, w, out, dims, nexts = g.type, g.in_dim, g.w, g.out, g.dims, g.nexts
+                if g.key in jobs16:
                     # up to sixteen tokens: the one-pass decode kernels with sixteen single-term tokens
-                    quant.gemv_packed16_dev(w, t, self._images16[key].ptr, out, dims, in_dim, count, 0, stream)
+                    quant.gemv_packed16_dev(w, t, g.image16, out, dims, in_dim, count, 0, stream)
                     continue
-                ws, nbytes = self._prefill_ws[key]
-                nexts = [self._next_input(e) for e in grp] if len(grp) >= 2 and int(t) in list_types else []
                 while dims:   # (the prefill counterpart of the qmatvec_many seam)
                     takes = quant.gemm_stream_takes(t, in_dim, sum(dims), count)
-                    if any(nexts) and (takes or quant.gemm_tall_takes(t, in_dim, dims, count)):
+                    tall = not takes and quant.gemm_tall_takes(t, in_dim, dims, count)
+                    if nexts and (takes or tall):
                         (quant.gemm_stream_pack_dev if takes else quant.gemm_tall_pack_dev)(
-                            w, t, ws.ptr, nbytes, out, dims, [n and n[1] for n in nexts], in_dim, count, stream)
+                            w, t, g.ws, g.nbytes, out, dims, [n and n[1] for n in nexts], in_dim, count, stream)
                         packed.update(n[0] for n in nexts if n)
                         break
                     if takes:
-                        quant.gemm_stream_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, 0, stream)
+                        quant.gemm_stream_dev(w, t, g.ws, g.nbytes, out, dims, in_dim, count, 0, stream)
                         break
-                    if quant.gemm_tall_takes(t, in_dim, dims, count):
-                        quant.gemm_tall_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, stream)
+                    if tall:
+                        quant.gemm_tall_dev(w, t, g.ws, g.nbytes, out, dims, in_dim, count, stream)
                         break
-                    if len(dims) >= 2 and int(t) in list_types:
-                        quant.gemm_packed_many_dev(w, t, ws.ptr, nbytes, out, dims, in_dim, count, stream)
+                    if len(dims) >= 2 and g.lists:
+                        quant.gemm_packed_many_dev(w, t, g.ws, g.nbytes, out, dims, in_dim, count, stream)
                         break
-                    quant.gemm_packed_dev(w[0], t, ws.ptr, nbytes, out[0], in_dim, dims[0], count, 0, stream)
+                    quant.gemm_packed_dev(w[0], t, g.ws, g.nbytes, out[0], in_dim, dims[0], count, 0, stream)
                     w, out, dims, nexts = w[1:], out[1:], dims[1:], nexts[1:]
 
     def _run_token(self, tok):

@@ -78,6 +78,27 @@ def test_runner_of_packed_outputs(gpu, tokens, w_type, down, monkeypatch):
         assert np.array_equal(results[0][k], results[1][k]), k
 
 
+def test_a_first_pass_asks_no_more_than_it_needs(gpu, monkeypatch):
+    """What a prefill of any length has to know of the projections is found when the runner is made, and a short prefill asks for none of the tiles of many tokens."""
+    rng = np.random.default_rng(3)
+    weights = Weights.synthetic(rng, [("q", "x", Q4_K, 2048, 2048), ("k", "x", Q4_K, 512, 2048), ("gate", "x", Q4_K, 11008, 2048), ("up", "x", Q4_K, 11008, 2048),
+                                      ("o", "q", Q4_K, 2048, 2048), ("down", "up", Q6_K, 2048, 11008)])
+    r = QwenProjectionStackRunner.from_weights(weights, 512, synth.make_activations(rng, 512, 2048).reshape(-1))
+    assert r._two_scratch is not None
+    asked = []
+    for owner, name in ((quant, "gemm_tall_takes"), (quant, "gemm_wide_two_takes"), (quant, "gemv_image_bytes"), (QwenProjectionStackRunner, "_next_input")):
+        f = getattr(owner, name)
+        monkeypatch.setattr(owner, name, lambda *a, f=f, name=name: (asked.append(name), f(*a))[1])
+    r.upload_weights()
+    r.reset_sequence()
+    for count, want in ((48, []), (512, ["gemm_tall_takes", "gemm_wide_two_takes"])):
+        r.active_tokens = count
+        r.run_sequence()
+        assert asked == want, count
+    r.read_outputs()
+    r.close()
+
+
 def test_refusals(gpu):
     bad = [([256, 256], [(Q6_K, 64, 1 << 30), None], Q6_K, "Unsupported quant type"), ([300], [(Q6_K, 64, 1 << 30)], Q4_K, "multiple of 256"),
            ([256], [(Q6_K, 64, 16)], Q4_K, "next_workspace too small"), ([256], [(8, 64, 1 << 30)], Q4_K, "Unsupported quant type")]
