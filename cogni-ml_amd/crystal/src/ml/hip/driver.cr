@@ -30,6 +30,7 @@ lib LibCogniHIP
   fun mlhip_graph_instantiate(exec : Void**, graph : Void*, flags : UInt64) : Int32
   fun mlhip_graph_upload(exec : Void*, stream : Void*) : Int32
   fun mlhip_graph_launch(exec : Void*, stream : Void*) : Int32
+  fun mlhip_graph_exec_kernels(exec : Void*) : Int32
   fun mlhip_graph_destroy(graph : Void*) : Int32
   fun mlhip_graph_exec_destroy(exec : Void*) : Int32
   fun mlhip_mem_alloc(dptr : Deviceptr*, bytesize : LibC::SizeT) : Int32

@@ -15,9 +15,11 @@
 // ---- graphs of a few kernels in a row ----------------------------------------------------------------------------------
 // hipGraphLaunch takes 16 us of host time whatever is in the graph, and leaves the device idle for 5 us between one graph and the
 // next; a plain launch takes 2.8 and leaves less than 1 (graphs of empty kernels, one to four of them, back to back: 16.2 to 18.4 us; one
-// kernel of 22.6 us 27.7, two 50.3). A decode step of the runners is two to four kernels one after the other, so a graph that is a chain
-// of up to CHAIN_MOST of this library's kernels and nothing else is launched as those kernels. Anything else - other nodes, branches, other modules'
-// kernels, instantiation flags - goes through hipGraphLaunch.
+// kernel of 22.6 us 27.7, two 50.3). A decode step of one runner is two to four kernels one after the other, so a graph that is a chain
+// of up to CHAIN_MOST of this library's kernels and nothing else is launched as those kernels. Anything else - longer chains (a step of many layers captured as
+// one graph, whose one idle gap is a small part of it), other nodes, branches, other modules' kernels, instantiation flags - goes through hipGraphLaunch.
+// Two launches of one executable on two streams are not ordered by hipGraphLaunch either (graphs of two kernels of 8.7 ms on one workgroup, one executable on two
+// streams 18.0 ms, on one stream twice 34.7).
 namespace {
 constexpr size_t CHAIN_MOST = 5;   // 14 us of launches
 struct Chain {
@@ -29,6 +31,33 @@ struct Chain {
 };
 std::mutex g_chain_mu;
 std::unordered_map<void*, std::shared_ptr<const Chain>> g_chains;   // by executable graph, until that is destroyed
+std::unordered_map<void*, std::shared_ptr<std::mutex>> g_launching;   // by stream, while a graph is being launched on it
+
+// Held while a graph is launched: a chain's kernels follow each other whole among the graphs that several threads launch on one stream, as single enqueues
+// would. A mutex for each stream, so that a launch that waits for room in its queue holds up no other stream's.
+class StreamLock {
+ public:
+  explicit StreamLock(void* stream) : stream_(stream) {
+    {
+      std::lock_guard<std::mutex> lk(g_chain_mu);
+      std::shared_ptr<std::mutex>& m = g_launching[stream];
+      if (!m) m = std::make_shared<std::mutex>();
+      mutex_ = m;
+    }
+    mutex_->lock();
+  }
+  ~StreamLock() {
+    mutex_->unlock();
+    std::lock_guard<std::mutex> lk(g_chain_mu);
+    if (mutex_.use_count() == 2) g_launching.erase(stream_);   // the table's and this one: nobody else waits
+  }
+  StreamLock(const StreamLock&) = delete;
+  StreamLock& operator=(const StreamLock&) = delete;
+
+ private:
+  void* stream_;
+  std::shared_ptr<std::mutex> mutex_;
+};
 
 // The chain a graph is, or null.
 std::shared_ptr<const Chain> chain_of(hipGraph_t graph) {
@@ -179,7 +208,14 @@ int mlhip_graph_upload(mlhip_graph_exec exec, mlhip_stream stream) {
   return (int)hipGraphUpload((hipGraphExec_t)exec, (hipStream_t)stream);
 }
 
+int32_t mlhip_graph_exec_kernels(mlhip_graph_exec exec) {
+  std::lock_guard<std::mutex> lk(g_chain_mu);
+  const auto it = g_chains.find(exec);
+  return it == g_chains.end() ? 0 : (int32_t)it->second->kernels.size();
+}
+
 int mlhip_graph_launch(mlhip_graph_exec exec, mlhip_stream stream) {
+  const StreamLock whole(stream);
   std::shared_ptr<const Chain> c;
   {
     std::lock_guard<std::mutex> lk(g_chain_mu);
