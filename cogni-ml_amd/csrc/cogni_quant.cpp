@@ -312,6 +312,7 @@ int cogni_quant_init(int32_t ordinal) {
 int cogni_quant_shutdown(void) {
   std::lock_guard<std::mutex> lk(g_mu);
   if (!g_rt.ready) return 0;
+  cogni_internal_drop_chains();
   (void)hipModuleUnload(g_rt.mod);
   if (g_rt.image_pool) (void)hipFree(g_rt.image_pool);
   g_rt = Runtime();

@@ -12,6 +12,8 @@ int cogni_internal_hip_fail(int hip_error, const char* what);
 int cogni_internal_noalloc_setup(int device);
 // Whether `function` (a hipFunction_t) is one of the library's kernels that it has looked up.
 int cogni_internal_is_kernel(const void* function);
+// Forgets the kernels that graphs are launched as: they go with the library's code object.
+void cogni_internal_drop_chains(void);
 #ifdef __cplusplus
 }
 #endif

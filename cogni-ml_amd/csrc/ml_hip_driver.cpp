@@ -103,6 +103,12 @@ std::shared_ptr<const Chain> chain_of(hipGraph_t graph) {
 
 extern "C" {
 
+void cogni_internal_drop_chains(void) {
+  std::unordered_map<void*, std::shared_ptr<const Chain>> gone;   // (destroyed outside the lock)
+  std::lock_guard<std::mutex> lk(g_chain_mu);
+  gone.swap(g_chains);
+}
+
 int mlhip_init(uint32_t flags) { return (int)hipInit(flags); }
 
 int mlhip_device_get(int32_t* device, int32_t ordinal) {

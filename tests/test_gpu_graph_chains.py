@@ -107,7 +107,7 @@ def wait(stream, after):
 
 
 def test_what_is_no_chain_goes_as_a_graph(gpu):
-    """Branches, nodes that do not depend on each other, another module's kernel, instantiation flags: not
+    """Branches, nodes that do not depend on each other, another module's kernel, instantiation flags, and chains that the library has been told to forget: not
     launched as kernels, and the values of the same work in order."""
     a, b = Layer(1), Layer(2)
     s, t = hip.HIPStream(), hip.HIPStream()
@@ -161,6 +161,14 @@ def test_what_is_no_chain_goes_as_a_graph(gpu):
                 assert np.array_equal(a.read(), want_a), body.__name__
                 assert want_b is None or np.array_equal(b.read(), want_b), body.__name__
             ex.close()
+        ex = captured(s, chain)
+        assert hip.lib().mlhip_graph_exec_kernels(ex._handle) == 3
+        hip.lib().cogni_internal_drop_chains()
+        assert hip.lib().mlhip_graph_exec_kernels(ex._handle) == 0
+        ex.launch(s)
+        s.synchronize()
+        assert np.array_equal(a.read(), once)
+        ex.close()
     finally:
         for o in [a, b, module, s, t] + events:
             o.close()
