@@ -1263,7 +1263,8 @@ static uint32_t gemm_splits_of(uint32_t tiles, uint32_t in_dim) {
 // costs per super-block against one of 192 rows is gemm_tile_cost (gemv_config.h), and the cheapest plan wins
 // (the 4096-row projections at 512 tokens: 88 tiles x 2 splits = 176 workgroups of 192 rows, or 128 x 2 = 256 of the
 // smaller ones). `split` false: the plan for a workspace without planes. COGNI_GEMM_N128=0 | 1 and COGNI_GEMM_WIDE=0 | 1
-// override the choice (measurement knobs: 1 takes that tile wherever its kernel can run; COGNI_GEMM_WIDE also of lists and gate | up).
+// override the choice (measurement knobs: 1 takes that tile wherever its kernel can run; COGNI_GEMM_WIDE also of lists of Q4_K and Q5_K and of gate | up, and
+// where it is set nothing goes to the 256-token tiles, at 0 no two matrices to their launch of 256-row tiles).
 struct GemmShape {
   uint32_t bn, splits;
 };
@@ -1450,7 +1451,7 @@ int cogni_gemm_packed_swiglu_dev(uint64_t w_gate, uint64_t w_up, uint32_t w_type
 }
 
 // Several matrices of one type and row length against one block of packed activations, as one launch: no k split (the list
-// is what fills the chip), the tile whose rounds of 256 workgroups cost least (gemm_tile_cost; the 256-row tile: Q4_K), the 64-token
+// is what fills the chip), the tile whose rounds of 256 workgroups cost least (gemm_list_rows), the 64-token
 // kernels for up to 64 tokens.
 namespace {
 struct GemmManyArgs {   // the kernels' first parameter (kernels/gemm_q4k.hpp)
@@ -1533,11 +1534,11 @@ int cogni_gemm_packed_swiglu_pack_dev(uint64_t w_gate, uint64_t w_up, uint32_t w
 // Launches of many tokens, tiles of 256 tokens x 256 rows (kernels/gemm_q4k_tall.hpp): the same packed activations and precision, each sum
 // added in one order of k (the kernels above add two halves), so not their bits.
 int32_t cogni_gemm_tall_takes(uint32_t w_type, uint32_t in_dim, const uint32_t* out_dims, uint32_t count, uint32_t tokens) {
-  if (!out_dims || count == 0 || count > 6) return 0;
+  if (!out_dims || count == 0 || count > 6 || gemm_wide_knob() >= 0) return 0;
   return gemm_tall_takes(w_type, in_dim, out_dims, count, tokens);
 }
 int32_t cogni_gemm_tall_swiglu_takes(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens) {
-  return gemm_tall_swiglu_takes(w_type, in_dim, out_dim, tokens);
+  return gemm_wide_knob() < 0 && gemm_tall_swiglu_takes(w_type, in_dim, out_dim, tokens);
 }
 // The packed inputs a list is to write: next_workspaces[i] (0: none) for a GEMM of type next_types[i] whose rows are out[i]'s values.
 static int gemm_next_of(const char* who, GemmNextArgs* next, const uint32_t* next_types, const uint64_t* next_workspaces, const size_t* next_bytes,
@@ -1733,6 +1734,7 @@ static bool wide_two_swaps(uint32_t type_a, uint32_t type_b) { return type_a != 
 int32_t cogni_gemm_wide_two_takes(uint32_t type_a, uint32_t in_dim_a, uint32_t out_dim_a, uint32_t type_b, uint32_t in_dim_b, uint32_t out_dim_b,
                                   uint32_t tokens) {
   unsigned sa, sb;
+  if (gemm_wide_knob() == 0) return 0;
   if (wide_two_swaps(type_a, type_b)) return gemm_wide_two_plan(type_b, in_dim_b, out_dim_b, type_a, in_dim_a, out_dim_a, tokens, &sa, &sb);
   return gemm_wide_two_plan(type_a, in_dim_a, out_dim_a, type_b, in_dim_b, out_dim_b, tokens, &sa, &sb);
 }
@@ -1809,7 +1811,7 @@ int32_t cogni_get_gemm_threshold(void) {
 // of single matrices (pack included, us, cogni_gemm_dev | these: 4096 -> 12288 at 700 | 1024 tokens 92.8 | 130.7 and 85.4 | 108.3, 4608 -> 8213 at 932 130.6 and 107.7,
 // 512 -> 11102 at 998 58.1 and 38.3, 8448 -> 11372 at 721 174.4 and 171.7; not taken: 1280 -> 10773 at 643, costs level, 50.2 and 50.5, 4096 -> 8192 at 1024 77.3 and 89.8).
 static bool matmul_takes_tall(uint32_t w_type, uint32_t in_dim, uint32_t out_dim, uint32_t tokens) {
-  if (!gemm_tall_takes(w_type, in_dim, &out_dim, 1, tokens)) return false;
+  if (gemm_wide_knob() >= 0 || !gemm_tall_takes(w_type, in_dim, &out_dim, 1, tokens)) return false;
   const unsigned long long mt = (tokens + 127ull) / 128ull;
   const unsigned rows = gemm_list_rows(w_type, in_dim, &out_dim, 1, tokens, -1);
   return 20 * gemm_fill_cost((mt + 1) / 2 * gemm_list_tiles(&out_dim, 1, 256), GEMM_TALL_COST) <

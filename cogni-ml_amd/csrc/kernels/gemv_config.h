@@ -321,8 +321,9 @@ static inline unsigned gemm_list_rows(unsigned type, unsigned in_dim, const unsi
   const unsigned of[3] = {192u, 128u, 256u};
   unsigned long long least = ~0ull;
   unsigned best = 192u, k, i;
-  if (type == 12u && knob == 1) return 256u;
-  for (k = 0; k < (tokens > 64u && knob != 0 && (type == 12u || in_dim / 256u <= GEMM_Q6W_MAX_KB) ? 3u : 2u); k++) {
+  const int can = type == 12u || in_dim / 256u <= GEMM_Q6W_MAX_KB;
+  if (knob == 1 && can) return 256u;
+  for (k = 0; k < (tokens > 64u && knob != 0 && can ? 3u : 2u); k++) {
     unsigned long long tiles = 0, cost;
     for (i = 0; i < count; i++) tiles += ((unsigned long long)out_dims[i] + of[k] - 1u) / of[k];
     cost = ((tokens + 127u) / 128u * tiles + GEMM_ROUND_TILES - 1) / GEMM_ROUND_TILES * gemm_tile_cost(type, of[k]);

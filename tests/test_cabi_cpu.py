@@ -542,3 +542,32 @@ def test_interleaved_term_kernels_are_taken_where_they_are_faster():
     for (t, m, n, k), us, pick in zip(asked, [v[1:] for c in timed for v in c[3:]], picks):
         assert us[pick] <= 1.02 * min(us), (t, m, n, k, us, pick)
     assert not any(picks[len(asked):])
+
+
+def test_the_knob_of_the_256_row_tiles_reaches_every_rule(monkeypatch):
+    """COGNI_GEMM_WIDE, for measurements: 1 takes the eight-wavefront tiles wherever there is a kernel (lists of Q5_K too), 0 takes none, and where it is set
+    nothing goes to the 256-token tiles."""
+    import subprocess
+    import tempfile
+    dims = [4096, 1024, 1024, 12288, 12288]
+
+    def takes():
+        return [quant.gemm_tall_takes(12, 4096, dims, 512), quant.gemm_tall_swiglu_takes(12, 4096, 12288, 512),
+                quant.gemm_wide_two_takes(12, 4096, 4096, 14, 12288, 4096, 512), quant.gemm_plan(14, 12288, 4096, 2048, 1 << 40)[0].endswith("wide_f16")]
+
+    monkeypatch.delenv("COGNI_GEMM_WIDE", raising=False)
+    assert takes() == [True] * 4
+    monkeypatch.setenv("COGNI_GEMM_WIDE", "0")
+    assert takes() == [False] * 4
+    monkeypatch.setenv("COGNI_GEMM_WIDE", "1")
+    assert takes() == [False, False, True, True]
+    src = '#include <cstdio>\n#include "gemv_config.h"\nint main() { unsigned t, k, r, m; int knob; while (std::scanf("%u %u %u %u %d", &t, &k, &r, &m, &knob) == 5) ' \
+          'std::printf("%u\\n", gemm_list_rows(t, k, &r, 1, m, knob)); }'
+    asked = [(t, 4096, 300, m, 1) for t in (12, 13) for m in (9, 64, 65, 500)] + [(13, 65536 * 256, 300, 500, 1)] + [(t, 4096, 30720, 512, 0) for t in (12, 13)]
+    with tempfile.TemporaryDirectory() as d:
+        open(os.path.join(d, "t.cpp"), "w").write(src)
+        subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "cogni-ml_amd", "csrc", "kernels"), "-o", os.path.join(d, "t"),
+                        os.path.join(d, "t.cpp")], check=True)
+        got = subprocess.run([os.path.join(d, "t")], input="\n".join("%d %d %d %d %d" % a for a in asked), capture_output=True, text=True, check=True)
+    got = [int(v) for v in got.stdout.split()]
+    assert got[:8] == [256] * 8 and all(v in (128, 192) for v in got[8:])

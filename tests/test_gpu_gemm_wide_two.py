@@ -96,6 +96,13 @@ def test_q5_k_lists_of_256_row_tiles(gpu, tokens, in_dim, dims):
         a.close()
 
 
+@pytest.mark.parametrize("tokens,in_dim,dims", [(9, 256, [300, 7]), (64, 512, [256, 1000]), (130, 768, [65, 513])])
+def test_q5_k_lists_where_the_knob_says_so(gpu, tokens, in_dim, dims, monkeypatch):
+    """COGNI_GEMM_WIDE=1: these tiles at every token count, the same bits."""
+    monkeypatch.setenv("COGNI_GEMM_WIDE", "1")
+    test_q5_k_lists_of_256_row_tiles(gpu, tokens, in_dim, dims)
+
+
 def test_what_is_not_taken(gpu):
     takes = quant.gemm_wide_two_takes
     o, down = (Q4_K, 4096, 4096), (Q6_K, 12288, 4096)
