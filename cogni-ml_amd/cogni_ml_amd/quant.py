@@ -671,7 +671,8 @@ def matvec_many(qws, x):
 
 
 # The calls a program issues one by one, read natively where their arguments are ordinary (csrc/py_calls.cpp; a pass of Q8_0 1024 -> 3584, one
-# token, through matmul_dev: 4.2 us in Python, 3.65 so). The functions above take what is not, and every call where the module is not built (no Python headers).
+# token, through matmul_dev: 4.2 us in Python, 3.65 so). The functions above take what is not, and every call where the module is not built (no Python headers). The native
+# calls have the library's addresses and do not ask hip.lib(), but while a sequence is noted (hip.issue).
 _matmul_dev, _gemv_dev, _dequantize_dev = matmul_dev, gemv_dev, dequantize_dev
 if hip.calls is not None:
     hip.calls.set_python(_matmul_dev, _gemv_dev, _dequantize_dev, _check, TensorType, ctypes.c_void_p)
