@@ -168,7 +168,8 @@ def issue(kept, key, launch, check_status):
     finally:
         _noting.on = False
         _count_noting(-1)
-    kept[key] = proxy.notes()
+    with _recording_lock:
+        kept[key] = proxy.notes()
 
 
 def _count_noting(by):
